@@ -264,7 +264,7 @@ struct GroupBuf {
   };
   struct HsumLaunch {
     uint32_t H, first, n_jobs, n_blocks;
-    bool vec;
+    bool whole_groups;  // every row length is a multiple of 8
   };
   std::vector<FtcLaunch> ftc;
   std::vector<HsumLaunch> hsum;
@@ -527,7 +527,7 @@ fdas_status build_group(fdas_engine* e, GroupBuf& g, const std::vector<Trial*>& 
       j.counts = reinterpret_cast<uint32_t*>(sm + l.counts);
       for (uint32_t k = 0; k < H; ++k) j.thr[k] = t->req.thresholds[k];
       L.n_blocks += (j.n_bins + kHsumBinsPerBlock - 1) / kHsumBinsPerBlock * j.n_row_chunks;
-      L.vec = L.vec && hsum_vec_ok(j.n_bins);
+      L.whole_groups = L.whole_groups && hsum_whole_groups(j.n_bins);
       for (uint32_t p = 0; p < H; ++p) {
         SelectJob& q = g.h_sel[js++];
         q.spill_key = j.spill_key + size_t(p) * spill;
@@ -616,7 +616,7 @@ fdas_status enqueue_group(fdas_engine* e, GroupBuf& g, const std::vector<Trial*>
       EHIP(e, launch_zero_u32(reinterpret_cast<uint32_t*>(t->small), uint32_t(t->lay.small_bytes / 4), B));
   }
   if (timing_events) EHIP(e, hipEventRecord(g.ev_hsum0, B));
-  for (const auto& L : g.hsum) EHIP(e, launch_hsum(g.d_hsum + L.first, L.n_jobs, L.n_blocks, L.H, L.vec, B));
+  for (const auto& L : g.hsum) EHIP(e, launch_hsum(g.d_hsum + L.first, L.n_jobs, L.n_blocks, L.H, B));
   if (timing_events) EHIP(e, hipEventRecord(g.ev_hsum1, B));
   EHIP(e, hipEventRecord(g.ev_hsum_done, B));
   EHIP(e, launch_select(g.d_sel, g.n_sel, B));
@@ -904,7 +904,7 @@ fdas_status time_shape(fdas_engine* e, uint32_t n_bins, uint32_t bank_id, uint32
           e,
           [&]() -> fdas_status {
             EHIP(e, launch_zero_u32(reinterpret_cast<uint32_t*>(t.small), uint32_t(lay.small_bytes / 4), e->s_ftc));
-            EHIP(e, launch_hsum(g.d_hsum, G, G * L1.n_blocks, L1.H, L1.vec, e->s_ftc));
+            EHIP(e, launch_hsum(g.d_hsum, G, G * L1.n_blocks, L1.H, e->s_ftc));
             return FDAS_OK;
           },
           3, &ms);
@@ -1618,7 +1618,7 @@ static fdas_status plan_enqueue_lagged(fdas_plan* p, bool capturing) {
     }
     const bool fuse = p->schedule == FDAS_SCHEDULE_FUSED && cur && prev && cur->ftc.size() == 1 &&
                       prev->hsum.size() == 1 && cur->ftc[0].tile == 1024 &&
-                      fused_supported(1024, prev->hsum[0].H, prev->hsum[0].vec);
+                      fused_supported(1024, prev->hsum[0].H, prev->hsum[0].whole_groups);
     if (cur) cur->launch_fused = fuse;
     if (prev) prev->hsum_fused = fuse;
     // Timing events bracket each kernel: the convolution (or the fused kernel)
@@ -1629,7 +1629,7 @@ static fdas_status plan_enqueue_lagged(fdas_plan* p, bool capturing) {
       const auto& S = prev->hsum[0];
       const auto& tw = e->twiddles.at(1024);
       EHIP(e, launch_fused(cur->d_ftc + F.first, F.n_jobs, F.n_items, tw.first, tw.second, prev->d_hsum + S.first,
-                           S.n_jobs, S.n_blocks, S.H, S.vec, A));
+                           S.n_jobs, S.n_blocks, S.H, A));
       if (!capturing) EHIP(e, hipEventRecord(cur->ev_ftc_t1, A));
     } else {
       if (cur) {
@@ -1643,7 +1643,7 @@ static fdas_status plan_enqueue_lagged(fdas_plan* p, bool capturing) {
       if (prev) {
         if (!capturing) EHIP(e, hipEventRecord(prev->ev_hsum0, A));
         for (const auto& L : prev->hsum)
-          EHIP(e, launch_hsum(prev->d_hsum + L.first, L.n_jobs, L.n_blocks, L.H, L.vec, A));
+          EHIP(e, launch_hsum(prev->d_hsum + L.first, L.n_jobs, L.n_blocks, L.H, A));
         if (!capturing) EHIP(e, hipEventRecord(prev->ev_hsum1, A));
       }
     }

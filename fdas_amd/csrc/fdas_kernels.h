@@ -13,8 +13,8 @@ namespace fdas {
 constexpr int kHsumThreads = 256;
 constexpr int kHsumBinsPerThread = 8;
 constexpr int kHsumBinsPerBlock = kHsumThreads * kHsumBinsPerThread;  // bins one HSUM workgroup covers
-// The 16-byte-load form of the summing kernel needs whole 8-bin groups.
-inline bool hsum_vec_ok(uint32_t n_bins) { return n_bins % kHsumBinsPerThread == 0; }
+// Rows of whole 8-bin groups (part of the rule for the fused kernel).
+inline bool hsum_whole_groups(uint32_t n_bins) { return n_bins % kHsumBinsPerThread == 0; }
 constexpr uint32_t kHsumRowsPerBlock = 11;  // target rows per HSUM workgroup (bounds the dense-hit tail)
 constexpr int kHsumWaveStage = 64;        // LDS staging entries per plane per wave before a global flush
 constexpr int kSelectThreads = 1024;
@@ -33,8 +33,8 @@ hipError_t launch_tiles(int tile, const float2* spectrum, uint32_t n_bins, uint3
                         uint32_t n_tiles, const float2* tw1, const float2* tw2, float2* out, hipStream_t stream);
 
 // Harmonic summing + thresholding + compaction into per-plane spill lists.
-// All jobs of one launch share n_harmonics; vec requires every job's n_bins % 4 == 0.
-hipError_t launch_hsum(const HsumJob* d_jobs, uint32_t n_jobs, uint32_t n_blocks, uint32_t n_harmonics, bool vec,
+// All jobs of one launch share n_harmonics; any row lengths go together.
+hipError_t launch_hsum(const HsumJob* d_jobs, uint32_t n_jobs, uint32_t n_blocks, uint32_t n_harmonics,
                        hipStream_t stream);
 
 // Per-plane cap (strongest first) and sort by (row, bin): power histogram and
@@ -55,12 +55,13 @@ hipError_t launch_hmax(const float* fop, uint32_t n_bins, uint32_t n_templates, 
 hipError_t launch_zero_u32(uint32_t* p, uint32_t n, hipStream_t stream);
 
 // One launch running both the FT convolution of ftc_jobs (1024-point tiles)
-// and the harmonic summing of hsum_jobs (n_harmonics planes; vec as in
-// launch_hsum) over a FOP written by an earlier launch; workgroups of the two
-// kinds are interleaved.  fused_supported tells which shapes it covers.
-bool fused_supported(uint32_t tile, uint32_t n_harmonics, bool vec);
+// and the harmonic summing of hsum_jobs (n_harmonics planes) over a FOP written
+// by an earlier launch; workgroups of the two kinds are interleaved.
+// fused_supported tells which shapes it covers (whole_groups: every row length
+// is a multiple of 8).
+bool fused_supported(uint32_t tile, uint32_t n_harmonics, bool whole_groups);
 hipError_t launch_fused(const FtcJob* ftc_jobs, uint32_t n_ftc_jobs, uint32_t n_items, const float2* tw1,
                         const float2* tw2, const HsumJob* hsum_jobs, uint32_t n_hsum_jobs, uint32_t n_blocks,
-                        uint32_t n_harmonics, bool vec, hipStream_t stream);
+                        uint32_t n_harmonics, hipStream_t stream);
 
 }  // namespace fdas

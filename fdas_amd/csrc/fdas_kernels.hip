@@ -390,61 +390,48 @@ struct RowLoads {
   float s[H][kHsumMaxSpan];
 };
 
-// Branch-free: H is a compile-time constant and the indexes are clamped, so
+// Branch-free: H is a compile-time constant and every index is in range, so
 // the compiler can count the loads in flight exactly (a load issued under a
 // condition makes it drain every outstanding load at the next use).
-//  VEC (n_bins % 8 == 0): f0 is clamped to the last 8 bins, so every index is
-//    in range; the own bins are two 16-byte loads, and so are the k = 2 bins
-//    (f0 / 2 is a multiple of 4); the k = 4 pair is one 8-byte load.
-//  otherwise: one load per value, each index clamped to the last bin, and the
-//    own bins past the end read as -inf, so no sum of theirs passes a threshold.
-template <bool VEC>
-__device__ __forceinline__ void hsum_load_own(float (&m)[kHsumBinsPerThread], const float* __restrict__ fop,
-                                              uint32_t n_bins, uint32_t r, uint32_t f0) {
+//
+// n_bins >= 8 may be any length: the loads need dword alignment only.  Bound by
+// HBM traffic as long as they stay wide: 16-byte loads of the own bins and of
+// the k = 2, 3 spans, narrower ones that the compiler merges for the rest, 9 per
+// row at H = 8.  With one dword load per value and a clamp on each (135 VGPRs,
+// 3 waves per SIMD) rows of odd length took 124 us per 700,001 bins x 43 rows,
+// against 57 us this way, and since a launch ran in one form for all its jobs,
+// one odd-length trial among five took the launch from 0.98 to 3.29 ms.
+//
+// A thread whose group of 8 crosses the end of its row reads on into the next
+// row (live_bits masks what it finds there); the plane's last row has no next
+// one, so hsum_block sums that row of the last wave bin by bin.
+//
+// For n_bins >= 8 a sub-harmonic span ends at (n_bins - 1) / 2 + 3 <= n_bins - 1
+// at most.
+template <int H>
+__device__ __forceinline__ void hsum_load_row(RowLoads<H>& L, const float* __restrict__ fop, uint32_t n_bins, int c,
+                                              uint32_t r, uint32_t f0) {
   const float* __restrict__ row = fop + size_t(r) * n_bins;
-  const uint32_t last = n_bins - 1;
-  if constexpr (VEC) {
-    const fdas_vf4 q0 = gld4(row, f0);
-    const fdas_vf4 q1 = gld4(row, f0 + 4);
-    m[0] = q0.x; m[1] = q0.y; m[2] = q0.z; m[3] = q0.w;
-    m[4] = q1.x; m[5] = q1.y; m[6] = q1.z; m[7] = q1.w;
-  } else {
-#pragma unroll
-    for (int b = 0; b < kHsumBinsPerThread; ++b) {
-      const float v = gld(row, min(f0 + uint32_t(b), last));
-      m[b] = (f0 + uint32_t(b) < n_bins) ? v : -INFINITY;
-    }
-  }
-}
-
-// The sub-harmonic spans of row r (harmonics 2..H) for the 8 bins from f0.
-template <int H, bool VEC>
-__device__ __forceinline__ void hsum_load_subs(RowLoads<H>& L, const float* __restrict__ fop, uint32_t n_bins, int c,
-                                               uint32_t r, uint32_t f0) {
-  const uint32_t last = n_bins - 1;
+  const fdas_vf4u q0 = gld4u(row, f0);
+  const fdas_vf4u q1 = gld4u(row, f0 + 4);
+  L.m[0] = q0.x; L.m[1] = q0.y; L.m[2] = q0.z; L.m[3] = q0.w;
+  L.m[4] = q1.x; L.m[5] = q1.y; L.m[6] = q1.z; L.m[7] = q1.w;
   const int t = int(r) - c;
 #pragma unroll
   for (int k = 2; k <= H; ++k) {
     const float* __restrict__ srow = fop + size_t(c + t / k) * n_bins;
     const uint32_t s0 = f0 / uint32_t(k);
-    if (VEC && k == 2) {
-      const fdas_vf4 q = gld4(srow, s0);
+    if (k == 2) {
+      const fdas_vf4u q = gld4u(srow, s0);
       L.s[k - 1][0] = q.x; L.s[k - 1][1] = q.y; L.s[k - 1][2] = q.z; L.s[k - 1][3] = q.w;
-    } else if (VEC && k == 4) {
-      const float2 q = gld2(reinterpret_cast<const float2*>(srow), s0 / 2);
+    } else if (k == 4) {
+      const fdas_vf2u q = gld2u(srow, s0);
       L.s[k - 1][0] = q.x; L.s[k - 1][1] = q.y;
     } else {
 #pragma unroll
-      for (int j = 0; j < hsum_span(k); ++j) L.s[k - 1][j] = gld(srow, VEC ? s0 + uint32_t(j) : min(s0 + uint32_t(j), last));
+      for (int j = 0; j < hsum_span(k); ++j) L.s[k - 1][j] = gld(srow, s0 + uint32_t(j));
     }
   }
-}
-
-template <int H, bool VEC>
-__device__ __forceinline__ void hsum_load_row(RowLoads<H>& L, const float* __restrict__ fop, uint32_t n_bins, int c,
-                                              uint32_t r, uint32_t f0) {
-  hsum_load_own<VEC>(L.m, fop, n_bins, r, f0);
-  hsum_load_subs<H, VEC>(L, fop, n_bins, c, r, f0);
 }
 
 // Bin b of the thread takes sub-harmonic value (f0 mod k + b) / k of its span:
@@ -546,12 +533,32 @@ __device__ __forceinline__ void hsum_row(Stage& st, const HsumJob& job, const Ro
   }
 }
 
+// One bin of one row, every hit placed by its own atomic: the bins that the
+// 16-byte loads cannot cover (below).
+template <int H>
+__device__ __forceinline__ void hsum_one_bin(const HsumJob& job, uint32_t r, uint32_t f) {
+  const int c = int(job.n_templates / 2), t = int(r) - c;
+  float v[H];
+#pragma unroll
+  for (int k = 1; k <= H; ++k) v[k - 1] = gld(job.fop, size_t(c + t / k) * job.n_bins + f / uint32_t(k));
+  float hp = v[0];
+#pragma unroll
+  for (int k = 1; k <= H; ++k) {
+    if (k > 1) hp += v[k - 1];
+    if (!(hp > job.thr[k - 1])) continue;
+    const uint32_t g = gatomic_add(job.counts + (k - 1), 1u);
+    if (g >= job.spill_cap) continue;
+    gst(job.spill_key, size_t(k - 1) * job.spill_cap + g, (r << kKeyBinBits) | f);
+    gst(job.spill_pwr, size_t(k - 1) * job.spill_cap + g, hp);
+  }
+}
+
 // HP_1 = FOP, HP_k = HP_{k-1} + FOP[trunc(t/k)][f/k] in FP32, in k order (hsum.py:93-120);
 // strict HP_k > thr_k (detect.cl.mako:81-83).  One workgroup covers 2048 bins
 // of a chunk of rows of its part, each thread 8 consecutive bins.  Rows are
 // processed in pairs with two register buffers: the loads of row r+1 are in
 // flight while row r is summed and thresholded.
-template <int H, bool VEC>
+template <int H>
 __device__ __forceinline__ void hsum_block(HsumStage<H>& st, const HsumJob* __restrict__ jobs, uint32_t n_jobs,
                                            uint32_t blk) {
   const HsumJob& job = jobs[find_job_hsum(jobs, n_jobs, blk)];
@@ -563,11 +570,26 @@ __device__ __forceinline__ void hsum_block(HsumStage<H>& st, const HsumJob* __re
   const float* __restrict__ fop = job.fop;
   const uint32_t local = blk - job.block_begin;
   const uint32_t chunk = local % job.n_row_chunks;  // row chunks of one bin block run side by side
-  const uint32_t f0 = (local / job.n_row_chunks) * uint32_t(kHsumBinsPerBlock) + uint32_t(tid * kHsumBinsPerThread);
-  // VEC: threads past the end read (and discard) the last 8 bins; both values are multiples of 8
-  const uint32_t fl = VEC ? min(f0, (n_bins - 8u) & ~7u) : f0;
+  const uint32_t block_f0 = (local / job.n_row_chunks) * uint32_t(kHsumBinsPerBlock);
+  const uint32_t f0 = block_f0 + uint32_t(tid * kHsumBinsPerThread);
   const uint32_t r_begin = job.row_begin + chunk * job.rows_per_block;
   const uint32_t r_last = min(r_begin + job.rows_per_block, job.row_begin + job.n_rows) - 1;
+  if (n_bins < uint32_t(kHsumBinsPerThread)) {  // rows shorter than one thread's bins
+    if (uint32_t(tid) < n_bins)
+      for (uint32_t r = r_begin; r <= r_last; ++r) hsum_one_bin<H>(job, r, uint32_t(tid));
+    return;
+  }
+  // The wave that ends in a partial group leaves the plane's last row to the
+  // whole workgroup, bin by bin (2 bins per thread).
+  constexpr uint32_t kWaveBins = 64u * kHsumBinsPerThread;
+  const uint32_t tail_f0 = (n_bins - 1u) / kWaveBins * kWaveBins;
+  const bool apart = n_bins % 8u != 0 && r_last + 1u == job.n_templates && tail_f0 - block_f0 < uint32_t(kHsumBinsPerBlock);
+  if (apart) {
+    for (uint32_t f = tail_f0 + uint32_t(tid); f < min(tail_f0 + kWaveBins, n_bins); f += kHsumThreads)
+      hsum_one_bin<H>(job, r_last, f);
+  }
+  // Threads past the end read (and discard) the row's last group of 8.
+  const uint32_t fl = min(f0, (n_bins - 1u) & ~7u);
   float thr[H];
   int thr_key[H];
   uint32_t wn[H], rk[H];
@@ -581,16 +603,19 @@ __device__ __forceinline__ void hsum_block(HsumStage<H>& st, const HsumJob* __re
 
   const bool live = f0 < n_bins;
   const uint64_t live_lanes = __ballot(live);
-  const uint32_t live_bits = live ? 0xffu : 0u;  // bins past the end read as -inf (or lie in the clamped copy)
-  RowLoads<H> a, b;
-  hsum_load_row<H, VEC>(a, fop, n_bins, c, r_begin, fl);
-  for (uint32_t r = r_begin;; r += 2) {
-    hsum_load_row<H, VEC>(b, fop, n_bins, c, min(r + 1, r_last), fl);
-    hsum_row<H>(st, job, a, r, fl, rk, thr, thr_key, live_lanes, live_bits, wn, wave);
-    if (r + 1 > r_last) break;
-    hsum_load_row<H, VEC>(a, fop, n_bins, c, min(r + 2, r_last), fl);
-    hsum_row<H>(st, job, b, r + 1, fl, rk, thr, thr_key, live_lanes, live_bits, wn, wave);
-    if (r + 2 > r_last) break;
+  const uint32_t live_bits = live ? (1u << min(n_bins - fl, 8u)) - 1u : 0u;
+  const uint32_t r_stop = apart && __ballot(fl + 8u > n_bins) != 0 ? r_last - 1u : r_last;
+  if (int(r_begin) <= int(r_stop)) {
+    RowLoads<H> a, b;
+    hsum_load_row<H>(a, fop, n_bins, c, r_begin, fl);
+    for (uint32_t r = r_begin;; r += 2) {
+      hsum_load_row<H>(b, fop, n_bins, c, min(r + 1, r_stop), fl);
+      hsum_row<H>(st, job, a, r, fl, rk, thr, thr_key, live_lanes, live_bits, wn, wave);
+      if (r + 1 > r_stop) break;
+      hsum_load_row<H>(a, fop, n_bins, c, min(r + 2, r_stop), fl);
+      hsum_row<H>(st, job, b, r + 1, fl, rk, thr, thr_key, live_lanes, live_bits, wn, wave);
+      if (r + 2 > r_stop) break;
+    }
   }
   // Flush what is left: one global atomic per plane for the whole workgroup.
   if (lane_id() == 0) {
@@ -619,40 +644,37 @@ __device__ __forceinline__ void hsum_block(HsumStage<H>& st, const HsumJob* __re
   }
 }
 
-template <int H, bool VEC>
+template <int H>
 __global__ __launch_bounds__(kHsumThreads) void hsum_kernel(const HsumJob* __restrict__ jobs, uint32_t n_jobs) {
   __shared__ HsumStage<H> st;
-  hsum_block<H, VEC>(st, jobs, n_jobs, blockIdx.x);
+  hsum_block<H>(st, jobs, n_jobs, blockIdx.x);
 }
 
 template <int H>
-static void launch_hsum_h(const HsumJob* d_jobs, uint32_t n_jobs, uint32_t n_blocks, bool vec, hipStream_t stream) {
-  if (vec)
-    hipLaunchKernelGGL((hsum_kernel<H, true>), dim3(n_blocks), dim3(kHsumThreads), 0, stream, d_jobs, n_jobs);
-  else
-    hipLaunchKernelGGL((hsum_kernel<H, false>), dim3(n_blocks), dim3(kHsumThreads), 0, stream, d_jobs, n_jobs);
+static void launch_hsum_h(const HsumJob* d_jobs, uint32_t n_jobs, uint32_t n_blocks, hipStream_t stream) {
+  hipLaunchKernelGGL(hsum_kernel<H>, dim3(n_blocks), dim3(kHsumThreads), 0, stream, d_jobs, n_jobs);
 }
 
 hipError_t launch_hsum(const HsumJob* d_jobs, uint32_t n_jobs, uint32_t n_blocks, uint32_t n_harmonics,
-                       bool vec, hipStream_t stream) {
+                       hipStream_t stream) {
   if (n_blocks == 0) return hipSuccess;
   switch (n_harmonics) {
-    case 1: launch_hsum_h<1>(d_jobs, n_jobs, n_blocks, vec, stream); break;
-    case 2: launch_hsum_h<2>(d_jobs, n_jobs, n_blocks, vec, stream); break;
-    case 3: launch_hsum_h<3>(d_jobs, n_jobs, n_blocks, vec, stream); break;
-    case 4: launch_hsum_h<4>(d_jobs, n_jobs, n_blocks, vec, stream); break;
-    case 5: launch_hsum_h<5>(d_jobs, n_jobs, n_blocks, vec, stream); break;
-    case 6: launch_hsum_h<6>(d_jobs, n_jobs, n_blocks, vec, stream); break;
-    case 7: launch_hsum_h<7>(d_jobs, n_jobs, n_blocks, vec, stream); break;
-    case 8: launch_hsum_h<8>(d_jobs, n_jobs, n_blocks, vec, stream); break;
-    case 9: launch_hsum_h<9>(d_jobs, n_jobs, n_blocks, vec, stream); break;
-    case 10: launch_hsum_h<10>(d_jobs, n_jobs, n_blocks, vec, stream); break;
-    case 11: launch_hsum_h<11>(d_jobs, n_jobs, n_blocks, vec, stream); break;
-    case 12: launch_hsum_h<12>(d_jobs, n_jobs, n_blocks, vec, stream); break;
-    case 13: launch_hsum_h<13>(d_jobs, n_jobs, n_blocks, vec, stream); break;
-    case 14: launch_hsum_h<14>(d_jobs, n_jobs, n_blocks, vec, stream); break;
-    case 15: launch_hsum_h<15>(d_jobs, n_jobs, n_blocks, vec, stream); break;
-    case 16: launch_hsum_h<16>(d_jobs, n_jobs, n_blocks, vec, stream); break;
+    case 1: launch_hsum_h<1>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 2: launch_hsum_h<2>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 3: launch_hsum_h<3>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 4: launch_hsum_h<4>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 5: launch_hsum_h<5>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 6: launch_hsum_h<6>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 7: launch_hsum_h<7>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 8: launch_hsum_h<8>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 9: launch_hsum_h<9>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 10: launch_hsum_h<10>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 11: launch_hsum_h<11>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 12: launch_hsum_h<12>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 13: launch_hsum_h<13>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 14: launch_hsum_h<14>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 15: launch_hsum_h<15>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 16: launch_hsum_h<16>(d_jobs, n_jobs, n_blocks, stream); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -676,7 +698,7 @@ union FusedLds {
   HsumStage<H> hsum;
 };
 
-template <int H, bool VEC>
+template <int H>
 __global__ __launch_bounds__(64 * kFtc1kWaves) __attribute__((amdgpu_waves_per_eu(3, 3))) void fused1k_kernel(
     const FtcJob* __restrict__ ftc_jobs, uint32_t n_ftc_jobs, uint32_t n_items, const float2* __restrict__ tw1,
     const float2* __restrict__ tw2, const HsumJob* __restrict__ hsum_jobs, uint32_t n_hsum_jobs,
@@ -692,26 +714,27 @@ __global__ __launch_bounds__(64 * kFtc1kWaves) __attribute__((amdgpu_waves_per_e
     fft.load_twiddles(tw1, tw2, lds.ftc.w2s, int(threadIdx.x) & 63, (threadIdx.x >> 6) == 0);
     ftc1k_item(lds.ftc, fft, ftc_jobs, n_ftc_jobs, a0);
   } else {
-    hsum_block<H, VEC>(lds.hsum, hsum_jobs, n_hsum_jobs, v - a0);
+    hsum_block<H>(lds.hsum, hsum_jobs, n_hsum_jobs, v - a0);
   }
 }
 
-bool fused_supported(uint32_t tile, uint32_t n_harmonics, bool vec) {
-  return tile == 1024 && (n_harmonics == 8 || (n_harmonics == 16 && vec));
+// 16 planes stay unfused when a row length is not a multiple of 8: the fused kernel's transform
+// rounds differently from ftconv1w_kernel's, so a plan's choice between them is part of its results.
+bool fused_supported(uint32_t tile, uint32_t n_harmonics, bool whole_groups) {
+  return tile == 1024 && (n_harmonics == 8 || (n_harmonics == 16 && whole_groups));
 }
 
 hipError_t launch_fused(const FtcJob* ftc_jobs, uint32_t n_ftc_jobs, uint32_t n_items, const float2* tw1,
                         const float2* tw2, const HsumJob* hsum_jobs, uint32_t n_hsum_jobs, uint32_t n_blocks,
-                        uint32_t n_harmonics, bool vec, hipStream_t stream) {
+                        uint32_t n_harmonics, hipStream_t stream) {
   const uint32_t grid = n_items + n_blocks;
   if (grid == 0) return hipSuccess;
   const dim3 block(64 * kFtc1kWaves);
-#define FDAS_FUSED(HH, VV)                                                                                          \
-  hipLaunchKernelGGL((fused1k_kernel<HH, VV>), dim3(grid), block, 0, stream, ftc_jobs, n_ftc_jobs, n_items, tw1, tw2, \
+#define FDAS_FUSED(HH)                                                                                         \
+  hipLaunchKernelGGL(fused1k_kernel<HH>, dim3(grid), block, 0, stream, ftc_jobs, n_ftc_jobs, n_items, tw1, tw2, \
                      hsum_jobs, n_hsum_jobs, n_blocks)
-  if (n_harmonics == 8 && vec) FDAS_FUSED(8, true);
-  else if (n_harmonics == 8) FDAS_FUSED(8, false);
-  else if (n_harmonics == 16 && vec) FDAS_FUSED(16, true);
+  if (n_harmonics == 8) FDAS_FUSED(8);
+  else if (n_harmonics == 16) FDAS_FUSED(16);
   else return hipErrorInvalidValue;
 #undef FDAS_FUSED
   return hipGetLastError();

@@ -29,6 +29,10 @@ namespace fdas {
 #define FDAS_GLOBAL __attribute__((address_space(1)))
 typedef float fdas_vf2 __attribute__((ext_vector_type(2)));
 typedef float fdas_vf4 __attribute__((ext_vector_type(4)));
+// The same read from any 4-byte boundary (rows whose length is not a multiple of 4):
+// gfx950 takes 8- and 16-byte global loads at dword alignment.
+typedef float fdas_vf2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float fdas_vf4u __attribute__((ext_vector_type(4), aligned(4)));
 
 template <typename T>
 __device__ __forceinline__ T gld(const T* p, size_t i) {
@@ -42,9 +46,12 @@ __device__ __forceinline__ float2 gld2(const float2* p, size_t i) {
   const fdas_vf2 v = ((const FDAS_GLOBAL fdas_vf2*)p)[i];
   return make_float2(v.x, v.y);
 }
-// Four consecutive floats p[i .. i+3]; p + i must be 16-byte aligned.
-__device__ __forceinline__ fdas_vf4 gld4(const float* p, size_t i) {
-  return *(const FDAS_GLOBAL fdas_vf4*)(p + i);
+// Two / four consecutive floats from p[i] on, at any dword alignment.
+__device__ __forceinline__ fdas_vf2u gld2u(const float* p, size_t i) {
+  return *(const FDAS_GLOBAL fdas_vf2u*)(p + i);
+}
+__device__ __forceinline__ fdas_vf4u gld4u(const float* p, size_t i) {
+  return *(const FDAS_GLOBAL fdas_vf4u*)(p + i);
 }
 // Streaming store: the data is read back only by a later kernel, so it is
 // written with the non-temporal hint and does not displace the cached
