@@ -291,7 +291,7 @@ fdas_status enqueue_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* 
   if ((st = record(ctx, s, EV_HSUM_K1)) != FDAS_OK) return st;
   HIPCK(ctx, hipEventRecord(s.hsum_done, s.stream));
   s.hsum_issued = true;
-  HIPCK(ctx, launch_select(s.d_sel, H, s.stream));
+  HIPCK(ctx, launch_select(s.d_sel, H, cap, s.stream));
   return FDAS_OK;
 }
 

@@ -619,7 +619,7 @@ fdas_status enqueue_group(fdas_engine* e, GroupBuf& g, const std::vector<Trial*>
   for (const auto& L : g.hsum) EHIP(e, launch_hsum(g.d_hsum + L.first, L.n_jobs, L.n_blocks, L.H, B));
   if (timing_events) EHIP(e, hipEventRecord(g.ev_hsum1, B));
   EHIP(e, hipEventRecord(g.ev_hsum_done, B));
-  EHIP(e, launch_select(g.d_sel, g.n_sel, B));
+  EHIP(e, launch_select(g.d_sel, g.n_sel, e->cfg.cands_per_harmonic, B));
   if (g.small_span) {
     EHIP(e, hipMemcpyAsync(g.h_span, g.small_span, g.span_bytes, hipMemcpyDeviceToHost, B));
   } else {
@@ -1650,7 +1650,7 @@ static fdas_status plan_enqueue_lagged(fdas_plan* p, bool capturing) {
     if (prev) {
       EHIP(e, hipEventRecord(prev->ev_hsum_done, A));
       EHIP(e, hipStreamWaitEvent(B, prev->ev_hsum_done, 0));
-      EHIP(e, launch_select(prev->d_sel, prev->n_sel, B));
+      EHIP(e, launch_select(prev->d_sel, prev->n_sel, e->cfg.cands_per_harmonic, B));
       if (prev->small_span) {
         EHIP(e, hipMemcpyAsync(prev->h_span, prev->small_span, prev->span_bytes, hipMemcpyDeviceToHost, B));
       } else {

@@ -17,7 +17,6 @@ constexpr int kHsumBinsPerBlock = kHsumThreads * kHsumBinsPerThread;  // bins on
 inline bool hsum_whole_groups(uint32_t n_bins) { return n_bins % kHsumBinsPerThread == 0; }
 constexpr uint32_t kHsumRowsPerBlock = 11;  // target rows per HSUM workgroup (bounds the dense-hit tail)
 constexpr int kHsumWaveStage = 64;        // LDS staging entries per plane per wave before a global flush
-constexpr int kSelectThreads = 1024;
 constexpr uint32_t kSelectMaxCap = 8192;  // largest per-plane cap the in-LDS sort handles
 constexpr uint32_t kSelectPool = 4096;    // boundary-bin entries resolved exactly in LDS
 constexpr uint32_t kSelectSlices = 64;    // workgroups per plane in the histogram / compaction passes
@@ -39,8 +38,9 @@ hipError_t launch_hsum(const HsumJob* d_jobs, uint32_t n_jobs, uint32_t n_blocks
 
 // Per-plane cap (strongest first) and sort by (row, bin): power histogram and
 // compaction over the spill lists (kSelectSlices workgroups per plane), then one
-// workgroup per plane resolves the boundary bin exactly and sorts.
-hipError_t launch_select(const SelectJob* d_jobs, uint32_t n_jobs, hipStream_t stream);
+// workgroup per plane resolves the boundary bin exactly and sorts.  cap: the
+// largest cap of the jobs.
+hipError_t launch_select(const SelectJob* d_jobs, uint32_t n_jobs, uint32_t cap, hipStream_t stream);
 
 // Harmonic plane HP_k over rows [row_begin, row_begin + n_rows) (debug / parity).
 hipError_t launch_hplane(const float* fop, uint32_t n_bins, uint32_t n_templates, uint32_t row_begin,

@@ -823,37 +823,32 @@ hipError_t launch_hmax(const float* fop, uint32_t n_bins, uint32_t n_templates, 
 // (row, bin) key first), returned sorted by key.
 // ---------------------------------------------------------------------------
 
-// Exclusive prefix sum over a workgroup of THREADS threads; *total gets the sum.
+// Inclusive prefix sum over the wave: row shifts inside each row of 16 lanes,
+// then the rows' totals broadcast upwards (VALU only; six LDS permutes take
+// about ten times as long).
+__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x111, 0xf, 0xf, false));  // row_shr:1
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x112, 0xf, 0xf, false));  // row_shr:2
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x114, 0xf, 0xf, false));  // row_shr:4
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x118, 0xf, 0xf, false));  // row_shr:8
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x142, 0xa, 0xf, false));  // row_bcast:15 into rows 1, 3
+  v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x143, 0xc, 0xf, false));  // row_bcast:31 into rows 2, 3
+  return v;
+}
+
+// Exclusive prefix sum over a workgroup of THREADS threads.  s_waves: one LDS
+// word per wave, not reused before the caller's next barrier.
 template <int THREADS>
-__device__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s_waves, uint32_t* total) {
-  constexpr int n_waves = THREADS / 64;
-  const int tid = threadIdx.x;
-  const int lane = int(lane_id());
-  const int wave = tid >> 6;
-  uint32_t x = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t y = __shfl_up(x, o);
-    if (lane >= o) x += y;
-  }
+__device__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s_waves) {
+  constexpr uint32_t n_waves = THREADS / 64;
+  static_assert(n_waves <= 16, "the waves' totals are scanned in one row of lanes");
+  const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
+  const uint32_t x = wave_inclusive_scan(v);
   if (lane == 63) s_waves[wave] = x;
   __syncthreads();
-  if (tid < 64) {
-    const uint32_t w = tid < n_waves ? s_waves[tid] : 0u;
-    uint32_t ws = w;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t y = __shfl_up(ws, o);
-      if (lane >= o) ws += y;
-    }
-    if (tid < n_waves) s_waves[tid] = ws - w;
-    if (tid == n_waves - 1) s_waves[32] = ws;
-  }
-  __syncthreads();
-  const uint32_t res = s_waves[wave] + x - v;
-  *total = s_waves[32];
-  __syncthreads();
-  return res;
+  const uint32_t w = lane < n_waves ? s_waves[lane] : 0u;
+  const uint32_t before = wave_inclusive_scan(w) - w;  // lane i: total of waves 0 .. i-1
+  return x - v + uint32_t(__builtin_amdgcn_readlane(int(before), __builtin_amdgcn_readfirstlane(int(wave))));
 }
 
 // Cut bin b*: the highest bin whose suffix count sum_{b >= b*} hist[b] reaches
@@ -876,8 +871,7 @@ __device__ void find_cut(const uint32_t* __restrict__ hist, uint32_t cap, uint32
     h[j] = gld(hist, kSelectBins - 1 - uint32_t(tid * PER + j));
     local += h[j];
   }
-  uint32_t total;
-  const uint32_t excl = block_exclusive_scan<THREADS>(local, s_waves, &total);
+  const uint32_t excl = block_exclusive_scan<THREADS>(local, s_waves);
   uint32_t bin, above;
   if (cut_in_share<PER>(h, excl, cap, uint32_t(tid * PER), &bin, &above)) {
     s_out[0] = bin;
@@ -914,86 +908,145 @@ __global__ __launch_bounds__(256) void cand_hist_kernel(const SelectJob* __restr
     if (h[i]) gatomic_add(job.hist + i, h[i]);
 }
 
+// Slots for the lanes that set take[u], u = 0 .. U-1, from a counter in LDS, with
+// one atomic per wave; slot[u] is meaningful where take[u] is set.
+template <int U>
+__device__ __forceinline__ void wave_append(uint32_t* counter, const bool (&take)[U], uint32_t (&slot)[U]) {
+  uint64_t mask[U];
+  uint32_t total = 0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    mask[u] = __ballot(take[u]);
+    slot[u] = total + lanes_below(mask[u]);
+    total += uint32_t(__builtin_popcountll(mask[u]));
+  }
+  if (total == 0) return;
+  uint32_t base = 0;
+  if (lane_id() == 0) base = atomicAdd(counter, total);
+  base = __shfl(base, 0);
+#pragma unroll
+  for (int u = 0; u < U; ++u) slot[u] += base;
+}
+
+// Copies the entries at or above the cut bin to the compact list.  Bound by
+// latency: a workgroup collects its slice's entries in LDS and reserves their
+// place in the list with one global atomic per flush.  (One returning global
+// atomic per wave with a hit, on the plane's one counter, made 2,500 of them
+// queue up for plane 1 of a 2^21-bin trial: 43 us per launch of 8 planes,
+// against 10 this way.)
 __global__ __launch_bounds__(256) void cand_compact_kernel(const SelectJob* __restrict__ jobs) {
   const SelectJob& job = jobs[blockIdx.y];
   const uint32_t n = min(gld(job.count, 0), job.spill_cap);
   if (n <= job.cap) return;
-  __shared__ uint32_t waves[40];
+  constexpr uint32_t kStep = 4 * 256, kStage = 2 * kStep;
+  __shared__ uint32_t waves[4];
   __shared__ uint32_t cut[2];
+  __shared__ uint32_t key[kStage];
+  __shared__ float pwr[kStage];
+  __shared__ uint32_t n_staged, g_base;
+  const int tid = threadIdx.x;
+  if (tid == 0) n_staged = 0;
   find_cut<256>(job.hist, job.cap, waves, cut);
   const uint32_t bstar = cut[0];
   const uint32_t tb = histogram_base(__float_as_uint(job.thr));
-  const int tid = threadIdx.x;
   const uint32_t per = (n + kSelectSlices - 1) / kSelectSlices;
   const uint32_t beg = blockIdx.x * per, end = min(beg + per, n);
-  for (uint32_t e0 = beg; e0 < end; e0 += 256) {
-    const uint32_t e = e0 + uint32_t(tid);
-    float v = -1.f;
-    uint32_t key = 0;
-    if (e < end) {
-      v = gld(job.spill_pwr, e);
-      key = gld(job.spill_key, e);
+  for (uint32_t e0 = beg; e0 < end; e0 += kStep) {
+    uint32_t k[4];
+    float v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const uint32_t e = min(e0 + uint32_t(u * 256 + tid), end - 1u);
+      v[u] = gld(job.spill_pwr, e);
+      k[u] = gld(job.spill_key, e);
     }
-    const bool sel = e < end && power_bin(__float_as_uint(v), tb) >= bstar;
-    const uint64_t mask = __ballot(sel);
-    if (mask == 0) continue;
-    const uint32_t lane = lane_id();
-    const uint32_t leader = uint32_t(__builtin_ctzll(mask));
-    uint32_t pos = 0;
-    if (lane == leader) pos = gatomic_add(job.compact_n, uint32_t(__builtin_popcountll(mask)));
-    pos = __shfl(pos, int(leader)) + lanes_below(mask);
-    if (sel && pos < job.compact_cap) {
-      gst(job.compact_key, pos, key);
-      gst(job.compact_pwr, pos, v);
+    bool sel[4];
+    uint32_t pos[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      sel[u] = e0 + uint32_t(u * 256 + tid) < end && power_bin(__float_as_uint(v[u]), tb) >= bstar;
+    wave_append(&n_staged, sel, pos);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (!sel[u]) continue;
+      key[pos[u]] = k[u];
+      pwr[pos[u]] = v[u];
     }
+    __syncthreads();
+    const uint32_t staged = n_staged;
+    __syncthreads();  // everyone has read it
+    if (staged > kStage - kStep || e0 + kStep >= end) {  // no room for another step, or done
+      if (tid == 0) {
+        g_base = staged ? gatomic_add(job.compact_n, staged) : 0u;
+        n_staged = 0;
+      }
+      __syncthreads();
+      const uint32_t base = g_base;
+      for (uint32_t i = tid; i < staged && base + i < job.compact_cap; i += 256) {
+        gst(job.compact_key, base + i, key[i]);
+        gst(job.compact_pwr, base + i, pwr[i]);
+      }
+    }
+    __syncthreads();
   }
 }
 
+constexpr int kSortBins = 256;  // values of one sort digit
+
+// LDS of one selection workgroup: up to CAP kept entries; the pool of the cut
+// bin's entries, the radix-select histogram and the sort's digit counters are
+// never live together.
+template <int THREADS, int CAP>
 struct SelectShared {
-  uint32_t key[kSelectMaxCap];
-  float pwr[kSelectMaxCap];
-  uint64_t pool[kSelectPool];
-  uint32_t hist[2048];
-  uint32_t waves[40];
+  static constexpr int kWaves = THREADS / 64;
+  static constexpr int kRow = kSortBins + 1;  // row stride of the counters: spreads a digit's over the banks
+  uint32_t key[CAP];
+  float pwr[CAP];
+  union {
+    uint64_t pool[kSelectPool];
+    uint32_t hist[2048];
+    uint32_t digit[kWaves * kRow];
+  };
+  uint32_t waves[kWaves];
   uint32_t misc[8];
 };
 
 // One radix-select digit pass: among values v with (v & mask) == prefix, find
 // the digit (bits [shift, shift+width)) holding the `rank`-th element counted
 // from the top (descending) or bottom (ascending).  Updates prefix/mask/rank.
-template <bool DESCENDING, typename Get>
-__device__ void radix_pass(SelectShared& sh, uint32_t n, Get get, uint32_t shift, uint32_t width, uint32_t& prefix,
+template <bool DESCENDING, int THREADS, class Shared, typename Get>
+__device__ void radix_pass(Shared& sh, uint32_t n, Get get, uint32_t shift, uint32_t width, uint32_t& prefix,
                            uint32_t& mask, uint32_t& rank) {
+  constexpr int PER = 2048 / THREADS;
   const int tid = threadIdx.x;
   const uint32_t nb = 1u << width;
-  for (uint32_t i = tid; i < 2048; i += kSelectThreads) sh.hist[i] = 0;
+  for (uint32_t i = tid; i < 2048; i += THREADS) sh.hist[i] = 0;
   __syncthreads();
-  for (uint32_t e = tid; e < n; e += kSelectThreads) {
+  for (uint32_t e = tid; e < n; e += THREADS) {
     const uint32_t v = get(e);
     if ((v & mask) == prefix) atomicAdd(&sh.hist[(v >> shift) & (nb - 1)], 1u);
   }
   __syncthreads();
-  // Thread t owns ordered positions u = 2t, 2t+1 (u counts from the selected end).
-  uint32_t h[2];
+  // Thread t owns ordered positions u = PER t .. PER t + PER - 1 (u counts from the selected end).
+  uint32_t h[PER], local = 0;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const uint32_t u = uint32_t(2 * tid + j);
+  for (int j = 0; j < PER; ++j) {
+    const uint32_t u = uint32_t(PER * tid + j);
     const uint32_t d = DESCENDING ? (nb - 1 - u) : u;
     h[j] = u < nb ? sh.hist[d] : 0u;
+    local += h[j];
   }
-  uint32_t total;
-  const uint32_t excl = block_exclusive_scan<kSelectThreads>(h[0] + h[1], sh.waves, &total);
-  if (excl < rank && rank <= excl + h[0] + h[1]) {
-    uint32_t u = uint32_t(2 * tid);
-    uint32_t r = rank - excl;
-    if (r > h[0]) {
-      r -= h[0];
-      u += 1;
+  const uint32_t excl = block_exclusive_scan<THREADS>(local, sh.waves);
+  uint32_t acc = excl;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    if (acc < rank && rank <= acc + h[j]) {
+      const uint32_t u = uint32_t(PER * tid + j);
+      sh.misc[0] = DESCENDING ? (nb - 1 - u) : u;
+      sh.misc[1] = rank - acc;
+      sh.misc[2] = h[j];
     }
-    const uint32_t d = DESCENDING ? (nb - 1 - u) : u;
-    sh.misc[0] = d;
-    sh.misc[1] = r;
-    sh.misc[2] = sh.hist[d];
+    acc += h[j];
   }
   __syncthreads();
   prefix |= sh.misc[0] << shift;
@@ -1002,45 +1055,136 @@ __device__ void radix_pass(SelectShared& sh, uint32_t n, Get get, uint32_t shift
   __syncthreads();
 }
 
-__device__ void bitonic_sort_by_key(SelectShared& sh, uint32_t n) {
-  const int tid = threadIdx.x;
-  uint32_t p2 = 1;
-  while (p2 < n) p2 <<= 1;
-  for (uint32_t i = n + tid; i < p2; i += kSelectThreads) {
-    sh.key[i] = 0xffffffffu;
-    sh.pwr[i] = 0.f;
+// Sorts the n kept entries by key (row, bin), ascending: a radix sort in place,
+// 8 bits a pass, over the bits that rows and bins really use (3 passes for a
+// spectrum of 2^17 bins and 85 templates, 4 for 2^21).  Bound by LDS latency and
+// barriers: an entry's place is its digit's start, plus what earlier waves and
+// the wave's earlier entries hold of that digit (one match by ballots), so a
+// pass takes 7 barriers, where the bitonic network took one for each of its 78
+// steps over 4096 entries.
+template <int THREADS, int CAP, class Shared>
+__device__ void sort_by_key(Shared& sh, uint32_t n) {
+  constexpr int E = CAP / THREADS, NW = THREADS / 64, ROW = Shared::kRow;
+  constexpr int PER = kSortBins * NW / THREADS;  // counters one thread scans
+  static_assert(PER * THREADS == kSortBins * NW, "whole counters per thread");
+  const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+  const uint32_t sub = (n + THREADS - 1) / THREADS;  // 64-entry runs of one wave
+  uint32_t key[E], place[E];
+  float pwr[E];
+  // Bits in use: bins below 2^nb, rows above them.
+  if (tid < 2) sh.misc[4 + tid] = 0;
+  __syncthreads();
+  uint32_t or_bin = 0, or_row = 0;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const uint32_t i = (wave * sub + uint32_t(e)) * 64 + lane;
+    key[e] = 0;
+    pwr[e] = 0.f;
+    place[e] = 0;
+    if (uint32_t(e) < sub && i < n) {
+      key[e] = sh.key[i];
+      pwr[e] = sh.pwr[i];
+      or_bin |= key[e] & ((1u << kKeyBinBits) - 1u);
+      or_row |= key[e] >> kKeyBinBits;
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    or_bin |= __shfl_xor(or_bin, o);
+    or_row |= __shfl_xor(or_row, o);
+  }
+  if (lane == 0) {
+    atomicOr(&sh.misc[4], or_bin);
+    atomicOr(&sh.misc[5], or_row);
   }
   __syncthreads();
-  for (uint32_t k = 2; k <= p2; k <<= 1) {
-    for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-      for (uint32_t i = tid; i < p2; i += kSelectThreads) {
-        const uint32_t ixj = i ^ j;
-        if (ixj > i) {
-          const uint32_t a = sh.key[i], b = sh.key[ixj];
-          const bool up = (i & k) == 0;
-          if ((a > b) == up) {
-            sh.key[i] = b;
-            sh.key[ixj] = a;
-            const float pa = sh.pwr[i];
-            sh.pwr[i] = sh.pwr[ixj];
-            sh.pwr[ixj] = pa;
-          }
-        }
+  const uint32_t nb = 32u - uint32_t(__builtin_clz(sh.misc[4] | 1u));
+  const uint32_t bits = nb + 32u - uint32_t(__builtin_clz(sh.misc[5] | 1u));
+  const uint32_t passes = (bits + 7u) / 8u, width = (bits + passes - 1u) / passes;  // digits of equal width, <= 8 bits
+  auto digit_of = [&](uint32_t k, uint32_t shift) {
+    const uint32_t packed = ((k >> kKeyBinBits) << nb) | (k & ((1u << kKeyBinBits) - 1u));
+    return (packed >> shift) & ((1u << width) - 1u);
+  };
+  uint32_t* mine = sh.digit + wave * ROW;
+  for (uint32_t shift = 0; shift < bits; shift += width) {
+    for (uint32_t i = tid; i < uint32_t(NW * ROW); i += THREADS) sh.digit[i] = 0;
+    __syncthreads();
+    // Lanes of the run that hold the same digit (its bits' ballots, complemented where the lane's bit is 0).
+    uint32_t same_lo[E], same_hi[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const uint64_t valid = __ballot(uint32_t(e) < sub && (wave * sub + uint32_t(e)) * 64 + lane < n);
+      same_lo[e] = uint32_t(valid);
+      same_hi[e] = uint32_t(valid >> 32);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (uint32_t(j) >= width) break;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int bit = -int((digit_of(key[e], shift) >> j) & 1u);  // all ones or zero
+        const uint64_t m = __ballot(bit != 0);
+        same_lo[e] &= ~(uint32_t(m) ^ uint32_t(bit));
+        same_hi[e] &= ~(uint32_t(m >> 32) ^ uint32_t(bit));
       }
-      __syncthreads();
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      if (uint32_t(e) >= sub) break;
+      const bool valid = (wave * sub + uint32_t(e)) * 64 + lane < n;
+      const uint32_t d = digit_of(key[e], shift);
+      const uint32_t below = __builtin_amdgcn_mbcnt_hi(same_hi[e], __builtin_amdgcn_mbcnt_lo(same_lo[e], 0u));
+      const uint32_t before = mine[d];
+      wave_lds_order();
+      place[e] = before + below;
+      if (valid && below == 0)
+        mine[d] = before + uint32_t(__builtin_popcount(same_lo[e])) + uint32_t(__builtin_popcount(same_hi[e]));
+      wave_lds_order();
+    }
+    __syncthreads();
+    uint32_t c[PER], local = 0;  // digit-major: all waves' counters of digit 0, of digit 1, ...
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const uint32_t q = tid * PER + uint32_t(j);
+      c[j] = sh.digit[(q % NW) * ROW + q / NW];
+      local += c[j];
+    }
+    uint32_t acc = block_exclusive_scan<THREADS>(local, sh.waves);
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const uint32_t q = tid * PER + uint32_t(j);
+      sh.digit[(q % NW) * ROW + q / NW] = acc;
+      acc += c[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      if (uint32_t(e) >= sub || (wave * sub + uint32_t(e)) * 64 + lane >= n) continue;
+      const uint32_t pos = mine[digit_of(key[e], shift)] + place[e];
+      sh.key[pos] = key[e];
+      sh.pwr[pos] = pwr[e];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const uint32_t i = (wave * sub + uint32_t(e)) * 64 + lane;
+      if (uint32_t(e) >= sub || i >= n) continue;
+      key[e] = sh.key[i];
+      pwr[e] = sh.pwr[i];
     }
   }
 }
 
+template <int THREADS>
 __device__ void bitonic_sort_u64(uint64_t* a, uint32_t n) {
   const int tid = threadIdx.x;
   uint32_t p2 = 1;
   while (p2 < n) p2 <<= 1;
-  for (uint32_t i = n + tid; i < p2; i += kSelectThreads) a[i] = ~0ull;
+  for (uint32_t i = n + tid; i < p2; i += THREADS) a[i] = ~0ull;
   __syncthreads();
   for (uint32_t k = 2; k <= p2; k <<= 1) {
     for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-      for (uint32_t i = tid; i < p2; i += kSelectThreads) {
+      for (uint32_t i = tid; i < p2; i += THREADS) {
         const uint32_t ixj = i ^ j;
         if (ixj > i) {
           const uint64_t x = a[i], y = a[ixj];
@@ -1055,18 +1199,47 @@ __device__ void bitonic_sort_u64(uint64_t* a, uint32_t n) {
   }
 }
 
+// Appends the `take` smallest of the pool's n entries (power descending, then
+// key ascending) to the kept list from `at` on.  A few hundred entries, the
+// usual size of the cut bin, are ranked by counting; a pool beyond
+// kCountedPool, where that would cost more than it saves (n^2 / THREADS
+// compares), is sorted.
+constexpr uint32_t kCountedPool = 1024;
+
+template <int THREADS, class Shared>
+__device__ void take_from_pool(Shared& sh, uint32_t n, uint32_t take, uint32_t at) {
+  const uint32_t tid = threadIdx.x;
+  auto keep = [&](uint32_t slot, uint64_t v) {
+    sh.key[slot] = uint32_t(v);
+    sh.pwr[slot] = __uint_as_float(order_key_inv(~uint32_t(v >> 32)));
+  };
+  if (n > kCountedPool) {
+    bitonic_sort_u64<THREADS>(sh.pool, n);
+    for (uint32_t i = tid; i < take && i < n; i += THREADS) keep(at + i, sh.pool[i]);
+    return;
+  }
+  for (uint32_t i = tid; i < n; i += THREADS) {
+    const uint64_t v = sh.pool[i];
+    uint32_t rank = 0;
+#pragma unroll 8
+    for (uint32_t q = 0; q < n; ++q) rank += sh.pool[q] < v ? 1u : 0u;
+    if (rank < take) keep(at + rank, v);
+  }
+}
+
 // Exact top-`cap` of the whole spill by radix select on (power desc, key asc).
 // Used when the boundary bin holds more entries than the LDS pool.
-__device__ uint32_t radix_select_spill(SelectShared& sh, const SelectJob& job, uint32_t n) {
+template <int THREADS, class Shared>
+__device__ uint32_t radix_select_spill(Shared& sh, const SelectJob& job, uint32_t n) {
   const int tid = threadIdx.x;
   const uint32_t cap = job.cap;
   const uint32_t* __restrict__ skey = job.spill_key;
   const float* __restrict__ spwr = job.spill_pwr;
   auto pkey = [&](uint32_t e) { return order_key(__float_as_uint(gld(spwr, e))); };
   uint32_t prefix = 0, mask = 0, rank = cap;
-  radix_pass<true>(sh, n, pkey, 21, 11, prefix, mask, rank);
-  radix_pass<true>(sh, n, pkey, 10, 11, prefix, mask, rank);
-  radix_pass<true>(sh, n, pkey, 0, 10, prefix, mask, rank);
+  radix_pass<true, THREADS>(sh, n, pkey, 21, 11, prefix, mask, rank);
+  radix_pass<true, THREADS>(sh, n, pkey, 10, 11, prefix, mask, rank);
+  radix_pass<true, THREADS>(sh, n, pkey, 0, 10, prefix, mask, rank);
   const uint32_t vkey = prefix;  // order key of the cap-th strongest power V
   const uint32_t n_equal = sh.misc[2];
   // `rank` entries with power == V are kept: the smallest keys among them.
@@ -1074,14 +1247,14 @@ __device__ uint32_t radix_select_spill(SelectShared& sh, const SelectJob& job, u
   if (n_equal > rank) {
     auto kbits = [&](uint32_t e) { return pkey(e) == vkey ? gld(skey, e) : 0xffffffffu; };
     uint32_t kp = 0, km = 0, kr = rank;
-    radix_pass<false>(sh, n, kbits, 21, 11, kp, km, kr);
-    radix_pass<false>(sh, n, kbits, 10, 11, kp, km, kr);
-    radix_pass<false>(sh, n, kbits, 0, 10, kp, km, kr);
+    radix_pass<false, THREADS>(sh, n, kbits, 21, 11, kp, km, kr);
+    radix_pass<false, THREADS>(sh, n, kbits, 10, 11, kp, km, kr);
+    radix_pass<false, THREADS>(sh, n, kbits, 0, 10, kp, km, kr);
     kmax = kp;
   }
   if (tid == 0) sh.misc[3] = 0;
   __syncthreads();
-  for (uint32_t e = tid; e < n; e += kSelectThreads) {
+  for (uint32_t e = tid; e < n; e += THREADS) {
     const float pv = gld(spwr, e);
     const uint32_t pk = order_key(__float_as_uint(pv));
     const uint32_t key = gld(skey, e);
@@ -1097,8 +1270,13 @@ __device__ uint32_t radix_select_spill(SelectShared& sh, const SelectJob& job, u
   return min(sh.misc[3], cap);
 }
 
-__global__ __launch_bounds__(kSelectThreads) void select_final_kernel(const SelectJob* __restrict__ jobs) {
-  __shared__ SelectShared sh;
+// One workgroup per plane: the kept entries, sorted.  CAP >= the job's cap.
+// Bound by latency (one workgroup's barriers and LDS round trips): 20 us for 8
+// planes that keep 4096 of 70,000 .. 173,000 entries, 13 of them in the sort, and
+// 9.7 us for a cap of 512 (with bitonic sorts of key and power: 75 and 16 us).
+template <int THREADS, int CAP>
+__global__ __launch_bounds__(THREADS) void select_final_kernel(const SelectJob* __restrict__ jobs) {
+  __shared__ SelectShared<THREADS, CAP> sh;
   const SelectJob& job = jobs[blockIdx.x];
   const int tid = threadIdx.x;
   const uint32_t n = min(gld(job.count, 0), job.spill_cap);
@@ -1106,13 +1284,13 @@ __global__ __launch_bounds__(kSelectThreads) void select_final_kernel(const Sele
 
   uint32_t kept;
   if (n <= cap) {
-    for (uint32_t e = tid; e < n; e += kSelectThreads) {
+    for (uint32_t e = tid; e < n; e += THREADS) {
       sh.key[e] = gld(job.spill_key, e);
       sh.pwr[e] = gld(job.spill_pwr, e);
     }
     kept = n;
   } else {
-    find_cut<kSelectThreads>(job.hist, cap, sh.waves, sh.misc);
+    find_cut<THREADS>(job.hist, cap, sh.waves, sh.misc);
     const uint32_t bstar = sh.misc[0], above = sh.misc[1];
     const uint32_t m = gld(job.compact_n, 0);
     const uint32_t pool_n = gld(job.hist, bstar);
@@ -1124,51 +1302,67 @@ __global__ __launch_bounds__(kSelectThreads) void select_final_kernel(const Sele
         sh.misc[4] = 0;
       }
       __syncthreads();
-      for (uint32_t e = tid; e < m; e += kSelectThreads) {
-        const float v = gld(job.compact_pwr, e);
-        const uint32_t key = gld(job.compact_key, e);
-        const uint32_t pb = __float_as_uint(v);
-        const uint32_t bin = power_bin(pb, tb);
-        if (bin > bstar) {
-          const uint32_t pos = atomicAdd(&sh.misc[3], 1u);
-          if (pos < cap) {
-            sh.key[pos] = key;
-            sh.pwr[pos] = v;
+      constexpr int U = 4;  // loads in flight per thread
+      for (uint32_t e0 = 0; e0 < m; e0 += U * THREADS) {
+        float v[U];
+        uint32_t key[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const uint32_t e = min(e0 + uint32_t(u * THREADS + tid), m - 1u);
+          v[u] = gld(job.compact_pwr, e);
+          key[u] = gld(job.compact_key, e);
+        }
+        bool strong[U], at_cut[U];
+        uint32_t pos[U], q[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const bool in = e0 + uint32_t(u * THREADS + tid) < m;
+          const uint32_t bin = power_bin(__float_as_uint(v[u]), tb);
+          strong[u] = in && bin > bstar;
+          at_cut[u] = in && bin == bstar;
+        }
+        wave_append(&sh.misc[3], strong, pos);
+        wave_append(&sh.misc[4], at_cut, q);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (strong[u] && pos[u] < cap) {
+            sh.key[pos[u]] = key[u];
+            sh.pwr[pos[u]] = v[u];
           }
-        } else if (bin == bstar) {
-          const uint32_t q = atomicAdd(&sh.misc[4], 1u);
-          if (q < kSelectPool) sh.pool[q] = (uint64_t(~order_key(pb)) << 32) | key;  // strongest first
+          if (at_cut[u] && q[u] < kSelectPool)
+            sh.pool[q[u]] = (uint64_t(~order_key(__float_as_uint(v[u]))) << 32) | key[u];  // strongest first
         }
       }
       __syncthreads();
-      const uint32_t n_pool = min(sh.misc[4], kSelectPool);
-      bitonic_sort_u64(sh.pool, n_pool);
-      const uint32_t take = cap - above;
-      for (uint32_t i = tid; i < take && i < n_pool; i += kSelectThreads) {
-        const uint64_t v = sh.pool[i];
-        sh.key[above + i] = uint32_t(v);
-        sh.pwr[above + i] = __uint_as_float(order_key_inv(~uint32_t(v >> 32)));
-      }
-      __syncthreads();
+      take_from_pool<THREADS>(sh, min(sh.misc[4], kSelectPool), cap - above, above);
       kept = cap;
     } else {
-      kept = radix_select_spill(sh, job, n);
+      kept = radix_select_spill<THREADS>(sh, job, n);
     }
   }
   __syncthreads();
-  bitonic_sort_by_key(sh, kept);
-  for (uint32_t e = tid; e < kept; e += kSelectThreads) {
+  sort_by_key<THREADS, CAP>(sh, kept);
+  __syncthreads();
+  for (uint32_t e = tid; e < kept; e += THREADS) {
     gst(job.out_key, e, sh.key[e]);
     gst(job.out_pwr, e, sh.pwr[e]);
   }
   if (tid == 0) gst(job.out_n, 0, kept);
 }
 
-hipError_t launch_select(const SelectJob* d_jobs, uint32_t n_jobs, hipStream_t stream) {
+hipError_t launch_select(const SelectJob* d_jobs, uint32_t n_jobs, uint32_t cap, hipStream_t stream) {
   if (n_jobs == 0) return hipSuccess;
+  if (cap > kSelectMaxCap) return hipErrorInvalidValue;
   hipLaunchKernelGGL(cand_hist_kernel, dim3(kSelectSlices, n_jobs), dim3(256), 0, stream, d_jobs);
   hipLaunchKernelGGL(cand_compact_kernel, dim3(kSelectSlices, n_jobs), dim3(256), 0, stream, d_jobs);
-  hipLaunchKernelGGL(select_final_kernel, dim3(n_jobs), dim3(kSelectThreads), 0, stream, d_jobs);
+  // The workgroup grows with the list.  With 1024 / 512 / 256 threads a cap of 4096 took 28 / 30 / 38 us and one
+  // of 512 took 11 / 10 / 11 us, where the small workgroup needs a quarter of the CU beside other kernels.
+  if (cap <= 1024)
+    hipLaunchKernelGGL((select_final_kernel<256, 1024>), dim3(n_jobs), dim3(256), 0, stream, d_jobs);
+  else if (cap <= 4096)
+    hipLaunchKernelGGL((select_final_kernel<1024, 4096>), dim3(n_jobs), dim3(1024), 0, stream, d_jobs);
+  else
+    hipLaunchKernelGGL((select_final_kernel<1024, 8192>), dim3(n_jobs), dim3(1024), 0, stream, d_jobs);
   return hipGetLastError();
 }
 

@@ -172,7 +172,7 @@ extern "C" fdas_status fdas_hsum_noalloc(const float* d_fop, uint32_t n_bins, ui
   if (e == hipSuccess) e = launch_zero_u32(compact_n, H * (1 + kSelectBins), s);
   const uint32_t blocks = (n_bins + kHsumBinsPerBlock - 1) / kHsumBinsPerBlock * j.n_row_chunks;
   if (e == hipSuccess) e = launch_hsum(&d_jobs->hsum, 1, blocks, H, s);
-  if (e == hipSuccess) e = launch_select(d_jobs->sel, H, s);
+  if (e == hipSuccess) e = launch_select(d_jobs->sel, H, cap, s);
   if (e != hipSuccess) return report(log, user, FDAS_EDEVICE, "kernel launch failed (%s)", hipGetErrorString(e));
   return FDAS_OK;
 }
