@@ -207,6 +207,7 @@ fdas_status record(fdas_ctx* ctx, DevSet& s, Ev e) {
 std::vector<FtcJob> plan_ftc_jobs(const fdas_ctx* ctx, const DevSet& s, uint32_t rb, uint32_t nr) {
   std::vector<FtcJob> jobs = plan_ftc_rows(ctx->cfg.tile, ctx->geo.n_bins, ctx->cfg.max_taps, s.row_taps, rb, nr,
                                            kMaxFtcJobs);
+  fit_ftc_items(jobs, ftconv_slots(ctx->cfg.tile));
   uint32_t item = 0;
   for (FtcJob& j : jobs) {
     j.spectrum = s.input;
@@ -257,7 +258,7 @@ fdas_status enqueue_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* 
   j.n_harmonics = H;
   j.spill_cap = ctx->spill;
   j.block_begin = 0;
-  hsum_row_chunks(nr, &j.rows_per_block, &j.n_row_chunks);
+  hsum_row_chunks(nr, &j.rows_per_block, &j.n_row_chunks, hsum_rows_for(j.n_bins, nr));
   j.spill_key = s.spill_key;
   j.spill_pwr = s.spill_pwr;
   j.counts = s.counts;

@@ -140,7 +140,7 @@ extern "C" fdas_status fdas_hsum_noalloc(const float* d_fop, uint32_t n_bins, ui
   j.n_harmonics = H;
   j.spill_cap = spill;
   j.block_begin = 0;
-  hsum_row_chunks(nr, &j.rows_per_block, &j.n_row_chunks);
+  hsum_row_chunks(nr, &j.rows_per_block, &j.n_row_chunks, hsum_rows_for(n_bins, nr));
   j.spill_key = spill_key;
   j.spill_pwr = spill_pwr;
   j.counts = d_counts + H;  // detections per plane, before the cap

@@ -71,6 +71,22 @@ std::vector<FtcJob> plan_ftc_rows(uint32_t tile, uint32_t n_bins, uint32_t max_t
   return jobs;
 }
 
+void fit_ftc_items(std::vector<FtcJob>& jobs, uint32_t slots) {
+  for (uint32_t target = 1; target < kFtcRowsPerItem; ++target) {
+    uint64_t items = 0;
+    for (const FtcJob& j : jobs) {
+      const uint32_t rows = ftc_rows_per_item(j.n_rows, target);
+      items += uint64_t(j.n_tiles) * ((j.n_rows + rows - 1) / rows);
+    }
+    if (items > slots) continue;
+    for (FtcJob& j : jobs) {
+      j.rows_per_item = ftc_rows_per_item(j.n_rows, target);
+      j.n_chunks = (j.n_rows + j.rows_per_item - 1) / j.rows_per_item;
+    }
+    return;
+  }
+}
+
 std::vector<float2> kernel_template_layout(const std::vector<std::complex<double>>& spec, uint32_t n_templates,
                                            uint32_t tile) {
   const uint32_t S = tile, NT = S / 16;
@@ -117,6 +133,12 @@ void make_twiddles(uint32_t tile, std::vector<float2>& tw1, std::vector<float2>&
       tw2[k * D + d] = make_float2(float(std::cos(a)), float(std::sin(a)));
     }
   }
+}
+
+uint32_t hsum_rows_for(uint32_t n_bins, uint32_t n_rows) {
+  const uint64_t row_blocks = uint64_t((n_bins + kHsumBinsPerBlock - 1) / kHsumBinsPerBlock) * n_rows;
+  if (row_blocks >= 65536) return kHsumRowsPerBlock;
+  return std::min(8u, std::max(1u, uint32_t(std::lround(std::sqrt(double(row_blocks) / 220.0)))));
 }
 
 void hsum_row_chunks(uint32_t n_rows, uint32_t* rows_per_block, uint32_t* n_row_chunks, uint32_t target) {

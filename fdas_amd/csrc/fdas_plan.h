@@ -15,7 +15,8 @@ namespace fdas {
 // Rows one FT-convolution work item convolves: enough to amortise the forward
 // transform of its tile, small enough for several items per tile.  `target` is
 // the preferred count; the rows are split into equal chunks of at most that.
-uint32_t ftc_rows_per_item(uint32_t n_rows, uint32_t target = 16);
+constexpr uint32_t kFtcRowsPerItem = 16;
+uint32_t ftc_rows_per_item(uint32_t n_rows, uint32_t target = kFtcRowsPerItem);
 
 // Splits rows [row_begin, row_begin + n_rows) into contiguous groups, each with
 // its own overlap (longest non-zero template of the group minus one, rounded up
@@ -25,7 +26,20 @@ uint32_t ftc_rows_per_item(uint32_t n_rows, uint32_t target = 16);
 // the tap extents; rows_target only sets how many rows one work item takes.
 std::vector<FtcJob> plan_ftc_rows(uint32_t tile, uint32_t n_bins, uint32_t max_taps,
                                   const std::vector<uint32_t>& row_taps, uint32_t row_begin, uint32_t n_rows,
-                                  uint32_t max_groups, uint32_t rows_target = 16);
+                                  uint32_t max_groups, uint32_t rows_target = kFtcRowsPerItem);
+
+// Fewer rows per item for a launch that would leave CUs idle: the smallest count
+// whose items are all resident at once (`slots` workgroups), so that a row's
+// latency, not the number of rows in a row, sets the span; launches with more
+// items than that at 16 rows keep 16, which spend the fewest forward transforms.
+// Measured, us per launch (1 trial), at 16 rows / at the count chosen here:
+//   4,999 bins x 33 templates, tile 1024: 28 / 8 (1 row)
+//   32,768 x 85, tile 2048: 39 / 15 (2; 1 row, two rounds of workgroups: 21)
+//   20,011 x 169, tile 4096: 49 / 17 (2)
+//   131,072 x 85, tile 2048: 42 / 29 (8); tile 1024: 38 / 27 (6)
+// and from 262,144 bins (tile 2048) on 16 rows are the fastest or within 3 %.
+// The FOP does not depend on it.
+void fit_ftc_items(std::vector<FtcJob>& jobs, uint32_t slots);
 
 // Template spectra (T x S, natural order, complex double) -> kernel layout
 // [t][slot][tid], scaled by 1/S (exact).
@@ -39,6 +53,15 @@ std::vector<std::complex<double>> taps_to_spectra(const float* taps_c64, uint32_
 
 // Twiddle tables of the S-point tile transform: w1[k][b] = W_S^(b k), w2[k][d] = W_(S/16)^(d k).
 void make_twiddles(uint32_t tile, std::vector<float2>& tw1, std::vector<float2>& tw2);
+
+// Rows per summing workgroup for a launch of one trial.  Short chunks fill the
+// chip where a plane is small (a chunk's rows follow one another, and each waits
+// for its loads); tall ones re-read fewer sub-harmonic rows.  Between, the best
+// height grew with the square root of the plane's size.  Measured, us at 11 rows /
+// at the height chosen here: 4,999 bins x 33 rows 30 / 8 (1 row); 32,768 x 85
+// 47 / 16 (2); 131,072 x 85 42 / 32 (5); 262,144 x 85 56 / 47 (7); 700,001 x 85
+// 89 / 82 (8); at 2^21 x 85 8 rows take 208 against 204 at 11.
+uint32_t hsum_rows_for(uint32_t n_bins, uint32_t n_rows);
 
 // HSUM workgroup row chunking for a part of n_rows rows (at most `target` rows per workgroup).
 void hsum_row_chunks(uint32_t n_rows, uint32_t* rows_per_block, uint32_t* n_row_chunks,
