@@ -51,6 +51,7 @@ struct DevSet {
   FtcJob* d_ftc = nullptr;
   HsumJob* d_hsum = nullptr;
   SelectJob* d_sel = nullptr;
+  float* quant = nullptr;          // quantile thresholds: block maxima, then [4H] thresholds, counts, order statistics
 
   FtcJob* h_ftc = nullptr;
   HsumJob* h_hsum = nullptr;
@@ -59,6 +60,7 @@ struct DevSet {
   float* h_out_pwr = nullptr;
   uint32_t* h_out_n = nullptr;
   uint32_t* h_counts = nullptr;
+  uint32_t* h_quant = nullptr;     // [4H] mirror of quant's tail
 
   hipStream_t stream = nullptr;
   hipEvent_t ev[EV_COUNT] = {};
@@ -242,7 +244,8 @@ fdas_status enqueue_ftc(fdas_ctx* ctx, DevSet& s, fdas_part part) {
   return FDAS_OK;
 }
 
-fdas_status enqueue_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr) {
+// Job descriptors of a summing pass over the part, on their way to the device.
+fdas_status stage_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr) {
   uint32_t rb, nr;
   part_rows(ctx, part, &rb, &nr);
   const uint32_t H = ctx->cfg.n_harmonics;
@@ -285,6 +288,14 @@ fdas_status enqueue_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* 
   HIPCK(ctx, hipMemcpyAsync(s.d_sel, s.h_sel, sizeof(SelectJob) * H, hipMemcpyHostToDevice, s.stream));
   HIPCK(ctx, hipEventRecord(s.staged_hsum, s.stream));
   s.hsum_pending = true;
+  return FDAS_OK;
+}
+
+// The summing and selection kernels of the staged jobs.
+fdas_status run_hsum(fdas_ctx* ctx, DevSet& s) {
+  const uint32_t H = ctx->cfg.n_harmonics;
+  const HsumJob& j = *s.h_hsum;
+  fdas_status st;
   HIPCK(ctx, launch_zero_u32(s.counts, H * (2 + kSelectBins), s.stream));
   const uint32_t blocks = (ctx->geo.n_bins + kHsumBinsPerBlock - 1) / kHsumBinsPerBlock * j.n_row_chunks;
   if ((st = record(ctx, s, EV_HSUM_K0)) != FDAS_OK) return st;
@@ -292,8 +303,13 @@ fdas_status enqueue_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* 
   if ((st = record(ctx, s, EV_HSUM_K1)) != FDAS_OK) return st;
   HIPCK(ctx, hipEventRecord(s.hsum_done, s.stream));
   s.hsum_issued = true;
-  HIPCK(ctx, launch_select(s.d_sel, H, cap, s.stream));
+  HIPCK(ctx, launch_select(s.d_sel, H, ctx->cfg.cands_per_harmonic, s.stream));
   return FDAS_OK;
+}
+
+fdas_status enqueue_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr) {
+  const fdas_status st = stage_hsum(ctx, s, part, thr);
+  return st == FDAS_OK ? run_hsum(ctx, s) : st;
 }
 
 fdas_status enqueue_readback(fdas_ctx* ctx, DevSet& s) {
@@ -368,6 +384,8 @@ void free_set(DevSet& s) {
   (void)hipFree(s.d_ftc);
   (void)hipFree(s.d_hsum);
   (void)hipFree(s.d_sel);
+  (void)hipFree(s.quant);
+  (void)hipHostFree(s.h_quant);
   (void)hipHostFree(s.h_ftc);
   (void)hipHostFree(s.h_hsum);
   (void)hipHostFree(s.h_sel);
@@ -940,10 +958,12 @@ extern "C" fdas_status fdas_retrieve_harmonic_plane(fdas_ctx* ctx, uint32_t k, f
 // over the M = rows * N values of the part, linear interpolation between the
 // order statistics around q (M - 1), in FP64, rounded once to float32.  The two
 // order statistics are the (n+1)-th and n-th largest values.  Instead of
-// sorting M values: the (n+1)-th largest block maximum B_k bounds the (n+1)-th
-// largest value from below (n+1 blocks hold a value >= B_k), so one summing
-// pass with threshold just below B_k spills every value >= B_k, among them the
-// n+1 largest, and those few are sorted on the host.
+// sorting M values: the (n+2)-th largest block maximum B_k bounds them from
+// below (n+2 blocks hold a value >= B_k), so one summing pass with a threshold
+// just below B_k spills every value >= B_k, and the two are found among those.
+// All of that runs on the device with one read-back; only planes with fewer
+// blocks than that, or more spilled values than the lists hold, bring the host
+// in, which bisects their thresholds.
 extern "C" fdas_status fdas_quantile_thresholds(fdas_ctx* ctx, uint32_t n_per_plane, fdas_part part, int set,
                                                 float* thresholds) {
   CHECK_SET(ctx, set);
@@ -959,97 +979,84 @@ extern "C" fdas_status fdas_quantile_thresholds(fdas_ctx* ctx, uint32_t n_per_pl
     return fail(ctx, FDAS_EINVAL, "candidates per plane %u outside 1 .. %llu", n_per_plane,
                 (unsigned long long)(M - 1));
   HIPCK(ctx, hipSetDevice(ctx->cfg.device));
-  fdas_status st = wait_staging(ctx, s.staged_hsum, s.hsum_pending);
-  if (st != FDAS_OK) return st;
-  HIPCK(ctx, hipStreamSynchronize(s.stream));
-  // 1. block maxima of every plane
-  const uint32_t nb = hmax_blocks(N, nr);
-  float* d_max = nullptr;
-  if ((st = dev_alloc(ctx, &d_max, size_t(H) * nb)) != FDAS_OK) return st;
-  std::vector<float> bmax(size_t(H) * nb);
-  hipError_t e = launch_hmax(s.fop, N, ctx->cfg.n_templates, rb, nr, H, d_max, s.stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(bmax.data(), d_max, sizeof(float) * bmax.size(), hipMemcpyDeviceToHost,
-                                          s.stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(s.stream);
-  (void)hipFree(d_max);
-  HIPCK(ctx, e);
-  // 2. per plane a threshold t with count(HP_k > t) >= n + 2 that fits the spill
-  //    lists: just below the (n+2)-th largest block maximum when there are that
-  //    many blocks, refined (or, without a bound, found) by bisection over the
-  //    bit patterns of non-negative floats, where each pass counts all planes.
-  const size_t want = size_t(std::min<uint64_t>(uint64_t(n_per_plane) + 2, M));  // a spare rank for rounding
-  auto value_of = [](int64_t b) { return b < 0 ? -INFINITY : __builtin_bit_cast(float, uint32_t(b)); };
-  std::vector<int64_t> lo_b(H, -1), hi_b(H, 0x7f800000);  // count(> lo) >= want, count(> hi) < want
-  for (uint32_t k = 0; k < H; ++k) {
-    std::vector<float> v(bmax.begin() + size_t(k) * nb, bmax.begin() + size_t(k + 1) * nb);
-    if (v.size() < want) continue;
-    std::nth_element(v.begin(), v.begin() + (want - 1), v.end(), std::greater<float>());
-    const float bound = std::nextafter(v[want - 1], -INFINITY);
-    lo_b[k] = bound < 0.f ? -1 : int64_t(__builtin_bit_cast(uint32_t, bound));
-  }
-  std::vector<float> thr(H);
-  std::vector<uint32_t> lo_count(H, 0);
-  bool probing = false;  // the last pass used a probe threshold for some plane
-  for (int pass = 0;; ++pass) {
-    // pass 0 measures the starting bounds; later passes bisect the planes that overflow
-    probing = false;
-    std::vector<int64_t> at(H);
-    for (uint32_t k = 0; k < H; ++k) {
-      at[k] = lo_b[k];
-      if (pass > 0 && lo_count[k] > ctx->spill) {
-        at[k] = lo_b[k] + (hi_b[k] - lo_b[k]) / 2;
-        probing = true;
-      }
-      thr[k] = value_of(at[k]);
-    }
-    if ((st = enqueue_hsum(ctx, s, part, thr.data())) != FDAS_OK) return st;
-    HIPCK(ctx, hipMemcpyAsync(s.h_counts, s.counts, sizeof(uint32_t) * H, hipMemcpyDeviceToHost, s.stream));
-    HIPCK(ctx, hipStreamSynchronize(s.stream));
-    bool all_fit = true;
-    for (uint32_t k = 0; k < H; ++k) {
-      const uint32_t c = s.h_counts[k];
-      if (pass == 0 || at[k] != lo_b[k]) {
-        if (c >= want) {
-          lo_b[k] = at[k];
-          lo_count[k] = c;
-        } else {
-          hi_b[k] = at[k];
-        }
-      }
-      if (lo_count[k] > ctx->spill) {
-        all_fit = false;
-        if (hi_b[k] - lo_b[k] <= 1)
-          return fail(ctx, FDAS_EOVERFLOW, "plane %u: %u values tie at the quantile, beyond the spill capacity %u",
-                      k + 1, lo_count[k], ctx->spill);
-      }
-    }
-    if (all_fit) break;
-  }
-  if (probing) {  // the spill lists hold a probe's entries: spill once more at the final thresholds
-    for (uint32_t k = 0; k < H; ++k) thr[k] = value_of(lo_b[k]);
-    if ((st = enqueue_hsum(ctx, s, part, thr.data())) != FDAS_OK) return st;
-    HIPCK(ctx, hipMemcpyAsync(s.h_counts, s.counts, sizeof(uint32_t) * H, hipMemcpyDeviceToHost, s.stream));
-    HIPCK(ctx, hipStreamSynchronize(s.stream));
-  }
-  s.cands_valid = false;  // the lists now belong to these thresholds, not to a search
+  fdas_status st;
+  const size_t most = size_t(H) * hmax_blocks(N, ctx->cfg.n_templates);
+  if (!s.quant && (st = dev_alloc(ctx, &s.quant, most + 4 * H)) != FDAS_OK) return st;
+  if (!s.h_quant && (st = host_alloc(ctx, &s.h_quant, 4 * H)) != FDAS_OK) return st;
+  float* d_thr = s.quant + most;                                  // [H] bounds
+  uint32_t* d_rank = reinterpret_cast<uint32_t*>(d_thr + H);      // [3H] counts, order statistics
+  const float* h_thr = reinterpret_cast<const float*>(s.h_quant);
+  const uint32_t* h_rank = s.h_quant + H;
   const double q = 1.0 - double(n_per_plane) / double(M);
   const double vi = q * double(M - 1);
   const uint64_t below = uint64_t(std::floor(vi));  // ascending rank of the lower order statistic
   const double g = vi - double(below);
+  // descending ranks of the two order statistics
+  const uint64_t r_lo = M - 1 - below, r_hi = below + 1 < M ? M - 2 - below : r_lo;
+  const uint64_t want = std::min<uint64_t>(uint64_t(n_per_plane) + 2, M);  // a spare rank for rounding
+  // One summing pass over the staged jobs and the order statistics of its spill.
+  auto spill_pass = [&]() -> fdas_status {
+    fdas_status r = run_hsum(ctx, s);
+    if (r != FDAS_OK) return r;
+    HIPCK(ctx, launch_quantile_rank(s.d_sel, H, uint32_t(r_lo), uint32_t(r_hi), d_rank, s.stream));
+    HIPCK(ctx, hipMemcpyAsync(s.h_quant, d_thr, sizeof(uint32_t) * 4 * H, hipMemcpyDeviceToHost, s.stream));
+    HIPCK(ctx, hipStreamSynchronize(s.stream));
+    return FDAS_OK;
+  };
+  s.cands_valid = false;  // the lists will belong to these thresholds, not to a search
+  std::vector<float> thr(H, -INFINITY);
+  if ((st = stage_hsum(ctx, s, part, thr.data())) != FDAS_OK) return st;
+  const uint32_t nb = hmax_blocks(N, nr);
+  HIPCK(ctx, launch_hmax(s.fop, N, ctx->cfg.n_templates, rb, nr, H, s.quant, s.stream));
+  HIPCK(ctx, launch_quantile_bound(s.quant, nb, uint32_t(std::min<uint64_t>(want, UINT32_MAX)), H, s.d_hsum, s.d_sel,
+                                   d_thr, s.stream));
+  if ((st = spill_pass()) != FDAS_OK) return st;
+  bool all_fit = true;
+  for (uint32_t k = 0; k < H; ++k) all_fit = all_fit && h_rank[k] <= ctx->spill;
+  if (!all_fit) {
+    // A threshold per plane with count(HP_k > t) >= want that fits the spill lists: the
+    // planes that overflow are bisected over the bit patterns of non-negative floats,
+    // where each pass counts all planes.
+    auto value_of = [](int64_t b) { return b < 0 ? -INFINITY : __builtin_bit_cast(float, uint32_t(b)); };
+    std::vector<int64_t> lo_b(H), hi_b(H, 0x7f800000);  // count(> lo) >= want, count(> hi) < want
+    std::vector<uint32_t> lo_count(h_rank, h_rank + H);
+    for (uint32_t k = 0; k < H; ++k) lo_b[k] = h_thr[k] < 0.f ? -1 : int64_t(__builtin_bit_cast(uint32_t, h_thr[k]));
+    for (;;) {
+      bool fit = true;
+      std::vector<int64_t> at(lo_b);
+      for (uint32_t k = 0; k < H; ++k) {
+        if (lo_count[k] > ctx->spill) {
+          fit = false;
+          if (hi_b[k] - lo_b[k] <= 1)
+            return fail(ctx, FDAS_EOVERFLOW, "plane %u: %u values tie at the quantile, beyond the spill capacity %u",
+                        k + 1, lo_count[k], ctx->spill);
+          at[k] = lo_b[k] + (hi_b[k] - lo_b[k]) / 2;
+        }
+        thr[k] = value_of(at[k]);
+      }
+      // the last pass spills at the final thresholds
+      if ((st = stage_hsum(ctx, s, part, thr.data())) != FDAS_OK) return st;
+      if ((st = spill_pass()) != FDAS_OK) return st;
+      if (fit) break;
+      for (uint32_t k = 0; k < H; ++k) {
+        if (at[k] == lo_b[k]) continue;
+        if (h_rank[k] >= want) {
+          lo_b[k] = at[k];
+          lo_count[k] = h_rank[k];
+        } else {
+          hi_b[k] = at[k];
+        }
+      }
+    }
+  }
   for (uint32_t k = 0; k < H; ++k) {
-    const uint32_t c = s.h_counts[k];
+    const uint32_t c = h_rank[k];
     if (c > ctx->spill)
       return fail(ctx, FDAS_EOVERFLOW, "plane %u: %u values above the bound exceed the spill capacity %u", k + 1, c,
                   ctx->spill);
-    std::vector<float> p(c);
-    if (c) HIPCK(ctx, hipMemcpy(p.data(), s.spill_pwr + size_t(k) * ctx->spill, sizeof(float) * c,
-                                hipMemcpyDeviceToHost));
-    // descending ranks of the two order statistics
-    const uint64_t r_lo = M - 1 - below, r_hi = below + 1 < M ? M - 2 - below : r_lo;
     if (r_lo >= c) return fail(ctx, FDAS_EDEVICE, "plane %u: only %u values spilled, need %llu", k + 1, c,
                                (unsigned long long)(r_lo + 1));
-    std::sort(p.begin(), p.end(), std::greater<float>());
-    const double lo = p[r_lo], hi = p[r_hi];
+    const double lo = __builtin_bit_cast(float, h_rank[H + k]), hi = __builtin_bit_cast(float, h_rank[2 * H + k]);
     thresholds[k] = float(lo * (1.0 - g) + hi * g);
   }
   return FDAS_OK;

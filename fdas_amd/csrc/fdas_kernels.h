@@ -57,6 +57,16 @@ uint32_t hmax_blocks(uint32_t n_bins, uint32_t n_rows);
 hipError_t launch_hmax(const float* fop, uint32_t n_bins, uint32_t n_templates, uint32_t row_begin, uint32_t n_rows,
                        uint32_t n_harmonics, float* out, hipStream_t stream);
 
+// The quantile thresholds' order statistics.  launch_quantile_bound sets the
+// thresholds of a summing job (and its n_harmonics selection jobs, and thr_out[H])
+// to bounds that `want` values of each plane lie above, from its nb block maxima;
+// launch_quantile_rank reads the planes' spill lists: out[3H] = detections, value
+// bits at descending rank r_lo, at r_hi.
+hipError_t launch_quantile_bound(const float* maxima, uint32_t nb, uint32_t want, uint32_t n_harmonics,
+                                 HsumJob* d_hsum, SelectJob* d_sel, float* thr_out, hipStream_t stream);
+hipError_t launch_quantile_rank(const SelectJob* d_sel, uint32_t n_harmonics, uint32_t r_lo, uint32_t r_hi,
+                                uint32_t* out, hipStream_t stream);
+
 hipError_t launch_zero_u32(uint32_t* p, uint32_t n, hipStream_t stream);
 
 // One launch running both the FT convolution of ftc_jobs (1024-point tiles)

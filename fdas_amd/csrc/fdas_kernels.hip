@@ -764,57 +764,125 @@ hipError_t launch_hplane(const float* fop, uint32_t n_bins, uint32_t n_templates
   return hipGetLastError();
 }
 
-// Largest HP_k, k = 1..n_harmonics, of each block of 256 bins x kHmaxRows rows of
-// rows [row_begin, row_begin + n_rows): out[k-1][block], block = y * gridDim.x + x.
-// HP_k is summed in FP32 in k order, as in hsum_kernel, so the values are the
-// ones the summing kernel thresholds.
+// Largest HP_k, k = 1..H, of each block of 256 bins x kHmaxRows rows of rows
+// [row_begin, row_begin + n_rows): out[k-1][block], block = row group * bin
+// blocks + bin block.  HP_k is summed in FP32 in k order, as in hsum_kernel, so
+// the values are the ones the summing kernel thresholds.
+//
+// Bound like the summing kernel, whose loads and sums it uses: a workgroup takes
+// 2048 bins, a thread 8 of them, with a maximum per plane in registers.  (One
+// bin per thread and a run-time number of planes took 215 us per 2^18 bins x 85
+// rows x 8 planes; this takes 30.)
 constexpr uint32_t kHmaxRows = 8;
+constexpr uint32_t kHmaxBins = 256;
 
-__global__ __launch_bounds__(256) void hmax_kernel(const float* __restrict__ fop, uint32_t n_bins,
-                                                   uint32_t n_templates, uint32_t row_begin, uint32_t n_rows,
-                                                   uint32_t n_harmonics, float* __restrict__ out) {
-  __shared__ float red[kMaxHarmonics][256 / 64];
-  const uint32_t f = blockIdx.x * 256u + threadIdx.x;
+template <int H>
+__global__ __launch_bounds__(kHsumThreads) void hmax_kernel(const float* __restrict__ fop, uint32_t n_bins,
+                                                            uint32_t n_templates, uint32_t row_begin, uint32_t n_rows,
+                                                            float* __restrict__ out) {
+  constexpr uint32_t kBlocks = uint32_t(kHsumBinsPerBlock) / kHmaxBins;  // per workgroup
+  __shared__ uint32_t red[H][kBlocks];                                   // order keys
+  const uint32_t tid = threadIdx.x, block_f0 = blockIdx.x * uint32_t(kHsumBinsPerBlock);
   const uint32_t r0 = row_begin + blockIdx.y * kHmaxRows;
-  const uint32_t r1 = min(r0 + kHmaxRows, row_begin + n_rows);
+  const uint32_t r_last = min(r0 + kHmaxRows, row_begin + n_rows) - 1;
   const int c = int(n_templates / 2);
-  float mx[kMaxHarmonics];
-  for (uint32_t k = 0; k < kMaxHarmonics; ++k) mx[k] = -INFINITY;
-  if (f < n_bins) {
-    for (uint32_t r = r0; r < r1; ++r) {
-      const int t = int(r) - c;
-      float hp = gld(fop, size_t(r) * n_bins + f);
-      mx[0] = fmaxf(mx[0], hp);
-      for (uint32_t k = 2; k <= n_harmonics; ++k) {
-        hp += gld(fop, size_t(c + t / int(k)) * n_bins + f / k);
-        mx[k - 1] = fmaxf(mx[k - 1], hp);
+  for (uint32_t i = tid; i < H * kBlocks; i += kHsumThreads)
+    (&red[0][0])[i] = order_key(__float_as_uint(-INFINITY));
+  __syncthreads();
+  // One bin of one row (the bins that the 16-byte loads cannot cover, as in hsum_block).
+  auto one_bin = [&](uint32_t r, uint32_t f) {
+    const int t = int(r) - c;
+    float hp = gld(fop, size_t(r) * n_bins + f);
+#pragma unroll
+    for (int k = 1; k <= H; ++k) {
+      if (k > 1) hp += gld(fop, size_t(c + t / k) * n_bins + f / uint32_t(k));
+      atomicMax(&red[k - 1][(f - block_f0) / kHmaxBins], order_key(__float_as_uint(fmaxf(-INFINITY, hp))));
+    }
+  };
+  if (n_bins < uint32_t(kHsumBinsPerThread)) {
+    if (tid < n_bins)
+      for (uint32_t r = r0; r <= r_last; ++r) one_bin(r, tid);
+  } else {
+    constexpr uint32_t kWaveBins = 64u * kHsumBinsPerThread;
+    const uint32_t tail_f0 = (n_bins - 1u) / kWaveBins * kWaveBins;
+    const bool apart =
+        n_bins % 8u != 0 && r_last + 1u == n_templates && tail_f0 - block_f0 < uint32_t(kHsumBinsPerBlock);
+    if (apart)
+      for (uint32_t f = tail_f0 + tid; f < min(tail_f0 + kWaveBins, n_bins); f += kHsumThreads) one_bin(r_last, f);
+    const uint32_t f0 = block_f0 + tid * uint32_t(kHsumBinsPerThread);
+    const uint32_t fl = min(f0, (n_bins - 1u) & ~7u);
+    const uint32_t live = f0 < n_bins ? min(n_bins - f0, 8u) : 0u;  // bins of this thread in the row
+    const uint32_t r_stop = apart && __ballot(fl + 8u > n_bins) != 0 ? r_last - 1u : r_last;
+    float mx[H];
+    uint32_t rk[H];
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+      mx[k] = -INFINITY;
+      rk[k] = fl % uint32_t(k + 1);
+    }
+    if (int(r0) <= int(r_stop)) {
+      RowLoads<H> a, b;
+      auto row_max = [&](const RowLoads<H>& L) {
+        float hp[kHsumBinsPerThread];
+#pragma unroll
+        for (int i = 0; i < kHsumBinsPerThread; ++i) hp[i] = uint32_t(i) < live ? L.m[i] : -INFINITY;
+#pragma unroll
+        for (int k = 1; k <= H; ++k) {
+          if (k > 1) hsum_add_k<H>(k, hp, L, rk);
+#pragma unroll
+          for (int i = 0; i < kHsumBinsPerThread; ++i) mx[k - 1] = fmaxf(mx[k - 1], hp[i]);
+        }
+      };
+      hsum_load_row<H>(a, fop, n_bins, c, r0, fl);
+      for (uint32_t r = r0;; r += 2) {
+        hsum_load_row<H>(b, fop, n_bins, c, min(r + 1, r_stop), fl);
+        row_max(a);
+        if (r + 1 > r_stop) break;
+        hsum_load_row<H>(a, fop, n_bins, c, min(r + 2, r_stop), fl);
+        row_max(b);
+        if (r + 2 > r_stop) break;
       }
     }
-  }
-  const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
-  for (uint32_t k = 0; k < n_harmonics; ++k) {
-    float v = mx[k];
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-    if (lane == 0) red[k][wave] = v;
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+      float v = mx[k];
+#pragma unroll
+      for (int o = 16; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
+      if ((tid & 31u) == 0) atomicMax(&red[k][tid / 32u], order_key(__float_as_uint(v)));
+    }
   }
   __syncthreads();
-  if (threadIdx.x < n_harmonics) {
-    const uint32_t k = threadIdx.x;
-    const float v = fmaxf(fmaxf(red[k][0], red[k][1]), fmaxf(red[k][2], red[k][3]));
-    gst(out, size_t(k) * (gridDim.x * gridDim.y) + blockIdx.y * gridDim.x + blockIdx.x, v);
+  const uint32_t bx = (n_bins + kHmaxBins - 1) / kHmaxBins, first = blockIdx.x * kBlocks;
+  const size_t nb = size_t(bx) * gridDim.y;
+  for (uint32_t i = tid; i < H * kBlocks; i += kHsumThreads) {
+    const uint32_t k = i / kBlocks, x = first + i % kBlocks;
+    if (x < bx) gst(out, k * nb + size_t(blockIdx.y) * bx + x, __uint_as_float(order_key_inv(red[k][i % kBlocks])));
   }
 }
 
 uint32_t hmax_blocks(uint32_t n_bins, uint32_t n_rows) {
-  return (n_bins + 255) / 256 * ((n_rows + kHmaxRows - 1) / kHmaxRows);
+  return (n_bins + kHmaxBins - 1) / kHmaxBins * ((n_rows + kHmaxRows - 1) / kHmaxRows);
+}
+
+template <int H = 1>
+static bool launch_hmax_h(uint32_t n_harmonics, dim3 grid, hipStream_t stream, const float* fop, uint32_t n_bins,
+                          uint32_t n_templates, uint32_t row_begin, uint32_t n_rows, float* out) {
+  if constexpr (H <= int(kMaxHarmonics)) {
+    if (n_harmonics != uint32_t(H))
+      return launch_hmax_h<H + 1>(n_harmonics, grid, stream, fop, n_bins, n_templates, row_begin, n_rows, out);
+    hipLaunchKernelGGL(hmax_kernel<H>, grid, dim3(kHsumThreads), 0, stream, fop, n_bins, n_templates, row_begin,
+                       n_rows, out);
+    return true;
+  }
+  return false;
 }
 
 hipError_t launch_hmax(const float* fop, uint32_t n_bins, uint32_t n_templates, uint32_t row_begin, uint32_t n_rows,
                        uint32_t n_harmonics, float* out, hipStream_t stream) {
   if (n_rows == 0 || n_bins == 0) return hipSuccess;
-  dim3 grid((n_bins + 255) / 256, (n_rows + kHmaxRows - 1) / kHmaxRows);
-  hipLaunchKernelGGL(hmax_kernel, grid, dim3(256), 0, stream, fop, n_bins, n_templates, row_begin, n_rows,
-                     n_harmonics, out);
+  dim3 grid((n_bins + kHsumBinsPerBlock - 1) / kHsumBinsPerBlock, (n_rows + kHmaxRows - 1) / kHmaxRows);
+  if (!launch_hmax_h(n_harmonics, grid, stream, fop, n_bins, n_templates, row_begin, n_rows, out))
+    return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
@@ -1022,9 +1090,13 @@ __device__ void radix_pass(Shared& sh, uint32_t n, Get get, uint32_t shift, uint
   const uint32_t nb = 1u << width;
   for (uint32_t i = tid; i < 2048; i += THREADS) sh.hist[i] = 0;
   __syncthreads();
-  for (uint32_t e = tid; e < n; e += THREADS) {
-    const uint32_t v = get(e);
-    if ((v & mask) == prefix) atomicAdd(&sh.hist[(v >> shift) & (nb - 1)], 1u);
+  for (uint32_t e0 = tid; e0 < n; e0 += 4 * THREADS) {
+    uint32_t v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = get(min(e0 + uint32_t(u * THREADS), n - 1u));
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (e0 + uint32_t(u * THREADS) < n && (v[u] & mask) == prefix) atomicAdd(&sh.hist[(v[u] >> shift) & (nb - 1)], 1u);
   }
   __syncthreads();
   // Thread t owns ordered positions u = PER t .. PER t + PER - 1 (u counts from the selected end).
@@ -1348,6 +1420,116 @@ __global__ __launch_bounds__(THREADS) void select_final_kernel(const SelectJob* 
     gst(job.out_pwr, e, sh.pwr[e]);
   }
   if (tid == 0) gst(job.out_n, 0, kept);
+}
+
+// ---------------------------------------------------------------------------
+// Quantile thresholds: order statistics of a plane
+// ---------------------------------------------------------------------------
+
+constexpr int kRankThreads = 1024;
+struct RankShared {
+  uint32_t hist[2048];
+  uint32_t waves[kRankThreads / 64];
+  uint32_t misc[8];
+};
+
+// The rank-th largest (1 = largest) of the order keys get(0) .. get(n-1), 1 <= rank <= n:
+// a radix select from the highest bit in which the keys differ, 11 bits a pass
+// (from the sign on, most keys would share their first digit, and its counter).
+template <typename Get>
+__device__ uint32_t radix_rank(RankShared& sh, uint32_t n, Get get, uint32_t rank) {
+  const uint32_t tid = threadIdx.x;
+  __syncthreads();  // earlier readers of sh are done
+  if (tid == 0) {
+    sh.misc[4] = 0;
+    sh.misc[5] = 0xffffffffu;
+  }
+  __syncthreads();
+  uint32_t any = 0, all = 0xffffffffu;
+  for (uint32_t e0 = tid; e0 < n; e0 += 4 * kRankThreads) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const uint32_t v = get(min(e0 + uint32_t(u * kRankThreads), n - 1u));
+      any |= v;
+      all &= v;
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    any |= __shfl_xor(any, o);
+    all &= __shfl_xor(all, o);
+  }
+  if (lane_id() == 0) {
+    atomicOr(&sh.misc[4], any);
+    atomicAnd(&sh.misc[5], all);
+  }
+  __syncthreads();
+  const uint32_t same = sh.misc[5], differ = sh.misc[4] ^ same;
+  __syncthreads();
+  if (differ == 0) return same;
+  uint32_t bits = 32u - uint32_t(__builtin_clz(differ));  // low bits still open
+  uint32_t mask = bits < 32u ? ~0u << bits : 0u, prefix = same & mask;
+  while (bits > 0) {
+    const uint32_t width = min(bits, 11u);
+    bits -= width;
+    radix_pass<true, kRankThreads>(sh, n, get, bits, width, prefix, mask, rank);
+  }
+  return prefix;
+}
+
+// thr_k just below the want-th largest of plane k's nb block maxima, or -inf when
+// there are fewer blocks or that value is not positive: at least `want` values
+// of the plane lie above it.  Written into the jobs of the summing pass that follows.
+__global__ __launch_bounds__(kRankThreads) void quantile_bound_kernel(const float* __restrict__ maxima, uint32_t nb,
+                                                                      uint32_t want, HsumJob* hsum, SelectJob* sel,
+                                                                      float* thr_out) {
+  __shared__ RankShared sh;
+  const uint32_t k = blockIdx.x;
+  float thr = -INFINITY;
+  if (nb >= want) {
+    auto key = [&](uint32_t e) { return order_key(__float_as_uint(gld(maxima, size_t(k) * nb + e))); };
+    const uint32_t v = order_key_inv(radix_rank(sh, nb, key, want));
+    if (v != 0 && (v & 0x80000000u) == 0) thr = __uint_as_float(v - 1u);
+  }
+  if (threadIdx.x == 0) {
+    hsum->thr[k] = thr;
+    sel[k].thr = thr;
+    thr_out[k] = thr;
+  }
+}
+
+// out = counts[H], then the values at the 0-based descending ranks r_lo and r_hi of
+// each plane's spilled powers (0 where the spill list does not hold the rank, or overflowed).
+__global__ __launch_bounds__(kRankThreads) void quantile_rank_kernel(const SelectJob* __restrict__ jobs, uint32_t r_lo,
+                                                                     uint32_t r_hi, uint32_t* __restrict__ out) {
+  __shared__ RankShared sh;
+  const uint32_t k = blockIdx.x, H = gridDim.x;
+  const SelectJob& job = jobs[k];
+  const uint32_t n = gld(job.count, 0);
+  uint32_t lo = 0, hi = 0;
+  if (n <= job.spill_cap && r_lo < n && r_hi < n) {
+    auto key = [&](uint32_t e) { return order_key(__float_as_uint(gld(job.spill_pwr, e))); };
+    lo = order_key_inv(radix_rank(sh, n, key, r_lo + 1));
+    hi = r_hi == r_lo ? lo : order_key_inv(radix_rank(sh, n, key, r_hi + 1));
+  }
+  if (threadIdx.x == 0) {
+    gst(out, k, n);
+    gst(out, H + k, lo);
+    gst(out, 2 * H + k, hi);
+  }
+}
+
+hipError_t launch_quantile_bound(const float* maxima, uint32_t nb, uint32_t want, uint32_t n_harmonics, HsumJob* d_hsum,
+                                 SelectJob* d_sel, float* thr_out, hipStream_t stream) {
+  hipLaunchKernelGGL(quantile_bound_kernel, dim3(n_harmonics), dim3(kRankThreads), 0, stream, maxima, nb, want, d_hsum,
+                     d_sel, thr_out);
+  return hipGetLastError();
+}
+
+hipError_t launch_quantile_rank(const SelectJob* d_sel, uint32_t n_harmonics, uint32_t r_lo, uint32_t r_hi,
+                                uint32_t* out, hipStream_t stream) {
+  hipLaunchKernelGGL(quantile_rank_kernel, dim3(n_harmonics), dim3(kRankThreads), 0, stream, d_sel, r_lo, r_hi, out);
+  return hipGetLastError();
 }
 
 hipError_t launch_select(const SelectJob* d_jobs, uint32_t n_jobs, uint32_t cap, hipStream_t stream) {
