@@ -42,36 +42,36 @@ struct DevSet {
   float* plane = nullptr;
   uint32_t* spill_key = nullptr;
   float* spill_pwr = nullptr;
+  // One allocation, read back from its start: lists (keys, powers), kept entries, detections;
+  // zeroed before each summing pass from `counts` on: detections, compact counts, histograms.
+  uint32_t* out_key = nullptr;     // [H][cap]
+  float* out_pwr = nullptr;        // [H][cap]
+  uint32_t* out_n = nullptr;       // [H]
   uint32_t* counts = nullptr;      // [H] detections, then [H] compact counts, then [H][kSelectBins] histograms
   uint32_t* compact_key = nullptr;
   float* compact_pwr = nullptr;
-  uint32_t* out_key = nullptr;
-  float* out_pwr = nullptr;
-  uint32_t* out_n = nullptr;
   FtcJob* d_ftc = nullptr;
   HsumJob* d_hsum = nullptr;
   SelectJob* d_sel = nullptr;
   float* quant = nullptr;          // quantile thresholds: block maxima, then [4H] thresholds, counts, order statistics
 
-  FtcJob* h_ftc = nullptr;
-  HsumJob* h_hsum = nullptr;
-  SelectJob* h_sel = nullptr;
-  uint32_t* h_out_key = nullptr;
+  FtcJob* h_ftc = nullptr;         // pinned staging of more than kPackFtcJobs row groups
+  JobPack pack;                    // the launches' job descriptors
+  uint32_t* h_out_key = nullptr;   // pinned mirror of the lists, kept entries and detections (one allocation)
   float* h_out_pwr = nullptr;
   uint32_t* h_out_n = nullptr;
   uint32_t* h_counts = nullptr;
+  bool lists_on_host = false;      // the mirror holds (or, in stream order, will hold) the last pass's lists
   uint32_t* h_quant = nullptr;     // [4H] mirror of quant's tail
 
   hipStream_t stream = nullptr;
   hipEvent_t ev[EV_COUNT] = {};
   hipEvent_t staged_ftc = nullptr;   // h_ftc may be rewritten once this completes
-  hipEvent_t staged_hsum = nullptr;  // h_hsum / h_sel may be rewritten once this completes
-  hipEvent_t hsum_done = nullptr;    // the set's last harmonic-summing kernel has finished
-  bool hsum_issued = false;          // hsum_done has been recorded at least once
+  bool hsum_issued = false;          // a harmonic-summing kernel (its end: ev[EV_HSUM_K1]) has been launched
   bool ftc_pending = false;
-  bool hsum_pending = false;
   bool ev_recorded[EV_COUNT] = {};
 
+  std::vector<FtcJob> ftc_plan[3];  // convolution jobs per part (empty: not planned for these templates)
   std::vector<uint32_t> row_taps;  // non-zero extent of each template row (sets per-group overlaps)
   bool templates = false;
   bool has_input = false;
@@ -206,9 +206,25 @@ fdas_status record(fdas_ctx* ctx, DevSet& s, Ev e) {
   return FDAS_OK;
 }
 
-std::vector<FtcJob> plan_ftc_jobs(const fdas_ctx* ctx, const DevSet& s, uint32_t rb, uint32_t nr) {
-  std::vector<FtcJob> jobs = plan_ftc_rows(ctx->cfg.tile, ctx->geo.n_bins, ctx->cfg.max_taps, s.row_taps, rb, nr,
-                                           kMaxFtcJobs);
+float elapsed(const DevSet& s, int a, int b) {
+  if (!s.ev_recorded[a] || !s.ev_recorded[b]) return 0.f;
+  float ms = 0.f;
+  if (hipEventElapsedTime(&ms, s.ev[a], s.ev[b]) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0.f;
+  }
+  return ms;
+}
+
+// The convolution jobs of the part.  Planned once per part and template bank: the
+// row grouping (a dynamic program over the rows, about 35 us on the host for 85) depends on
+// nothing else that changes between launches.
+const std::vector<FtcJob>& ftc_jobs(const fdas_ctx* ctx, DevSet& s, fdas_part part) {
+  std::vector<FtcJob>& jobs = s.ftc_plan[part];
+  if (!jobs.empty()) return jobs;
+  uint32_t rb, nr;
+  part_rows(ctx, part, &rb, &nr);
+  jobs = plan_ftc_rows(ctx->cfg.tile, ctx->geo.n_bins, ctx->cfg.max_taps, s.row_taps, rb, nr, kMaxFtcJobs);
   fit_ftc_items(jobs, ftconv_slots(ctx->cfg.tile));
   uint32_t item = 0;
   for (FtcJob& j : jobs) {
@@ -221,37 +237,33 @@ std::vector<FtcJob> plan_ftc_jobs(const fdas_ctx* ctx, const DevSet& s, uint32_t
   return jobs;
 }
 
-fdas_status enqueue_ftc(fdas_ctx* ctx, DevSet& s, fdas_part part) {
-  uint32_t rb, nr;
-  part_rows(ctx, part, &rb, &nr);
-  fdas_status st = wait_staging(ctx, s.staged_ftc, s.ftc_pending);
+// The convolution jobs of the part into the pack (or, beyond its size, the pinned staging array).
+// Returns the work items; *n_jobs = jobs.
+fdas_status fill_ftc(fdas_ctx* ctx, DevSet& s, fdas_part part, uint32_t* n_jobs, uint32_t* n_items) {
+  const std::vector<FtcJob>& jobs = ftc_jobs(ctx, s, part);
+  *n_jobs = uint32_t(jobs.size());
+  *n_items = jobs.back().item_begin + jobs.back().n_tiles * jobs.back().n_chunks;
+  s.pack.n_ftc = 0;
+  if (jobs.size() <= kPackFtcJobs) {
+    std::copy(jobs.begin(), jobs.end(), s.pack.ftc);
+    s.pack.n_ftc = *n_jobs;
+    return FDAS_OK;
+  }
+  const fdas_status st = wait_staging(ctx, s.staged_ftc, s.ftc_pending);
   if (st != FDAS_OK) return st;
-  const std::vector<FtcJob> jobs = plan_ftc_jobs(ctx, s, rb, nr);
   std::copy(jobs.begin(), jobs.end(), s.h_ftc);
-  const uint32_t n_items = jobs.back().item_begin + jobs.back().n_tiles * jobs.back().n_chunks;
   HIPCK(ctx, hipMemcpyAsync(s.d_ftc, s.h_ftc, sizeof(FtcJob) * jobs.size(), hipMemcpyHostToDevice, s.stream));
   HIPCK(ctx, hipEventRecord(s.staged_ftc, s.stream));
   s.ftc_pending = true;
-  // The two sets' kernels take turns: this convolution starts once the other
-  // set's last summing kernel has finished (both kinds of kernel are VALU-bound,
-  // and side by side they only slow each other down), while that set's
-  // selection and read-back, and this set's input copy, still overlap.
-  const DevSet& other = &s == &ctx->set[0] ? ctx->set[1] : ctx->set[0];
-  if (other.hsum_issued) HIPCK(ctx, hipStreamWaitEvent(s.stream, other.hsum_done, 0));
-  if ((st = record(ctx, s, EV_FTC_K)) != FDAS_OK) return st;
-  HIPCK(ctx, launch_ftconv(int(ctx->cfg.tile), s.d_ftc, uint32_t(jobs.size()), n_items, ctx->tw1, ctx->tw2,
-                           n_items, s.stream));
   return FDAS_OK;
 }
 
-// Job descriptors of a summing pass over the part, on their way to the device.
-fdas_status stage_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr) {
+// The summing and selection jobs of a pass over the part into the pack.
+void fill_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr) {
   uint32_t rb, nr;
   part_rows(ctx, part, &rb, &nr);
   const uint32_t H = ctx->cfg.n_harmonics;
-  fdas_status st = wait_staging(ctx, s.staged_hsum, s.hsum_pending);
-  if (st != FDAS_OK) return st;
-  HsumJob& j = *s.h_hsum;
+  HsumJob& j = s.pack.hsum;
   j = HsumJob{};
   j.fop = s.fop;
   j.n_bins = ctx->geo.n_bins;
@@ -268,7 +280,7 @@ fdas_status stage_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* th
   for (uint32_t k = 0; k < H; ++k) j.thr[k] = thr[k];
   const uint32_t cap = ctx->cfg.cands_per_harmonic, ccap = cap + kSelectPool;
   for (uint32_t p = 0; p < H; ++p) {
-    SelectJob& q = s.h_sel[p];
+    SelectJob& q = s.pack.sel[p];
     q.spill_key = s.spill_key + size_t(p) * ctx->spill;
     q.spill_pwr = s.spill_pwr + size_t(p) * ctx->spill;
     q.count = s.counts + p;
@@ -284,40 +296,84 @@ fdas_status stage_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* th
     q.out_pwr = s.out_pwr + size_t(p) * cap;
     q.out_n = s.out_n + p;
   }
-  HIPCK(ctx, hipMemcpyAsync(s.d_hsum, s.h_hsum, sizeof(HsumJob), hipMemcpyHostToDevice, s.stream));
-  HIPCK(ctx, hipMemcpyAsync(s.d_sel, s.h_sel, sizeof(SelectJob) * H, hipMemcpyHostToDevice, s.stream));
-  HIPCK(ctx, hipEventRecord(s.staged_hsum, s.stream));
-  s.hsum_pending = true;
+  s.pack.n_sel = H;
+}
+
+// Takes the pack's jobs to the device, with the counters cleared when a summing pass is among them.
+fdas_status put_jobs(fdas_ctx* ctx, DevSet& s) {
+  ZeroSpan zero;
+  if (s.pack.n_sel) zero = {s.counts, ctx->cfg.n_harmonics * (2 + kSelectBins)};
+  HIPCK(ctx, launch_put_jobs(s.pack, s.d_ftc, s.d_hsum, s.d_sel, zero, {}, s.stream));
+  s.pack.n_ftc = s.pack.n_sel = 0;
   return FDAS_OK;
 }
 
-// The summing and selection kernels of the staged jobs.
+fdas_status run_ftc(fdas_ctx* ctx, DevSet& s, uint32_t n_jobs, uint32_t n_items) {
+  // The two sets' kernels take turns: this convolution starts once the other
+  // set's last summing kernel has finished (both kinds of kernel are VALU-bound,
+  // and side by side they only slow each other down), while that set's
+  // selection and read-back, and this set's input copy, still overlap.
+  const DevSet& other = &s == &ctx->set[0] ? ctx->set[1] : ctx->set[0];
+  if (other.hsum_issued) HIPCK(ctx, hipStreamWaitEvent(s.stream, other.ev[EV_HSUM_K1], 0));
+  HIPCK(ctx, launch_ftconv(int(ctx->cfg.tile), s.d_ftc, n_jobs, n_items, ctx->tw1, ctx->tw2, n_items, s.stream,
+                           {s.ev[EV_FTC_K], s.ev[EV_FTC]}));
+  s.ev_recorded[EV_FTC_K] = s.ev_recorded[EV_FTC] = true;
+  return FDAS_OK;
+}
+
+// The summing and selection kernels of the jobs on the device.
 fdas_status run_hsum(fdas_ctx* ctx, DevSet& s) {
   const uint32_t H = ctx->cfg.n_harmonics;
-  const HsumJob& j = *s.h_hsum;
-  fdas_status st;
-  HIPCK(ctx, launch_zero_u32(s.counts, H * (2 + kSelectBins), s.stream));
+  const HsumJob& j = s.pack.hsum;
+  s.lists_on_host = false;
   const uint32_t blocks = (ctx->geo.n_bins + kHsumBinsPerBlock - 1) / kHsumBinsPerBlock * j.n_row_chunks;
-  if ((st = record(ctx, s, EV_HSUM_K0)) != FDAS_OK) return st;
-  HIPCK(ctx, launch_hsum(s.d_hsum, 1, blocks, H, s.stream));
-  if ((st = record(ctx, s, EV_HSUM_K1)) != FDAS_OK) return st;
-  HIPCK(ctx, hipEventRecord(s.hsum_done, s.stream));
+  HIPCK(ctx, launch_hsum(s.d_hsum, 1, blocks, H, s.stream, {s.ev[EV_HSUM_K0], s.ev[EV_HSUM_K1]}));
   s.hsum_issued = true;
-  HIPCK(ctx, launch_select(s.d_sel, H, ctx->cfg.cands_per_harmonic, s.stream));
+  HIPCK(ctx, launch_select(s.d_sel, H, ctx->cfg.cands_per_harmonic, s.stream, s.ev[EV_HSUM]));
+  s.ev_recorded[EV_HSUM_K0] = s.ev_recorded[EV_HSUM_K1] = s.ev_recorded[EV_HSUM] = true;
   return FDAS_OK;
+}
+
+fdas_status enqueue_ftc(fdas_ctx* ctx, DevSet& s, fdas_part part) {
+  uint32_t n_jobs, n_items;
+  fdas_status st = fill_ftc(ctx, s, part, &n_jobs, &n_items);
+  if (st != FDAS_OK) return st;
+  if (s.pack.n_ftc && (st = put_jobs(ctx, s)) != FDAS_OK) return st;
+  return run_ftc(ctx, s, n_jobs, n_items);
 }
 
 fdas_status enqueue_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr) {
-  const fdas_status st = stage_hsum(ctx, s, part, thr);
+  fill_hsum(ctx, s, part, thr);
+  const fdas_status st = put_jobs(ctx, s);
   return st == FDAS_OK ? run_hsum(ctx, s) : st;
 }
 
+// Convolution and summing of one launch, their jobs taken to the device together.
+fdas_status enqueue_search(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr) {
+  uint32_t n_jobs, n_items;
+  fdas_status st = fill_ftc(ctx, s, part, &n_jobs, &n_items);
+  if (st != FDAS_OK) return st;
+  fill_hsum(ctx, s, part, thr);
+  if ((st = put_jobs(ctx, s)) != FDAS_OK) return st;
+  if ((st = run_ftc(ctx, s, n_jobs, n_items)) != FDAS_OK) return st;
+  return run_hsum(ctx, s);
+}
+
 fdas_status enqueue_readback(fdas_ctx* ctx, DevSet& s) {
-  const uint32_t H = ctx->cfg.n_harmonics, cap = ctx->cfg.cands_per_harmonic;
-  HIPCK(ctx, hipMemcpyAsync(s.h_out_key, s.out_key, sizeof(uint32_t) * H * cap, hipMemcpyDeviceToHost, s.stream));
-  HIPCK(ctx, hipMemcpyAsync(s.h_out_pwr, s.out_pwr, sizeof(float) * H * cap, hipMemcpyDeviceToHost, s.stream));
-  HIPCK(ctx, hipMemcpyAsync(s.h_out_n, s.out_n, sizeof(uint32_t) * H, hipMemcpyDeviceToHost, s.stream));
-  HIPCK(ctx, hipMemcpyAsync(s.h_counts, s.counts, sizeof(uint32_t) * H, hipMemcpyDeviceToHost, s.stream));
+  const size_t H = ctx->cfg.n_harmonics, cap = ctx->cfg.cands_per_harmonic;
+  HIPCK(ctx, hipMemcpyAsync(s.h_out_key, s.out_key, sizeof(uint32_t) * (2 * H * cap + 2 * H), hipMemcpyDeviceToHost,
+                            s.stream));
+  s.lists_on_host = true;
+  return FDAS_OK;
+}
+
+// The last pass's lists in the pinned mirror: copied unless that pass has read them back.
+fdas_status lists_to_host(fdas_ctx* ctx, DevSet& s) {
+  if (!s.lists_on_host) {
+    const fdas_status st = enqueue_readback(ctx, s);
+    if (st != FDAS_OK) return st;
+  }
+  HIPCK(ctx, hipStreamSynchronize(s.stream));
   return FDAS_OK;
 }
 
@@ -362,7 +418,6 @@ fdas_status flush_gated(fdas_ctx* ctx, int set) {
   s.gated = false;
   fdas_status st = enqueue_hsum(ctx, s, s.gated_part, s.gated_thr);
   if (st != FDAS_OK) return st;
-  if ((st = record(ctx, s, EV_HSUM)) != FDAS_OK) return st;
   if ((st = enqueue_readback(ctx, s)) != FDAS_OK) return st;
   return record(ctx, s, EV_XFER);
 }
@@ -375,29 +430,19 @@ void free_set(DevSet& s) {
   (void)hipFree(s.plane);
   (void)hipFree(s.spill_key);
   (void)hipFree(s.spill_pwr);
-  (void)hipFree(s.counts);
   (void)hipFree(s.compact_key);
   (void)hipFree(s.compact_pwr);
-  (void)hipFree(s.out_key);
-  (void)hipFree(s.out_pwr);
-  (void)hipFree(s.out_n);
+  (void)hipFree(s.out_key);  // and out_pwr, out_n, counts
   (void)hipFree(s.d_ftc);
   (void)hipFree(s.d_hsum);
   (void)hipFree(s.d_sel);
   (void)hipFree(s.quant);
   (void)hipHostFree(s.h_quant);
   (void)hipHostFree(s.h_ftc);
-  (void)hipHostFree(s.h_hsum);
-  (void)hipHostFree(s.h_sel);
-  (void)hipHostFree(s.h_out_key);
-  (void)hipHostFree(s.h_out_pwr);
-  (void)hipHostFree(s.h_out_n);
-  (void)hipHostFree(s.h_counts);
+  (void)hipHostFree(s.h_out_key);  // and h_out_pwr, h_out_n, h_counts
   for (auto& e : s.ev)
     if (e) (void)hipEventDestroy(e);
   if (s.staged_ftc) (void)hipEventDestroy(s.staged_ftc);
-  if (s.staged_hsum) (void)hipEventDestroy(s.staged_hsum);
-  if (s.hsum_done) (void)hipEventDestroy(s.hsum_done);
   if (s.stream) (void)hipStreamDestroy(s.stream);
   s = DevSet{};
 }
@@ -518,31 +563,27 @@ extern "C" fdas_status fdas_create(const fdas_config* cfg, fdas_log_fn log, void
     if ((st = dev_alloc(ctx, &s.fop, T * N)) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.spill_key, H * ctx->spill)) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.spill_pwr, H * ctx->spill)) != FDAS_OK) return bail(st);
-    if ((st = dev_alloc(ctx, &s.counts, H * (2 + kSelectBins))) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.compact_key, H * (cap + kSelectPool))) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.compact_pwr, H * (cap + kSelectPool))) != FDAS_OK) return bail(st);
-    if ((st = dev_alloc(ctx, &s.out_key, H * cap)) != FDAS_OK) return bail(st);
-    if ((st = dev_alloc(ctx, &s.out_pwr, H * cap)) != FDAS_OK) return bail(st);
-    if ((st = dev_alloc(ctx, &s.out_n, H)) != FDAS_OK) return bail(st);
+    if ((st = dev_alloc(ctx, &s.out_key, 2 * H * cap + H * (3 + kSelectBins))) != FDAS_OK) return bail(st);
+    s.out_pwr = reinterpret_cast<float*>(s.out_key + H * cap);
+    s.out_n = s.out_key + 2 * H * cap;
+    s.counts = s.out_n + H;
     if ((st = dev_alloc(ctx, &s.d_ftc, kMaxFtcJobs)) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.d_hsum, 1)) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.d_sel, H)) != FDAS_OK) return bail(st);
     if ((st = host_alloc(ctx, &s.h_ftc, kMaxFtcJobs)) != FDAS_OK) return bail(st);
-    if ((st = host_alloc(ctx, &s.h_hsum, 1)) != FDAS_OK) return bail(st);
-    if ((st = host_alloc(ctx, &s.h_sel, H)) != FDAS_OK) return bail(st);
-    if ((st = host_alloc(ctx, &s.h_out_key, H * cap)) != FDAS_OK) return bail(st);
-    if ((st = host_alloc(ctx, &s.h_out_pwr, H * cap)) != FDAS_OK) return bail(st);
-    if ((st = host_alloc(ctx, &s.h_out_n, H)) != FDAS_OK) return bail(st);
-    if ((st = host_alloc(ctx, &s.h_counts, H)) != FDAS_OK) return bail(st);
+    if ((st = host_alloc(ctx, &s.h_out_key, 2 * H * cap + 2 * H)) != FDAS_OK) return bail(st);
+    s.h_out_pwr = reinterpret_cast<float*>(s.h_out_key + H * cap);
+    s.h_out_n = s.h_out_key + 2 * H * cap;
+    s.h_counts = s.h_out_n + H;
     std::memset(s.h_out_n, 0, sizeof(uint32_t) * H);
     std::memset(s.h_counts, 0, sizeof(uint32_t) * H);
     if (hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) != hipSuccess)
       return bail(fail(ctx, FDAS_EDEVICE, "stream creation failed"));
     for (auto& ev : s.ev)
       if (hipEventCreate(&ev) != hipSuccess) return bail(fail(ctx, FDAS_EDEVICE, "event creation failed"));
-    if (hipEventCreateWithFlags(&s.staged_ftc, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&s.staged_hsum, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&s.hsum_done, hipEventDisableTiming) != hipSuccess)
+    if (hipEventCreateWithFlags(&s.staged_ftc, hipEventDisableTiming) != hipSuccess)
       return bail(fail(ctx, FDAS_EDEVICE, "event creation failed"));
     // a FOP that was never written reads as zeros
     if (hipMemset(s.fop, 0, T * N * sizeof(float)) != hipSuccess ||
@@ -596,6 +637,11 @@ static fdas_status upload_spectra(fdas_ctx* ctx, int set, const std::vector<std:
   return FDAS_OK;
 }
 
+static void set_row_taps(DevSet& s, const std::vector<uint32_t>& taps) {
+  s.row_taps = taps;
+  for (auto& plan : s.ftc_plan) plan.clear();
+}
+
 // Natural bin of entry i of a row stored in 4-parallel FFT order:
 // stored[4m + j] = natural[bitrev2(j) * S/4 + m] (tmpl-gen.py:145-153, ft_conv.py:185-194).
 static inline uint32_t p4_natural_index(uint32_t i, uint32_t S) {
@@ -608,7 +654,7 @@ extern "C" fdas_status fdas_upload_templates(fdas_ctx* ctx, const float* spectra
   CHECK_SET(ctx, set);
   if (!spectra_c64) return fail(ctx, FDAS_EINVAL, "null template pointer");
   // spectra do not reveal the tap extent exactly: every row uses the configured max_taps
-  ctx->set[set].row_taps.assign(ctx->cfg.n_templates, ctx->cfg.max_taps);
+  set_row_taps(ctx->set[set], std::vector<uint32_t>(ctx->cfg.n_templates, ctx->cfg.max_taps));
   const uint32_t S = ctx->cfg.tile, T = ctx->cfg.n_templates;
   const bool p4 = (ctx->cfg.flags & FDAS_FLAG_REFERENCE_FFT_ORDER) != 0;
   std::vector<std::complex<double>> spec(size_t(T) * S);
@@ -636,7 +682,7 @@ extern "C" fdas_status fdas_upload_template_taps(fdas_ctx* ctx, const float* tap
   std::vector<uint32_t> extent;
   const std::vector<std::complex<double>> spec = taps_to_spectra(taps_c64, T, n_taps, ctx->cfg.max_taps, S, extent);
   fdas_status st = upload_spectra(ctx, set, spec);
-  if (st == FDAS_OK) ctx->set[set].row_taps = extent;
+  if (st == FDAS_OK) set_row_taps(ctx->set[set], extent);
   return st;
 }
 
@@ -706,7 +752,6 @@ extern "C" fdas_status fdas_perform_ft_convolution(fdas_ctx* ctx, fdas_part part
   HIPCK(ctx, hipSetDevice(ctx->cfg.device));
   if ((st = record(ctx, s, EV_INPUT)) != FDAS_OK) return st;
   if ((st = enqueue_ftc(ctx, s, part)) != FDAS_OK) return st;
-  if ((st = record(ctx, s, EV_FTC)) != FDAS_OK) return st;
   HIPCK(ctx, hipEventSynchronize(s.ev[EV_FTC]));
   s.fop_valid = true;
   s.cands_valid = false;
@@ -732,17 +777,34 @@ extern "C" fdas_status fdas_perform_harmonic_summing(fdas_ctx* ctx, const float*
   if (!thr) return FDAS_ESTATE;
   HIPCK(ctx, hipSetDevice(ctx->cfg.device));
   fdas_status st;
-  if ((st = record(ctx, s, EV_FTC)) != FDAS_OK) return st;
   if ((st = enqueue_hsum(ctx, s, part, thr)) != FDAS_OK) return st;
-  if ((st = record(ctx, s, EV_HSUM)) != FDAS_OK) return st;
   if ((st = enqueue_readback(ctx, s)) != FDAS_OK) return st;
   if ((st = record(ctx, s, EV_XFER)) != FDAS_OK) return st;
   HIPCK(ctx, hipEventSynchronize(s.ev[EV_XFER]));
   s.cands_valid = true;
   float ms = 0.f;
-  (void)hipEventElapsedTime(&ms, s.ev[EV_HSUM_K0], s.ev[EV_HSUM]);
+  ms = elapsed(s, EV_HSUM_K0, EV_HSUM_K1) + elapsed(s, EV_HSUM_K1, EV_HSUM);
   info(ctx, "Harmonic summing duration: %.3f ms", double(ms));
   return overflow_status(ctx, s);
+}
+
+// The work of a launch once its spectrum is on its way: convolution, and summing,
+// selection and read-back unless they are held (sync pipeline).
+static fdas_status enqueue_launch(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr, uint32_t* det_loc,
+                                  float* det_pwr) {
+  fdas_status st = ctx->sync_pipeline ? enqueue_ftc(ctx, s, part) : enqueue_search(ctx, s, part, thr);
+  if (st != FDAS_OK) return st;
+  s.launched = true;
+  s.user_loc = det_loc;
+  s.user_pwr = det_pwr;
+  if (ctx->sync_pipeline) {
+    s.gated = true;
+    s.gated_part = part;
+    for (uint32_t k = 0; k < ctx->cfg.n_harmonics; ++k) s.gated_thr[k] = thr[k];
+    return FDAS_OK;
+  }
+  if ((st = enqueue_readback(ctx, s)) != FDAS_OK) return st;
+  return record(ctx, s, EV_XFER);
 }
 
 extern "C" fdas_status fdas_launch(fdas_ctx* ctx, const float* spectrum_c64, const float* thresholds, uint32_t* det_loc,
@@ -764,21 +826,7 @@ extern "C" fdas_status fdas_launch(fdas_ctx* ctx, const float* spectrum_c64, con
   if (s.gated && (st = flush_gated(ctx, set)) != FDAS_OK) return st;
   if ((st = upload_input(ctx, s, spectrum_c64, hipMemcpyHostToDevice)) != FDAS_OK) return st;
   if ((st = record(ctx, s, EV_INPUT)) != FDAS_OK) return st;
-  if ((st = enqueue_ftc(ctx, s, part)) != FDAS_OK) return st;
-  if ((st = record(ctx, s, EV_FTC)) != FDAS_OK) return st;
-  s.launched = true;
-  s.user_loc = det_loc;
-  s.user_pwr = det_pwr;
-  if (ctx->sync_pipeline) {
-    s.gated = true;
-    s.gated_part = part;
-    for (uint32_t k = 0; k < ctx->cfg.n_harmonics; ++k) s.gated_thr[k] = thr[k];
-    return FDAS_OK;
-  }
-  if ((st = enqueue_hsum(ctx, s, part, thr)) != FDAS_OK) return st;
-  if ((st = record(ctx, s, EV_HSUM)) != FDAS_OK) return st;
-  if ((st = enqueue_readback(ctx, s)) != FDAS_OK) return st;
-  return record(ctx, s, EV_XFER);
+  return enqueue_launch(ctx, s, part, thr, det_loc, det_pwr);
 }
 
 extern "C" fdas_status fdas_launch_resident(fdas_ctx* ctx, const float* thresholds, uint32_t* det_loc,
@@ -800,21 +848,7 @@ extern "C" fdas_status fdas_launch_resident(fdas_ctx* ctx, const float* threshol
   if (s.gated && (st = flush_gated(ctx, set)) != FDAS_OK) return st;
   if ((st = record(ctx, s, EV_START)) != FDAS_OK) return st;
   if ((st = record(ctx, s, EV_INPUT)) != FDAS_OK) return st;
-  if ((st = enqueue_ftc(ctx, s, part)) != FDAS_OK) return st;
-  if ((st = record(ctx, s, EV_FTC)) != FDAS_OK) return st;
-  s.launched = true;
-  s.user_loc = det_loc;
-  s.user_pwr = det_pwr;
-  if (ctx->sync_pipeline) {
-    s.gated = true;
-    s.gated_part = part;
-    for (uint32_t k = 0; k < ctx->cfg.n_harmonics; ++k) s.gated_thr[k] = thr[k];
-    return FDAS_OK;
-  }
-  if ((st = enqueue_hsum(ctx, s, part, thr)) != FDAS_OK) return st;
-  if ((st = record(ctx, s, EV_HSUM)) != FDAS_OK) return st;
-  if ((st = enqueue_readback(ctx, s)) != FDAS_OK) return st;
-  return record(ctx, s, EV_XFER);
+  return enqueue_launch(ctx, s, part, thr, det_loc, det_pwr);
 }
 
 extern "C" fdas_status fdas_wait(fdas_ctx* ctx, int set) {
@@ -899,9 +933,8 @@ extern "C" fdas_status fdas_retrieve_candidates(fdas_ctx* ctx, uint32_t* det_loc
     return fail(ctx, FDAS_EUNSUPPORTED, "T=%u/H=%u do not fit the 32-bit candidate layout; use the wide API",
                 ctx->cfg.n_templates, ctx->cfg.n_harmonics);
   HIPCK(ctx, hipSetDevice(ctx->cfg.device));
-  fdas_status st;
-  if ((st = enqueue_readback(ctx, s)) != FDAS_OK) return st;
-  HIPCK(ctx, hipStreamSynchronize(s.stream));
+  const fdas_status st = lists_to_host(ctx, s);
+  if (st != FDAS_OK) return st;
   to_reference_lists(ctx, s, det_loc, det_pwr);
   return FDAS_OK;
 }
@@ -912,9 +945,8 @@ extern "C" fdas_status fdas_retrieve_candidates_wide(fdas_ctx* ctx, fdas_candida
   DevSet& s = ctx->set[set];
   if (!out && capacity) return fail(ctx, FDAS_EINVAL, "null candidate pointer");
   HIPCK(ctx, hipSetDevice(ctx->cfg.device));
-  fdas_status st;
-  if ((st = enqueue_readback(ctx, s)) != FDAS_OK) return st;
-  HIPCK(ctx, hipStreamSynchronize(s.stream));
+  const fdas_status st = lists_to_host(ctx, s);
+  if (st != FDAS_OK) return st;
   const uint32_t H = ctx->cfg.n_harmonics, cap = ctx->cfg.cands_per_harmonic;
   const int c = int(ctx->c);
   uint32_t w = 0;
@@ -996,7 +1028,7 @@ extern "C" fdas_status fdas_quantile_thresholds(fdas_ctx* ctx, uint32_t n_per_pl
   const uint64_t want = std::min<uint64_t>(uint64_t(n_per_plane) + 2, M);  // a spare rank for rounding
   // One summing pass over the staged jobs and the order statistics of its spill.
   auto spill_pass = [&]() -> fdas_status {
-    fdas_status r = run_hsum(ctx, s);
+    const fdas_status r = run_hsum(ctx, s);
     if (r != FDAS_OK) return r;
     HIPCK(ctx, launch_quantile_rank(s.d_sel, H, uint32_t(r_lo), uint32_t(r_hi), d_rank, s.stream));
     HIPCK(ctx, hipMemcpyAsync(s.h_quant, d_thr, sizeof(uint32_t) * 4 * H, hipMemcpyDeviceToHost, s.stream));
@@ -1005,7 +1037,8 @@ extern "C" fdas_status fdas_quantile_thresholds(fdas_ctx* ctx, uint32_t n_per_pl
   };
   s.cands_valid = false;  // the lists will belong to these thresholds, not to a search
   std::vector<float> thr(H, -INFINITY);
-  if ((st = stage_hsum(ctx, s, part, thr.data())) != FDAS_OK) return st;
+  fill_hsum(ctx, s, part, thr.data());
+  if ((st = put_jobs(ctx, s)) != FDAS_OK) return st;
   const uint32_t nb = hmax_blocks(N, nr);
   HIPCK(ctx, launch_hmax(s.fop, N, ctx->cfg.n_templates, rb, nr, H, s.quant, s.stream));
   HIPCK(ctx, launch_quantile_bound(s.quant, nb, uint32_t(std::min<uint64_t>(want, UINT32_MAX)), H, s.d_hsum, s.d_sel,
@@ -1035,7 +1068,8 @@ extern "C" fdas_status fdas_quantile_thresholds(fdas_ctx* ctx, uint32_t n_per_pl
         thr[k] = value_of(at[k]);
       }
       // the last pass spills at the final thresholds
-      if ((st = stage_hsum(ctx, s, part, thr.data())) != FDAS_OK) return st;
+      fill_hsum(ctx, s, part, thr.data());
+      if ((st = put_jobs(ctx, s)) != FDAS_OK) return st;
       if ((st = spill_pass()) != FDAS_OK) return st;
       if (fit) break;
       for (uint32_t k = 0; k < H; ++k) {
@@ -1060,16 +1094,6 @@ extern "C" fdas_status fdas_quantile_thresholds(fdas_ctx* ctx, uint32_t n_per_pl
     thresholds[k] = float(lo * (1.0 - g) + hi * g);
   }
   return FDAS_OK;
-}
-
-static float elapsed(const DevSet& s, int a, int b) {
-  if (!s.ev_recorded[a] || !s.ev_recorded[b]) return 0.f;
-  float ms = 0.f;
-  if (hipEventElapsedTime(&ms, s.ev[a], s.ev[b]) != hipSuccess) {
-    (void)hipGetLastError();
-    return 0.f;
-  }
-  return ms;
 }
 
 extern "C" fdas_status fdas_get_stage_times(fdas_ctx* ctx, int set, float* ms6) {
@@ -1103,7 +1127,7 @@ extern "C" void fdas_print_stats(fdas_ctx* ctx, int set, int reset) {
        double(acc), double(acc - ctx->pipeline_accum));
   info(ctx, "  Preparation duration: %.3f ms", double(elapsed(s, EV_START, EV_INPUT)));
   info(ctx, "  FT convolution and IFFT duration: %.3f ms", double(elapsed(s, EV_FTC_K, EV_FTC)));
-  info(ctx, "  Harmonic summing duration: %.3f ms", double(elapsed(s, EV_HSUM_K0, EV_HSUM)));
+  info(ctx, "  Harmonic summing duration: %.3f ms", double(elapsed(s, EV_HSUM_K0, EV_HSUM_K1) + elapsed(s, EV_HSUM_K1, EV_HSUM)));
   info(ctx, "  Total duration: %.3f ms", double(elapsed(s, EV_START, EV_XFER)));
   ctx->pipeline_accum = acc;
 }
@@ -1114,6 +1138,9 @@ extern "C" void fdas_print_events(fdas_ctx* ctx, int set) {
   float t[EV_COUNT] = {};
   for (int e = 0; e < EV_COUNT; ++e)
     if (s.ev_recorded[e]) (void)hipEventElapsedTime(&t[e], ctx->epoch, s.ev[e]);
+  // A kernel's start and end are events of one dispatch, and against another event both give its end.
+  t[EV_FTC_K] = t[EV_FTC] - elapsed(s, EV_FTC_K, EV_FTC);
+  t[EV_HSUM_K0] = t[EV_HSUM_K1] - elapsed(s, EV_HSUM_K0, EV_HSUM_K1);
   char buf[256];
   std::snprintf(buf, sizeof(buf), "@@@,%c,%.6f,%.6f,%.6f,%.6f,%.6f,%.6f,%.6f,%.6f", set == FDAS_SET_A ? 'A' : 'B',
                 double(t[EV_START]), double(t[EV_INPUT]), double(t[EV_FTC_K]), double(t[EV_FTC]),

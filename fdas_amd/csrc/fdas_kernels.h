@@ -23,6 +23,14 @@ constexpr uint32_t kSelectSlices = 64;    // workgroups per plane in the histogr
 
 int ftconv_threads(int tile);
 
+// Events of a launch's own dispatch: `start` takes its begin, `stop` its end.  They
+// ride on the dispatch packet; an event recorded between two kernels is a packet of
+// its own there and keeps the second one waiting (about 5 us each).  Not for
+// launches under stream capture.
+struct LaunchEvents {
+  hipEvent_t start = nullptr, stop = nullptr;
+};
+
 // Workgroups of the FT-convolution kernel that run at once on the 256 CUs: 12 one-wave
 // workgroups per CU (3 waves per SIMD) for 1024-point tiles; 8 waves per CU in
 // workgroups of 2 and 4 for 2048 and 4096.
@@ -30,7 +38,7 @@ inline uint32_t ftconv_slots(uint32_t tile) { return 256u * (tile == 1024 ? 12u 
 
 // Fused FT convolution over a list of jobs (all with the same tile size).
 hipError_t launch_ftconv(int tile, const FtcJob* d_jobs, uint32_t n_jobs, uint32_t n_items, const float2* tw1,
-                         const float2* tw2, uint32_t grid, hipStream_t stream);
+                         const float2* tw2, uint32_t grid, hipStream_t stream, LaunchEvents ev = {});
 
 // Forward transform of every tile of one spectrum, natural bin order (debug / drop-in retrieve_tiles).
 hipError_t launch_tiles(int tile, const float2* spectrum, uint32_t n_bins, uint32_t overlap, uint32_t payload,
@@ -39,13 +47,14 @@ hipError_t launch_tiles(int tile, const float2* spectrum, uint32_t n_bins, uint3
 // Harmonic summing + thresholding + compaction into per-plane spill lists.
 // All jobs of one launch share n_harmonics; any row lengths go together.
 hipError_t launch_hsum(const HsumJob* d_jobs, uint32_t n_jobs, uint32_t n_blocks, uint32_t n_harmonics,
-                       hipStream_t stream);
+                       hipStream_t stream, LaunchEvents ev = {});
 
 // Per-plane cap (strongest first) and sort by (row, bin): power histogram and
 // compaction over the spill lists (kSelectSlices workgroups per plane), then one
 // workgroup per plane resolves the boundary bin exactly and sorts.  cap: the
-// largest cap of the jobs.
-hipError_t launch_select(const SelectJob* d_jobs, uint32_t n_jobs, uint32_t cap, hipStream_t stream);
+// largest cap of the jobs; stop: event of the last kernel's end.
+hipError_t launch_select(const SelectJob* d_jobs, uint32_t n_jobs, uint32_t cap, hipStream_t stream,
+                         hipEvent_t stop = nullptr);
 
 // Harmonic plane HP_k over rows [row_begin, row_begin + n_rows) (debug / parity).
 hipError_t launch_hplane(const float* fop, uint32_t n_bins, uint32_t n_templates, uint32_t row_begin,
@@ -68,6 +77,23 @@ hipError_t launch_quantile_rank(const SelectJob* d_sel, uint32_t n_harmonics, ui
                                 uint32_t* out, hipStream_t stream);
 
 hipError_t launch_zero_u32(uint32_t* p, uint32_t n, hipStream_t stream);
+
+// The job descriptors of one trial's launches, taken to the device as the argument
+// of a kernel that also clears up to two spans of counters: one launch in place of
+// three copies and a fill.
+constexpr uint32_t kPackFtcJobs = 16;
+struct JobPack {
+  FtcJob ftc[kPackFtcJobs];
+  HsumJob hsum;
+  SelectJob sel[kMaxHarmonics];
+  uint32_t n_ftc = 0, n_sel = 0;  // descriptors to write (the summing job goes with the selection jobs)
+};
+struct ZeroSpan {
+  uint32_t* p = nullptr;
+  uint32_t n = 0;
+};
+hipError_t launch_put_jobs(const JobPack& pack, FtcJob* d_ftc, HsumJob* d_hsum, SelectJob* d_sel, ZeroSpan a,
+                           ZeroSpan b, hipStream_t stream);
 
 // One launch running both the FT convolution of ftc_jobs (1024-point tiles)
 // and the harmonic summing of hsum_jobs (n_harmonics planes) over a FOP written

@@ -10,6 +10,7 @@
 //  select_kernel  per-plane cap (strongest first) and (row, bin) ordering of the
 //                 detections; replaces the reference's overwrite-oldest ring
 //                 (detect.cl.mako:106-115) with a deterministic rule.
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <climits>
@@ -287,16 +288,26 @@ __global__ __launch_bounds__(S / 16) void tiles_kernel(const float2* __restrict_
   for (int s = 0; s < 16; ++s) o[F::slot_bin(tid, s)] = v[s];
 }
 
+// A launch, with its events on the dispatch itself where there are any.
+template <class... Params, class... Args>
+static void launch(void (*kernel)(Params...), uint32_t grid, uint32_t block, hipStream_t stream, LaunchEvents ev,
+                   Args... args) {
+  if (ev.start || ev.stop)
+    hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(block), 0, stream, ev.start, ev.stop, 0, args...);
+  else
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), 0, stream, args...);
+}
+
 int ftconv_threads(int tile) { return tile == 1024 ? 64 : tile / 16; }
 
 hipError_t launch_ftconv(int tile, const FtcJob* d_jobs, uint32_t n_jobs, uint32_t n_items, const float2* tw1,
-                         const float2* tw2, uint32_t grid, hipStream_t stream) {
+                         const float2* tw2, uint32_t grid, hipStream_t stream, LaunchEvents ev) {
   if (n_items == 0) return hipSuccess;
   if (grid == 0 || grid > n_items) grid = n_items;
   switch (tile) {
-    case 1024: hipLaunchKernelGGL(ftconv1w_kernel, dim3(grid), dim3(64), 0, stream, d_jobs, n_jobs, n_items, tw1, tw2); break;
-    case 2048: hipLaunchKernelGGL(ftconv_kernel<2048>, dim3(grid), dim3(128), 0, stream, d_jobs, n_jobs, n_items, tw1, tw2); break;
-    case 4096: hipLaunchKernelGGL(ftconv_kernel<4096>, dim3(grid), dim3(256), 0, stream, d_jobs, n_jobs, n_items, tw1, tw2); break;
+    case 1024: launch(ftconv1w_kernel, grid, 64, stream, ev, d_jobs, n_jobs, n_items, tw1, tw2); break;
+    case 2048: launch(ftconv_kernel<2048>, grid, 128, stream, ev, d_jobs, n_jobs, n_items, tw1, tw2); break;
+    case 4096: launch(ftconv_kernel<4096>, grid, 256, stream, ev, d_jobs, n_jobs, n_items, tw1, tw2); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -651,30 +662,31 @@ __global__ __launch_bounds__(kHsumThreads) void hsum_kernel(const HsumJob* __res
 }
 
 template <int H>
-static void launch_hsum_h(const HsumJob* d_jobs, uint32_t n_jobs, uint32_t n_blocks, hipStream_t stream) {
-  hipLaunchKernelGGL(hsum_kernel<H>, dim3(n_blocks), dim3(kHsumThreads), 0, stream, d_jobs, n_jobs);
+static void launch_hsum_h(const HsumJob* d_jobs, uint32_t n_jobs, uint32_t n_blocks, hipStream_t stream,
+                          LaunchEvents ev) {
+  launch(hsum_kernel<H>, n_blocks, kHsumThreads, stream, ev, d_jobs, n_jobs);
 }
 
 hipError_t launch_hsum(const HsumJob* d_jobs, uint32_t n_jobs, uint32_t n_blocks, uint32_t n_harmonics,
-                       hipStream_t stream) {
+                       hipStream_t stream, LaunchEvents ev) {
   if (n_blocks == 0) return hipSuccess;
   switch (n_harmonics) {
-    case 1: launch_hsum_h<1>(d_jobs, n_jobs, n_blocks, stream); break;
-    case 2: launch_hsum_h<2>(d_jobs, n_jobs, n_blocks, stream); break;
-    case 3: launch_hsum_h<3>(d_jobs, n_jobs, n_blocks, stream); break;
-    case 4: launch_hsum_h<4>(d_jobs, n_jobs, n_blocks, stream); break;
-    case 5: launch_hsum_h<5>(d_jobs, n_jobs, n_blocks, stream); break;
-    case 6: launch_hsum_h<6>(d_jobs, n_jobs, n_blocks, stream); break;
-    case 7: launch_hsum_h<7>(d_jobs, n_jobs, n_blocks, stream); break;
-    case 8: launch_hsum_h<8>(d_jobs, n_jobs, n_blocks, stream); break;
-    case 9: launch_hsum_h<9>(d_jobs, n_jobs, n_blocks, stream); break;
-    case 10: launch_hsum_h<10>(d_jobs, n_jobs, n_blocks, stream); break;
-    case 11: launch_hsum_h<11>(d_jobs, n_jobs, n_blocks, stream); break;
-    case 12: launch_hsum_h<12>(d_jobs, n_jobs, n_blocks, stream); break;
-    case 13: launch_hsum_h<13>(d_jobs, n_jobs, n_blocks, stream); break;
-    case 14: launch_hsum_h<14>(d_jobs, n_jobs, n_blocks, stream); break;
-    case 15: launch_hsum_h<15>(d_jobs, n_jobs, n_blocks, stream); break;
-    case 16: launch_hsum_h<16>(d_jobs, n_jobs, n_blocks, stream); break;
+    case 1: launch_hsum_h<1>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 2: launch_hsum_h<2>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 3: launch_hsum_h<3>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 4: launch_hsum_h<4>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 5: launch_hsum_h<5>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 6: launch_hsum_h<6>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 7: launch_hsum_h<7>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 8: launch_hsum_h<8>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 9: launch_hsum_h<9>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 10: launch_hsum_h<10>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 11: launch_hsum_h<11>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 12: launch_hsum_h<12>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 13: launch_hsum_h<13>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 14: launch_hsum_h<14>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 15: launch_hsum_h<15>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 16: launch_hsum_h<16>(d_jobs, n_jobs, n_blocks, stream, ev); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -1532,19 +1544,17 @@ hipError_t launch_quantile_rank(const SelectJob* d_sel, uint32_t n_harmonics, ui
   return hipGetLastError();
 }
 
-hipError_t launch_select(const SelectJob* d_jobs, uint32_t n_jobs, uint32_t cap, hipStream_t stream) {
+hipError_t launch_select(const SelectJob* d_jobs, uint32_t n_jobs, uint32_t cap, hipStream_t stream, hipEvent_t stop) {
   if (n_jobs == 0) return hipSuccess;
   if (cap > kSelectMaxCap) return hipErrorInvalidValue;
   hipLaunchKernelGGL(cand_hist_kernel, dim3(kSelectSlices, n_jobs), dim3(256), 0, stream, d_jobs);
   hipLaunchKernelGGL(cand_compact_kernel, dim3(kSelectSlices, n_jobs), dim3(256), 0, stream, d_jobs);
   // The workgroup grows with the list.  With 1024 / 512 / 256 threads a cap of 4096 took 28 / 30 / 38 us and one
   // of 512 took 11 / 10 / 11 us, where the small workgroup needs a quarter of the CU beside other kernels.
-  if (cap <= 1024)
-    hipLaunchKernelGGL((select_final_kernel<256, 1024>), dim3(n_jobs), dim3(256), 0, stream, d_jobs);
-  else if (cap <= 4096)
-    hipLaunchKernelGGL((select_final_kernel<1024, 4096>), dim3(n_jobs), dim3(1024), 0, stream, d_jobs);
-  else
-    hipLaunchKernelGGL((select_final_kernel<1024, 8192>), dim3(n_jobs), dim3(1024), 0, stream, d_jobs);
+  const LaunchEvents ev{nullptr, stop};
+  if (cap <= 1024) launch(select_final_kernel<256, 1024>, n_jobs, 256, stream, ev, d_jobs);
+  else if (cap <= 4096) launch(select_final_kernel<1024, 4096>, n_jobs, 1024, stream, ev, d_jobs);
+  else launch(select_final_kernel<1024, 8192>, n_jobs, 1024, stream, ev, d_jobs);
   return hipGetLastError();
 }
 
@@ -1556,6 +1566,31 @@ hipError_t launch_zero_u32(uint32_t* p, uint32_t n, hipStream_t stream) {
   if (n == 0) return hipSuccess;
   const uint32_t blocks = min((n + 255u) / 256u, 1024u);
   hipLaunchKernelGGL(zero_u32_kernel, dim3(blocks), dim3(256), 0, stream, p, n);
+  return hipGetLastError();
+}
+
+static_assert(sizeof(JobPack) <= 3584, "job descriptors must fit a kernel argument block");
+
+__global__ __launch_bounds__(256) void put_jobs_kernel(JobPack pack, FtcJob* ftc, HsumJob* hsum, SelectJob* sel,
+                                                       ZeroSpan a, ZeroSpan b) {
+  const uint32_t tid = blockIdx.x * 256u + threadIdx.x, stride = gridDim.x * 256u;
+  for (uint32_t i = tid; i < a.n; i += stride) a.p[i] = 0u;
+  for (uint32_t i = tid; i < b.n; i += stride) b.p[i] = 0u;
+  auto copy = [&](const void* src, void* dst, uint32_t bytes) {
+    for (uint32_t i = tid; i < bytes / 4u; i += stride)
+      static_cast<uint32_t*>(dst)[i] = static_cast<const uint32_t*>(src)[i];
+  };
+  copy(pack.ftc, ftc, pack.n_ftc * uint32_t(sizeof(FtcJob)));
+  if (pack.n_sel) {
+    copy(&pack.hsum, hsum, uint32_t(sizeof(HsumJob)));
+    copy(pack.sel, sel, pack.n_sel * uint32_t(sizeof(SelectJob)));
+  }
+}
+
+hipError_t launch_put_jobs(const JobPack& pack, FtcJob* d_ftc, HsumJob* d_hsum, SelectJob* d_sel, ZeroSpan a,
+                           ZeroSpan b, hipStream_t stream) {
+  const uint32_t blocks = min(1u + (a.n + b.n) / 1024u, 64u);
+  hipLaunchKernelGGL(put_jobs_kernel, dim3(blocks), dim3(256), 0, stream, pack, d_ftc, d_hsum, d_sel, a, b);
   return hipGetLastError();
 }
 

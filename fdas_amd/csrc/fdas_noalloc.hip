@@ -29,20 +29,13 @@ namespace {
 
 constexpr int kMaxDevices = 64;
 
-// Job descriptors of one call, written into the scratch by a kernel that takes
-// them as its argument (no host-to-device copy from pageable memory).
+// Job descriptors of one call, in the scratch.
 struct NoallocJobs {
   HsumJob hsum;
   SelectJob sel[kMaxHarmonics];
 };
-static_assert(sizeof(NoallocJobs) <= 3072, "job descriptors must fit a kernel argument block");
 constexpr uint64_t kJobsBytes = 4096;
-
-__global__ void put_jobs_kernel(NoallocJobs jobs, NoallocJobs* dst) {
-  const uint32_t* src = reinterpret_cast<const uint32_t*>(&jobs);
-  uint32_t* out = reinterpret_cast<uint32_t*>(dst);
-  for (uint32_t i = threadIdx.x; i < sizeof(NoallocJobs) / 4; i += blockDim.x) out[i] = src[i];
-}
+static_assert(sizeof(NoallocJobs) <= kJobsBytes, "job descriptors must fit their place in the scratch");
 
 std::mutex g_mu;
 void* g_scratch[kMaxDevices] = {};
@@ -130,7 +123,8 @@ extern "C" fdas_status fdas_hsum_noalloc(const float* d_fop, uint32_t n_bins, ui
   uint32_t* spill_key = reinterpret_cast<uint32_t*>(base + o_spill);
   float* spill_pwr = reinterpret_cast<float*>(base + o_spill + 4ull * H * spill);
 
-  NoallocJobs jobs{};
+  JobPack jobs{};
+  jobs.n_sel = H;
   HsumJob& j = jobs.hsum;
   j.fop = d_fop;
   j.n_bins = n_bins;
@@ -165,11 +159,9 @@ extern "C" fdas_status fdas_hsum_noalloc(const float* d_fop, uint32_t n_bins, ui
   hipStream_t s = static_cast<hipStream_t>(stream);
   // Every call shares this device's scratch and keeps no state between calls:
   // what must start at zero (counters, histograms, the caller's counts) is
-  // cleared by fill kernels first.
-  hipLaunchKernelGGL(put_jobs_kernel, dim3(1), dim3(256), 0, s, jobs, d_jobs);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = launch_zero_u32(d_counts, 2 * H, s);
-  if (e == hipSuccess) e = launch_zero_u32(compact_n, H * (1 + kSelectBins), s);
+  // cleared by the kernel that brings the job descriptors.
+  hipError_t e = launch_put_jobs(jobs, nullptr, &d_jobs->hsum, d_jobs->sel, {d_counts, 2 * H},
+                                 {compact_n, H * (1 + kSelectBins)}, s);
   const uint32_t blocks = (n_bins + kHsumBinsPerBlock - 1) / kHsumBinsPerBlock * j.n_row_chunks;
   if (e == hipSuccess) e = launch_hsum(&d_jobs->hsum, 1, blocks, H, s);
   if (e == hipSuccess) e = launch_select(d_jobs->sel, H, cap, s);
