@@ -16,7 +16,6 @@ constexpr int kHsumBinsPerBlock = kHsumThreads * kHsumBinsPerThread;  // bins on
 // Rows of whole 8-bin groups (part of the rule for the fused kernel).
 inline bool hsum_whole_groups(uint32_t n_bins) { return n_bins % kHsumBinsPerThread == 0; }
 constexpr uint32_t kHsumRowsPerBlock = 11;  // target rows per HSUM workgroup (bounds the dense-hit tail)
-constexpr int kHsumWaveStage = 64;        // LDS staging entries per plane per wave before a global flush
 constexpr uint32_t kSelectMaxCap = 8192;  // largest per-plane cap the in-LDS sort handles
 constexpr uint32_t kSelectPool = 4096;    // boundary-bin entries resolved exactly in LDS
 constexpr uint32_t kSelectSlices = 64;    // workgroups per plane in the histogram / compaction passes

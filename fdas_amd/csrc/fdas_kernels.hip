@@ -349,30 +349,66 @@ __device__ __forceinline__ uint32_t wave_prefix_small(uint32_t v, uint32_t& tota
   return excl;
 }
 
-// Per-wave detection staging: each wave owns kHsumWaveStage LDS slots per
-// plane and a wave-uniform fill count.  A full stage is flushed by the wave
-// alone (one global atomic for up to 64 entries); what is left at the end is
-// flushed with one atomic per plane per workgroup.
+// Per-wave detection staging.  A lane with a hit stages its whole group, 8 sums
+// and their first key, in one slot of its wave's list for the plane; the bins
+// that pass are picked out when the list is flushed, by 8 lanes per group.  So a
+// hit costs the row loop one ballot and three LDS writes: picking the bins there
+// (compares, a prefix sum and a store per bin, inlined for each plane and
+// register buffer) took about 170 instructions, and two rows in three have a
+// wave with a hit at six-sigma thresholds.  8 trials of 2^21 bins x 85 rows x 8
+// planes 1.645 -> 1.617 ms (memory bound), 2^20 x 85 x 16 1.54 -> 1.48.
 template <int H>
 struct HsumStage {
-  static constexpr int kCap = kHsumWaveStage;
-  uint32_t key[kHsumThreads / 64][H][kCap];
-  float pwr[kHsumThreads / 64][H][kCap];
-  uint32_t n[kHsumThreads / 64][H];
+  static constexpr uint32_t kGroups = H <= 8 ? 24 : 12;  // LDS for 5 and 4 workgroups per CU
+  float sum[kHsumThreads / 64][H][kGroups][kHsumBinsPerThread];
+  uint32_t key[kHsumThreads / 64][H][kGroups];  // row << kKeyBinBits | f0
+  uint32_t n[kHsumThreads / 64][H];             // groups, then (at the end) hits
   uint32_t base[kHsumThreads / 64][H];
 };
 
-// Writes the wave's n staged entries of plane p to the global spill list.
+// One bin of each of 8 staged groups, first, first + 1, ...: this lane's value and key,
+// and whether it is a hit of the plane.
 template <class Stage>
-__device__ __forceinline__ void wave_flush(Stage& st, const HsumJob& job, uint32_t wave, uint32_t p, uint32_t n) {
-  const uint32_t lane = lane_id();
-  uint32_t g = 0;
-  if (lane == 0) g = gatomic_add(job.counts + p, n);
-  g = __shfl(g, 0);
-  if (lane < n && g + lane < job.spill_cap) {
-    gst(job.spill_key, size_t(p) * job.spill_cap + g + lane, st.key[wave][p][lane]);
-    gst(job.spill_pwr, size_t(p) * job.spill_cap + g + lane, st.pwr[wave][p][lane]);
+__device__ __forceinline__ bool staged_bin(const Stage& st, uint32_t wave, uint32_t p, uint32_t first, uint32_t n,
+                                           float thr, uint32_t n_bins, float* v, uint32_t* key) {
+  const uint32_t lane = lane_id(), g = first + lane / 8u, b = lane % 8u;
+  if (g >= n) return false;
+  *v = st.sum[wave][p][g][b];
+  *key = st.key[wave][p][g] + b;
+  return *v > thr && (*key & ((1u << kKeyBinBits) - 1u)) < n_bins;
+}
+
+__device__ __forceinline__ void spill_hit(const HsumJob& job, uint32_t p, uint32_t slot, uint32_t key, float v) {
+  if (slot >= job.spill_cap) return;  // counted, not kept
+  gst(job.spill_key, size_t(p) * job.spill_cap + slot, key);
+  gst(job.spill_pwr, size_t(p) * job.spill_cap + slot, v);
+}
+
+// Writes the hits of the wave's n staged groups of plane p to the global spill
+// list, with one global atomic.
+template <class Stage>
+__device__ __forceinline__ void wave_flush(Stage& st, const HsumJob& job, uint32_t wave, uint32_t p, uint32_t n,
+                                           float thr) {
+  constexpr int kSteps = int((Stage::kGroups + 7) / 8);
+  wave_lds_order();
+  float v[kSteps];
+  uint32_t key[kSteps], slot[kSteps], total = 0;
+  bool hit[kSteps];
+#pragma unroll
+  for (int s = 0; s < kSteps; ++s) {
+    hit[s] = staged_bin(st, wave, p, uint32_t(8 * s), n, thr, job.n_bins, &v[s], &key[s]);
+    const uint64_t m = __ballot(hit[s]);
+    slot[s] = total + lanes_below(m);
+    total += uint32_t(__builtin_popcountll(m));
   }
+  wave_lds_order();  // the stage is rewritten next
+  if (total == 0) return;
+  uint32_t base = 0;
+  if (lane_id() == 0) base = gatomic_add(job.counts + p, total);
+  base = __shfl(base, 0);
+#pragma unroll
+  for (int s = 0; s < kSteps; ++s)
+    if (hit[s]) spill_hit(job, p, base + slot[s], key[s], v[s]);
 }
 
 __device__ __forceinline__ uint32_t find_job_hsum(const HsumJob* __restrict__ jobs, uint32_t n_jobs, uint32_t blk) {
@@ -446,12 +482,16 @@ __device__ __forceinline__ void hsum_load_row(RowLoads<H>& L, const float* __res
 }
 
 // Bin b of the thread takes sub-harmonic value (f0 mod k + b) / k of its span:
-// b / k when f0 mod k < k (b / k + 1) - b, else the next one.  rk[k-1] = f0 mod k.
+// b / k when f0 mod k < k (b / k + 1) - b, else the next one.  rk[k-1] = f0 mod k
+// is a multiple of g = gcd(8, k), so the edge may be rounded up to one: that
+// drops the selects no residue reaches, and bins share their compares (35 in
+// place of 49 for k = 9 .. 15; 1.61 -> 1.54 ms per 8 trials of 2^20 bins x 85 rows
+// x 16 planes, no change at 8 planes).
 template <int K>
 __device__ __forceinline__ float hsum_sub(const float (&s)[kHsumMaxSpan], uint32_t rk, int b) {
-  const int lo = b / K;
-  const int edge = K * (lo + 1) - b;  // f0 mod k at which bin b moves to the next value
-  if (edge > K - hsum_gcd8(K)) return s[lo];  // no f0 mod k reaches it
+  const int lo = b / K, g = hsum_gcd8(K);
+  const int edge = (K * (lo + 1) - b + g - 1) / g * g;  // f0 mod k at which bin b moves to the next value
+  if (edge > K - g) return s[lo];  // no f0 mod k reaches it
   return rk >= uint32_t(edge) ? s[lo + 1] : s[lo];
 }
 
@@ -501,45 +541,41 @@ __device__ __forceinline__ void hsum_row(Stage& st, const HsumJob& job, const Ro
 #pragma unroll
   for (int k = 1; k <= H; ++k) {
     if (k > 1) hsum_add_k<H>(k, hp, L, rk);
-    if ((__ballot(group_max(hp) >= thr_key[k - 1]) & live_lanes) == 0) continue;
-    // The wave's hits in lane order, each lane's in bin order: one prefix sum
-    // over the per-lane counts places them all.
-    uint32_t bits = 0;
-#pragma unroll
-    for (int b = 0; b < kHsumBinsPerThread; ++b) bits |= (hp[b] > thr[k - 1]) ? (1u << b) : 0u;
-    bits &= live_bits;
-    uint32_t total;
-    uint32_t pos = wave_prefix_small(uint32_t(__builtin_popcount(bits)), total);
-    if (wn[k - 1] + total > uint32_t(Stage::kCap)) {
-      wave_flush(st, job, wave, uint32_t(k - 1), wn[k - 1]);
+    const uint64_t groups = __ballot(group_max(hp) >= thr_key[k - 1]) & live_lanes;
+    if (groups == 0) continue;
+    const uint32_t n_groups = uint32_t(__builtin_popcountll(groups));
+    if (wn[k - 1] + n_groups > Stage::kGroups) {
+      wave_flush(st, job, wave, uint32_t(k - 1), wn[k - 1], thr[k - 1]);
       wn[k - 1] = 0;
     }
-    if (total > uint32_t(Stage::kCap)) {
-      // more than a stage holds: straight to the spill list (entries past its end are counted, not kept)
+    if (n_groups > Stage::kGroups) {
+      // more than the stage holds (a strong signal, a low threshold): straight to the spill list,
+      // the wave's hits in lane order, each lane's in bin order
+      uint32_t bits = 0;
+#pragma unroll
+      for (int b = 0; b < kHsumBinsPerThread; ++b) bits |= (hp[b] > thr[k - 1]) ? (1u << b) : 0u;
+      bits &= live_bits;
+      uint32_t total;
+      const uint32_t pos = wave_prefix_small(uint32_t(__builtin_popcount(bits)), total);
       uint32_t g = 0;
       if (lane_id() == 0) g = gatomic_add(job.counts + (k - 1), total);
       g = __shfl(g, 0) + pos;
 #pragma unroll
       for (int b = 0; b < kHsumBinsPerThread; ++b) {
         if ((bits >> b) & 1u) {
-          if (g < job.spill_cap) {
-            gst(job.spill_key, size_t(k - 1) * job.spill_cap + g, (r << kKeyBinBits) | (f0 + uint32_t(b)));
-            gst(job.spill_pwr, size_t(k - 1) * job.spill_cap + g, hp[b]);
-          }
+          spill_hit(job, uint32_t(k - 1), g, (r << kKeyBinBits) | (f0 + uint32_t(b)), hp[b]);
           ++g;
         }
       }
     } else {
-      pos += wn[k - 1];
+      if ((groups >> lane_id()) & 1u) {
+        const uint32_t slot = wn[k - 1] + lanes_below(groups);
+        float* __restrict__ to = st.sum[wave][k - 1][slot];
 #pragma unroll
-      for (int b = 0; b < kHsumBinsPerThread; ++b) {
-        if ((bits >> b) & 1u) {
-          st.key[wave][k - 1][pos] = (r << kKeyBinBits) | (f0 + uint32_t(b));
-          st.pwr[wave][k - 1][pos] = hp[b];
-          ++pos;
-        }
+        for (int b = 0; b < kHsumBinsPerThread; ++b) to[b] = hp[b];
+        st.key[wave][k - 1][slot] = (r << kKeyBinBits) | f0;
       }
-      wn[k - 1] += total;
+      wn[k - 1] += n_groups;
     }
   }
 }
@@ -633,30 +669,46 @@ __device__ __forceinline__ void hsum_block(HsumStage<H>& st, const HsumJob* __re
 #pragma unroll
     for (int k = 0; k < H; ++k) st.n[wave][k] = wn[k];
   }
-  __syncthreads();
-  if (tid < H) {
-    uint32_t total = 0;
-    for (uint32_t w = 0; w < uint32_t(kHsumThreads / 64); ++w) {
-      st.base[w][tid] = total;
-      total += st.n[w][tid];
-    }
-    const uint32_t g = total ? gatomic_add(job.counts + tid, total) : 0u;
-    for (uint32_t w = 0; w < uint32_t(kHsumThreads / 64); ++w) st.base[w][tid] += g;
+  wave_lds_order();
+  float v;
+  uint32_t key;
+  for (uint32_t k = 0; k < uint32_t(H); ++k) {
+    const uint32_t n = __builtin_amdgcn_readfirstlane(st.n[wave][k]);
+    uint32_t hits = 0;
+    for (uint32_t first = 0; first < n; first += 8)
+      hits += uint32_t(__builtin_popcountll(__ballot(staged_bin(st, wave, k, first, n, job.thr[k], n_bins, &v, &key))));
+    if (lane_id() == 0) st.base[wave][k] = hits;
   }
   __syncthreads();
-  const uint32_t lane = lane_id();
+  if (tid < H) {
+    uint32_t total = 0, before[kHsumThreads / 64];
 #pragma unroll
-  for (int k = 0; k < H; ++k) {
-    const uint32_t g = st.base[wave][k] + lane;
-    if (lane < wn[k] && g < job.spill_cap) {
-      gst(job.spill_key, size_t(k) * job.spill_cap + g, st.key[wave][k][lane]);
-      gst(job.spill_pwr, size_t(k) * job.spill_cap + g, st.pwr[wave][k][lane]);
+    for (uint32_t w = 0; w < uint32_t(kHsumThreads / 64); ++w) {
+      before[w] = total;
+      total += st.base[w][tid];
+    }
+    const uint32_t g = total ? gatomic_add(job.counts + tid, total) : 0u;
+#pragma unroll
+    for (uint32_t w = 0; w < uint32_t(kHsumThreads / 64); ++w) st.base[w][tid] = g + before[w];
+  }
+  __syncthreads();
+  for (uint32_t k = 0; k < uint32_t(H); ++k) {
+    const uint32_t n = __builtin_amdgcn_readfirstlane(st.n[wave][k]);
+    uint32_t at = __builtin_amdgcn_readfirstlane(st.base[wave][k]);
+    for (uint32_t first = 0; first < n; first += 8) {
+      const bool hit = staged_bin(st, wave, k, first, n, job.thr[k], n_bins, &v, &key);
+      const uint64_t m = __ballot(hit);
+      if (hit) spill_hit(job, k, at + lanes_below(m), key, v);
+      at += uint32_t(__builtin_popcountll(m));
     }
   }
 }
 
+// 15 and 16 planes are held to 128 registers (they take 129 and 131 unasked): four
+// waves per SIMD in place of three, 1.49 -> 1.30 ms per 8 trials of 2^20 bins x 85 rows
+// x 16 planes.
 template <int H>
-__global__ __launch_bounds__(kHsumThreads) void hsum_kernel(const HsumJob* __restrict__ jobs, uint32_t n_jobs) {
+__global__ __launch_bounds__(kHsumThreads) __attribute__((amdgpu_waves_per_eu(H >= 15 ? 4 : 1))) void hsum_kernel(const HsumJob* __restrict__ jobs, uint32_t n_jobs) {
   __shared__ HsumStage<H> st;
   hsum_block<H>(st, jobs, n_jobs, blockIdx.x);
 }
