@@ -30,10 +30,10 @@ struct LaunchEvents {
   hipEvent_t start = nullptr, stop = nullptr;
 };
 
-// Workgroups of the FT-convolution kernel that run at once on the 256 CUs: 12 one-wave
-// workgroups per CU (3 waves per SIMD) for 1024-point tiles; 8 waves per CU in
-// workgroups of 2 and 4 for 2048 and 4096.
-inline uint32_t ftconv_slots(uint32_t tile) { return 256u * (tile == 1024 ? 12u : tile == 2048 ? 4u : 2u); }
+// Workgroups of the FT-convolution kernel that run at once on the 256 CUs, at three
+// waves per SIMD: 12 one-wave workgroups per CU for 1024-point tiles, 6 and 3 of two
+// and four waves for 2048 and 4096.
+inline uint32_t ftconv_slots(uint32_t tile) { return 256u * 12u * 1024u / tile; }
 
 // Fused FT convolution over a list of jobs (all with the same tile size).
 hipError_t launch_ftconv(int tile, const FtcJob* d_jobs, uint32_t n_jobs, uint32_t n_items, const float2* tw1,

@@ -34,21 +34,26 @@ __device__ __forceinline__ uint32_t find_job_ftc(const FtcJob* __restrict__ jobs
   return lo;
 }
 
+// 2048- and 4096-point tiles, S / 16 threads (2 and 4 waves) per workgroup.
+//
+// Bound by VALU issue and, for a launch of a round or two, by latency.  Held to 168
+// registers (three waves per SIMD): F2 twiddles in LDS, one exchange buffer, template
+// spectra loaded when they are used.  With everything in registers, two buffers and
+// the template prefetched one row ahead (232 / 221 VGPRs, two waves) a trial of
+// 85 templates took, 2048-point tiles: 50 us at 2^18 bins, 114 at 700,001, 350 at
+// 2^21, against 46, 99 and 336; 4096-point tiles at 2^21: 373 against 338.  The FMA
+// forms are spelled out to give the FOP that kernel gave, bit for bit.
 template <int S>
-__global__ __launch_bounds__(S / 16) void ftconv_kernel(const FtcJob* __restrict__ jobs, uint32_t n_jobs,
-                                                        uint32_t n_items, const float2* __restrict__ tw1,
-                                                        const float2* __restrict__ tw2) {
-  using F = TileFFT<S>;
+__global__ __launch_bounds__(S / 16) __attribute__((amdgpu_waves_per_eu(3, 3))) void ftconv_kernel(
+    const FtcJob* __restrict__ jobs, uint32_t n_jobs, uint32_t n_items, const float2* __restrict__ tw1,
+    const float2* __restrict__ tw2) {
+  using F = TileFFTLean<S>;
   constexpr int NT = F::NT;
-  // A one-wave workgroup (S = 1024) barriers for free: it keeps one LDS buffer
-  // (8.7 KB), so more workgroups fit beside it on a CU.  Wider tiles keep two
-  // buffers and save two barriers per inverse transform.
-  constexpr bool kSingle = (S == 1024);
   __shared__ float2 la[F::LDS_ELEMS];
-  __shared__ float2 lb[kSingle ? 1 : F::LDS_ELEMS];
+  __shared__ float2 w2[F::W2_ELEMS];
   const int tid = threadIdx.x;
   F fft;
-  fft.load_twiddles(tw1, tw2, tid);
+  fft.load_twiddles(tw1, tw2, w2, tid);
 
   for (uint32_t item = blockIdx.x; item < n_items; item += gridDim.x) {
     const FtcJob* job = jobs + find_job_ftc(jobs, n_jobs, item);
@@ -78,28 +83,12 @@ __global__ __launch_bounds__(S / 16) void ftconv_kernel(const FtcJob* __restrict
     const float2* __restrict__ hbase = static_cast<const float2*>(job->hperm);
     const uint32_t out0 = tile * payload;  // FOP bin of tile sample s = overlap
 
-    // Template spectra are loaded one row ahead: the first row's before the
-    // forward transform, every next row's as soon as this row's has been used,
-    // so the loads have a whole transform to complete (and they precede this
-    // row's FOP stores: loads and stores share one in-order completion counter,
-    // so a load issued after the stores would wait for them).
-    float2 hn[16];
-#pragma unroll
-    for (int s = 0; s < 16; ++s) hn[s] = gld2(hbase + size_t(r_begin) * S + tid, size_t(s * NT));
     fft.forward(xf, la, tid);
     for (uint32_t r = r_begin; r < r_end; ++r) {
       float2 v[16];
 #pragma unroll
-      for (int s = 0; s < 16; ++s) v[s] = cmul(xf[s], hn[s]);
-      {
-        const float2* __restrict__ h = hbase + size_t(min(r + 1, r_end - 1)) * S + tid;  // unconditional: no branch
-#pragma unroll
-        for (int s = 0; s < 16; ++s) hn[s] = gld2(h, size_t(s * NT));
-      }
-      if constexpr (kSingle)
-        fft.inverse_single(v, la, tid);
-      else
-        fft.inverse(v, la, lb, tid);
+      for (int s = 0; s < 16; ++s) v[s] = cmul_f0(xf[s], gld2(hbase + size_t(r) * S + tid, size_t(s * NT)));
+      fft.inverse(v, la, tid);
       // Slot a of this thread is FOP bin out0 + NT*a + tid - overlap: one base
       // address per row and a constant offset per slot (the store's immediate).
       float* __restrict__ out = job->fop + size_t(r) * n_bins + (ptrdiff_t(out0) + tid - ptrdiff_t(overlap));

@@ -37,7 +37,8 @@ std::vector<FtcJob> plan_ftc_rows(uint32_t tile, uint32_t n_bins, uint32_t max_t
 //   32,768 x 85, tile 2048: 39 / 15 (2; 1 row, two rounds of workgroups: 21)
 //   20,011 x 169, tile 4096: 49 / 17 (2)
 //   131,072 x 85, tile 2048: 42 / 29 (8); tile 1024: 38 / 27 (6)
-// and from 262,144 bins (tile 2048) on 16 rows are the fastest or within 3 %.
+// (2048 and 4096 with two waves per SIMD; three since), and where one round needs
+// more than 16 rows, 16 are the fastest or within 3 %.
 // The FOP does not depend on it.
 void fit_ftc_items(std::vector<FtcJob>& jobs, uint32_t slots);
 

@@ -72,6 +72,18 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
 __device__ __forceinline__ float2 cmulc(float2 a, float2 b) {
   return make_float2(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y);
 }
+// The same products with the fused multiply-add of each part spelled out, for code whose results must not
+// depend on where the compiler keeps the operands (contraction otherwise picks the fused product by that):
+// a b with the first product of either part fused last / first, and a conj(b).
+__device__ __forceinline__ float2 cmul_f0(float2 a, float2 b) {
+  return make_float2(fmaf(a.x, b.x, -(a.y * b.y)), fmaf(a.y, b.x, a.x * b.y));
+}
+__device__ __forceinline__ float2 cmul_f2(float2 a, float2 b) {
+  return make_float2(fmaf(a.x, b.x, -(a.y * b.y)), fmaf(a.x, b.y, a.y * b.x));
+}
+__device__ __forceinline__ float2 cmulc_f3(float2 a, float2 b) {
+  return make_float2(fmaf(a.x, b.x, a.y * b.y), fmaf(a.y, b.x, -(a.x * b.y)));
+}
 // a * W with W = conj(w) for the inverse direction (DIR = +1), w for DIR = -1.
 template <int DIR>
 __device__ __forceinline__ float2 ctw(float2 a, float2 w) {
@@ -311,62 +323,6 @@ struct TileFFT {
     apply_dftD<-1>(v);
   }
 
-  // Inverse transform of spectrum slots v -> v[a] = out[NT*a + tid] (unnormalised).
-  // Uses two LDS buffers: a (pair layout) and b (row layout).  The caller must
-  // ensure no thread still reads `a` from a previous forward pass.
-  __device__ __forceinline__ void inverse(float2 (&v)[16], float2* __restrict__ la, float2* __restrict__ lb,
-                                          int tid) const {
-    apply_dftD<+1>(v);
-#pragma unroll
-    for (int i = 0; i < PAIRS; ++i)
-#pragma unroll
-      for (int dd = 0; dd < D; ++dd) la[dd * RS2 + tid + NT * i] = v[i * D + dd];
-    __syncthreads();
-    const int ka = tid & 15, d = tid >> 4;
-#pragma unroll
-    for (int kc = 0; kc < 16; ++kc) v[kc] = la[d * RS2 + 16 * kc + ka];
-#pragma unroll
-    for (int k = 1; k < 16; ++k) v[k] = cmulc(v[k], w2[k]);
-    dft16<+1>(v);
-#pragma unroll
-    for (int c = 0; c < 16; ++c) lb[ka * RS1 + D * c + d] = v[c];
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 16; ++k) v[k] = lb[k * RS1 + tid];
-#pragma unroll
-    for (int k = 1; k < 16; ++k) v[k] = cmulc(v[k], w1[k]);
-    dft16<+1>(v);
-  }
-
-  // As inverse(), with one LDS buffer for both exchanges (half the LDS, two more
-  // barriers).  Starts with a barrier, so the caller's previous readers of `lds`
-  // are done before it is rewritten.
-  __device__ __forceinline__ void inverse_single(float2 (&v)[16], float2* __restrict__ lds, int tid) const {
-    apply_dftD<+1>(v);
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < PAIRS; ++i)
-#pragma unroll
-      for (int dd = 0; dd < D; ++dd) lds[dd * RS2 + tid + NT * i] = v[i * D + dd];
-    __syncthreads();
-    const int ka = tid & 15, d = tid >> 4;
-#pragma unroll
-    for (int kc = 0; kc < 16; ++kc) v[kc] = lds[d * RS2 + 16 * kc + ka];
-#pragma unroll
-    for (int k = 1; k < 16; ++k) v[k] = cmulc(v[k], w2[k]);
-    dft16<+1>(v);
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < 16; ++c) lds[ka * RS1 + D * c + d] = v[c];
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 16; ++k) v[k] = lds[k * RS1 + tid];
-#pragma unroll
-    for (int k = 1; k < 16; ++k) v[k] = cmulc(v[k], w1[k]);
-    dft16<+1>(v);
-  }
-
- private:
   template <int DIR>
   __device__ __forceinline__ static void apply_dftD(float2 (&v)[16]) {
     if constexpr (PAIRS == 1) {
@@ -383,6 +339,88 @@ struct TileFFT {
   }
 };
 
+
+// TileFFT<S> with few live registers, for the convolution of 2048- and 4096-point
+// tiles: the F2 twiddles W_NT^(d k) come from an LDS table (w2[k * D + d]; 30 registers
+// less), and one LDS buffer serves both exchanges (half the LDS, two more barriers
+// per transform).
+template <int S>
+struct TileFFTLean {
+  using F = TileFFT<S>;
+  static constexpr int NT = F::NT, D = F::D, PAIRS = F::PAIRS, RS1 = F::RS1, RS2 = F::RS2;
+  static constexpr int LDS_ELEMS = F::LDS_ELEMS;
+  static constexpr int W2_ELEMS = 16 * D;
+
+  float2 w1[16];                  // W_S^(tid * ka)
+  const float2* __restrict__ w2;  // LDS
+
+  // w2_lds is read after the caller's next barrier.
+  __device__ __forceinline__ void load_twiddles(const float2* __restrict__ tw1, const float2* __restrict__ tw2,
+                                                float2* __restrict__ w2_lds, int tid) {
+    w1[0] = make_float2(1.f, 0.f);
+#pragma unroll
+    for (int k = 1; k < 16; ++k) w1[k] = tw1[k * NT + tid];
+    for (int i = tid; i < W2_ELEMS; i += NT) w2_lds[i] = tw2[i];
+    w2 = w2_lds;
+  }
+
+  // x[a] = tile[NT * a + tid] -> spectrum slots (TileFFT slot_bin order).  Ends with
+  // a barrier after the last LDS read.
+  __device__ __forceinline__ void forward(float2 (&v)[16], float2* __restrict__ lds, int tid) const {
+    dft16<-1>(v);
+#pragma unroll
+    for (int k = 1; k < 16; ++k) v[k] = cmul(v[k], w1[k]);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) lds[k * RS1 + tid] = v[k];
+    __syncthreads();
+    const int ka = tid & 15, d = tid >> 4;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) v[c] = lds[ka * RS1 + D * c + d];
+    __syncthreads();
+    dft16<-1>(v);
+#pragma unroll
+    for (int k = 1; k < 16; ++k) {
+      const float2 w = w2[k * D + d];
+      v[k] = k % 5 == 0 ? cmul_f0(v[k], w) : cmul_f2(v[k], w);
+    }
+#pragma unroll
+    for (int kc = 0; kc < 16; ++kc) lds[d * RS2 + 16 * kc + ka] = v[kc];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PAIRS; ++i)
+#pragma unroll
+      for (int dd = 0; dd < D; ++dd) v[i * D + dd] = lds[dd * RS2 + tid + NT * i];
+    __syncthreads();
+    F::template apply_dftD<-1>(v);
+  }
+
+  // Spectrum slots -> v[a] = out[NT * a + tid] (unnormalised inverse).  Starts with a
+  // barrier, so the caller's previous readers of `lds` are done before it is rewritten.
+  __device__ __forceinline__ void inverse(float2 (&v)[16], float2* __restrict__ lds, int tid) const {
+    F::template apply_dftD<+1>(v);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PAIRS; ++i)
+#pragma unroll
+      for (int dd = 0; dd < D; ++dd) lds[dd * RS2 + tid + NT * i] = v[i * D + dd];
+    __syncthreads();
+    const int ka = tid & 15, d = tid >> 4;
+#pragma unroll
+    for (int kc = 0; kc < 16; ++kc) v[kc] = lds[d * RS2 + 16 * kc + ka];
+#pragma unroll
+    for (int k = 1; k < 16; ++k) v[k] = cmulc_f3(v[k], w2[k * D + d]);
+    dft16<+1>(v);
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 16; ++c) lds[ka * RS1 + D * c + d] = v[c];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 16; ++k) v[k] = lds[k * RS1 + tid];
+#pragma unroll
+    for (int k = 1; k < 16; ++k) v[k] = cmulc(v[k], w1[k]);
+    dft16<+1>(v);
+  }
+};
 
 // ---------------------------------------------------------------------------
 // One-wave 1024-point transform whose first exchange stays in registers.
