@@ -31,8 +31,8 @@ namespace {
 constexpr uint32_t kMaxFtcJobs = 64;  // row groups per FT-convolution launch
 
 // Events per launch: START, INPUT (spectrum in place), FTC_K (FT-convolution kernel start), FTC (its end),
-// HSUM_K0 / HSUM_K1 (harmonic-summing kernel start / end), HSUM (selection end), XFER (lists read back).
-enum Ev { EV_START = 0, EV_INPUT, EV_FTC_K, EV_FTC, EV_HSUM_K0, EV_HSUM_K1, EV_HSUM, EV_XFER, EV_COUNT };
+// HSUM_K0 / HSUM_K1 (harmonic-summing kernel start / end), HSUM (selection end, with the lists in host memory).
+enum Ev { EV_START = 0, EV_INPUT, EV_FTC_K, EV_FTC, EV_HSUM_K0, EV_HSUM_K1, EV_HSUM, EV_COUNT };
 
 struct DevSet {
   float2* input = nullptr;
@@ -42,11 +42,6 @@ struct DevSet {
   float* plane = nullptr;
   uint32_t* spill_key = nullptr;
   float* spill_pwr = nullptr;
-  // One allocation, read back from its start: lists (keys, powers), kept entries, detections;
-  // zeroed before each summing pass from `counts` on: detections, compact counts, histograms.
-  uint32_t* out_key = nullptr;     // [H][cap]
-  float* out_pwr = nullptr;        // [H][cap]
-  uint32_t* out_n = nullptr;       // [H]
   uint32_t* counts = nullptr;      // [H] detections, then [H] compact counts, then [H][kSelectBins] histograms
   uint32_t* compact_key = nullptr;
   float* compact_pwr = nullptr;
@@ -57,11 +52,11 @@ struct DevSet {
 
   FtcJob* h_ftc = nullptr;         // pinned staging of more than kPackFtcJobs row groups
   JobPack pack;                    // the launches' job descriptors
-  uint32_t* h_out_key = nullptr;   // pinned mirror of the lists, kept entries and detections (one allocation)
-  float* h_out_pwr = nullptr;
-  uint32_t* h_out_n = nullptr;
-  uint32_t* h_counts = nullptr;
-  bool lists_on_host = false;      // the mirror holds (or, in stream order, will hold) the last pass's lists
+  // The lists, in pinned host memory that the selection kernel writes (one allocation).
+  uint32_t* h_out_key = nullptr;   // [H][cap]
+  float* h_out_pwr = nullptr;      // [H][cap]
+  uint32_t* h_out_n = nullptr;     // [H] kept entries
+  uint32_t* h_counts = nullptr;    // [H] detections
   uint32_t* h_quant = nullptr;     // [4H] mirror of quant's tail
 
   hipStream_t stream = nullptr;
@@ -179,9 +174,9 @@ fdas_status dev_alloc(fdas_ctx* ctx, T** p, size_t count) {
 }
 
 template <typename T>
-fdas_status host_alloc(fdas_ctx* ctx, T** p, size_t count) {
+fdas_status host_alloc(fdas_ctx* ctx, T** p, size_t count, unsigned flags = 0) {
   *p = nullptr;
-  hipError_t e = hipHostMalloc(reinterpret_cast<void**>(p), std::max<size_t>(count, 1) * sizeof(T), 0);
+  hipError_t e = hipHostMalloc(reinterpret_cast<void**>(p), std::max<size_t>(count, 1) * sizeof(T), flags);
   if (e != hipSuccess) {
     (void)hipGetLastError();
     *p = nullptr;
@@ -292,9 +287,10 @@ void fill_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr) {
     q.compact_key = s.compact_key + size_t(p) * ccap;
     q.compact_pwr = s.compact_pwr + size_t(p) * ccap;
     q.compact_n = s.counts + H + p;
-    q.out_key = s.out_key + size_t(p) * cap;
-    q.out_pwr = s.out_pwr + size_t(p) * cap;
-    q.out_n = s.out_n + p;
+    q.out_key = s.h_out_key + size_t(p) * cap;
+    q.out_pwr = s.h_out_pwr + size_t(p) * cap;
+    q.out_n = s.h_out_n + p;
+    q.out_count = s.h_counts + p;
   }
   s.pack.n_sel = H;
 }
@@ -312,7 +308,7 @@ fdas_status run_ftc(fdas_ctx* ctx, DevSet& s, uint32_t n_jobs, uint32_t n_items)
   // The two sets' kernels take turns: this convolution starts once the other
   // set's last summing kernel has finished (both kinds of kernel are VALU-bound,
   // and side by side they only slow each other down), while that set's
-  // selection and read-back, and this set's input copy, still overlap.
+  // selection, and this set's input copy, still overlap.
   const DevSet& other = &s == &ctx->set[0] ? ctx->set[1] : ctx->set[0];
   if (other.hsum_issued) HIPCK(ctx, hipStreamWaitEvent(s.stream, other.ev[EV_HSUM_K1], 0));
   HIPCK(ctx, launch_ftconv(int(ctx->cfg.tile), s.d_ftc, n_jobs, n_items, ctx->tw1, ctx->tw2, n_items, s.stream,
@@ -325,7 +321,6 @@ fdas_status run_ftc(fdas_ctx* ctx, DevSet& s, uint32_t n_jobs, uint32_t n_items)
 fdas_status run_hsum(fdas_ctx* ctx, DevSet& s) {
   const uint32_t H = ctx->cfg.n_harmonics;
   const HsumJob& j = s.pack.hsum;
-  s.lists_on_host = false;
   const uint32_t blocks = (ctx->geo.n_bins + kHsumBinsPerBlock - 1) / kHsumBinsPerBlock * j.n_row_chunks;
   HIPCK(ctx, launch_hsum(s.d_hsum, 1, blocks, H, s.stream, {s.ev[EV_HSUM_K0], s.ev[EV_HSUM_K1]}));
   s.hsum_issued = true;
@@ -357,24 +352,6 @@ fdas_status enqueue_search(fdas_ctx* ctx, DevSet& s, fdas_part part, const float
   if ((st = put_jobs(ctx, s)) != FDAS_OK) return st;
   if ((st = run_ftc(ctx, s, n_jobs, n_items)) != FDAS_OK) return st;
   return run_hsum(ctx, s);
-}
-
-fdas_status enqueue_readback(fdas_ctx* ctx, DevSet& s) {
-  const size_t H = ctx->cfg.n_harmonics, cap = ctx->cfg.cands_per_harmonic;
-  HIPCK(ctx, hipMemcpyAsync(s.h_out_key, s.out_key, sizeof(uint32_t) * (2 * H * cap + 2 * H), hipMemcpyDeviceToHost,
-                            s.stream));
-  s.lists_on_host = true;
-  return FDAS_OK;
-}
-
-// The last pass's lists in the pinned mirror: copied unless that pass has read them back.
-fdas_status lists_to_host(fdas_ctx* ctx, DevSet& s) {
-  if (!s.lists_on_host) {
-    const fdas_status st = enqueue_readback(ctx, s);
-    if (st != FDAS_OK) return st;
-  }
-  HIPCK(ctx, hipStreamSynchronize(s.stream));
-  return FDAS_OK;
 }
 
 // Converts the staged lists to the reference's 32-bit layout (gen_info.h:62-73).
@@ -416,10 +393,7 @@ fdas_status flush_gated(fdas_ctx* ctx, int set) {
   DevSet& s = ctx->set[set];
   if (!s.gated) return FDAS_OK;
   s.gated = false;
-  fdas_status st = enqueue_hsum(ctx, s, s.gated_part, s.gated_thr);
-  if (st != FDAS_OK) return st;
-  if ((st = enqueue_readback(ctx, s)) != FDAS_OK) return st;
-  return record(ctx, s, EV_XFER);
+  return enqueue_hsum(ctx, s, s.gated_part, s.gated_thr);
 }
 
 void free_set(DevSet& s) {
@@ -432,7 +406,7 @@ void free_set(DevSet& s) {
   (void)hipFree(s.spill_pwr);
   (void)hipFree(s.compact_key);
   (void)hipFree(s.compact_pwr);
-  (void)hipFree(s.out_key);  // and out_pwr, out_n, counts
+  (void)hipFree(s.counts);
   (void)hipFree(s.d_ftc);
   (void)hipFree(s.d_hsum);
   (void)hipFree(s.d_sel);
@@ -565,15 +539,12 @@ extern "C" fdas_status fdas_create(const fdas_config* cfg, fdas_log_fn log, void
     if ((st = dev_alloc(ctx, &s.spill_pwr, H * ctx->spill)) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.compact_key, H * (cap + kSelectPool))) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.compact_pwr, H * (cap + kSelectPool))) != FDAS_OK) return bail(st);
-    if ((st = dev_alloc(ctx, &s.out_key, 2 * H * cap + H * (3 + kSelectBins))) != FDAS_OK) return bail(st);
-    s.out_pwr = reinterpret_cast<float*>(s.out_key + H * cap);
-    s.out_n = s.out_key + 2 * H * cap;
-    s.counts = s.out_n + H;
+    if ((st = dev_alloc(ctx, &s.counts, H * (2 + kSelectBins))) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.d_ftc, kMaxFtcJobs)) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.d_hsum, 1)) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.d_sel, H)) != FDAS_OK) return bail(st);
     if ((st = host_alloc(ctx, &s.h_ftc, kMaxFtcJobs)) != FDAS_OK) return bail(st);
-    if ((st = host_alloc(ctx, &s.h_out_key, 2 * H * cap + 2 * H)) != FDAS_OK) return bail(st);
+    if ((st = host_alloc(ctx, &s.h_out_key, 2 * H * cap + 2 * H, hipHostMallocCoherent)) != FDAS_OK) return bail(st);
     s.h_out_pwr = reinterpret_cast<float*>(s.h_out_key + H * cap);
     s.h_out_n = s.h_out_key + 2 * H * cap;
     s.h_counts = s.h_out_n + H;
@@ -587,7 +558,6 @@ extern "C" fdas_status fdas_create(const fdas_config* cfg, fdas_log_fn log, void
       return bail(fail(ctx, FDAS_EDEVICE, "event creation failed"));
     // a FOP that was never written reads as zeros
     if (hipMemset(s.fop, 0, T * N * sizeof(float)) != hipSuccess ||
-        hipMemset(s.out_n, 0, H * sizeof(uint32_t)) != hipSuccess ||
         hipMemset(s.counts, 0, H * (2 + kSelectBins) * sizeof(uint32_t)) != hipSuccess)
       return bail(fail(ctx, FDAS_EDEVICE, "buffer initialisation failed"));
   }
@@ -778,9 +748,7 @@ extern "C" fdas_status fdas_perform_harmonic_summing(fdas_ctx* ctx, const float*
   HIPCK(ctx, hipSetDevice(ctx->cfg.device));
   fdas_status st;
   if ((st = enqueue_hsum(ctx, s, part, thr)) != FDAS_OK) return st;
-  if ((st = enqueue_readback(ctx, s)) != FDAS_OK) return st;
-  if ((st = record(ctx, s, EV_XFER)) != FDAS_OK) return st;
-  HIPCK(ctx, hipEventSynchronize(s.ev[EV_XFER]));
+  HIPCK(ctx, hipEventSynchronize(s.ev[EV_HSUM]));
   s.cands_valid = true;
   float ms = 0.f;
   ms = elapsed(s, EV_HSUM_K0, EV_HSUM_K1) + elapsed(s, EV_HSUM_K1, EV_HSUM);
@@ -788,8 +756,8 @@ extern "C" fdas_status fdas_perform_harmonic_summing(fdas_ctx* ctx, const float*
   return overflow_status(ctx, s);
 }
 
-// The work of a launch once its spectrum is on its way: convolution, and summing,
-// selection and read-back unless they are held (sync pipeline).
+// The work of a launch once its spectrum is on its way: convolution, and summing
+// and selection unless they are held (sync pipeline).
 static fdas_status enqueue_launch(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr, uint32_t* det_loc,
                                   float* det_pwr) {
   fdas_status st = ctx->sync_pipeline ? enqueue_ftc(ctx, s, part) : enqueue_search(ctx, s, part, thr);
@@ -801,10 +769,8 @@ static fdas_status enqueue_launch(fdas_ctx* ctx, DevSet& s, fdas_part part, cons
     s.gated = true;
     s.gated_part = part;
     for (uint32_t k = 0; k < ctx->cfg.n_harmonics; ++k) s.gated_thr[k] = thr[k];
-    return FDAS_OK;
   }
-  if ((st = enqueue_readback(ctx, s)) != FDAS_OK) return st;
-  return record(ctx, s, EV_XFER);
+  return FDAS_OK;
 }
 
 extern "C" fdas_status fdas_launch(fdas_ctx* ctx, const float* spectrum_c64, const float* thresholds, uint32_t* det_loc,
@@ -858,7 +824,7 @@ extern "C" fdas_status fdas_wait(fdas_ctx* ctx, int set) {
   HIPCK(ctx, hipSetDevice(ctx->cfg.device));
   fdas_status st;
   if (s.gated && (st = flush_gated(ctx, set)) != FDAS_OK) return st;
-  HIPCK(ctx, hipEventSynchronize(s.ev[EV_XFER]));
+  HIPCK(ctx, hipEventSynchronize(s.ev[EV_HSUM]));
   s.launched = false;
   s.fop_valid = true;
   s.cands_valid = true;
@@ -933,8 +899,7 @@ extern "C" fdas_status fdas_retrieve_candidates(fdas_ctx* ctx, uint32_t* det_loc
     return fail(ctx, FDAS_EUNSUPPORTED, "T=%u/H=%u do not fit the 32-bit candidate layout; use the wide API",
                 ctx->cfg.n_templates, ctx->cfg.n_harmonics);
   HIPCK(ctx, hipSetDevice(ctx->cfg.device));
-  const fdas_status st = lists_to_host(ctx, s);
-  if (st != FDAS_OK) return st;
+  HIPCK(ctx, hipStreamSynchronize(s.stream));
   to_reference_lists(ctx, s, det_loc, det_pwr);
   return FDAS_OK;
 }
@@ -945,8 +910,7 @@ extern "C" fdas_status fdas_retrieve_candidates_wide(fdas_ctx* ctx, fdas_candida
   DevSet& s = ctx->set[set];
   if (!out && capacity) return fail(ctx, FDAS_EINVAL, "null candidate pointer");
   HIPCK(ctx, hipSetDevice(ctx->cfg.device));
-  const fdas_status st = lists_to_host(ctx, s);
-  if (st != FDAS_OK) return st;
+  HIPCK(ctx, hipStreamSynchronize(s.stream));
   const uint32_t H = ctx->cfg.n_harmonics, cap = ctx->cfg.cands_per_harmonic;
   const int c = int(ctx->c);
   uint32_t w = 0;
@@ -1104,8 +1068,8 @@ extern "C" fdas_status fdas_get_stage_times(fdas_ctx* ctx, int set, float* ms6) 
   ms6[1] = elapsed(s, EV_FTC_K, EV_FTC);
   ms6[2] = elapsed(s, EV_HSUM_K0, EV_HSUM_K1);
   ms6[3] = elapsed(s, EV_HSUM_K1, EV_HSUM);
-  ms6[4] = elapsed(s, EV_HSUM, EV_XFER);
-  ms6[5] = elapsed(s, EV_START, EV_XFER);
+  ms6[4] = 0.f;  // the selection writes the lists to host memory
+  ms6[5] = elapsed(s, EV_START, EV_HSUM);
   return FDAS_OK;
 }
 
@@ -1114,7 +1078,7 @@ extern "C" void fdas_print_stats(fdas_ctx* ctx, int set, int reset) {
   const DevSet& s = ctx->set[set];
   float t0 = 0.f, t1 = 0.f;
   (void)hipEventElapsedTime(&t0, ctx->epoch, s.ev[EV_START]);
-  (void)hipEventElapsedTime(&t1, ctx->epoch, s.ev[EV_XFER]);
+  (void)hipEventElapsedTime(&t1, ctx->epoch, s.ev[EV_HSUM]);
   if (reset) {
     ctx->pipeline_start = t0;
     ctx->pipeline_accum = 0.f;
@@ -1128,7 +1092,7 @@ extern "C" void fdas_print_stats(fdas_ctx* ctx, int set, int reset) {
   info(ctx, "  Preparation duration: %.3f ms", double(elapsed(s, EV_START, EV_INPUT)));
   info(ctx, "  FT convolution and IFFT duration: %.3f ms", double(elapsed(s, EV_FTC_K, EV_FTC)));
   info(ctx, "  Harmonic summing duration: %.3f ms", double(elapsed(s, EV_HSUM_K0, EV_HSUM_K1) + elapsed(s, EV_HSUM_K1, EV_HSUM)));
-  info(ctx, "  Total duration: %.3f ms", double(elapsed(s, EV_START, EV_XFER)));
+  info(ctx, "  Total duration: %.3f ms", double(elapsed(s, EV_START, EV_HSUM)));
   ctx->pipeline_accum = acc;
 }
 
@@ -1144,7 +1108,7 @@ extern "C" void fdas_print_events(fdas_ctx* ctx, int set) {
   char buf[256];
   std::snprintf(buf, sizeof(buf), "@@@,%c,%.6f,%.6f,%.6f,%.6f,%.6f,%.6f,%.6f,%.6f", set == FDAS_SET_A ? 'A' : 'B',
                 double(t[EV_START]), double(t[EV_INPUT]), double(t[EV_FTC_K]), double(t[EV_FTC]),
-                double(t[EV_HSUM_K0]), double(t[EV_HSUM_K1]), double(t[EV_HSUM]), double(t[EV_XFER]));
+                double(t[EV_HSUM_K0]), double(t[EV_HSUM_K1]), double(t[EV_HSUM]), double(t[EV_HSUM]));
   emit(ctx, FDAS_LOG_INFO, buf);
 }
 

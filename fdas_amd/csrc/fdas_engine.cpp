@@ -4,8 +4,8 @@
 // (FDAS.cpp:282-615).  Here an engine keeps banks, twiddles and a device arena
 // bounded by an HBM budget; trials of any N, bank, harmonic count and part are
 // cut into groups.  One group's FT convolution runs on the convolution stream
-// while the previous group's harmonic summing, selection and read-back run on
-// the summing stream, so the VALU-bound convolution overlaps the HBM-bound
+// while the previous group's harmonic summing and selection run on the
+// summing stream, so the VALU-bound convolution overlaps the HBM-bound
 // summing.  The same group machinery serves fixed batches (plans, optionally
 // captured once as a HIP graph) and a continuous-batching request loop.
 #include <hip/hip_runtime.h>
@@ -177,37 +177,40 @@ struct Shape {
   uint32_t n_items = 0;
 };
 
-// Byte offsets of one trial's device state, in two parts.  The small part
-// (lists, counters, selection histogram) is zeroed before every run and read
-// back; the large part (selection pool, spill lists, input copy, FOP) is not.
-// Plans keep the small parts of all their trials in one array, so a group
-// zeroes and reads back its trials with one launch and one copy.
+// Byte offsets of one trial's device state, in two parts, and of its lists in host
+// memory.  The small part (counters, selection histogram) is cleared before every
+// run; the large part (selection pool, spill lists, input copy, FOP) is not.  The
+// selection kernel writes the lists to pinned host memory itself.
 struct TrialLayout {
   // small part, from its base
-  uint64_t out_n, counts, out_key, out_pwr, compact_n, hist, small_bytes;
-  uint64_t readback_bytes;  // out_n .. out_pwr
+  uint64_t counts, compact_n, hist, small_bytes;
   // large part, from its base
   uint64_t compact_key, compact_pwr, spill_key, spill_pwr, input, fop, large_bytes;
   uint64_t total;  // small_bytes + large_bytes
+  // lists, from the trial's base in host memory
+  uint64_t out_n, out_count, out_key, out_pwr, host_bytes;
 };
 
 TrialLayout trial_layout(uint32_t n_bins, uint32_t T, uint32_t H, uint32_t cap, uint32_t spill, bool own_input) {
   TrialLayout l{};
   uint64_t o = 0;
-  l.out_n = o;
-  o += 4ull * H;
   l.counts = o;
   o += 4ull * H;
-  l.out_key = o;
-  o += 4ull * H * cap;
-  l.out_pwr = o;
-  o += 4ull * H * cap;
-  l.readback_bytes = o;
   l.compact_n = o;
   o += 4ull * H;
   l.hist = o;
   o += 4ull * H * kSelectBins;
   l.small_bytes = align_up(o);
+  o = 0;
+  l.out_n = o;
+  o += 4ull * H;
+  l.out_count = o;
+  o += 4ull * H;
+  l.out_key = o;
+  o += 4ull * H * cap;
+  l.out_pwr = o;
+  o += 4ull * H * cap;
+  l.host_bytes = align_up(o);
   const uint64_t ccap = uint64_t(cap) + kSelectPool;
   o = 0;
   l.compact_key = o;
@@ -238,12 +241,15 @@ struct Trial {
   char* small = nullptr;          // device small part (served trials: also the arena block)
   char* mem = nullptr;            // device large part
   const float2* input = nullptr;  // device spectrum
-  char* h_read = nullptr;         // pinned mirror of the small part
+  char* h_lists = nullptr;        // pinned host memory of the lists
   double t_submit = 0.0;
 };
 
 // Device and pinned job arrays of one group, and its launch list.
 struct GroupBuf {
+  // One device array and its pinned twin: FT-convolution, summing and selection jobs.
+  char* d_jobs = nullptr;
+  char* h_jobs = nullptr;
   FtcJob* d_ftc = nullptr;
   FtcJob* h_ftc = nullptr;
   uint32_t ftc_cap = 0;
@@ -256,7 +262,8 @@ struct GroupBuf {
   // ev_ftc1 / ev_done order the streams; ev_ftc0 / ev_ftc_t1 / ev_hsum0 / ev_hsum1 only time the kernels.
   hipEvent_t ev_ftc0 = nullptr, ev_ftc1 = nullptr, ev_hsum0 = nullptr, ev_hsum1 = nullptr, ev_done = nullptr;
   hipEvent_t ev_ftc_t1 = nullptr;
-  hipEvent_t ev_hsum_done = nullptr;  // harmonic summing finished (the next group's convolution waits on it)
+  hipEvent_t ev_hsum_done = nullptr;  // harmonic summing finished (the selection waits on it)
+  hipEvent_t ev_up = nullptr;          // served groups: jobs and host spectra uploaded, counters cleared
   bool launch_fused = false;           // this group's convolution ran in a fused kernel (with the previous summing)
   bool hsum_fused = false;             // this group's summing ran in the next group's fused kernel
   struct FtcLaunch {
@@ -269,10 +276,6 @@ struct GroupBuf {
   std::vector<FtcLaunch> ftc;
   std::vector<HsumLaunch> hsum;
   uint32_t n_sel = 0;
-  // Small parts of the group's trials when they are one contiguous span (plans).
-  char* small_span = nullptr;
-  char* h_span = nullptr;
-  uint64_t span_bytes = 0;
 };
 
 }  // namespace
@@ -288,7 +291,7 @@ struct fdas_engine {
   std::vector<std::unique_ptr<Bank>> banks;
   std::map<std::tuple<uint32_t, uint32_t, uint32_t>, std::unique_ptr<Shape>> shapes;
   std::map<uint32_t, std::pair<float2*, float2*>> twiddles;  // tile -> (tw1, tw2)
-  hipStream_t s_ftc = nullptr, s_hsum = nullptr;
+  hipStream_t s_ftc = nullptr, s_hsum = nullptr, s_up = nullptr;  // s_up: uploads of served groups
   float2* tune_input = nullptr;  // 2^22 bins of seeded complex noise, E|X|^2 = 1 (tuning input)
   uint32_t n_cu = 0;
   std::string device_key;        // device name, architecture and CU count (tuning-cache key)
@@ -305,15 +308,14 @@ struct fdas_engine {
   struct Ctx {
     GroupBuf buf;
     std::vector<Trial> trials;
-    char* h_read = nullptr;
-    uint64_t h_read_cap = 0;
+    char* h_lists = nullptr;
+    uint64_t h_lists_cap = 0;
     bool busy = false;
     uint64_t seq = 0;
   };
   std::vector<Ctx> ctxs;
   uint64_t launch_seq = 0;
   std::vector<fdas_plan*> plans;   // live plans, which hold arena memory (guarded by api_mu)
-  hipEvent_t last_hsum = nullptr;  // summing-done event of the last served group
   fdas_engine_stats stats{};
 };
 
@@ -325,7 +327,8 @@ struct fdas_plan {
   std::vector<char*> regions;
   std::vector<char*> inputs;  // plan-owned device copies of host spectra (nullptr for device spectra)
   char* small_all = nullptr;  // small parts of all trials, in trial order
-  char* h_read = nullptr;     // its pinned mirror
+  uint64_t small_bytes = 0;
+  char* h_lists = nullptr;    // lists of all trials, in trial order (pinned host memory)
   uint64_t region_bytes = 0;
   hipEvent_t ev_start = nullptr, ev_end = nullptr;
   hipGraph_t graph = nullptr;
@@ -406,9 +409,9 @@ fdas_status dev_alloc(fdas_engine* e, T** p, size_t count) {
 }
 
 template <typename T>
-fdas_status host_alloc(fdas_engine* e, T** p, size_t count) {
+fdas_status host_alloc(fdas_engine* e, T** p, size_t count, unsigned flags = 0) {
   *p = nullptr;
-  const hipError_t r = hipHostMalloc(reinterpret_cast<void**>(p), std::max<size_t>(count, 1) * sizeof(T), 0);
+  const hipError_t r = hipHostMalloc(reinterpret_cast<void**>(p), std::max<size_t>(count, 1) * sizeof(T), flags);
   if (r != hipSuccess) {
     (void)hipGetLastError();
     *p = nullptr;
@@ -419,13 +422,9 @@ fdas_status host_alloc(fdas_engine* e, T** p, size_t count) {
 }
 
 void free_group(GroupBuf& g) {
-  (void)hipFree(g.d_ftc);
-  (void)hipFree(g.d_hsum);
-  (void)hipFree(g.d_sel);
-  (void)hipHostFree(g.h_ftc);
-  (void)hipHostFree(g.h_hsum);
-  (void)hipHostFree(g.h_sel);
-  for (hipEvent_t ev : {g.ev_ftc0, g.ev_ftc1, g.ev_hsum0, g.ev_hsum1, g.ev_done, g.ev_ftc_t1, g.ev_hsum_done})
+  (void)hipFree(g.d_jobs);
+  (void)hipHostFree(g.h_jobs);
+  for (hipEvent_t ev : {g.ev_ftc0, g.ev_ftc1, g.ev_hsum0, g.ev_hsum1, g.ev_done, g.ev_ftc_t1, g.ev_hsum_done, g.ev_up})
     if (ev) (void)hipEventDestroy(ev);
   g = GroupBuf{};
 }
@@ -433,45 +432,37 @@ void free_group(GroupBuf& g) {
 fdas_status group_events(fdas_engine* e, GroupBuf& g) {
   for (hipEvent_t* ev : {&g.ev_ftc0, &g.ev_ftc1, &g.ev_hsum0, &g.ev_hsum1, &g.ev_done, &g.ev_ftc_t1})
     if (!*ev) EHIP(e, hipEventCreate(ev));
-  if (!g.ev_hsum_done) EHIP(e, hipEventCreateWithFlags(&g.ev_hsum_done, hipEventDisableTiming));
+  for (hipEvent_t* ev : {&g.ev_hsum_done, &g.ev_up})
+    if (!*ev) EHIP(e, hipEventCreateWithFlags(ev, hipEventDisableTiming));
   return FDAS_OK;
 }
 
 // Grows the job arrays of g to hold at least the given counts.
 fdas_status group_reserve(fdas_engine* e, GroupBuf& g, uint32_t n_ftc, uint32_t n_hsum, uint32_t n_sel) {
-  fdas_status st;
-  if (n_ftc > g.ftc_cap) {
-    (void)hipFree(g.d_ftc);
-    (void)hipHostFree(g.h_ftc);
-    g.d_ftc = nullptr;
-    g.h_ftc = nullptr;
-    g.ftc_cap = 0;
-    if ((st = dev_alloc(e, &g.d_ftc, n_ftc)) != FDAS_OK || (st = host_alloc(e, &g.h_ftc, n_ftc)) != FDAS_OK) return st;
-    g.ftc_cap = n_ftc;
-  }
-  if (n_hsum > g.hsum_cap) {
-    (void)hipFree(g.d_hsum);
-    (void)hipHostFree(g.h_hsum);
-    g.d_hsum = nullptr;
-    g.h_hsum = nullptr;
-    g.hsum_cap = 0;
-    if ((st = dev_alloc(e, &g.d_hsum, n_hsum)) != FDAS_OK || (st = host_alloc(e, &g.h_hsum, n_hsum)) != FDAS_OK)
-      return st;
-    g.hsum_cap = n_hsum;
-  }
-  if (n_sel > g.sel_cap) {
-    (void)hipFree(g.d_sel);
-    (void)hipHostFree(g.h_sel);
-    g.d_sel = nullptr;
-    g.h_sel = nullptr;
-    g.sel_cap = 0;
-    if ((st = dev_alloc(e, &g.d_sel, n_sel)) != FDAS_OK || (st = host_alloc(e, &g.h_sel, n_sel)) != FDAS_OK) return st;
-    g.sel_cap = n_sel;
+  if (n_ftc > g.ftc_cap || n_hsum > g.hsum_cap || n_sel > g.sel_cap) {
+    (void)hipFree(g.d_jobs);
+    (void)hipHostFree(g.h_jobs);
+    g.d_jobs = g.h_jobs = nullptr;
+    const uint32_t cf = std::max(n_ftc, g.ftc_cap), ch = std::max(n_hsum, g.hsum_cap), cs = std::max(n_sel, g.sel_cap);
+    g.ftc_cap = g.hsum_cap = g.sel_cap = 0;
+    const uint64_t o_hsum = align_up(sizeof(FtcJob) * uint64_t(cf)), o_sel = o_hsum + align_up(sizeof(HsumJob) * uint64_t(ch));
+    const uint64_t bytes = o_sel + sizeof(SelectJob) * uint64_t(cs);
+    fdas_status st;
+    if ((st = dev_alloc(e, &g.d_jobs, bytes)) != FDAS_OK || (st = host_alloc(e, &g.h_jobs, bytes)) != FDAS_OK) return st;
+    g.d_ftc = reinterpret_cast<FtcJob*>(g.d_jobs);
+    g.h_ftc = reinterpret_cast<FtcJob*>(g.h_jobs);
+    g.d_hsum = reinterpret_cast<HsumJob*>(g.d_jobs + o_hsum);
+    g.h_hsum = reinterpret_cast<HsumJob*>(g.h_jobs + o_hsum);
+    g.d_sel = reinterpret_cast<SelectJob*>(g.d_jobs + o_sel);
+    g.h_sel = reinterpret_cast<SelectJob*>(g.h_jobs + o_sel);
+    g.ftc_cap = cf;
+    g.hsum_cap = ch;
+    g.sel_cap = cs;
   }
   return group_events(e, g);
 }
 
-// Fills the host job arrays of a group of placed trials (mem, input, h_read set)
+// Fills the host job arrays of a group of placed trials (mem, input, h_lists set)
 // and its launch list: FT-convolution jobs grouped by tile, summing jobs by H.
 fdas_status build_group(fdas_engine* e, GroupBuf& g, const std::vector<Trial*>& trials) {
   const uint32_t cap = e->cfg.cands_per_harmonic, ccap = cap + kSelectPool;
@@ -541,9 +532,10 @@ fdas_status build_group(fdas_engine* e, GroupBuf& g, const std::vector<Trial*>& 
         q.compact_key = reinterpret_cast<uint32_t*>(m + l.compact_key) + size_t(p) * ccap;
         q.compact_pwr = reinterpret_cast<float*>(m + l.compact_pwr) + size_t(p) * ccap;
         q.compact_n = reinterpret_cast<uint32_t*>(sm + l.compact_n) + p;
-        q.out_key = reinterpret_cast<uint32_t*>(sm + l.out_key) + size_t(p) * cap;
-        q.out_pwr = reinterpret_cast<float*>(sm + l.out_pwr) + size_t(p) * cap;
-        q.out_n = reinterpret_cast<uint32_t*>(sm + l.out_n) + p;
+        q.out_key = reinterpret_cast<uint32_t*>(t->h_lists + l.out_key) + size_t(p) * cap;
+        q.out_pwr = reinterpret_cast<float*>(t->h_lists + l.out_pwr) + size_t(p) * cap;
+        q.out_n = reinterpret_cast<uint32_t*>(t->h_lists + l.out_n) + p;
+        q.out_count = reinterpret_cast<uint32_t*>(t->h_lists + l.out_count) + p;
       }
     }
     L.n_jobs = jh - L.first;
@@ -551,55 +543,25 @@ fdas_status build_group(fdas_engine* e, GroupBuf& g, const std::vector<Trial*>& 
   }
   g.n_sel = js;
   (void)n_sel;
-  // One zeroing launch and one read-back copy when the small parts are contiguous.
-  g.small_span = nullptr;
-  g.h_span = nullptr;
-  g.span_bytes = 0;
-  bool contiguous = !trials.empty();
-  for (size_t i = 1; i < trials.size() && contiguous; ++i)
-    contiguous = trials[i]->small == trials[i - 1]->small + trials[i - 1]->lay.small_bytes &&
-                 trials[i]->h_read == trials[i - 1]->h_read + trials[i - 1]->lay.small_bytes;
-  if (contiguous) {
-    g.small_span = trials.front()->small;
-    g.h_span = trials.front()->h_read;
-    g.span_bytes = uint64_t(trials.back()->small - trials.front()->small) + trials.back()->lay.small_bytes;
-  }
   return FDAS_OK;
 }
 
-fdas_status upload_group(fdas_engine* e, GroupBuf& g, uint32_t n_ftc, uint32_t n_hsum, hipStream_t s) {
-  EHIP(e, hipMemcpyAsync(g.d_ftc, g.h_ftc, sizeof(FtcJob) * n_ftc, hipMemcpyHostToDevice, s));
-  EHIP(e, hipMemcpyAsync(g.d_hsum, g.h_hsum, sizeof(HsumJob) * n_hsum, hipMemcpyHostToDevice, s));
-  EHIP(e, hipMemcpyAsync(g.d_sel, g.h_sel, sizeof(SelectJob) * g.n_sel, hipMemcpyHostToDevice, s));
+fdas_status upload_group(fdas_engine* e, GroupBuf& g, hipStream_t s) {
+  const uint64_t bytes = uint64_t(reinterpret_cast<char*>(g.h_sel + g.n_sel) - g.h_jobs);
+  EHIP(e, hipMemcpyAsync(g.d_jobs, g.h_jobs, bytes, hipMemcpyHostToDevice, s));
   return FDAS_OK;
 }
 
-uint32_t group_ftc_jobs(const GroupBuf& g) {
-  uint32_t n = 0;
-  for (const auto& L : g.ftc) n += L.n_jobs;
-  return n;
-}
-
-uint32_t group_hsum_jobs(const GroupBuf& g) {
-  uint32_t n = 0;
-  for (const auto& L : g.hsum) n += L.n_jobs;
-  return n;
-}
-
-// Enqueues one group: convolution on s_ftc, then (after its end event) zeroing,
-// summing, selection and read-back on s_hsum.  wait_before: an event s_ftc waits
-// on first (the group whose memory this one reuses), or nullptr.  prev_hsum: the
-// previous group's summing-done event, or nullptr: the convolution starts after
-// it, since the two kernels only slow each other down when they share the CUs
-// (both VALU-heavy), while the selection and read-back that follow the summing
-// still run beside the next convolution.  Timing events bracket the two kernels
-// (not under graph capture, where this runtime rejects externally visible
-// event records).
-fdas_status enqueue_group(fdas_engine* e, GroupBuf& g, const std::vector<Trial*>& trials, hipEvent_t wait_before,
-                          hipEvent_t prev_hsum, bool timing_events) {
-  hipStream_t A = e->s_ftc, B = e->s_hsum;
+// Enqueues one group: convolution on s_ftc, summing on s_ftc too (lagged) or on s_hsum beside the next group's
+// convolution, selection on s_hsum.  wait_before: an event s_ftc waits on first, or nullptr.  With the summing on
+// s_ftc the two kernels, which only slow each other down when they share the CUs (both VALU-heavy), take turns,
+// while the selection still runs beside the next convolution; with the summing on s_hsum it would also wait for the
+// previous group's selection, whose 1024-thread workgroups wait for a free CU behind the convolution (twelve served
+// requests: 7.36 ms, and 6.73 ms on s_ftc, with the uploads and clears on s_up).  Timing events bracket the two kernels (not under
+// graph capture, where this runtime rejects externally visible event records).
+fdas_status enqueue_group(fdas_engine* e, GroupBuf& g, hipEvent_t wait_before, bool lagged, bool timing_events) {
+  hipStream_t A = e->s_ftc, B = e->s_hsum, S = lagged ? A : B;
   if (wait_before) EHIP(e, hipStreamWaitEvent(A, wait_before, 0));
-  if (prev_hsum) EHIP(e, hipStreamWaitEvent(A, prev_hsum, 0));
   if (timing_events) EHIP(e, hipEventRecord(g.ev_ftc0, A));
   for (const auto& L : g.ftc) {
     const auto& tw = e->twiddles.at(L.tile);
@@ -607,47 +569,48 @@ fdas_status enqueue_group(fdas_engine* e, GroupBuf& g, const std::vector<Trial*>
                           ftc_grid(e, L.n_items), A));
   }
   if (timing_events) EHIP(e, hipEventRecord(g.ev_ftc_t1, A));
-  EHIP(e, hipEventRecord(g.ev_ftc1, A));
-  EHIP(e, hipStreamWaitEvent(B, g.ev_ftc1, 0));
-  if (g.small_span) {
-    EHIP(e, launch_zero_u32(reinterpret_cast<uint32_t*>(g.small_span), uint32_t(g.span_bytes / 4), B));
-  } else {
-    for (const Trial* t : trials)
-      EHIP(e, launch_zero_u32(reinterpret_cast<uint32_t*>(t->small), uint32_t(t->lay.small_bytes / 4), B));
+  if (!lagged) {
+    EHIP(e, hipEventRecord(g.ev_ftc1, A));
+    EHIP(e, hipStreamWaitEvent(B, g.ev_ftc1, 0));
+    EHIP(e, launch_clear_counters(g.d_sel, g.n_sel, B));
   }
-  if (timing_events) EHIP(e, hipEventRecord(g.ev_hsum0, B));
-  for (const auto& L : g.hsum) EHIP(e, launch_hsum(g.d_hsum + L.first, L.n_jobs, L.n_blocks, L.H, B));
-  if (timing_events) EHIP(e, hipEventRecord(g.ev_hsum1, B));
-  EHIP(e, hipEventRecord(g.ev_hsum_done, B));
+  if (timing_events) EHIP(e, hipEventRecord(g.ev_hsum0, S));
+  for (const auto& L : g.hsum) EHIP(e, launch_hsum(g.d_hsum + L.first, L.n_jobs, L.n_blocks, L.H, S));
+  if (timing_events) EHIP(e, hipEventRecord(g.ev_hsum1, S));
+  if (lagged) {
+    EHIP(e, hipEventRecord(g.ev_hsum_done, A));
+    EHIP(e, hipStreamWaitEvent(B, g.ev_hsum_done, 0));
+  }
   EHIP(e, launch_select(g.d_sel, g.n_sel, e->cfg.cands_per_harmonic, B));
-  if (g.small_span) {
-    EHIP(e, hipMemcpyAsync(g.h_span, g.small_span, g.span_bytes, hipMemcpyDeviceToHost, B));
-  } else {
-    for (const Trial* t : trials)
-      EHIP(e, hipMemcpyAsync(t->h_read, t->small, t->lay.readback_bytes, hipMemcpyDeviceToHost, B));
-  }
   EHIP(e, hipEventRecord(g.ev_done, B));
   return FDAS_OK;
 }
 
-// Copies a completed trial's lists from its pinned read-back area to the result.
+// Copies a completed trial's lists from their pinned host memory to the result (entries past a plane's kept
+// ones: 0).
 void finish_result(const fdas_engine* e, const Trial& t, fdas_result* r) {
   const uint32_t H = t.req.n_harmonics, cap = e->cfg.cands_per_harmonic;
-  const uint32_t* out_n = reinterpret_cast<const uint32_t*>(t.h_read + t.lay.out_n);
-  const uint32_t* counts = reinterpret_cast<const uint32_t*>(t.h_read + t.lay.counts);
-  const uint32_t* key = reinterpret_cast<const uint32_t*>(t.h_read + t.lay.out_key);
-  const float* pwr = reinterpret_cast<const float*>(t.h_read + t.lay.out_pwr);
+  const uint32_t* out_n = reinterpret_cast<const uint32_t*>(t.h_lists + t.lay.out_n);
+  const uint32_t* counts = reinterpret_cast<const uint32_t*>(t.h_lists + t.lay.out_count);
+  const uint32_t* key = reinterpret_cast<const uint32_t*>(t.h_lists + t.lay.out_key);
+  const float* pwr = reinterpret_cast<const float*>(t.h_lists + t.lay.out_pwr);
   r->tag = t.req.tag;
   r->n_harmonics = H;
   r->tile = t.shape->tile;
   r->status = FDAS_OK;
+  auto put = [cap](void* dst, const void* src, uint32_t p, uint32_t n) {
+    char* d = static_cast<char*>(dst) + 4ull * p * cap;
+    std::memcpy(d, static_cast<const char*>(src) + 4ull * p * cap, 4ull * n);
+    std::memset(d + 4ull * n, 0, 4ull * (cap - n));
+  };
   for (uint32_t p = 0; p < kMaxHarmonics; ++p) {
     r->n_detected[p] = p < H ? counts[p] : 0;
     r->n_kept[p] = p < H ? std::min(out_n[p], cap) : 0;
-    if (p < H && counts[p] > t.spill) r->status = FDAS_EOVERFLOW;
+    if (p >= H) continue;
+    if (counts[p] > t.spill) r->status = FDAS_EOVERFLOW;
+    if (r->key) put(r->key, key, p, r->n_kept[p]);
+    if (r->power) put(r->power, pwr, p, r->n_kept[p]);
   }
-  if (r->key) std::memcpy(r->key, key, sizeof(uint32_t) * H * cap);
-  if (r->power) std::memcpy(r->power, pwr, sizeof(float) * H * cap);
 }
 
 fdas_status validate_request(fdas_engine* e, const fdas_request* q) {
@@ -898,7 +861,7 @@ fdas_status time_shape(fdas_engine* e, uint32_t n_bins, uint32_t bank_id, uint32
         g.h_hsum[c].fop = fop_of(c);
         g.h_hsum[c].block_begin = c * L1.n_blocks;
       }
-      if ((st = upload_group(e, g, 0, G, e->s_ftc)) != FDAS_OK) break;
+      if ((st = upload_group(e, g, e->s_ftc)) != FDAS_OK) break;
       float ms = FLT_MAX;
       st = time_best(
           e,
@@ -1122,37 +1085,41 @@ bool admit(fdas_engine* e, fdas_engine::Ctx& c, bool others_in_flight, bool& mem
     picked.push_back(t);
   }
   if (picked.empty()) return progress;
-  // Pinned read-back area of the context.
-  uint64_t rb = 0;
-  for (const Trial& t : picked) rb += t.lay.small_bytes;
-  if (rb > c.h_read_cap) {
-    (void)hipHostFree(c.h_read);
-    c.h_read = nullptr;
-    c.h_read_cap = 0;
-    if (host_alloc(e, &c.h_read, rb) == FDAS_OK) c.h_read_cap = rb;
+  // Host memory of the context's lists.
+  uint64_t lists = 0;
+  for (const Trial& t : picked) lists += t.lay.host_bytes;
+  if (lists > c.h_lists_cap) {
+    (void)hipHostFree(c.h_lists);
+    c.h_lists = nullptr;
+    c.h_lists_cap = 0;
+    if (host_alloc(e, &c.h_lists, lists, hipHostMallocCoherent) == FDAS_OK) c.h_lists_cap = lists;
   }
-  fdas_status st = c.h_read ? FDAS_OK : FDAS_ENOMEM;
+  fdas_status st = c.h_lists ? FDAS_OK : FDAS_ENOMEM;
   uint64_t off = 0;
   std::vector<Trial*> ptrs;
+  // Uploads go on a stream of their own, beside the kernels of the groups in flight.
   for (Trial& t : picked) {
-    t.h_read = c.h_read + off;
-    off += t.lay.small_bytes;
+    t.h_lists = c.h_lists + off;
+    off += t.lay.host_bytes;
     if (t.req.flags & FDAS_REQ_DEVICE_SPECTRUM) {
       t.input = static_cast<const float2*>(t.req.spectrum);
     } else {
       t.input = reinterpret_cast<const float2*>(t.mem + t.lay.input);
       if (st == FDAS_OK && hipMemcpyAsync(t.mem + t.lay.input, t.req.spectrum, 8ull * t.req.n_bins,
-                                          hipMemcpyHostToDevice, e->s_ftc) != hipSuccess)
+                                          hipMemcpyHostToDevice, e->s_up) != hipSuccess)
         st = fail(e, FDAS_EDEVICE, "spectrum upload of request %llu failed", (unsigned long long)t.req.tag);
     }
     ptrs.push_back(&t);
   }
   if (st == FDAS_OK) st = build_group(e, c.buf, ptrs);
-  if (st == FDAS_OK) st = upload_group(e, c.buf, group_ftc_jobs(c.buf), group_hsum_jobs(c.buf), e->s_ftc);
-  if (st == FDAS_OK) st = enqueue_group(e, c.buf, ptrs, nullptr, e->last_hsum, false);
-  if (st == FDAS_OK) e->last_hsum = c.buf.ev_hsum_done;
+  if (st == FDAS_OK) st = upload_group(e, c.buf, e->s_up);
+  if (st == FDAS_OK && (launch_clear_counters(c.buf.d_sel, c.buf.n_sel, e->s_up) != hipSuccess ||
+                        hipEventRecord(c.buf.ev_up, e->s_up) != hipSuccess))
+    st = fail(e, FDAS_EDEVICE, "upload of a served group failed");
+  if (st == FDAS_OK) st = enqueue_group(e, c.buf, c.buf.ev_up, /*lagged=*/true, false);
   if (st != FDAS_OK) {
     // The streams may hold part of the group: drain them before the memory goes back.
+    (void)hipStreamSynchronize(e->s_up);
     (void)hipStreamSynchronize(e->s_ftc);
     (void)hipStreamSynchronize(e->s_hsum);
     for (Trial& t : picked) {
@@ -1251,6 +1218,7 @@ static fdas_status engine_init(fdas_engine* e) {
     if (ch == ' ' || ch == '\t' || ch == '|') ch = '_';
   EHIP(e, hipStreamCreateWithFlags(&e->s_ftc, hipStreamNonBlocking));
   EHIP(e, hipStreamCreateWithFlags(&e->s_hsum, hipStreamNonBlocking));
+  EHIP(e, hipStreamCreateWithFlags(&e->s_up, hipStreamNonBlocking));
   for (uint32_t tile : kTileSizes) {
     std::vector<float2> tw1, tw2;
     make_twiddles(tile, tw1, tw2);
@@ -1322,11 +1290,12 @@ void fdas_engine_destroy(fdas_engine* e) {
     std::lock_guard<std::mutex> lk(e->api_mu);
     while (!e->plans.empty()) plan_release(e, e->plans.back());
   }
+  if (e->s_up) (void)hipStreamSynchronize(e->s_up);
   if (e->s_ftc) (void)hipStreamSynchronize(e->s_ftc);
   if (e->s_hsum) (void)hipStreamSynchronize(e->s_hsum);
   for (auto& c : e->ctxs) {
     free_group(c.buf);
-    (void)hipHostFree(c.h_read);
+    (void)hipHostFree(c.h_lists);
   }
   for (auto& b : e->banks)
     for (auto& kv : b->spectra) (void)hipFree(kv.second);
@@ -1338,6 +1307,7 @@ void fdas_engine_destroy(fdas_engine* e) {
   e->arena.reset();
   if (e->s_ftc) (void)hipStreamDestroy(e->s_ftc);
   if (e->s_hsum) (void)hipStreamDestroy(e->s_hsum);
+  if (e->s_up) (void)hipStreamDestroy(e->s_up);
   delete e;
 }
 
@@ -1494,7 +1464,7 @@ fdas_status fdas_plan_create(fdas_engine* e, const fdas_request* reqs, uint32_t 
     for (char* r : p->regions) e->arena->free(r);
     for (char* m : p->inputs) e->arena->free(m);
     for (auto& b : p->bufs) free_group(b);
-    (void)hipHostFree(p->h_read);
+    (void)hipHostFree(p->h_lists);
     if (p->ev_start) (void)hipEventDestroy(p->ev_start);
     if (p->ev_end) (void)hipEventDestroy(p->ev_end);
     return st;
@@ -1520,22 +1490,26 @@ fdas_status fdas_plan_create(fdas_engine* e, const fdas_request* reqs, uint32_t 
       return cleanup(fail(e, FDAS_ENOMEM, "no room in the HBM budget for the device copy of spectrum %u", i));
     p->region_bytes += align_up(8ull * p->trials[i].req.n_bins);
   }
-  // Small parts of all trials in one array (and its pinned mirror), in trial order.
-  uint64_t rb = 0;
-  for (const Trial& t : p->trials) rb += t.lay.small_bytes;
+  // Small parts of all trials in one array, and their lists in one host array, in trial order.
+  uint64_t lists = 0;
+  for (const Trial& t : p->trials) {
+    p->small_bytes += t.lay.small_bytes;
+    lists += t.lay.host_bytes;
+  }
   {
     hipError_t herr = hipSuccess;
-    p->small_all = e->arena->alloc(rb, &herr);
-    if (!p->small_all) return cleanup(fail(e, FDAS_ENOMEM, "no room in the HBM budget for the plan's lists"));
-    p->region_bytes += align_up(rb);
+    p->small_all = e->arena->alloc(p->small_bytes, &herr);
+    if (!p->small_all) return cleanup(fail(e, FDAS_ENOMEM, "no room in the HBM budget for the plan's counters"));
+    p->region_bytes += align_up(p->small_bytes);
   }
-  fdas_status st = host_alloc(e, &p->h_read, rb);
+  fdas_status st = host_alloc(e, &p->h_lists, lists, hipHostMallocCoherent);
   if (st != FDAS_OK) return cleanup(st);
-  uint64_t roff = 0;
+  uint64_t soff = 0, loff = 0;
   for (Trial& t : p->trials) {
-    t.small = p->small_all + roff;
-    t.h_read = p->h_read + roff;
-    roff += t.lay.small_bytes;
+    t.small = p->small_all + soff;
+    t.h_lists = p->h_lists + loff;
+    soff += t.lay.small_bytes;
+    loff += t.lay.host_bytes;
   }
   p->bufs.resize(n_groups);
   for (uint32_t g = 0; g < n_groups; ++g) {
@@ -1550,9 +1524,7 @@ fdas_status fdas_plan_create(fdas_engine* e, const fdas_request* reqs, uint32_t 
       ptrs.push_back(&t);
     }
     if ((st = build_group(e, p->bufs[g], ptrs)) != FDAS_OK) return cleanup(st);
-    if ((st = upload_group(e, p->bufs[g], group_ftc_jobs(p->bufs[g]), group_hsum_jobs(p->bufs[g]), e->s_ftc)) !=
-        FDAS_OK)
-      return cleanup(st);
+    if ((st = upload_group(e, p->bufs[g], e->s_ftc)) != FDAS_OK) return cleanup(st);
   }
   if (hipStreamSynchronize(e->s_ftc) != hipSuccess) return cleanup(fail(e, FDAS_EDEVICE, "job upload failed"));
   if (hipEventCreate(&p->ev_start) != hipSuccess || hipEventCreate(&p->ev_end) != hipSuccess)
@@ -1584,9 +1556,7 @@ fdas_status fdas_plan_set_request(fdas_plan* p, uint32_t i, const void* spectrum
     for (uint32_t j : p->groups[g]) ptrs.push_back(&p->trials[j]);
     fdas_status st = build_group(e, p->bufs[g], ptrs);
     if (st != FDAS_OK) return st;
-    if ((st = upload_group(e, p->bufs[g], group_ftc_jobs(p->bufs[g]), group_hsum_jobs(p->bufs[g]), e->s_ftc)) !=
-        FDAS_OK)
-      return st;
+    if ((st = upload_group(e, p->bufs[g], e->s_ftc)) != FDAS_OK) return st;
     EHIP(e, hipStreamSynchronize(e->s_ftc));
   }
   return FDAS_OK;
@@ -1596,26 +1566,17 @@ fdas_status fdas_plan_set_request(fdas_plan* p, uint32_t i, const void* spectrum
 // (g = 0..G) runs group g's FT convolution together with group g-1's harmonic
 // summing, as one fused kernel when the pair's shapes allow it (1024-point
 // tiles, one summing shape), else as consecutive kernels.  Group g-1's
-// selection and read-back follow on stream B beside launch g+1.
+// selection follows on stream B beside launch g+1.
 static fdas_status plan_enqueue_lagged(fdas_plan* p, bool capturing) {
   fdas_engine* e = p->eng;
   hipStream_t A = e->s_ftc, B = e->s_hsum;
   const uint32_t R = uint32_t(p->regions.size()), G = uint32_t(p->groups.size());
-  std::vector<std::vector<Trial*>> ptrs(G);
-  for (uint32_t g = 0; g < G; ++g)
-    for (uint32_t i : p->groups[g]) ptrs[g].push_back(&p->trials[i]);
+  // The counters of all groups at once (the small parts are not shared like the regions).
+  EHIP(e, launch_zero_u32(reinterpret_cast<uint32_t*>(p->small_all), uint32_t(p->small_bytes / 4), A));
   for (uint32_t g = 0; g <= G; ++g) {
     GroupBuf* cur = g < G ? &p->bufs[g] : nullptr;    // convolved in this launch
     GroupBuf* prev = g > 0 ? &p->bufs[g - 1] : nullptr;  // summed in this launch
     if (cur && g >= R) EHIP(e, hipStreamWaitEvent(A, p->bufs[g - R].ev_done, 0));  // its region is free again
-    if (prev) {
-      if (prev->small_span) {
-        EHIP(e, launch_zero_u32(reinterpret_cast<uint32_t*>(prev->small_span), uint32_t(prev->span_bytes / 4), A));
-      } else {
-        for (const Trial* t : ptrs[g - 1])
-          EHIP(e, launch_zero_u32(reinterpret_cast<uint32_t*>(t->small), uint32_t(t->lay.small_bytes / 4), A));
-      }
-    }
     const bool fuse = p->schedule == FDAS_SCHEDULE_FUSED && cur && prev && cur->ftc.size() == 1 &&
                       prev->hsum.size() == 1 && cur->ftc[0].tile == 1024 &&
                       fused_supported(1024, prev->hsum[0].H, prev->hsum[0].whole_groups);
@@ -1651,12 +1612,6 @@ static fdas_status plan_enqueue_lagged(fdas_plan* p, bool capturing) {
       EHIP(e, hipEventRecord(prev->ev_hsum_done, A));
       EHIP(e, hipStreamWaitEvent(B, prev->ev_hsum_done, 0));
       EHIP(e, launch_select(prev->d_sel, prev->n_sel, e->cfg.cands_per_harmonic, B));
-      if (prev->small_span) {
-        EHIP(e, hipMemcpyAsync(prev->h_span, prev->small_span, prev->span_bytes, hipMemcpyDeviceToHost, B));
-      } else {
-        for (const Trial* t : ptrs[g - 1])
-          EHIP(e, hipMemcpyAsync(t->h_read, t->small, t->lay.readback_bytes, hipMemcpyDeviceToHost, B));
-      }
       EHIP(e, hipEventRecord(prev->ev_done, B));
     }
   }
@@ -1665,15 +1620,13 @@ static fdas_status plan_enqueue_lagged(fdas_plan* p, bool capturing) {
 }
 
 // Two streams: group g's convolution (stream A) runs beside group g-1's
-// summing, selection and read-back (stream B).
+// summing and selection (stream B).
 static fdas_status plan_enqueue_streams(fdas_plan* p, bool capturing) {
   fdas_engine* e = p->eng;
   const uint32_t R = uint32_t(p->regions.size());
   for (uint32_t g = 0; g < p->groups.size(); ++g) {
-    std::vector<Trial*> ptrs;
-    for (uint32_t i : p->groups[g]) ptrs.push_back(&p->trials[i]);
-    const fdas_status st =
-        enqueue_group(e, p->bufs[g], ptrs, g >= R ? p->bufs[g - R].ev_done : nullptr, nullptr, !capturing);
+    const fdas_status st = enqueue_group(e, p->bufs[g], g >= R ? p->bufs[g - R].ev_done : nullptr, /*lagged=*/false,
+                                         !capturing);
     if (st != FDAS_OK) return st;
   }
   EHIP(e, hipStreamWaitEvent(e->s_ftc, p->bufs.back().ev_done, 0));  // join the summing stream
@@ -1787,7 +1740,7 @@ static void plan_release(fdas_engine* e, fdas_plan* p) {
   for (char* r : p->regions) e->arena->free(r);
   for (char* m : p->inputs) e->arena->free(m);
   if (p->small_all) e->arena->free(p->small_all);
-  (void)hipHostFree(p->h_read);
+  (void)hipHostFree(p->h_lists);
   if (p->ev_start) (void)hipEventDestroy(p->ev_start);
   if (p->ev_end) (void)hipEventDestroy(p->ev_end);
   e->plans.erase(std::find(e->plans.begin(), e->plans.end(), p));

@@ -57,9 +57,13 @@ struct SelectJob {
   uint32_t* compact_key;      // [compact_cap] entries at or above the cut bin
   float* compact_pwr;
   uint32_t* compact_n;        // zeroed per run
+  // Results, in device memory or in pinned host memory (coherent), which the kernel writes directly: at most
+  // 12 bytes per entry against a copy command of 8 to 16 us per trial.  A single trial of 32768 bins took 126 us
+  // with the copy and takes 106 us without; twelve served requests 7.36 ms and 6.73 ms (see enqueue_group).
   uint32_t* out_key;          // [cap] sorted by key
   float* out_pwr;
   uint32_t* out_n;            // kept entries
+  uint32_t* out_count;        // detections (nullptr: not wanted)
 };
 
 }  // namespace fdas

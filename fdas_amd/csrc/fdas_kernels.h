@@ -75,6 +75,9 @@ hipError_t launch_quantile_bound(const float* maxima, uint32_t nb, uint32_t want
 hipError_t launch_quantile_rank(const SelectJob* d_sel, uint32_t n_harmonics, uint32_t r_lo, uint32_t r_hi,
                                 uint32_t* out, hipStream_t stream);
 
+// Clears what a summing and selection pass counts in (detections, compact counts, histograms).
+hipError_t launch_clear_counters(const SelectJob* d_jobs, uint32_t n_jobs, hipStream_t stream);
+
 hipError_t launch_zero_u32(uint32_t* p, uint32_t n, hipStream_t stream);
 
 // The job descriptors of one trial's launches, taken to the device as the argument

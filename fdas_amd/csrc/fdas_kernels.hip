@@ -1404,7 +1404,7 @@ __global__ __launch_bounds__(THREADS) void select_final_kernel(const SelectJob* 
   __shared__ SelectShared<THREADS, CAP> sh;
   const SelectJob& job = jobs[blockIdx.x];
   const int tid = threadIdx.x;
-  const uint32_t n = min(gld(job.count, 0), job.spill_cap);
+  const uint32_t detected = gld(job.count, 0), n = min(detected, job.spill_cap);
   const uint32_t cap = job.cap;
 
   uint32_t kept;
@@ -1472,7 +1472,11 @@ __global__ __launch_bounds__(THREADS) void select_final_kernel(const SelectJob* 
     gst(job.out_key, e, sh.key[e]);
     gst(job.out_pwr, e, sh.pwr[e]);
   }
-  if (tid == 0) gst(job.out_n, 0, kept);
+  if (tid == 0) {
+    gst(job.out_n, 0, kept);
+    if (job.out_count) gst(job.out_count, 0, detected);
+  }
+  __threadfence_system();  // the results may be in host memory
 }
 
 // ---------------------------------------------------------------------------
@@ -1596,6 +1600,22 @@ hipError_t launch_select(const SelectJob* d_jobs, uint32_t n_jobs, uint32_t cap,
   if (cap <= 1024) launch(select_final_kernel<256, 1024>, n_jobs, 256, stream, ev, d_jobs);
   else if (cap <= 4096) launch(select_final_kernel<1024, 4096>, n_jobs, 1024, stream, ev, d_jobs);
   else launch(select_final_kernel<1024, 8192>, n_jobs, 1024, stream, ev, d_jobs);
+  return hipGetLastError();
+}
+
+// The counters and histograms of a group's selection jobs to zero.
+__global__ __launch_bounds__(256) void clear_counters_kernel(const SelectJob* __restrict__ jobs) {
+  const SelectJob& job = jobs[blockIdx.x];
+  for (uint32_t i = threadIdx.x; i < kSelectBins; i += 256) gst(job.hist, i, 0u);
+  if (threadIdx.x == 0) {
+    gst(job.compact_n, 0, 0u);
+    gst(const_cast<uint32_t*>(job.count), 0, 0u);
+  }
+}
+
+hipError_t launch_clear_counters(const SelectJob* d_jobs, uint32_t n_jobs, hipStream_t stream) {
+  if (n_jobs == 0) return hipSuccess;
+  hipLaunchKernelGGL(clear_counters_kernel, dim3(n_jobs), dim3(256), 0, stream, d_jobs);
   return hipGetLastError();
 }
 

@@ -155,6 +155,7 @@ extern "C" fdas_status fdas_hsum_noalloc(const float* d_fop, uint32_t n_bins, ui
     q.out_key = d_key + size_t(p) * cap;
     q.out_pwr = d_power + size_t(p) * cap;
     q.out_n = d_counts + p;
+    q.out_count = nullptr;  // the summing kernel counts in d_counts + H itself
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   // Every call shares this device's scratch and keeps no state between calls:

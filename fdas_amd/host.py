@@ -268,7 +268,10 @@ class FDAS:
         self._lib.fdas_print_events(self._ctx, ab)
 
     def stage_times(self, ab) -> np.ndarray:
-        """[input, FT-conv kernel, HSUM kernel, selection, read-back, total] in ms of the last run on ab."""
+        """[input, FT-conv kernel, HSUM kernel, selection, read-back, total] in ms of the last run on ab.
+
+        The selection writes the lists to host memory, so the read-back is 0.
+        """
         out = np.zeros(6, dtype=np.float32)
         self._lib.fdas_get_stage_times(self._ctx, ab, N.fptr(out))
         return out

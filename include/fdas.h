@@ -188,7 +188,8 @@ fdas_status fdas_quantile_thresholds(fdas_ctx* ctx, uint32_t n_per_plane, fdas_p
 
 /* Device durations in ms of the last run on `set` (HIP events on the set's
  * stream): [0] input, [1] FT-convolution kernel, [2] harmonic-summing kernel,
- * [3] candidate selection, [4] candidate read-back, [5] total. */
+ * [3] candidate selection, [4] candidate read-back (0: the selection writes the
+ * lists to host memory), [5] total. */
 fdas_status fdas_get_stage_times(fdas_ctx* ctx, int set, float* ms6);
 
 /* Device enumeration for the platform / device selectors of
