@@ -30,9 +30,15 @@ namespace {
 
 constexpr uint32_t kMaxFtcJobs = 64;  // row groups per FT-convolution launch
 
-// Events per launch: START, INPUT (spectrum in place), FTC_K (FT-convolution kernel start), FTC (its end),
-// HSUM_K0 / HSUM_K1 (harmonic-summing kernel start / end), HSUM (selection end, with the lists in host memory).
-enum Ev { EV_START = 0, EV_INPUT, EV_FTC_K, EV_FTC, EV_HSUM_K0, EV_HSUM_K1, EV_HSUM, EV_COUNT };
+// Device times of a launch (clock ticks, in pinned host memory, 0: not taken): START, INPUT (spectrum in place),
+// FTC_K (FT-convolution kernel start), FTC (its end where no summing follows at once), HSUM_K0 (harmonic-summing
+// kernel start), HSUM_K1 (selection start), then the end of each plane's selection.
+enum Stamp { ST_START = 0, ST_INPUT, ST_FTC_K, ST_FTC, ST_HSUM_K0, ST_HSUM_K1, ST_ENDS, ST_COUNT = ST_ENDS + kMaxHarmonics };
+
+// Host spectra up to this size are taken through pinned memory by a kernel; larger ones by a copy command.  Launch and
+// wait with 5 templates, by copy command and by kernel: 74 and 44 us at 4096 bins, 73 and 62 at 32768, 109 and 93 at
+// 2^17 (1 MiB), 139 and 138 at 2^18, 199 and 210 at 2^19, where the host's copy costs more than the signal saves.
+constexpr size_t kStagedInput = 1 << 20;
 
 struct DevSet {
   float2* input = nullptr;
@@ -60,11 +66,15 @@ struct DevSet {
   uint32_t* h_quant = nullptr;     // [4H] mirror of quant's tail
 
   hipStream_t stream = nullptr;
-  hipEvent_t ev[EV_COUNT] = {};
+  uint64_t* h_stamp = nullptr;       // [ST_COUNT] pinned
+  bool ftc_to_hsum = false;          // the summing followed the convolution at once: its start is the other's end
+  float2* h_input = nullptr;         // pinned staging of small host spectra
+  bool input_pending = false;        // h_input may still be read by the device
+  hipEvent_t hsum_done = nullptr;    // end of the last summing kernel, where the other set is in use
   hipEvent_t staged_ftc = nullptr;   // h_ftc may be rewritten once this completes
-  bool hsum_issued = false;          // a harmonic-summing kernel (its end: ev[EV_HSUM_K1]) has been launched
+  bool used = false;                 // a convolution has been launched
+  bool hsum_recorded = false;        // hsum_done has been recorded
   bool ftc_pending = false;
-  bool ev_recorded[EV_COUNT] = {};
 
   std::vector<FtcJob> ftc_plan[3];  // convolution jobs per part (empty: not planned for these templates)
   std::vector<uint32_t> row_taps;  // non-zero extent of each template row (sets per-group overlaps)
@@ -97,7 +107,8 @@ struct fdas_ctx {
   float2* tw1 = nullptr;
   float2* tw2 = nullptr;
   DevSet set[2];
-  hipEvent_t epoch = nullptr;
+  uint64_t epoch = 0;       // device clock at creation
+  double clock_khz = 1e5;
   bool sync_pipeline = false;
   // print_stats state; the reference keeps it file-static (FDAS.cpp:640-641)
   float pipeline_start = 0.f;
@@ -195,20 +206,45 @@ fdas_status wait_staging(fdas_ctx* ctx, hipEvent_t ev, bool& pending) {
   return FDAS_OK;
 }
 
-fdas_status record(fdas_ctx* ctx, DevSet& s, Ev e) {
-  HIPCK(ctx, hipEventRecord(s.ev[e], s.stream));
-  s.ev_recorded[e] = true;
+void clear_stamps(DevSet& s, int from, int to) {
+  for (int i = from; i <= to; ++i) reinterpret_cast<volatile uint64_t*>(s.h_stamp)[i] = 0;
+}
+
+fdas_status stamp(fdas_ctx* ctx, DevSet& s, Stamp at) {
+  HIPCK(ctx, launch_stamp(s.stream, s.h_stamp + at));
   return FDAS_OK;
 }
 
-float elapsed(const DevSet& s, int a, int b) {
-  if (!s.ev_recorded[a] || !s.ev_recorded[b]) return 0.f;
-  float ms = 0.f;
-  if (hipEventElapsedTime(&ms, s.ev[a], s.ev[b]) != hipSuccess) {
-    (void)hipGetLastError();
-    return 0.f;
+// The clock at a stamp (ST_ENDS: the last plane's), 0 where it was not taken.
+uint64_t clock_at(const fdas_ctx* ctx, const DevSet& s, int at) {
+  const volatile uint64_t* t = s.h_stamp;
+  if (at == ST_FTC && s.ftc_to_hsum) at = ST_HSUM_K0;
+  if (at != ST_ENDS) return t[at];
+  uint64_t last = 0;
+  for (uint32_t p = 0; p < ctx->cfg.n_harmonics; ++p) {
+    const uint64_t v = t[ST_ENDS + p];
+    if (v == 0) return 0;
+    last = std::max(last, v);
   }
-  return ms;
+  return last;
+}
+
+float elapsed(const fdas_ctx* ctx, const DevSet& s, int a, int b) {
+  const uint64_t ta = clock_at(ctx, s, a), tb = clock_at(ctx, s, b);
+  return ta && tb > ta ? float(double(tb - ta) / ctx->clock_khz) : 0.f;
+}
+
+// Milliseconds since creation, 0 where the stamp was not taken.
+float since_epoch(const fdas_ctx* ctx, const DevSet& s, int at) {
+  const uint64_t t = clock_at(ctx, s, at);
+  return t > ctx->epoch ? float(double(t - ctx->epoch) / ctx->clock_khz) : 0.f;
+}
+
+// Waits for the set's stream: lists and stamps are in host memory, the staged spectrum has been read.
+fdas_status drain(fdas_ctx* ctx, DevSet& s) {
+  HIPCK(ctx, hipStreamSynchronize(s.stream));
+  s.input_pending = false;
+  return FDAS_OK;
 }
 
 // The convolution jobs of the part.  Planned once per part and template bank: the
@@ -296,10 +332,10 @@ void fill_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr) {
 }
 
 // Takes the pack's jobs to the device, with the counters cleared when a summing pass is among them.
-fdas_status put_jobs(fdas_ctx* ctx, DevSet& s) {
+fdas_status put_jobs(fdas_ctx* ctx, DevSet& s, uint64_t* stamp = nullptr, uint64_t* stamp2 = nullptr) {
   ZeroSpan zero;
   if (s.pack.n_sel) zero = {s.counts, ctx->cfg.n_harmonics * (2 + kSelectBins)};
-  HIPCK(ctx, launch_put_jobs(s.pack, s.d_ftc, s.d_hsum, s.d_sel, zero, {}, s.stream));
+  HIPCK(ctx, launch_put_jobs(s.pack, s.d_ftc, s.d_hsum, s.d_sel, zero, {}, s.stream, stamp, stamp2));
   s.pack.n_ftc = s.pack.n_sel = 0;
   return FDAS_OK;
 }
@@ -310,10 +346,10 @@ fdas_status run_ftc(fdas_ctx* ctx, DevSet& s, uint32_t n_jobs, uint32_t n_items)
   // and side by side they only slow each other down), while that set's
   // selection, and this set's input copy, still overlap.
   const DevSet& other = &s == &ctx->set[0] ? ctx->set[1] : ctx->set[0];
-  if (other.hsum_issued) HIPCK(ctx, hipStreamWaitEvent(s.stream, other.ev[EV_HSUM_K1], 0));
+  if (other.hsum_recorded) HIPCK(ctx, hipStreamWaitEvent(s.stream, other.hsum_done, 0));
+  s.used = true;
   HIPCK(ctx, launch_ftconv(int(ctx->cfg.tile), s.d_ftc, n_jobs, n_items, ctx->tw1, ctx->tw2, n_items, s.stream,
-                           {s.ev[EV_FTC_K], s.ev[EV_FTC]}));
-  s.ev_recorded[EV_FTC_K] = s.ev_recorded[EV_FTC] = true;
+                           s.h_stamp + ST_FTC_K));
   return FDAS_OK;
 }
 
@@ -322,34 +358,54 @@ fdas_status run_hsum(fdas_ctx* ctx, DevSet& s) {
   const uint32_t H = ctx->cfg.n_harmonics;
   const HsumJob& j = s.pack.hsum;
   const uint32_t blocks = (ctx->geo.n_bins + kHsumBinsPerBlock - 1) / kHsumBinsPerBlock * j.n_row_chunks;
-  HIPCK(ctx, launch_hsum(s.d_hsum, 1, blocks, H, s.stream, {s.ev[EV_HSUM_K0], s.ev[EV_HSUM_K1]}));
-  s.hsum_issued = true;
-  HIPCK(ctx, launch_select(s.d_sel, H, ctx->cfg.cands_per_harmonic, s.stream, s.ev[EV_HSUM]));
-  s.ev_recorded[EV_HSUM_K0] = s.ev_recorded[EV_HSUM_K1] = s.ev_recorded[EV_HSUM] = true;
+  HIPCK(ctx, launch_hsum(s.d_hsum, 1, blocks, H, s.stream, s.h_stamp + ST_HSUM_K0));
+  const DevSet& other = &s == &ctx->set[0] ? ctx->set[1] : ctx->set[0];
+  if (other.used) {  // its next convolution waits for this summing
+    HIPCK(ctx, hipEventRecord(s.hsum_done, s.stream));
+    s.hsum_recorded = true;
+  }
+  HIPCK(ctx, launch_select(s.d_sel, H, ctx->cfg.cands_per_harmonic, s.stream, s.h_stamp + ST_HSUM_K1,
+                           s.h_stamp + ST_ENDS));
   return FDAS_OK;
 }
 
-fdas_status enqueue_ftc(fdas_ctx* ctx, DevSet& s, fdas_part part) {
+// Convolution alone.  start: the sequence starts here (no input step before it).
+fdas_status enqueue_ftc(fdas_ctx* ctx, DevSet& s, fdas_part part, bool start) {
+  clear_stamps(s, start ? ST_START : ST_INPUT, ST_FTC);
+  s.ftc_to_hsum = false;
+  uint64_t* const at_start = start ? s.h_stamp + ST_START : nullptr;
   uint32_t n_jobs, n_items;
   fdas_status st = fill_ftc(ctx, s, part, &n_jobs, &n_items);
   if (st != FDAS_OK) return st;
-  if (s.pack.n_ftc && (st = put_jobs(ctx, s)) != FDAS_OK) return st;
-  return run_ftc(ctx, s, n_jobs, n_items);
+  // (with no jobs in the pack the kernel takes the stamps only)
+  if ((st = put_jobs(ctx, s, s.h_stamp + ST_INPUT, at_start)) != FDAS_OK) return st;
+  if ((st = run_ftc(ctx, s, n_jobs, n_items)) != FDAS_OK) return st;
+  return stamp(ctx, s, ST_FTC);
+}
+
+// A summing pass on its own: the convolution's end is kept, the pass's times are not taken yet.
+void restart_hsum_stamps(DevSet& s) {
+  if (s.ftc_to_hsum) s.h_stamp[ST_FTC] = s.h_stamp[ST_HSUM_K0];
+  s.ftc_to_hsum = false;
+  clear_stamps(s, ST_HSUM_K0, ST_COUNT - 1);
 }
 
 fdas_status enqueue_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr) {
+  restart_hsum_stamps(s);
   fill_hsum(ctx, s, part, thr);
   const fdas_status st = put_jobs(ctx, s);
   return st == FDAS_OK ? run_hsum(ctx, s) : st;
 }
 
 // Convolution and summing of one launch, their jobs taken to the device together.
-fdas_status enqueue_search(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr) {
+fdas_status enqueue_search(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr, bool start) {
+  clear_stamps(s, start ? ST_START : ST_INPUT, ST_COUNT - 1);
+  s.ftc_to_hsum = true;
   uint32_t n_jobs, n_items;
   fdas_status st = fill_ftc(ctx, s, part, &n_jobs, &n_items);
   if (st != FDAS_OK) return st;
   fill_hsum(ctx, s, part, thr);
-  if ((st = put_jobs(ctx, s)) != FDAS_OK) return st;
+  if ((st = put_jobs(ctx, s, s.h_stamp + ST_INPUT, start ? s.h_stamp + ST_START : nullptr)) != FDAS_OK) return st;
   if ((st = run_ftc(ctx, s, n_jobs, n_items)) != FDAS_OK) return st;
   return run_hsum(ctx, s);
 }
@@ -414,8 +470,9 @@ void free_set(DevSet& s) {
   (void)hipHostFree(s.h_quant);
   (void)hipHostFree(s.h_ftc);
   (void)hipHostFree(s.h_out_key);  // and h_out_pwr, h_out_n, h_counts
-  for (auto& e : s.ev)
-    if (e) (void)hipEventDestroy(e);
+  if (s.hsum_done) (void)hipEventDestroy(s.hsum_done);
+  (void)hipHostFree(s.h_stamp);
+  (void)hipHostFree(s.h_input);
   if (s.staged_ftc) (void)hipEventDestroy(s.staged_ftc);
   if (s.stream) (void)hipStreamDestroy(s.stream);
   s = DevSet{};
@@ -494,7 +551,6 @@ extern "C" fdas_status fdas_create(const fdas_config* cfg, fdas_log_fn log, void
     for (auto& set : ctx->set) free_set(set);
     (void)hipFree(ctx->tw1);
     (void)hipFree(ctx->tw2);
-    if (ctx->epoch) (void)hipEventDestroy(ctx->epoch);
     delete ctx;
     return s;
   };
@@ -528,7 +584,9 @@ extern "C" fdas_status fdas_create(const fdas_config* cfg, fdas_log_fn log, void
     fail(ctx, FDAS_EDEVICE, "twiddle upload failed");
     return bail(FDAS_EDEVICE);
   }
-  if (hipEventCreate(&ctx->epoch) != hipSuccess) return bail(fail(ctx, FDAS_EDEVICE, "event creation failed"));
+  int khz = 0;
+  if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, cfg->device) == hipSuccess && khz > 0)
+    ctx->clock_khz = khz;
 
   const size_t N = cfg->n_bins, T = cfg->n_templates, H = cfg->n_harmonics, cap = cfg->cands_per_harmonic;
   for (auto& s : ctx->set) {
@@ -552,17 +610,22 @@ extern "C" fdas_status fdas_create(const fdas_config* cfg, fdas_log_fn log, void
     std::memset(s.h_counts, 0, sizeof(uint32_t) * H);
     if (hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) != hipSuccess)
       return bail(fail(ctx, FDAS_EDEVICE, "stream creation failed"));
-    for (auto& ev : s.ev)
-      if (hipEventCreate(&ev) != hipSuccess) return bail(fail(ctx, FDAS_EDEVICE, "event creation failed"));
-    if (hipEventCreateWithFlags(&s.staged_ftc, hipEventDisableTiming) != hipSuccess)
+    if ((st = host_alloc(ctx, &s.h_stamp, ST_COUNT, hipHostMallocCoherent)) != FDAS_OK) return bail(st);
+    clear_stamps(s, 0, ST_COUNT - 1);
+    if (N * sizeof(float2) <= kStagedInput && (st = host_alloc(ctx, &s.h_input, N)) != FDAS_OK) return bail(st);
+    if (hipEventCreateWithFlags(&s.hsum_done, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&s.staged_ftc, hipEventDisableTiming) != hipSuccess)
       return bail(fail(ctx, FDAS_EDEVICE, "event creation failed"));
     // a FOP that was never written reads as zeros
     if (hipMemset(s.fop, 0, T * N * sizeof(float)) != hipSuccess ||
         hipMemset(s.counts, 0, H * (2 + kSelectBins) * sizeof(uint32_t)) != hipSuccess)
       return bail(fail(ctx, FDAS_EDEVICE, "buffer initialisation failed"));
   }
-  if (hipDeviceSynchronize() != hipSuccess) return bail(fail(ctx, FDAS_EDEVICE, "device synchronisation failed"));
-  (void)hipEventRecord(ctx->epoch, ctx->set[0].stream);
+  uint64_t* const clock = ctx->set[0].h_stamp;
+  if (launch_stamp(ctx->set[0].stream, clock) != hipSuccess || hipDeviceSynchronize() != hipSuccess)
+    return bail(fail(ctx, FDAS_EDEVICE, "device synchronisation failed"));
+  ctx->epoch = *static_cast<volatile uint64_t*>(clock);
+  *clock = 0;
   info(ctx, "Geometry: N=%u, T=%u, S=%u, overlap=%u, payload=%u, tiles=%u, H=%u, cap=%u, spill=%u", cfg->n_bins,
        cfg->n_templates, S, ctx->geo.overlap, ctx->geo.payload, ctx->geo.n_tiles, cfg->n_harmonics,
        cfg->cands_per_harmonic, ctx->spill);
@@ -578,7 +641,6 @@ extern "C" void fdas_destroy(fdas_ctx* ctx) {
   for (auto& s : ctx->set) free_set(s);
   (void)hipFree(ctx->tw1);
   (void)hipFree(ctx->tw2);
-  if (ctx->epoch) (void)hipEventDestroy(ctx->epoch);
   delete ctx;
 }
 
@@ -666,15 +728,49 @@ extern "C" fdas_status fdas_upload_thresholds(fdas_ctx* ctx, const float* thresh
   return FDAS_OK;
 }
 
+// Whether this device can read the whole spectrum where it is: device memory of its own, 8-byte aligned.
+static bool readable_spectrum(const fdas_ctx* ctx, const void* src, size_t bytes) {
+  hipPointerAttribute_t attr{};
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipPointerGetAttributes(&attr, src) != hipSuccess ||
+      hipMemGetAddressRange(&base, &size, const_cast<void*>(src)) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  const uintptr_t p = reinterpret_cast<uintptr_t>(src), b = reinterpret_cast<uintptr_t>(base);
+  return attr.type == hipMemoryTypeDevice && attr.device == ctx->cfg.device && p % sizeof(float2) == 0 && p >= b &&
+         size >= bytes && p - b <= size - bytes;
+}
+
+// The spectrum into the set's buffer.  By a kernel, which the next one follows within 2 us, where it can be read:
+// device memory, and host memory up to kStagedInput after a copy to pinned memory, as the runtime also makes one; a
+// copy command's completion signal takes about 10 us to let the next kernel start.
 static fdas_status upload_input(fdas_ctx* ctx, DevSet& s, const void* src, hipMemcpyKind kind) {
+  const size_t bytes = sizeof(float2) * ctx->geo.n_bins;
   fdas_status st;
-  if ((st = record(ctx, s, EV_START)) != FDAS_OK) return st;
-  HIPCK(ctx, hipMemcpyAsync(s.input, src, sizeof(float2) * ctx->geo.n_bins, kind, s.stream));
+  if (s.input_pending && (st = drain(ctx, s)) != FDAS_OK) return st;
+  clear_stamps(s, 0, ST_COUNT - 1);
+  s.ftc_to_hsum = false;
+  const float2* from = nullptr;
+  if (kind == hipMemcpyHostToDevice && s.h_input) {
+    std::memcpy(s.h_input, src, bytes);
+    s.input_pending = true;
+    from = s.h_input;
+  } else if (kind == hipMemcpyDeviceToDevice && readable_spectrum(ctx, src, bytes)) {
+    from = static_cast<const float2*>(src);
+  }
+  if (from) {
+    HIPCK(ctx, launch_copy_spectrum(from, s.input, ctx->geo.n_bins, s.stream, s.h_stamp + ST_START,
+                                    s.h_stamp + ST_INPUT));
+  } else {
+    if ((st = stamp(ctx, s, ST_START)) != FDAS_OK) return st;
+    HIPCK(ctx, hipMemcpyAsync(s.input, src, bytes, kind, s.stream));
+  }
   s.has_input = true;
   s.fop_valid = false;
   s.cands_valid = false;
   s.tiles_valid = false;
-  for (int e = EV_INPUT; e < EV_COUNT; ++e) s.ev_recorded[e] = false;
   return FDAS_OK;
 }
 
@@ -688,12 +784,10 @@ extern "C" fdas_status fdas_perform_input_tiling(fdas_ctx* ctx, const float* spe
   if ((st = upload_input(ctx, s, spectrum_c64, hipMemcpyHostToDevice)) != FDAS_OK) return st;
   HIPCK(ctx, launch_tiles(int(ctx->cfg.tile), s.input, ctx->geo.n_bins, ctx->geo.overlap, ctx->geo.payload,
                           ctx->geo.n_tiles, ctx->tw1, ctx->tw2, s.tiles, s.stream));
-  if ((st = record(ctx, s, EV_INPUT)) != FDAS_OK) return st;
-  HIPCK(ctx, hipEventSynchronize(s.ev[EV_INPUT]));
+  if ((st = stamp(ctx, s, ST_INPUT)) != FDAS_OK) return st;
+  if ((st = drain(ctx, s)) != FDAS_OK) return st;
   s.tiles_valid = true;
-  float ms = 0.f;
-  (void)hipEventElapsedTime(&ms, s.ev[EV_START], s.ev[EV_INPUT]);
-  info(ctx, "Preparation duration: %.3f ms", double(ms));
+  info(ctx, "Preparation duration: %.3f ms", double(elapsed(ctx, s, ST_START, ST_INPUT)));
   return FDAS_OK;
 }
 
@@ -702,9 +796,7 @@ extern "C" fdas_status fdas_set_input_device(fdas_ctx* ctx, const void* d_spectr
   if (!d_spectrum_c64) return fail(ctx, FDAS_EINVAL, "null device spectrum");
   DevSet& s = ctx->set[set];
   HIPCK(ctx, hipSetDevice(ctx->cfg.device));
-  fdas_status st;
-  if ((st = upload_input(ctx, s, d_spectrum_c64, hipMemcpyDeviceToDevice)) != FDAS_OK) return st;
-  return record(ctx, s, EV_INPUT);
+  return upload_input(ctx, s, d_spectrum_c64, hipMemcpyDeviceToDevice);
 }
 
 static fdas_status check_ready_ftc(fdas_ctx* ctx, const DevSet& s, fdas_part part) {
@@ -720,14 +812,11 @@ extern "C" fdas_status fdas_perform_ft_convolution(fdas_ctx* ctx, fdas_part part
   fdas_status st = check_ready_ftc(ctx, s, part);
   if (st != FDAS_OK) return st;
   HIPCK(ctx, hipSetDevice(ctx->cfg.device));
-  if ((st = record(ctx, s, EV_INPUT)) != FDAS_OK) return st;
-  if ((st = enqueue_ftc(ctx, s, part)) != FDAS_OK) return st;
-  HIPCK(ctx, hipEventSynchronize(s.ev[EV_FTC]));
+  if ((st = enqueue_ftc(ctx, s, part, false)) != FDAS_OK) return st;
+  if ((st = drain(ctx, s)) != FDAS_OK) return st;
   s.fop_valid = true;
   s.cands_valid = false;
-  float ms = 0.f;
-  (void)hipEventElapsedTime(&ms, s.ev[EV_FTC_K], s.ev[EV_FTC]);
-  info(ctx, "FT convolution and IFFT duration: %.3f ms", double(ms));
+  info(ctx, "FT convolution and IFFT duration: %.3f ms", double(elapsed(ctx, s, ST_FTC_K, ST_FTC)));
   return FDAS_OK;
 }
 
@@ -748,19 +837,18 @@ extern "C" fdas_status fdas_perform_harmonic_summing(fdas_ctx* ctx, const float*
   HIPCK(ctx, hipSetDevice(ctx->cfg.device));
   fdas_status st;
   if ((st = enqueue_hsum(ctx, s, part, thr)) != FDAS_OK) return st;
-  HIPCK(ctx, hipEventSynchronize(s.ev[EV_HSUM]));
+  if ((st = drain(ctx, s)) != FDAS_OK) return st;
   s.cands_valid = true;
-  float ms = 0.f;
-  ms = elapsed(s, EV_HSUM_K0, EV_HSUM_K1) + elapsed(s, EV_HSUM_K1, EV_HSUM);
-  info(ctx, "Harmonic summing duration: %.3f ms", double(ms));
+  info(ctx, "Harmonic summing duration: %.3f ms", double(elapsed(ctx, s, ST_HSUM_K0, ST_ENDS)));
   return overflow_status(ctx, s);
 }
 
 // The work of a launch once its spectrum is on its way: convolution, and summing
 // and selection unless they are held (sync pipeline).
 static fdas_status enqueue_launch(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr, uint32_t* det_loc,
-                                  float* det_pwr) {
-  fdas_status st = ctx->sync_pipeline ? enqueue_ftc(ctx, s, part) : enqueue_search(ctx, s, part, thr);
+                                  float* det_pwr, bool resident) {
+  fdas_status st =
+      ctx->sync_pipeline ? enqueue_ftc(ctx, s, part, resident) : enqueue_search(ctx, s, part, thr, resident);
   if (st != FDAS_OK) return st;
   s.launched = true;
   s.user_loc = det_loc;
@@ -791,8 +879,7 @@ extern "C" fdas_status fdas_launch(fdas_ctx* ctx, const float* spectrum_c64, con
   if (ctx->sync_pipeline && (st = flush_gated(ctx, 1 - set)) != FDAS_OK) return st;
   if (s.gated && (st = flush_gated(ctx, set)) != FDAS_OK) return st;
   if ((st = upload_input(ctx, s, spectrum_c64, hipMemcpyHostToDevice)) != FDAS_OK) return st;
-  if ((st = record(ctx, s, EV_INPUT)) != FDAS_OK) return st;
-  return enqueue_launch(ctx, s, part, thr, det_loc, det_pwr);
+  return enqueue_launch(ctx, s, part, thr, det_loc, det_pwr, false);
 }
 
 extern "C" fdas_status fdas_launch_resident(fdas_ctx* ctx, const float* thresholds, uint32_t* det_loc,
@@ -812,9 +899,7 @@ extern "C" fdas_status fdas_launch_resident(fdas_ctx* ctx, const float* threshol
   fdas_status st;
   if (ctx->sync_pipeline && (st = flush_gated(ctx, 1 - set)) != FDAS_OK) return st;
   if (s.gated && (st = flush_gated(ctx, set)) != FDAS_OK) return st;
-  if ((st = record(ctx, s, EV_START)) != FDAS_OK) return st;
-  if ((st = record(ctx, s, EV_INPUT)) != FDAS_OK) return st;
-  return enqueue_launch(ctx, s, part, thr, det_loc, det_pwr);
+  return enqueue_launch(ctx, s, part, thr, det_loc, det_pwr, true);
 }
 
 extern "C" fdas_status fdas_wait(fdas_ctx* ctx, int set) {
@@ -824,7 +909,7 @@ extern "C" fdas_status fdas_wait(fdas_ctx* ctx, int set) {
   HIPCK(ctx, hipSetDevice(ctx->cfg.device));
   fdas_status st;
   if (s.gated && (st = flush_gated(ctx, set)) != FDAS_OK) return st;
-  HIPCK(ctx, hipEventSynchronize(s.ev[EV_HSUM]));
+  if ((st = drain(ctx, s)) != FDAS_OK) return st;
   s.launched = false;
   s.fop_valid = true;
   s.cands_valid = true;
@@ -882,10 +967,11 @@ extern "C" fdas_status fdas_inject_fop(fdas_ctx* ctx, const float* fop, int set)
   HIPCK(ctx, hipSetDevice(ctx->cfg.device));
   const size_t n = size_t(ctx->cfg.n_templates) * ctx->geo.n_bins;
   fdas_status st;
-  if ((st = record(ctx, s, EV_START)) != FDAS_OK) return st;
-  if ((st = record(ctx, s, EV_INPUT)) != FDAS_OK) return st;
+  clear_stamps(s, ST_START, ST_FTC);
+  s.ftc_to_hsum = false;
+  HIPCK(ctx, launch_stamp(s.stream, s.h_stamp + ST_START, s.h_stamp + ST_INPUT));
   HIPCK(ctx, hipMemcpyAsync(s.fop, fop, n * sizeof(float), hipMemcpyHostToDevice, s.stream));
-  if ((st = record(ctx, s, EV_FTC)) != FDAS_OK) return st;
+  if ((st = stamp(ctx, s, ST_FTC)) != FDAS_OK) return st;
   s.fop_valid = true;
   s.cands_valid = false;
   return FDAS_OK;
@@ -999,6 +1085,7 @@ extern "C" fdas_status fdas_quantile_thresholds(fdas_ctx* ctx, uint32_t n_per_pl
     HIPCK(ctx, hipStreamSynchronize(s.stream));
     return FDAS_OK;
   };
+  restart_hsum_stamps(s);
   s.cands_valid = false;  // the lists will belong to these thresholds, not to a search
   std::vector<float> thr(H, -INFINITY);
   fill_hsum(ctx, s, part, thr.data());
@@ -1064,21 +1151,19 @@ extern "C" fdas_status fdas_get_stage_times(fdas_ctx* ctx, int set, float* ms6) 
   CHECK_SET(ctx, set);
   if (!ms6) return fail(ctx, FDAS_EINVAL, "null output");
   const DevSet& s = ctx->set[set];
-  ms6[0] = elapsed(s, EV_START, EV_INPUT);
-  ms6[1] = elapsed(s, EV_FTC_K, EV_FTC);
-  ms6[2] = elapsed(s, EV_HSUM_K0, EV_HSUM_K1);
-  ms6[3] = elapsed(s, EV_HSUM_K1, EV_HSUM);
+  ms6[0] = elapsed(ctx, s, ST_START, ST_INPUT);
+  ms6[1] = elapsed(ctx, s, ST_FTC_K, ST_FTC);
+  ms6[2] = elapsed(ctx, s, ST_HSUM_K0, ST_HSUM_K1);
+  ms6[3] = elapsed(ctx, s, ST_HSUM_K1, ST_ENDS);
   ms6[4] = 0.f;  // the selection writes the lists to host memory
-  ms6[5] = elapsed(s, EV_START, EV_HSUM);
+  ms6[5] = elapsed(ctx, s, ST_START, ST_ENDS);
   return FDAS_OK;
 }
 
 extern "C" void fdas_print_stats(fdas_ctx* ctx, int set, int reset) {
   if (!ctx || (set != FDAS_SET_A && set != FDAS_SET_B)) return;
   const DevSet& s = ctx->set[set];
-  float t0 = 0.f, t1 = 0.f;
-  (void)hipEventElapsedTime(&t0, ctx->epoch, s.ev[EV_START]);
-  (void)hipEventElapsedTime(&t1, ctx->epoch, s.ev[EV_HSUM]);
+  const float t0 = since_epoch(ctx, s, ST_START), t1 = since_epoch(ctx, s, ST_ENDS);
   if (reset) {
     ctx->pipeline_start = t0;
     ctx->pipeline_accum = 0.f;
@@ -1089,26 +1174,22 @@ extern "C" void fdas_print_stats(fdas_ctx* ctx, int set, int reset) {
   const float acc = t1 - ctx->pipeline_start;
   info(ctx, "Launch  #%u%c complete @ %.3f ms II ~ %.3f ms", ctx->pipeline_launches, set == FDAS_SET_A ? 'A' : 'B',
        double(acc), double(acc - ctx->pipeline_accum));
-  info(ctx, "  Preparation duration: %.3f ms", double(elapsed(s, EV_START, EV_INPUT)));
-  info(ctx, "  FT convolution and IFFT duration: %.3f ms", double(elapsed(s, EV_FTC_K, EV_FTC)));
-  info(ctx, "  Harmonic summing duration: %.3f ms", double(elapsed(s, EV_HSUM_K0, EV_HSUM_K1) + elapsed(s, EV_HSUM_K1, EV_HSUM)));
-  info(ctx, "  Total duration: %.3f ms", double(elapsed(s, EV_START, EV_HSUM)));
+  info(ctx, "  Preparation duration: %.3f ms", double(elapsed(ctx, s, ST_START, ST_INPUT)));
+  info(ctx, "  FT convolution and IFFT duration: %.3f ms", double(elapsed(ctx, s, ST_FTC_K, ST_FTC)));
+  info(ctx, "  Harmonic summing duration: %.3f ms", double(elapsed(ctx, s, ST_HSUM_K0, ST_ENDS)));
+  info(ctx, "  Total duration: %.3f ms", double(elapsed(ctx, s, ST_START, ST_ENDS)));
   ctx->pipeline_accum = acc;
 }
 
 extern "C" void fdas_print_events(fdas_ctx* ctx, int set) {
   if (!ctx || !ctx->log || (set != FDAS_SET_A && set != FDAS_SET_B)) return;
   const DevSet& s = ctx->set[set];
-  float t[EV_COUNT] = {};
-  for (int e = 0; e < EV_COUNT; ++e)
-    if (s.ev_recorded[e]) (void)hipEventElapsedTime(&t[e], ctx->epoch, s.ev[e]);
-  // A kernel's start and end are events of one dispatch, and against another event both give its end.
-  t[EV_FTC_K] = t[EV_FTC] - elapsed(s, EV_FTC_K, EV_FTC);
-  t[EV_HSUM_K0] = t[EV_HSUM_K1] - elapsed(s, EV_HSUM_K0, EV_HSUM_K1);
+  float t[ST_ENDS + 1];
+  for (int i = 0; i <= ST_ENDS; ++i) t[i] = since_epoch(ctx, s, i);
   char buf[256];
   std::snprintf(buf, sizeof(buf), "@@@,%c,%.6f,%.6f,%.6f,%.6f,%.6f,%.6f,%.6f,%.6f", set == FDAS_SET_A ? 'A' : 'B',
-                double(t[EV_START]), double(t[EV_INPUT]), double(t[EV_FTC_K]), double(t[EV_FTC]),
-                double(t[EV_HSUM_K0]), double(t[EV_HSUM_K1]), double(t[EV_HSUM]), double(t[EV_HSUM]));
+                double(t[ST_START]), double(t[ST_INPUT]), double(t[ST_FTC_K]), double(t[ST_FTC]),
+                double(t[ST_HSUM_K0]), double(t[ST_HSUM_K1]), double(t[ST_ENDS]), double(t[ST_ENDS]));
   emit(ctx, FDAS_LOG_INFO, buf);
 }
 

@@ -22,13 +22,10 @@ constexpr uint32_t kSelectSlices = 64;    // workgroups per plane in the histogr
 
 int ftconv_threads(int tile);
 
-// Events of a launch's own dispatch: `start` takes its begin, `stop` its end.  They
-// ride on the dispatch packet; an event recorded between two kernels is a packet of
-// its own there and keeps the second one waiting (about 5 us each).  Not for
-// launches under stream capture.
-struct LaunchEvents {
-  hipEvent_t start = nullptr, stop = nullptr;
-};
+// Times of a launch sequence are read on the device: a kernel given a `stamp` has its first workgroup write the
+// device's constant-rate clock there (pinned host memory) as it starts.  An event between two kernels is a packet of
+// its own, or a signal on the dispatch, that keeps the second kernel waiting for 5 to 9 us; with three events in it a
+// launch of 32768 bins took 106 us, and 88 without.
 
 // Workgroups of the FT-convolution kernel that run at once on the 256 CUs, at three
 // waves per SIMD: 12 one-wave workgroups per CU for 1024-point tiles, 6 and 3 of two
@@ -37,7 +34,7 @@ inline uint32_t ftconv_slots(uint32_t tile) { return 256u * 12u * 1024u / tile; 
 
 // Fused FT convolution over a list of jobs (all with the same tile size).
 hipError_t launch_ftconv(int tile, const FtcJob* d_jobs, uint32_t n_jobs, uint32_t n_items, const float2* tw1,
-                         const float2* tw2, uint32_t grid, hipStream_t stream, LaunchEvents ev = {});
+                         const float2* tw2, uint32_t grid, hipStream_t stream, uint64_t* stamp = nullptr);
 
 // Forward transform of every tile of one spectrum, natural bin order (debug / drop-in retrieve_tiles).
 hipError_t launch_tiles(int tile, const float2* spectrum, uint32_t n_bins, uint32_t overlap, uint32_t payload,
@@ -46,14 +43,14 @@ hipError_t launch_tiles(int tile, const float2* spectrum, uint32_t n_bins, uint3
 // Harmonic summing + thresholding + compaction into per-plane spill lists.
 // All jobs of one launch share n_harmonics; any row lengths go together.
 hipError_t launch_hsum(const HsumJob* d_jobs, uint32_t n_jobs, uint32_t n_blocks, uint32_t n_harmonics,
-                       hipStream_t stream, LaunchEvents ev = {});
+                       hipStream_t stream, uint64_t* stamp = nullptr);
 
 // Per-plane cap (strongest first) and sort by (row, bin): power histogram and
 // compaction over the spill lists (kSelectSlices workgroups per plane), then one
 // workgroup per plane resolves the boundary bin exactly and sorts.  cap: the
-// largest cap of the jobs; stop: event of the last kernel's end.
+// largest cap of the jobs; ends[n_jobs]: when each plane's lists were complete.
 hipError_t launch_select(const SelectJob* d_jobs, uint32_t n_jobs, uint32_t cap, hipStream_t stream,
-                         hipEvent_t stop = nullptr);
+                         uint64_t* stamp = nullptr, uint64_t* ends = nullptr);
 
 // Harmonic plane HP_k over rows [row_begin, row_begin + n_rows) (debug / parity).
 hipError_t launch_hplane(const float* fop, uint32_t n_bins, uint32_t n_templates, uint32_t row_begin,
@@ -95,7 +92,14 @@ struct ZeroSpan {
   uint32_t n = 0;
 };
 hipError_t launch_put_jobs(const JobPack& pack, FtcJob* d_ftc, HsumJob* d_hsum, SelectJob* d_sel, ZeroSpan a,
-                           ZeroSpan b, hipStream_t stream);
+                           ZeroSpan b, hipStream_t stream, uint64_t* stamp = nullptr, uint64_t* stamp2 = nullptr);
+
+// n spectrum bins from device or pinned host memory (8-byte aligned); `end`: the last workgroup's end.
+hipError_t launch_copy_spectrum(const float2* src, float2* dst, uint32_t n, hipStream_t stream, uint64_t* stamp,
+                                uint64_t* end);
+
+// A stamp where no kernel of the sequence starts.
+hipError_t launch_stamp(hipStream_t stream, uint64_t* stamp, uint64_t* stamp2 = nullptr);
 
 // One launch running both the FT convolution of ftc_jobs (1024-point tiles)
 // and the harmonic summing of hsum_jobs (n_harmonics planes) over a FOP written

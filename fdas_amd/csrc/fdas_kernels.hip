@@ -25,6 +25,10 @@ namespace fdas {
 // FT convolution
 // ---------------------------------------------------------------------------
 
+__device__ __forceinline__ void put_stamp(uint64_t* stamp) {
+  if (stamp && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *stamp = wall_clock64();
+}
+
 __device__ __forceinline__ uint32_t find_job_ftc(const FtcJob* __restrict__ jobs, uint32_t n_jobs, uint32_t item) {
   uint32_t lo = 0, hi = n_jobs;
   while (hi - lo > 1) {
@@ -46,7 +50,8 @@ __device__ __forceinline__ uint32_t find_job_ftc(const FtcJob* __restrict__ jobs
 template <int S>
 __global__ __launch_bounds__(S / 16) __attribute__((amdgpu_waves_per_eu(3, 3))) void ftconv_kernel(
     const FtcJob* __restrict__ jobs, uint32_t n_jobs, uint32_t n_items, const float2* __restrict__ tw1,
-    const float2* __restrict__ tw2) {
+    const float2* __restrict__ tw2, uint64_t* stamp) {
+  put_stamp(stamp);
   using F = TileFFTLean<S>;
   constexpr int NT = F::NT;
   __shared__ float2 la[F::LDS_ELEMS];
@@ -198,7 +203,8 @@ __device__ __forceinline__ void ftc1k_item(Ftc1kLds& L, const WaveFFT1k<true>& f
 // workgroup).  164 VGPRs: three waves per SIMD.
 __global__ __launch_bounds__(64) void ftconv1w_kernel(const FtcJob* __restrict__ jobs, uint32_t n_jobs,
                                                       uint32_t n_items, const float2* __restrict__ tw1,
-                                                      const float2* __restrict__ tw2) {
+                                                      const float2* __restrict__ tw2, uint64_t* stamp) {
+  put_stamp(stamp);
   using F = WaveFFT1kLean;
   constexpr int NT = F::NT;
   constexpr int S = F::S;
@@ -277,26 +283,16 @@ __global__ __launch_bounds__(S / 16) void tiles_kernel(const float2* __restrict_
   for (int s = 0; s < 16; ++s) o[F::slot_bin(tid, s)] = v[s];
 }
 
-// A launch, with its events on the dispatch itself where there are any.
-template <class... Params, class... Args>
-static void launch(void (*kernel)(Params...), uint32_t grid, uint32_t block, hipStream_t stream, LaunchEvents ev,
-                   Args... args) {
-  if (ev.start || ev.stop)
-    hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(block), 0, stream, ev.start, ev.stop, 0, args...);
-  else
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), 0, stream, args...);
-}
-
 int ftconv_threads(int tile) { return tile == 1024 ? 64 : tile / 16; }
 
 hipError_t launch_ftconv(int tile, const FtcJob* d_jobs, uint32_t n_jobs, uint32_t n_items, const float2* tw1,
-                         const float2* tw2, uint32_t grid, hipStream_t stream, LaunchEvents ev) {
+                         const float2* tw2, uint32_t grid, hipStream_t stream, uint64_t* stamp) {
   if (n_items == 0) return hipSuccess;
   if (grid == 0 || grid > n_items) grid = n_items;
   switch (tile) {
-    case 1024: launch(ftconv1w_kernel, grid, 64, stream, ev, d_jobs, n_jobs, n_items, tw1, tw2); break;
-    case 2048: launch(ftconv_kernel<2048>, grid, 128, stream, ev, d_jobs, n_jobs, n_items, tw1, tw2); break;
-    case 4096: launch(ftconv_kernel<4096>, grid, 256, stream, ev, d_jobs, n_jobs, n_items, tw1, tw2); break;
+    case 1024: ftconv1w_kernel<<<grid, 64, 0, stream>>>(d_jobs, n_jobs, n_items, tw1, tw2, stamp); break;
+    case 2048: ftconv_kernel<2048><<<grid, 128, 0, stream>>>(d_jobs, n_jobs, n_items, tw1, tw2, stamp); break;
+    case 4096: ftconv_kernel<4096><<<grid, 256, 0, stream>>>(d_jobs, n_jobs, n_items, tw1, tw2, stamp); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -697,37 +693,39 @@ __device__ __forceinline__ void hsum_block(HsumStage<H>& st, const HsumJob* __re
 // waves per SIMD in place of three, 1.49 -> 1.30 ms per 8 trials of 2^20 bins x 85 rows
 // x 16 planes.
 template <int H>
-__global__ __launch_bounds__(kHsumThreads) __attribute__((amdgpu_waves_per_eu(H >= 15 ? 4 : 1))) void hsum_kernel(const HsumJob* __restrict__ jobs, uint32_t n_jobs) {
+__global__ __launch_bounds__(kHsumThreads) __attribute__((amdgpu_waves_per_eu(H >= 15 ? 4 : 1))) void hsum_kernel(
+    const HsumJob* __restrict__ jobs, uint32_t n_jobs, uint64_t* stamp) {
+  put_stamp(stamp);
   __shared__ HsumStage<H> st;
   hsum_block<H>(st, jobs, n_jobs, blockIdx.x);
 }
 
 template <int H>
 static void launch_hsum_h(const HsumJob* d_jobs, uint32_t n_jobs, uint32_t n_blocks, hipStream_t stream,
-                          LaunchEvents ev) {
-  launch(hsum_kernel<H>, n_blocks, kHsumThreads, stream, ev, d_jobs, n_jobs);
+                          uint64_t* stamp) {
+  hsum_kernel<H><<<n_blocks, kHsumThreads, 0, stream>>>(d_jobs, n_jobs, stamp);
 }
 
 hipError_t launch_hsum(const HsumJob* d_jobs, uint32_t n_jobs, uint32_t n_blocks, uint32_t n_harmonics,
-                       hipStream_t stream, LaunchEvents ev) {
+                       hipStream_t stream, uint64_t* stamp) {
   if (n_blocks == 0) return hipSuccess;
   switch (n_harmonics) {
-    case 1: launch_hsum_h<1>(d_jobs, n_jobs, n_blocks, stream, ev); break;
-    case 2: launch_hsum_h<2>(d_jobs, n_jobs, n_blocks, stream, ev); break;
-    case 3: launch_hsum_h<3>(d_jobs, n_jobs, n_blocks, stream, ev); break;
-    case 4: launch_hsum_h<4>(d_jobs, n_jobs, n_blocks, stream, ev); break;
-    case 5: launch_hsum_h<5>(d_jobs, n_jobs, n_blocks, stream, ev); break;
-    case 6: launch_hsum_h<6>(d_jobs, n_jobs, n_blocks, stream, ev); break;
-    case 7: launch_hsum_h<7>(d_jobs, n_jobs, n_blocks, stream, ev); break;
-    case 8: launch_hsum_h<8>(d_jobs, n_jobs, n_blocks, stream, ev); break;
-    case 9: launch_hsum_h<9>(d_jobs, n_jobs, n_blocks, stream, ev); break;
-    case 10: launch_hsum_h<10>(d_jobs, n_jobs, n_blocks, stream, ev); break;
-    case 11: launch_hsum_h<11>(d_jobs, n_jobs, n_blocks, stream, ev); break;
-    case 12: launch_hsum_h<12>(d_jobs, n_jobs, n_blocks, stream, ev); break;
-    case 13: launch_hsum_h<13>(d_jobs, n_jobs, n_blocks, stream, ev); break;
-    case 14: launch_hsum_h<14>(d_jobs, n_jobs, n_blocks, stream, ev); break;
-    case 15: launch_hsum_h<15>(d_jobs, n_jobs, n_blocks, stream, ev); break;
-    case 16: launch_hsum_h<16>(d_jobs, n_jobs, n_blocks, stream, ev); break;
+    case 1: launch_hsum_h<1>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
+    case 2: launch_hsum_h<2>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
+    case 3: launch_hsum_h<3>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
+    case 4: launch_hsum_h<4>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
+    case 5: launch_hsum_h<5>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
+    case 6: launch_hsum_h<6>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
+    case 7: launch_hsum_h<7>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
+    case 8: launch_hsum_h<8>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
+    case 9: launch_hsum_h<9>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
+    case 10: launch_hsum_h<10>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
+    case 11: launch_hsum_h<11>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
+    case 12: launch_hsum_h<12>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
+    case 13: launch_hsum_h<13>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
+    case 14: launch_hsum_h<14>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
+    case 15: launch_hsum_h<15>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
+    case 16: launch_hsum_h<16>(d_jobs, n_jobs, n_blocks, stream, stamp); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -1001,7 +999,8 @@ __device__ void find_cut(const uint32_t* __restrict__ hist, uint32_t cap, uint32
   __syncthreads();
 }
 
-__global__ __launch_bounds__(256) void cand_hist_kernel(const SelectJob* __restrict__ jobs) {
+__global__ __launch_bounds__(256) void cand_hist_kernel(const SelectJob* __restrict__ jobs, uint64_t* stamp) {
+  put_stamp(stamp);
   const SelectJob& job = jobs[blockIdx.y];
   const uint32_t n = min(gld(job.count, 0), job.spill_cap);
   if (n <= job.cap) return;
@@ -1400,7 +1399,7 @@ __device__ uint32_t radix_select_spill(Shared& sh, const SelectJob& job, uint32_
 // planes that keep 4096 of 70,000 .. 173,000 entries, 13 of them in the sort, and
 // 9.7 us for a cap of 512 (with bitonic sorts of key and power: 75 and 16 us).
 template <int THREADS, int CAP>
-__global__ __launch_bounds__(THREADS) void select_final_kernel(const SelectJob* __restrict__ jobs) {
+__global__ __launch_bounds__(THREADS) void select_final_kernel(const SelectJob* __restrict__ jobs, uint64_t* ends) {
   __shared__ SelectShared<THREADS, CAP> sh;
   const SelectJob& job = jobs[blockIdx.x];
   const int tid = threadIdx.x;
@@ -1477,6 +1476,7 @@ __global__ __launch_bounds__(THREADS) void select_final_kernel(const SelectJob* 
     if (job.out_count) gst(job.out_count, 0, detected);
   }
   __threadfence_system();  // the results may be in host memory
+  if (ends && tid == 0) ends[blockIdx.x] = wall_clock64();
 }
 
 // ---------------------------------------------------------------------------
@@ -1589,17 +1589,17 @@ hipError_t launch_quantile_rank(const SelectJob* d_sel, uint32_t n_harmonics, ui
   return hipGetLastError();
 }
 
-hipError_t launch_select(const SelectJob* d_jobs, uint32_t n_jobs, uint32_t cap, hipStream_t stream, hipEvent_t stop) {
+hipError_t launch_select(const SelectJob* d_jobs, uint32_t n_jobs, uint32_t cap, hipStream_t stream, uint64_t* stamp,
+                         uint64_t* ends) {
   if (n_jobs == 0) return hipSuccess;
   if (cap > kSelectMaxCap) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(cand_hist_kernel, dim3(kSelectSlices, n_jobs), dim3(256), 0, stream, d_jobs);
+  hipLaunchKernelGGL(cand_hist_kernel, dim3(kSelectSlices, n_jobs), dim3(256), 0, stream, d_jobs, stamp);
   hipLaunchKernelGGL(cand_compact_kernel, dim3(kSelectSlices, n_jobs), dim3(256), 0, stream, d_jobs);
   // The workgroup grows with the list.  With 1024 / 512 / 256 threads a cap of 4096 took 28 / 30 / 38 us and one
   // of 512 took 11 / 10 / 11 us, where the small workgroup needs a quarter of the CU beside other kernels.
-  const LaunchEvents ev{nullptr, stop};
-  if (cap <= 1024) launch(select_final_kernel<256, 1024>, n_jobs, 256, stream, ev, d_jobs);
-  else if (cap <= 4096) launch(select_final_kernel<1024, 4096>, n_jobs, 1024, stream, ev, d_jobs);
-  else launch(select_final_kernel<1024, 8192>, n_jobs, 1024, stream, ev, d_jobs);
+  if (cap <= 1024) select_final_kernel<256, 1024><<<n_jobs, 256, 0, stream>>>(d_jobs, ends);
+  else if (cap <= 4096) select_final_kernel<1024, 4096><<<n_jobs, 1024, 0, stream>>>(d_jobs, ends);
+  else select_final_kernel<1024, 8192><<<n_jobs, 1024, 0, stream>>>(d_jobs, ends);
   return hipGetLastError();
 }
 
@@ -1633,7 +1633,10 @@ hipError_t launch_zero_u32(uint32_t* p, uint32_t n, hipStream_t stream) {
 static_assert(sizeof(JobPack) <= 3584, "job descriptors must fit a kernel argument block");
 
 __global__ __launch_bounds__(256) void put_jobs_kernel(JobPack pack, FtcJob* ftc, HsumJob* hsum, SelectJob* sel,
-                                                       ZeroSpan a, ZeroSpan b) {
+                                                       ZeroSpan a, ZeroSpan b, uint64_t* stamp,
+                                                       uint64_t* stamp2) {
+  put_stamp(stamp);
+  put_stamp(stamp2);
   const uint32_t tid = blockIdx.x * 256u + threadIdx.x, stride = gridDim.x * 256u;
   for (uint32_t i = tid; i < a.n; i += stride) a.p[i] = 0u;
   for (uint32_t i = tid; i < b.n; i += stride) b.p[i] = 0u;
@@ -1649,9 +1652,44 @@ __global__ __launch_bounds__(256) void put_jobs_kernel(JobPack pack, FtcJob* ftc
 }
 
 hipError_t launch_put_jobs(const JobPack& pack, FtcJob* d_ftc, HsumJob* d_hsum, SelectJob* d_sel, ZeroSpan a,
-                           ZeroSpan b, hipStream_t stream) {
+                           ZeroSpan b, hipStream_t stream, uint64_t* stamp, uint64_t* stamp2) {
   const uint32_t blocks = min(1u + (a.n + b.n) / 1024u, 64u);
-  hipLaunchKernelGGL(put_jobs_kernel, dim3(blocks), dim3(256), 0, stream, pack, d_ftc, d_hsum, d_sel, a, b);
+  hipLaunchKernelGGL(put_jobs_kernel, dim3(blocks), dim3(256), 0, stream, pack, d_ftc, d_hsum, d_sel, a, b,
+                     stamp, stamp2);
+  return hipGetLastError();
+}
+
+// Bound by the source: pinned host memory or HBM.
+__global__ __launch_bounds__(256) void copy_spectrum_kernel(const float2* __restrict__ src, float2* __restrict__ dst,
+                                                            uint32_t n, uint64_t* stamp, uint64_t* end) {
+  put_stamp(stamp);
+  const uint32_t step = gridDim.x * 256u;
+  for (uint64_t i0 = blockIdx.x * 256u + threadIdx.x; i0 < n; i0 += 4ull * step) {
+    float2 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = gld2(src, size_t(min(i0 + uint64_t(u) * step, uint64_t(n - 1u))));
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (i0 + uint64_t(u) * step < n) dst[i0 + uint64_t(u) * step] = v[u];
+  }
+  if (end && blockIdx.x == gridDim.x - 1u && threadIdx.x == 0) *end = wall_clock64();
+}
+
+hipError_t launch_copy_spectrum(const float2* src, float2* dst, uint32_t n, hipStream_t stream, uint64_t* stamp,
+                                uint64_t* end) {
+  if (n == 0) return hipSuccess;
+  const uint32_t blocks = min((n + 1023u) / 1024u, 2048u);
+  copy_spectrum_kernel<<<blocks, 256, 0, stream>>>(src, dst, n, stamp, end);
+  return hipGetLastError();
+}
+
+__global__ void stamp_kernel(uint64_t* stamp, uint64_t* stamp2) {
+  put_stamp(stamp);
+  put_stamp(stamp2);
+}
+
+hipError_t launch_stamp(hipStream_t stream, uint64_t* stamp, uint64_t* stamp2) {
+  stamp_kernel<<<1, 64, 0, stream>>>(stamp, stamp2);
   return hipGetLastError();
 }
 
