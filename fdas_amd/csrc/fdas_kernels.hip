@@ -975,8 +975,8 @@ __device__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s_waves) {
 // counts every spilled entry and there are more than `cap` of them, so a cut
 // exists; the defaults (bin 0, nothing above) keep b* inside the histogram
 // regardless.
-template <int THREADS>
-__device__ void find_cut(const uint32_t* __restrict__ hist, uint32_t cap, uint32_t* s_waves, uint32_t* s_out) {
+template <int THREADS, class Bin>
+__device__ void find_cut(Bin hist_bin, uint32_t cap, uint32_t* s_waves, uint32_t* s_out) {
   constexpr int PER = int(kSelectBins) / THREADS;
   const int tid = threadIdx.x;
   if (tid == 0) {
@@ -987,7 +987,7 @@ __device__ void find_cut(const uint32_t* __restrict__ hist, uint32_t cap, uint32
   uint32_t local = 0;
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    h[j] = gld(hist, kSelectBins - 1 - uint32_t(tid * PER + j));
+    h[j] = hist_bin(kSelectBins - 1 - uint32_t(tid * PER + j));
     local += h[j];
   }
   const uint32_t excl = block_exclusive_scan<THREADS>(local, s_waves);
@@ -999,11 +999,16 @@ __device__ void find_cut(const uint32_t* __restrict__ hist, uint32_t cap, uint32
   __syncthreads();
 }
 
+// Planes of no more detections than the compact list holds are left to the last kernel, which reads the spill list
+// itself; for them the histogram and the compaction are two empty kernels.  With that and sort_by_runs the selection
+// of 8 planes of cap 512 takes 11 us at 4,999 bins x 33 templates and 12 at 32,768 x 85; it took 22 and 18.
+__device__ __forceinline__ bool select_direct(const SelectJob& job, uint32_t n) { return n <= job.compact_cap; }
+
 __global__ __launch_bounds__(256) void cand_hist_kernel(const SelectJob* __restrict__ jobs, uint64_t* stamp) {
   put_stamp(stamp);
   const SelectJob& job = jobs[blockIdx.y];
   const uint32_t n = min(gld(job.count, 0), job.spill_cap);
-  if (n <= job.cap) return;
+  if (select_direct(job, n)) return;
   __shared__ uint32_t h[kSelectBins];
   const int tid = threadIdx.x;
   for (uint32_t i = tid; i < kSelectBins; i += 256) h[i] = 0;
@@ -1057,7 +1062,7 @@ __device__ __forceinline__ void wave_append(uint32_t* counter, const bool (&take
 __global__ __launch_bounds__(256) void cand_compact_kernel(const SelectJob* __restrict__ jobs) {
   const SelectJob& job = jobs[blockIdx.y];
   const uint32_t n = min(gld(job.count, 0), job.spill_cap);
-  if (n <= job.cap) return;
+  if (select_direct(job, n)) return;
   constexpr uint32_t kStep = 4 * 256, kStage = 2 * kStep;
   __shared__ uint32_t waves[4];
   __shared__ uint32_t cut[2];
@@ -1066,7 +1071,7 @@ __global__ __launch_bounds__(256) void cand_compact_kernel(const SelectJob* __re
   __shared__ uint32_t n_staged, g_base;
   const int tid = threadIdx.x;
   if (tid == 0) n_staged = 0;
-  find_cut<256>(job.hist, job.cap, waves, cut);
+  find_cut<256>([&](uint32_t b) { return gld(job.hist, b); }, job.cap, waves, cut);
   const uint32_t bstar = cut[0];
   const uint32_t tb = histogram_base(__float_as_uint(job.thr));
   const uint32_t per = (n + kSelectSlices - 1) / kSelectSlices;
@@ -1177,6 +1182,85 @@ __device__ void radix_pass(Shared& sh, uint32_t n, Get get, uint32_t shift, uint
   mask |= (nb - 1) << shift;
   rank = sh.misc[1];
   __syncthreads();
+}
+
+// v of the lane whose index differs in the bits of M.
+template <int M>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+  if constexpr (M == 1) return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0xb1, 0xf, 0xf, true));  // quad_perm
+  if constexpr (M == 2) return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x4e, 0xf, 0xf, true));
+  if constexpr (M == 8) return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x128, 0xf, 0xf, true));  // row_ror:8
+  if constexpr (M == 4 || M == 16) return uint32_t(__builtin_amdgcn_ds_swizzle(int(v), (M << 10) | 0x1f));
+  return uint32_t(__shfl_xor(int(v), M));
+}
+
+// Bitonic sort of a wave's 64 K keys, ascending; lane l holds entries K l .. K l + K - 1.
+template <int K, int SIZE = 2, int STRIDE = 1>
+__device__ __forceinline__ void wave_sort(uint32_t (&a)[K]) {
+  if constexpr (SIZE <= 64 * K) {
+    const uint32_t lane = lane_id();
+    if constexpr (STRIDE >= K) {
+      constexpr int M = STRIDE / K;
+      const bool keep_min = ((lane & M) == 0) == ((lane & (SIZE / K)) == 0);
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const uint32_t other = lane_xor<M>(a[k]);
+        a[k] = keep_min ? min(a[k], other) : max(a[k], other);
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        if (k & STRIDE) continue;
+        const bool up = SIZE < K ? (k & SIZE) == 0 : (lane & (SIZE / K)) == 0;
+        const uint32_t lo = min(a[k], a[k + STRIDE]), hi = max(a[k], a[k + STRIDE]);
+        a[k] = up ? lo : hi;
+        a[k + STRIDE] = up ? hi : lo;
+      }
+    }
+    if constexpr (STRIDE > 1) wave_sort<K, SIZE, STRIDE / 2>(a);
+    else wave_sort<K, SIZE * 2, SIZE>(a);
+  }
+}
+
+// Sorts n <= 64 K entries per wave by key (all different), ascending.  Each wave sorts its entries' keys in
+// registers, and an entry's place is the number of smaller keys in every wave's run, by binary searches: 3 barriers,
+// where the radix sort takes 7 a pass.  For workgroups of 4 waves: 512 entries in about 2 us against 5 (3 passes) and
+// 6.7 (4 passes); the searches grow with the number of runs, and 16 runs of 256 would take longer than the passes.
+template <int K, int THREADS, class Shared>
+__device__ void sort_by_runs(Shared& sh, uint32_t n) {
+  constexpr uint32_t RUN = 64 * K;
+  uint32_t* runs = reinterpret_cast<uint32_t*>(sh.pool);
+  uint32_t key[K], sorted[K], place[K];
+  float pwr[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const uint32_t i = threadIdx.x * K + uint32_t(k);
+    key[k] = i < n ? sh.key[i] : 0xffffffffu;
+    pwr[k] = i < n ? sh.pwr[i] : 0.f;
+    sorted[k] = key[k];
+    place[k] = 0;
+  }
+  wave_sort<K>(sorted);
+#pragma unroll
+  for (int k = 0; k < K; ++k) runs[threadIdx.x * K + uint32_t(k)] = sorted[k];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t w = 0; w < THREADS / 64; ++w) {
+    const uint32_t* run = runs + w * RUN;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      uint32_t c = 0;  // keys of the run below this one
+#pragma unroll
+      for (uint32_t s = RUN / 2; s > 0; s /= 2) c += run[c + s - 1] < key[k] ? s : 0u;
+      place[k] += c + (run[c] < key[k] ? 1u : 0u);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    if (threadIdx.x * K + uint32_t(k) >= n) continue;
+    sh.key[place[k]] = key[k];
+    sh.pwr[place[k]] = pwr[k];
+  }
 }
 
 // Sorts the n kept entries by key (row, bin), ascending: a radix sort in place,
@@ -1395,9 +1479,11 @@ __device__ uint32_t radix_select_spill(Shared& sh, const SelectJob& job, uint32_
 }
 
 // One workgroup per plane: the kept entries, sorted.  CAP >= the job's cap.
-// Bound by latency (one workgroup's barriers and LDS round trips): 20 us for 8
-// planes that keep 4096 of 70,000 .. 173,000 entries, 13 of them in the sort, and
-// 9.7 us for a cap of 512 (with bitonic sorts of key and power: 75 and 16 us).
+// Bound by latency (one workgroup's barriers and LDS round trips): 19 us for 8
+// planes that keep 4096 of 70,000 .. 173,000 entries, 13.6 of them in the sort (with
+// bitonic sorts of key and power 75).  Results in host memory need no fence of the
+// kernel's own: the stream's or event's synchronisation makes them visible, and the
+// fence, which writes back the L2, took 2 to 4 us.
 template <int THREADS, int CAP>
 __global__ __launch_bounds__(THREADS) void select_final_kernel(const SelectJob* __restrict__ jobs, uint64_t* ends) {
   __shared__ SelectShared<THREADS, CAP> sh;
@@ -1414,27 +1500,45 @@ __global__ __launch_bounds__(THREADS) void select_final_kernel(const SelectJob* 
     }
     kept = n;
   } else {
-    find_cut<THREADS>(job.hist, cap, sh.waves, sh.misc);
+    constexpr int U = THREADS == 256 ? 8 : 4;  // loads in flight per thread
+    const uint32_t tb = histogram_base(__float_as_uint(job.thr));
+    const bool direct = select_direct(job, n);
+    if (direct) {
+      for (uint32_t i = tid; i < kSelectBins; i += THREADS) sh.hist[i] = 0;
+      __syncthreads();
+      for (uint32_t e0 = tid; e0 < n; e0 += U * THREADS) {
+        uint32_t v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = __float_as_uint(gld(job.spill_pwr, min(e0 + uint32_t(u * THREADS), n - 1u)));
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (e0 + uint32_t(u * THREADS) < n) atomicAdd(&sh.hist[power_bin(v[u], tb)], 1u);
+      }
+      __syncthreads();
+      find_cut<THREADS>([&](uint32_t b) { return sh.hist[b]; }, cap, sh.waves, sh.misc);
+    } else {
+      find_cut<THREADS>([&](uint32_t b) { return gld(job.hist, b); }, cap, sh.waves, sh.misc);
+    }
     const uint32_t bstar = sh.misc[0], above = sh.misc[1];
-    const uint32_t m = gld(job.compact_n, 0);
-    const uint32_t pool_n = gld(job.hist, bstar);
+    const uint32_t m = direct ? n : gld(job.compact_n, 0);
+    const uint32_t pool_n = direct ? sh.hist[bstar] : gld(job.hist, bstar);
+    const uint32_t* list_key = direct ? job.spill_key : job.compact_key;
+    const float* list_pwr = direct ? job.spill_pwr : job.compact_pwr;
     __syncthreads();
     if (m <= job.compact_cap && pool_n <= kSelectPool && above < cap) {
-      const uint32_t tb = histogram_base(__float_as_uint(job.thr));
       if (tid == 0) {
         sh.misc[3] = 0;
         sh.misc[4] = 0;
       }
       __syncthreads();
-      constexpr int U = 4;  // loads in flight per thread
       for (uint32_t e0 = 0; e0 < m; e0 += U * THREADS) {
         float v[U];
         uint32_t key[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           const uint32_t e = min(e0 + uint32_t(u * THREADS + tid), m - 1u);
-          v[u] = gld(job.compact_pwr, e);
-          key[u] = gld(job.compact_key, e);
+          v[u] = gld(list_pwr, e);
+          key[u] = gld(list_key, e);
         }
         bool strong[U], at_cut[U];
         uint32_t pos[U], q[U];
@@ -1465,7 +1569,13 @@ __global__ __launch_bounds__(THREADS) void select_final_kernel(const SelectJob* 
     }
   }
   __syncthreads();
-  sort_by_key<THREADS, CAP>(sh, kept);
+  if constexpr (CAP <= 4 * THREADS && THREADS == 256) {
+    if (kept <= THREADS) sort_by_runs<1, THREADS>(sh, kept);
+    else if (kept <= 2 * THREADS) sort_by_runs<2, THREADS>(sh, kept);
+    else sort_by_runs<4, THREADS>(sh, kept);
+  } else {
+    sort_by_key<THREADS, CAP>(sh, kept);
+  }
   __syncthreads();
   for (uint32_t e = tid; e < kept; e += THREADS) {
     gst(job.out_key, e, sh.key[e]);
@@ -1475,7 +1585,6 @@ __global__ __launch_bounds__(THREADS) void select_final_kernel(const SelectJob* 
     gst(job.out_n, 0, kept);
     if (job.out_count) gst(job.out_count, 0, detected);
   }
-  __threadfence_system();  // the results may be in host memory
   if (ends && tid == 0) ends[blockIdx.x] = wall_clock64();
 }
 
