@@ -48,7 +48,7 @@ struct DevSet {
   float* plane = nullptr;
   uint32_t* spill_key = nullptr;
   float* spill_pwr = nullptr;
-  uint32_t* counts = nullptr;      // [H] detections, then [H] compact counts, then [H][kSelectBins] histograms
+  uint32_t* counts = nullptr;      // [H][kPlaneCounters]
   uint32_t* compact_key = nullptr;
   float* compact_pwr = nullptr;
   FtcJob* d_ftc = nullptr;
@@ -314,15 +314,15 @@ void fill_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr) {
     SelectJob& q = s.pack.sel[p];
     q.spill_key = s.spill_key + size_t(p) * ctx->spill;
     q.spill_pwr = s.spill_pwr + size_t(p) * ctx->spill;
-    q.count = s.counts + p;
+    q.count = s.counts + size_t(p) * kPlaneCounters;
     q.spill_cap = ctx->spill;
     q.cap = cap;
     q.thr = thr[p];
     q.compact_cap = ccap;
-    q.hist = s.counts + 2 * H + size_t(p) * kSelectBins;
+    q.hist = s.counts + size_t(p) * kPlaneCounters + 2;
     q.compact_key = s.compact_key + size_t(p) * ccap;
     q.compact_pwr = s.compact_pwr + size_t(p) * ccap;
-    q.compact_n = s.counts + H + p;
+    q.compact_n = s.counts + size_t(p) * kPlaneCounters + 1;
     q.out_key = s.h_out_key + size_t(p) * cap;
     q.out_pwr = s.h_out_pwr + size_t(p) * cap;
     q.out_n = s.h_out_n + p;
@@ -334,8 +334,8 @@ void fill_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr) {
 // Takes the pack's jobs to the device, with the counters cleared when a summing pass is among them.
 fdas_status put_jobs(fdas_ctx* ctx, DevSet& s, uint64_t* stamp = nullptr, uint64_t* stamp2 = nullptr) {
   ZeroSpan zero;
-  if (s.pack.n_sel) zero = {s.counts, ctx->cfg.n_harmonics * (2 + kSelectBins)};
-  HIPCK(ctx, launch_put_jobs(s.pack, s.d_ftc, s.d_hsum, s.d_sel, zero, {}, s.stream, stamp, stamp2));
+  if (s.pack.n_sel) zero = {s.counts, ctx->cfg.n_harmonics * kPlaneCounters};
+  HIPCK(ctx, launch_put_jobs(s.pack, s.d_ftc, s.d_hsum, s.d_sel, zero, s.stream, stamp, stamp2));
   s.pack.n_ftc = s.pack.n_sel = 0;
   return FDAS_OK;
 }
@@ -597,7 +597,7 @@ extern "C" fdas_status fdas_create(const fdas_config* cfg, fdas_log_fn log, void
     if ((st = dev_alloc(ctx, &s.spill_pwr, H * ctx->spill)) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.compact_key, H * (cap + kSelectPool))) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.compact_pwr, H * (cap + kSelectPool))) != FDAS_OK) return bail(st);
-    if ((st = dev_alloc(ctx, &s.counts, H * (2 + kSelectBins))) != FDAS_OK) return bail(st);
+    if ((st = dev_alloc(ctx, &s.counts, H * kPlaneCounters)) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.d_ftc, kMaxFtcJobs)) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.d_hsum, 1)) != FDAS_OK) return bail(st);
     if ((st = dev_alloc(ctx, &s.d_sel, H)) != FDAS_OK) return bail(st);
@@ -618,7 +618,7 @@ extern "C" fdas_status fdas_create(const fdas_config* cfg, fdas_log_fn log, void
       return bail(fail(ctx, FDAS_EDEVICE, "event creation failed"));
     // a FOP that was never written reads as zeros
     if (hipMemset(s.fop, 0, T * N * sizeof(float)) != hipSuccess ||
-        hipMemset(s.counts, 0, H * (2 + kSelectBins) * sizeof(uint32_t)) != hipSuccess)
+        hipMemset(s.counts, 0, H * kPlaneCounters * sizeof(uint32_t)) != hipSuccess)
       return bail(fail(ctx, FDAS_EDEVICE, "buffer initialisation failed"));
   }
   uint64_t* const clock = ctx->set[0].h_stamp;

@@ -183,7 +183,7 @@ struct Shape {
 // selection kernel writes the lists to pinned host memory itself.
 struct TrialLayout {
   // small part, from its base
-  uint64_t counts, compact_n, hist, small_bytes;
+  uint64_t counters, small_bytes;
   // large part, from its base
   uint64_t compact_key, compact_pwr, spill_key, spill_pwr, input, fop, large_bytes;
   uint64_t total;  // small_bytes + large_bytes
@@ -194,12 +194,8 @@ struct TrialLayout {
 TrialLayout trial_layout(uint32_t n_bins, uint32_t T, uint32_t H, uint32_t cap, uint32_t spill, bool own_input) {
   TrialLayout l{};
   uint64_t o = 0;
-  l.counts = o;
-  o += 4ull * H;
-  l.compact_n = o;
-  o += 4ull * H;
-  l.hist = o;
-  o += 4ull * H * kSelectBins;
+  l.counters = o;
+  o += 4ull * H * kPlaneCounters;
   l.small_bytes = align_up(o);
   o = 0;
   l.out_n = o;
@@ -515,7 +511,7 @@ fdas_status build_group(fdas_engine* e, GroupBuf& g, const std::vector<Trial*>& 
       hsum_row_chunks(j.n_rows, &j.rows_per_block, &j.n_row_chunks, t->shape->hsum_rows);
       j.spill_key = reinterpret_cast<uint32_t*>(m + l.spill_key);
       j.spill_pwr = reinterpret_cast<float*>(m + l.spill_pwr);
-      j.counts = reinterpret_cast<uint32_t*>(sm + l.counts);
+      j.counts = reinterpret_cast<uint32_t*>(sm + l.counters);
       for (uint32_t k = 0; k < H; ++k) j.thr[k] = t->req.thresholds[k];
       L.n_blocks += (j.n_bins + kHsumBinsPerBlock - 1) / kHsumBinsPerBlock * j.n_row_chunks;
       L.whole_groups = L.whole_groups && hsum_whole_groups(j.n_bins);
@@ -523,15 +519,15 @@ fdas_status build_group(fdas_engine* e, GroupBuf& g, const std::vector<Trial*>& 
         SelectJob& q = g.h_sel[js++];
         q.spill_key = j.spill_key + size_t(p) * spill;
         q.spill_pwr = j.spill_pwr + size_t(p) * spill;
-        q.count = j.counts + p;
+        q.count = j.counts + size_t(p) * kPlaneCounters;
         q.spill_cap = spill;
         q.cap = cap;
         q.thr = t->req.thresholds[p];
         q.compact_cap = ccap;
-        q.hist = reinterpret_cast<uint32_t*>(sm + l.hist) + size_t(p) * kSelectBins;
+        q.hist = j.counts + size_t(p) * kPlaneCounters + 2;
         q.compact_key = reinterpret_cast<uint32_t*>(m + l.compact_key) + size_t(p) * ccap;
         q.compact_pwr = reinterpret_cast<float*>(m + l.compact_pwr) + size_t(p) * ccap;
-        q.compact_n = reinterpret_cast<uint32_t*>(sm + l.compact_n) + p;
+        q.compact_n = j.counts + size_t(p) * kPlaneCounters + 1;
         q.out_key = reinterpret_cast<uint32_t*>(t->h_lists + l.out_key) + size_t(p) * cap;
         q.out_pwr = reinterpret_cast<float*>(t->h_lists + l.out_pwr) + size_t(p) * cap;
         q.out_n = reinterpret_cast<uint32_t*>(t->h_lists + l.out_n) + p;

@@ -41,7 +41,7 @@ struct HsumJob {
   uint32_t pad_;
   uint32_t* spill_key;    // [H][spill_cap] row << 22 | bin
   float* spill_pwr;       // [H][spill_cap]
-  uint32_t* counts;       // [H] detections per plane (may exceed spill_cap)
+  uint32_t* counts;       // detections of plane k at [k * kPlaneCounters] (may exceed spill_cap)
   float thr[kMaxHarmonics];
 };
 
@@ -63,7 +63,7 @@ struct SelectJob {
   uint32_t* out_key;          // [cap] sorted by key
   float* out_pwr;
   uint32_t* out_n;            // kept entries
-  uint32_t* out_count;        // detections (nullptr: not wanted)
+  uint32_t* out_count;        // detections
 };
 
 }  // namespace fdas

@@ -78,7 +78,7 @@ hipError_t launch_clear_counters(const SelectJob* d_jobs, uint32_t n_jobs, hipSt
 hipError_t launch_zero_u32(uint32_t* p, uint32_t n, hipStream_t stream);
 
 // The job descriptors of one trial's launches, taken to the device as the argument
-// of a kernel that also clears up to two spans of counters: one launch in place of
+// of a kernel that also clears the counters: one launch in place of
 // three copies and a fill.
 constexpr uint32_t kPackFtcJobs = 16;
 struct JobPack {
@@ -91,8 +91,8 @@ struct ZeroSpan {
   uint32_t* p = nullptr;
   uint32_t n = 0;
 };
-hipError_t launch_put_jobs(const JobPack& pack, FtcJob* d_ftc, HsumJob* d_hsum, SelectJob* d_sel, ZeroSpan a,
-                           ZeroSpan b, hipStream_t stream, uint64_t* stamp = nullptr, uint64_t* stamp2 = nullptr);
+hipError_t launch_put_jobs(const JobPack& pack, FtcJob* d_ftc, HsumJob* d_hsum, SelectJob* d_sel, ZeroSpan zero,
+                           hipStream_t stream, uint64_t* stamp = nullptr, uint64_t* stamp2 = nullptr);
 
 // n spectrum bins from device or pinned host memory (8-byte aligned); `end`: the last workgroup's end.
 hipError_t launch_copy_spectrum(const float2* src, float2* dst, uint32_t n, hipStream_t stream, uint64_t* stamp,

@@ -347,8 +347,7 @@ struct HsumStage {
   static constexpr uint32_t kGroups = H <= 8 ? 24 : 12;  // LDS for 5 and 4 workgroups per CU
   float sum[kHsumThreads / 64][H][kGroups][kHsumBinsPerThread];
   uint32_t key[kHsumThreads / 64][H][kGroups];  // row << kKeyBinBits | f0
-  uint32_t n[kHsumThreads / 64][H];             // groups, then (at the end) hits
-  uint32_t base[kHsumThreads / 64][H];
+  uint32_t n[H][kHsumThreads / 64];             // groups of each wave, at the end
 };
 
 // One bin of each of 8 staged groups, first, first + 1, ...: this lane's value and key,
@@ -389,7 +388,7 @@ __device__ __forceinline__ void wave_flush(Stage& st, const HsumJob& job, uint32
   wave_lds_order();  // the stage is rewritten next
   if (total == 0) return;
   uint32_t base = 0;
-  if (lane_id() == 0) base = gatomic_add(job.counts + p, total);
+  if (lane_id() == 0) base = gatomic_add(job.counts + size_t(p) * kPlaneCounters, total);
   base = __shfl(base, 0);
 #pragma unroll
   for (int s = 0; s < kSteps; ++s)
@@ -543,7 +542,7 @@ __device__ __forceinline__ void hsum_row(Stage& st, const HsumJob& job, const Ro
       uint32_t total;
       const uint32_t pos = wave_prefix_small(uint32_t(__builtin_popcount(bits)), total);
       uint32_t g = 0;
-      if (lane_id() == 0) g = gatomic_add(job.counts + (k - 1), total);
+      if (lane_id() == 0) g = gatomic_add(job.counts + size_t((k - 1)) * kPlaneCounters, total);
       g = __shfl(g, 0) + pos;
 #pragma unroll
       for (int b = 0; b < kHsumBinsPerThread; ++b) {
@@ -565,6 +564,77 @@ __device__ __forceinline__ void hsum_row(Stage& st, const HsumJob& job, const Ro
   }
 }
 
+// Writes what the workgroup has staged to the spill lists, with one global atomic per plane.  Many launches are one
+// round of workgroups and end with this, so its latency counts.  A wave takes whole planes, the groups of all four
+// waves' lists in steps of 8: the waves share a strong signal that one of them has staged, and each wave reserves
+// places for its planes with one instruction and needs no second barrier.  (Each wave counting its own lists of all
+// planes, one after another, then workgroup totals: 4,999 bins x 33 rows x 8 planes with two tones 10 us against 6.8,
+// 32,768 x 85 14.7 against 12.8 at 2 rows a workgroup, 2^20 x 85 x 16 planes 169 against 161.)
+template <int H>
+__device__ __forceinline__ void flush_rest(HsumStage<H>& st, const HsumJob& job, const uint32_t (&wn)[H]) {
+  constexpr uint32_t kWaves = kHsumThreads / 64, kPlanes = (uint32_t(H) + kWaves - 1) / kWaves;  // planes of a wave
+  const uint32_t lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint32_t mine = 0;
+#pragma unroll
+  for (int k = 0; k < H; ++k)
+    if (lane == uint32_t(k)) mine = wn[k];
+  if (lane < uint32_t(H)) st.n[lane][wave] = mine;
+  __syncthreads();
+  uint32_t at[kPlanes][kWaves], n[kPlanes];  // where each wave's groups begin in the plane's list; its length
+#pragma unroll
+  for (uint32_t i = 0; i < kPlanes; ++i) {
+    const uint32_t p = wave + i * kWaves;
+    n[i] = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kWaves; ++w) {
+      at[i][w] = n[i];
+      n[i] += p < uint32_t(H) ? __builtin_amdgcn_readfirstlane(st.n[p][w]) : 0u;
+    }
+  }
+  // This lane's bin of the groups first .. first + 7 of the wave's plane i.
+  auto staged = [&](uint32_t i, uint32_t first, float* v, uint32_t* key) {
+    const uint32_t p = wave + i * kWaves, g = first + lane / 8u;
+    uint32_t w = 0, begin = 0;
+#pragma unroll
+    for (uint32_t x = 1; x < kWaves; ++x) {
+      if (g < at[i][x]) continue;
+      w = x;
+      begin = at[i][x];
+    }
+    if (g >= n[i]) return false;
+    *v = st.sum[w][p][g - begin][lane % 8u];
+    *key = st.key[w][p][g - begin] + lane % 8u;
+    return *v > job.thr[p] && (*key & ((1u << kKeyBinBits) - 1u)) < job.n_bins;
+  };
+  uint32_t key[kPlanes], hits = 0, x;
+  float v[kPlanes], y;
+  uint64_t m[kPlanes];  // hits of the first 8 groups, most often all of them
+#pragma unroll
+  for (uint32_t i = 0; i < kPlanes; ++i) m[i] = __ballot(staged(i, 0, &v[i], &key[i]));
+#pragma unroll
+  for (uint32_t i = 0; i < kPlanes; ++i) {
+    uint32_t total = uint32_t(__builtin_popcountll(m[i]));
+    for (uint32_t first = 8; first < n[i]; first += 8)
+      total += uint32_t(__builtin_popcountll(__ballot(staged(i, first, &y, &x))));
+    if (lane == i) hits = total;
+  }
+  uint32_t place = 0;
+  if (hits) place = gatomic_add(job.counts + size_t(wave + lane * kWaves) * kPlaneCounters, hits);
+#pragma unroll
+  for (uint32_t i = 0; i < kPlanes; ++i) {
+    const uint32_t p = wave + i * kWaves;
+    uint32_t to = uint32_t(__builtin_amdgcn_readlane(int(place), int(i)));
+    if ((m[i] >> lane) & 1u) spill_hit(job, p, to + lanes_below(m[i]), key[i], v[i]);
+    to += uint32_t(__builtin_popcountll(m[i]));
+    for (uint32_t first = 8; first < n[i]; first += 8) {
+      const bool hit = staged(i, first, &y, &x);
+      const uint64_t mask = __ballot(hit);
+      if (hit) spill_hit(job, p, to + lanes_below(mask), x, y);
+      to += uint32_t(__builtin_popcountll(mask));
+    }
+  }
+}
+
 // One bin of one row, every hit placed by its own atomic: the bins that the
 // 16-byte loads cannot cover (below).
 template <int H>
@@ -578,7 +648,7 @@ __device__ __forceinline__ void hsum_one_bin(const HsumJob& job, uint32_t r, uin
   for (int k = 1; k <= H; ++k) {
     if (k > 1) hp += v[k - 1];
     if (!(hp > job.thr[k - 1])) continue;
-    const uint32_t g = gatomic_add(job.counts + (k - 1), 1u);
+    const uint32_t g = gatomic_add(job.counts + size_t((k - 1)) * kPlaneCounters, 1u);
     if (g >= job.spill_cap) continue;
     gst(job.spill_key, size_t(k - 1) * job.spill_cap + g, (r << kKeyBinBits) | f);
     gst(job.spill_pwr, size_t(k - 1) * job.spill_cap + g, hp);
@@ -649,51 +719,14 @@ __device__ __forceinline__ void hsum_block(HsumStage<H>& st, const HsumJob* __re
       if (r + 2 > r_stop) break;
     }
   }
-  // Flush what is left: one global atomic per plane for the whole workgroup.
-  if (lane_id() == 0) {
-#pragma unroll
-    for (int k = 0; k < H; ++k) st.n[wave][k] = wn[k];
-  }
-  wave_lds_order();
-  float v;
-  uint32_t key;
-  for (uint32_t k = 0; k < uint32_t(H); ++k) {
-    const uint32_t n = __builtin_amdgcn_readfirstlane(st.n[wave][k]);
-    uint32_t hits = 0;
-    for (uint32_t first = 0; first < n; first += 8)
-      hits += uint32_t(__builtin_popcountll(__ballot(staged_bin(st, wave, k, first, n, job.thr[k], n_bins, &v, &key))));
-    if (lane_id() == 0) st.base[wave][k] = hits;
-  }
-  __syncthreads();
-  if (tid < H) {
-    uint32_t total = 0, before[kHsumThreads / 64];
-#pragma unroll
-    for (uint32_t w = 0; w < uint32_t(kHsumThreads / 64); ++w) {
-      before[w] = total;
-      total += st.base[w][tid];
-    }
-    const uint32_t g = total ? gatomic_add(job.counts + tid, total) : 0u;
-#pragma unroll
-    for (uint32_t w = 0; w < uint32_t(kHsumThreads / 64); ++w) st.base[w][tid] = g + before[w];
-  }
-  __syncthreads();
-  for (uint32_t k = 0; k < uint32_t(H); ++k) {
-    const uint32_t n = __builtin_amdgcn_readfirstlane(st.n[wave][k]);
-    uint32_t at = __builtin_amdgcn_readfirstlane(st.base[wave][k]);
-    for (uint32_t first = 0; first < n; first += 8) {
-      const bool hit = staged_bin(st, wave, k, first, n, job.thr[k], n_bins, &v, &key);
-      const uint64_t m = __ballot(hit);
-      if (hit) spill_hit(job, k, at + lanes_below(m), key, v);
-      at += uint32_t(__builtin_popcountll(m));
-    }
-  }
+  flush_rest(st, job, wn);
 }
 
-// 15 and 16 planes are held to 128 registers (they take 129 and 131 unasked): four
-// waves per SIMD in place of three, 1.49 -> 1.30 ms per 8 trials of 2^20 bins x 85 rows
-// x 16 planes.
+// Up to 8 planes are held to the registers of 5 and 6 waves per SIMD, as many as the LDS allows from 5 planes on, and
+// 15 and 16 planes to 128 registers: four waves per SIMD in place of three, 1.49 -> 1.30 ms per 8 trials of 2^20 bins
+// x 85 rows x 16 planes.
 template <int H>
-__global__ __launch_bounds__(kHsumThreads) __attribute__((amdgpu_waves_per_eu(H >= 15 ? 4 : 1))) void hsum_kernel(
+__global__ __launch_bounds__(kHsumThreads) __attribute__((amdgpu_waves_per_eu(H >= 15 ? 4 : H > 8 ? 1 : H > 4 ? 5 : 6))) void hsum_kernel(
     const HsumJob* __restrict__ jobs, uint32_t n_jobs, uint64_t* stamp) {
   put_stamp(stamp);
   __shared__ HsumStage<H> st;
@@ -1583,7 +1616,7 @@ __global__ __launch_bounds__(THREADS) void select_final_kernel(const SelectJob* 
   }
   if (tid == 0) {
     gst(job.out_n, 0, kept);
-    if (job.out_count) gst(job.out_count, 0, detected);
+    gst(job.out_count, 0, detected);
   }
   if (ends && tid == 0) ends[blockIdx.x] = wall_clock64();
 }
@@ -1742,13 +1775,12 @@ hipError_t launch_zero_u32(uint32_t* p, uint32_t n, hipStream_t stream) {
 static_assert(sizeof(JobPack) <= 3584, "job descriptors must fit a kernel argument block");
 
 __global__ __launch_bounds__(256) void put_jobs_kernel(JobPack pack, FtcJob* ftc, HsumJob* hsum, SelectJob* sel,
-                                                       ZeroSpan a, ZeroSpan b, uint64_t* stamp,
+                                                       ZeroSpan zero, uint64_t* stamp,
                                                        uint64_t* stamp2) {
   put_stamp(stamp);
   put_stamp(stamp2);
   const uint32_t tid = blockIdx.x * 256u + threadIdx.x, stride = gridDim.x * 256u;
-  for (uint32_t i = tid; i < a.n; i += stride) a.p[i] = 0u;
-  for (uint32_t i = tid; i < b.n; i += stride) b.p[i] = 0u;
+  for (uint32_t i = tid; i < zero.n; i += stride) zero.p[i] = 0u;
   auto copy = [&](const void* src, void* dst, uint32_t bytes) {
     for (uint32_t i = tid; i < bytes / 4u; i += stride)
       static_cast<uint32_t*>(dst)[i] = static_cast<const uint32_t*>(src)[i];
@@ -1760,11 +1792,11 @@ __global__ __launch_bounds__(256) void put_jobs_kernel(JobPack pack, FtcJob* ftc
   }
 }
 
-hipError_t launch_put_jobs(const JobPack& pack, FtcJob* d_ftc, HsumJob* d_hsum, SelectJob* d_sel, ZeroSpan a,
-                           ZeroSpan b, hipStream_t stream, uint64_t* stamp, uint64_t* stamp2) {
-  const uint32_t blocks = min(1u + (a.n + b.n) / 1024u, 64u);
-  hipLaunchKernelGGL(put_jobs_kernel, dim3(blocks), dim3(256), 0, stream, pack, d_ftc, d_hsum, d_sel, a, b,
-                     stamp, stamp2);
+hipError_t launch_put_jobs(const JobPack& pack, FtcJob* d_ftc, HsumJob* d_hsum, SelectJob* d_sel, ZeroSpan zero,
+                           hipStream_t stream, uint64_t* stamp, uint64_t* stamp2) {
+  const uint32_t blocks = min(1u + zero.n / 1024u, 64u);
+  hipLaunchKernelGGL(put_jobs_kernel, dim3(blocks), dim3(256), 0, stream, pack, d_ftc, d_hsum, d_sel, zero, stamp,
+                     stamp2);
   return hipGetLastError();
 }
 

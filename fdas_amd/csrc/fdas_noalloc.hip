@@ -23,7 +23,8 @@ using namespace fdas;
 // The scratch: one copy per GPU, alive until the process ends.  Host code
 // never passes this name to a kernel (on the host it is only a stand-in for
 // the symbol); it uses the per-device address from hipGetSymbolAddress.
-static __device__ __align__(256) unsigned char scratch[FDAS_NOALLOC_SCRATCH_BYTES];
+constexpr uint64_t kCountBytes = 256;  // the planes' detection counts, beyond the documented limit
+static __device__ __align__(256) unsigned char scratch[FDAS_NOALLOC_SCRATCH_BYTES + kCountBytes];
 
 namespace {
 
@@ -116,8 +117,8 @@ extern "C" fdas_status fdas_hsum_noalloc(const float* d_fop, uint32_t n_bins, ui
   if (part == FDAS_POSITIVE) rb = n_templates / 2, nr = n_templates / 2 + 1;
 
   NoallocJobs* d_jobs = reinterpret_cast<NoallocJobs*>(base);
-  uint32_t* compact_n = reinterpret_cast<uint32_t*>(base + o_counts);
-  uint32_t* hist = compact_n + H;
+  uint32_t* counters = reinterpret_cast<uint32_t*>(base + o_counts);
+  base += kCountBytes;
   uint32_t* compact_key = reinterpret_cast<uint32_t*>(base + o_compact);
   float* compact_pwr = reinterpret_cast<float*>(base + o_compact + 4ull * H * ccap);
   uint32_t* spill_key = reinterpret_cast<uint32_t*>(base + o_spill);
@@ -137,32 +138,31 @@ extern "C" fdas_status fdas_hsum_noalloc(const float* d_fop, uint32_t n_bins, ui
   hsum_row_chunks(nr, &j.rows_per_block, &j.n_row_chunks, hsum_rows_for(n_bins, nr));
   j.spill_key = spill_key;
   j.spill_pwr = spill_pwr;
-  j.counts = d_counts + H;  // detections per plane, before the cap
+  j.counts = counters;
   for (uint32_t k = 0; k < H; ++k) j.thr[k] = thresholds[k];
   for (uint32_t p = 0; p < H; ++p) {
     SelectJob& q = jobs.sel[p];
     q.spill_key = spill_key + size_t(p) * spill;
     q.spill_pwr = spill_pwr + size_t(p) * spill;
-    q.count = d_counts + H + p;
+    q.count = counters + size_t(p) * kPlaneCounters;
     q.spill_cap = spill;
     q.cap = cap;
     q.thr = thresholds[p];
     q.compact_cap = ccap;
-    q.hist = hist + size_t(p) * kSelectBins;
+    q.hist = counters + size_t(p) * kPlaneCounters + 2;
     q.compact_key = compact_key + size_t(p) * ccap;
     q.compact_pwr = compact_pwr + size_t(p) * ccap;
-    q.compact_n = compact_n + p;
+    q.compact_n = counters + size_t(p) * kPlaneCounters + 1;
     q.out_key = d_key + size_t(p) * cap;
     q.out_pwr = d_power + size_t(p) * cap;
     q.out_n = d_counts + p;
-    q.out_count = nullptr;  // the summing kernel counts in d_counts + H itself
+    q.out_count = d_counts + H + p;  // detections per plane, before the cap
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   // Every call shares this device's scratch and keeps no state between calls:
-  // what must start at zero (counters, histograms, the caller's counts) is
-  // cleared by the kernel that brings the job descriptors.
-  hipError_t e = launch_put_jobs(jobs, nullptr, &d_jobs->hsum, d_jobs->sel, {d_counts, 2 * H},
-                                 {compact_n, H * (1 + kSelectBins)}, s);
+  // what must start at zero (counters, histograms) is cleared by the kernel that
+  // brings the job descriptors.
+  hipError_t e = launch_put_jobs(jobs, nullptr, &d_jobs->hsum, d_jobs->sel, {counters, H * kPlaneCounters}, s);
   const uint32_t blocks = (n_bins + kHsumBinsPerBlock - 1) / kHsumBinsPerBlock * j.n_row_chunks;
   if (e == hipSuccess) e = launch_hsum(&d_jobs->hsum, 1, blocks, H, s);
   if (e == hipSuccess) e = launch_select(d_jobs->sel, H, cap, s);

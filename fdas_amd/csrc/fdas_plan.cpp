@@ -137,8 +137,7 @@ void make_twiddles(uint32_t tile, std::vector<float2>& tw1, std::vector<float2>&
 
 uint32_t hsum_rows_for(uint32_t n_bins, uint32_t n_rows) {
   const uint64_t row_blocks = uint64_t((n_bins + kHsumBinsPerBlock - 1) / kHsumBinsPerBlock) * n_rows;
-  if (row_blocks >= 65536) return kHsumRowsPerBlock;
-  return std::min(8u, std::max(1u, uint32_t(std::lround(std::sqrt(double(row_blocks) / 220.0)))));
+  return std::min(kHsumRowsPerBlock, std::max(1u, uint32_t(std::lround(std::sqrt(double(row_blocks) / 100.0)))));
 }
 
 void hsum_row_chunks(uint32_t n_rows, uint32_t* rows_per_block, uint32_t* n_row_chunks, uint32_t target) {

@@ -57,11 +57,13 @@ void make_twiddles(uint32_t tile, std::vector<float2>& tw1, std::vector<float2>&
 
 // Rows per summing workgroup for a launch of one trial.  Short chunks fill the
 // chip where a plane is small (a chunk's rows follow one another, and each waits
-// for its loads); tall ones re-read fewer sub-harmonic rows.  Between, the best
-// height grew with the square root of the plane's size.  Measured, us at 11 rows /
-// at the height chosen here: 4,999 bins x 33 rows 30 / 8 (1 row); 32,768 x 85
-// 47 / 16 (2); 131,072 x 85 42 / 32 (5); 262,144 x 85 56 / 47 (7); 700,001 x 85
-// 89 / 82 (8); at 2^21 x 85 8 rows take 208 against 204 at 11.
+// for its loads); tall ones re-read fewer sub-harmonic rows and send fewer additions
+// to each plane's detection count, which take turns at about 6 ns.  Between, the best
+// height grows with the square root of the plane's size.  Measured, us of the kernel
+// at 8 planes and 2 / 4 / 8 / 11 rows: 4,999 bins x 33 rows (4 planes; 1 row 4.7)
+// 5.7 / 9.0 / 15 / 21; 20,011 x 169 15 / 14 / 23 / 31; 32,768 x 85 12.7 / 10.6 / 18 / 22;
+// 100,003 x 85 31 / 22 / 17 / 17; 262,144 x 85 70 / 44 / 33 / 34; 700,001 x 85
+// 175 / 105 / 72 / 65; 2^21 x 85 510 / 302 / 200 / 196, and 203 at 15.
 uint32_t hsum_rows_for(uint32_t n_bins, uint32_t n_rows);
 
 // HSUM workgroup row chunking for a part of n_rows rows (at most `target` rows per workgroup).

@@ -20,6 +20,10 @@ namespace fdas {
 
 constexpr uint32_t kSelectBins = 2048;  // power histogram bins (256 per octave above the threshold)
 
+// A plane's counters, one after another: detections, compact-list entries, histogram.  So far apart, the planes'
+// detection counts are in cache lines of their own: a workgroup of the summing adds to each of them once.
+constexpr uint32_t kPlaneCounters = 2 + kSelectBins;
+
 // a > b (as floats, no NaN)  <=>  order_key(a) > order_key(b).
 __host__ __device__ inline uint32_t order_key(uint32_t bits) {
   return (bits & 0x80000000u) ? ~bits : (bits | 0x80000000u);
