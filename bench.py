@@ -54,15 +54,15 @@ HBM_PEAK_GBS = 8000.0
 # HBM bytes per launch (rocprofv3 FETCH_SIZE x2.000 + WRITE_SIZE x1.000, calibrated
 # on a copy kernel) for the batched workload at N=2^21, T=85, tile 1024, 8 trials
 # per launch; profiles/batched_n2p21_t85_h8_tile1024_traffic.txt.
-MEASURED_TRAFFIC = {("ftconv1w_kernel", 8): 6869.7e6, ("hsum_kernel<8,true>", 8): 9302.7e6}
+MEASURED_TRAFFIC = {("ftconv1w_kernel", 8): 6852.2e6, ("hsum_kernel<8>", 8): 9243.6e6}
 # VALU wave-instructions per launch (rocprofv3 SQ_INSTS_VALU) at the same shape;
 # profiles/batched_n2p21_t85_h8_tile1024_instructions.txt.  Issue rate: 256 CUs x
 # 4 SIMDs, one wave64 VALU instruction per 4 cycles per SIMD at 2.4 GHz.
-MEASURED_VALU = {("ftconv1w_kernel", 8): 1050558056, ("hsum_kernel<8,true>", 8): 510989349}
+MEASURED_VALU = {("ftconv1w_kernel", 8): 1050779416, ("hsum_kernel<8>", 8): 422009166}
 VALU_ISSUE_PER_S = 256 * 4 * 2.4e9 / 4
 # Shader clock the kernel runs at (amd-smi median while it runs alone, bench.py --forms batched,power);
 # profiles/power_clock_n2p21_t85_tile1024.txt.  The FT convolution holds the board at its power limit.
-MEASURED_CLOCK_GHZ = {"ftconv1w_kernel": 2.112, "hsum_kernel<8,true>": 2.385}
+MEASURED_CLOCK_GHZ = {"ftconv1w_kernel": 2.112, "hsum_kernel<8>": 2.385}
 FP32_PEAK_TFLOPS = 157.3
 N_METRIC = 1 << 21
 T_METRIC = 85
@@ -734,7 +734,7 @@ def main():
             kernels = {
                 ftc_kernel_name(tile): {"ms": batched["ftc_span_ms"],
                                         "bytes": ftc_bytes(N_METRIC, T_METRIC, tile, trials_per_launch)},
-                "hsum_kernel<8,true>": {"ms": batched["hsum_span_ms"],
+                "hsum_kernel<8>": {"ms": batched["hsum_span_ms"],
                                         "bytes": hsum_bytes(N_METRIC, T_METRIC, n_cands, trials_per_launch)},
             }
         workload = (f"batched uniform: {args.batch} DM trials per step, N=2^21 bins, 85 templates x 421 taps, "
@@ -747,7 +747,7 @@ def main():
             raise SystemExit("bench.py: --forms needs batched or single for the headline value")
         value, ms_per_step, steps, trials_per_launch = st["value"], st["ms_per_trial"], 30, 1
         kernels = {ftc_kernel_name(tile): {"ms": st["ftconv_ms"], "bytes": ftc_bytes(N_METRIC, T_METRIC, tile)},
-                   "hsum_kernel<8,true>": {"ms": st["hsum_ms"], "bytes": hsum_bytes(N_METRIC, T_METRIC, 8 * CAP)}}
+                   "hsum_kernel<8>": {"ms": st["hsum_ms"], "bytes": hsum_bytes(N_METRIC, T_METRIC, 8 * CAP)}}
         workload = "single-trial FDAS, N=2^21 bins, 85 templates x 421 taps, 8 harmonics, spectra resident"
         in_flight = "2 trials (buffer sets A/B)"
 
