@@ -89,6 +89,8 @@ struct DevSet {
   bool launched = false;
   uint32_t* user_loc = nullptr;
   float* user_pwr = nullptr;
+  bool delivered = false;  // the caller's arrays hold the launch's lists, the set's own hold another pass's
+  uint32_t delivered_counts[kMaxHarmonics] = {};
   bool gated = false;
   fdas_part gated_part = FDAS_ALL;
   float gated_thr[kMaxHarmonics] = {};
@@ -435,14 +437,22 @@ void to_reference_lists(const fdas_ctx* ctx, const DevSet& s, uint32_t* loc, flo
 
 bool reference_format_ok(const fdas_ctx* ctx) { return ctx->cfg.n_templates <= 127 && ctx->cfg.n_harmonics <= 8; }
 
-fdas_status overflow_status(fdas_ctx* ctx, const DevSet& s) {
+// counts: [H] detections
+fdas_status overflow_status(fdas_ctx* ctx, const uint32_t* counts) {
   for (uint32_t p = 0; p < ctx->cfg.n_harmonics; ++p)
-    if (s.h_counts[p] > ctx->spill)
+    if (counts[p] > ctx->spill)
       return fail(ctx, FDAS_EOVERFLOW,
                   "plane %u: %u detections exceed the spill capacity %u; lists are incomplete (raise the "
                   "threshold or spill_per_harmonic)",
-                  p + 1, s.h_counts[p], ctx->spill);
+                  p + 1, counts[p], ctx->spill);
   return FDAS_OK;
+}
+
+// The finished launch's lists to the caller's arrays before another pass overwrites the set's.
+void deliver_early(const fdas_ctx* ctx, DevSet& s) {
+  to_reference_lists(ctx, s, s.user_loc, s.user_pwr);
+  std::copy(s.h_counts, s.h_counts + ctx->cfg.n_harmonics, s.delivered_counts);
+  s.delivered = true;
 }
 
 fdas_status flush_gated(fdas_ctx* ctx, int set) {
@@ -839,8 +849,9 @@ extern "C" fdas_status fdas_perform_harmonic_summing(fdas_ctx* ctx, const float*
   if ((st = enqueue_hsum(ctx, s, part, thr)) != FDAS_OK) return st;
   if ((st = drain(ctx, s)) != FDAS_OK) return st;
   s.cands_valid = true;
+  s.delivered = false;
   info(ctx, "Harmonic summing duration: %.3f ms", double(elapsed(ctx, s, ST_HSUM_K0, ST_ENDS)));
-  return overflow_status(ctx, s);
+  return overflow_status(ctx, s.h_counts);
 }
 
 // The work of a launch once its spectrum is on its way: convolution, and summing
@@ -851,6 +862,7 @@ static fdas_status enqueue_launch(fdas_ctx* ctx, DevSet& s, fdas_part part, cons
       ctx->sync_pipeline ? enqueue_ftc(ctx, s, part, resident) : enqueue_search(ctx, s, part, thr, resident);
   if (st != FDAS_OK) return st;
   s.launched = true;
+  s.delivered = false;
   s.user_loc = det_loc;
   s.user_pwr = det_pwr;
   if (ctx->sync_pipeline) {
@@ -913,8 +925,9 @@ extern "C" fdas_status fdas_wait(fdas_ctx* ctx, int set) {
   s.launched = false;
   s.fop_valid = true;
   s.cands_valid = true;
+  if (s.delivered) return overflow_status(ctx, s.delivered_counts);
   to_reference_lists(ctx, s, s.user_loc, s.user_pwr);
-  return overflow_status(ctx, s);
+  return overflow_status(ctx, s.h_counts);
 }
 
 extern "C" fdas_status fdas_end_pipeline(fdas_ctx* ctx, int set) {
@@ -1012,7 +1025,7 @@ extern "C" fdas_status fdas_retrieve_candidates_wide(fdas_ctx* ctx, fdas_candida
     }
   }
   if (n_written) *n_written = w;
-  return overflow_status(ctx, s);
+  return overflow_status(ctx, s.h_counts);
 }
 
 extern "C" fdas_status fdas_retrieve_harmonic_plane(fdas_ctx* ctx, uint32_t k, float* plane, fdas_part part,
@@ -1085,6 +1098,10 @@ extern "C" fdas_status fdas_quantile_thresholds(fdas_ctx* ctx, uint32_t n_per_pl
     HIPCK(ctx, hipStreamSynchronize(s.stream));
     return FDAS_OK;
   };
+  if (s.launched && !s.gated && !s.delivered) {
+    if ((st = drain(ctx, s)) != FDAS_OK) return st;
+    deliver_early(ctx, s);
+  }
   restart_hsum_stamps(s);
   s.cands_valid = false;  // the lists will belong to these thresholds, not to a search
   std::vector<float> thr(H, -INFINITY);

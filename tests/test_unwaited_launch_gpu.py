@@ -1,0 +1,59 @@
+"""GPU test of calls on a buffer set whose launch has not been waited for."""
+
+import numpy as np
+import pytest
+
+from fdas_amd import synth
+from fdas_amd.host import FDAS
+
+from test_gpu_parity import bank_for, make, spectrum
+
+pytestmark = pytest.mark.gpu
+
+N, T, H, CAP = 20000, 21, 4, 64
+
+
+@pytest.fixture
+def search():
+    bank = bank_for(T)
+    f = make(N, n_templates=T, max_taps=bank.shape[1], tile=1024, n_harmonics=H, cands_per_harmonic=CAP)
+    assert f.upload_template_taps(bank, FDAS.A), f.last_error
+    x = spectrum(N, 2)
+    yield f, x, synth.noise_thresholds(x, H)
+    f.close()
+
+
+def arrays(f):
+    n = f.get_candidate_list_sz()
+    return np.zeros(n, np.uint32), np.zeros(n, np.float32)
+
+
+def test_quantile_thresholds_before_wait_leave_the_launch_its_lists(search):
+    """wait() hands over the lists of the launch, also where the quantile thresholds of the set's plane were taken
+    between the two; the set's own lists are then the quantile pass's (fewer entries: 3 per plane asked for)."""
+    f, x, thr = search
+    want = arrays(f)
+    assert f.launch(x, thr, *want, 2, FDAS.A) and f.wait(FDAS.A), f.last_error
+    assert all((want[1][k * CAP:(k + 1) * CAP] > 0).all() for k in range(H))  # full lists
+    q0 = f.quantile_thresholds(3, 2, FDAS.A)
+    of_quantile = arrays(f)
+    assert f.retrieve_candidates(*of_quantile, FDAS.A)
+    assert (of_quantile[1] > 0).sum() < H * CAP
+    for again in range(2):
+        got = arrays(f)
+        assert f.launch_resident(thr, *got, 2, FDAS.A), f.last_error
+        for _ in range(1 + again):
+            assert np.array_equal(f.quantile_thresholds(3, 2, FDAS.A), q0)
+        assert f.wait(FDAS.A), f.last_error
+        assert all(np.array_equal(a, b) for a, b in zip(got, want))
+        after = arrays(f)
+        assert f.retrieve_candidates(*after, FDAS.A)
+        assert all(np.array_equal(a, b) for a, b in zip(after, of_quantile))
+    # a summing pass after it replaces the lists, as it does those of a launch
+    got, summed = arrays(f), arrays(f)
+    assert f.launch_resident(thr, *got, 2, FDAS.A), f.last_error
+    f.quantile_thresholds(3, 2, FDAS.A)
+    assert f.perform_harmonic_summing(thr * 2, 2, FDAS.A), f.last_error
+    assert f.retrieve_candidates(*summed, FDAS.A) and f.wait(FDAS.A), f.last_error
+    assert all(np.array_equal(a, b) for a, b in zip(got, summed))
+    assert not np.array_equal(got[0], want[0])
