@@ -67,6 +67,7 @@ struct DevSet {
 
   hipStream_t stream = nullptr;
   uint64_t* h_stamp = nullptr;       // [ST_COUNT] pinned
+  bool in_flight = false;            // work was enqueued since the stream was last waited for
   bool ftc_to_hsum = false;          // the summing followed the convolution at once: its start is the other's end
   float2* h_input = nullptr;         // pinned staging of small host spectra
   bool input_pending = false;        // h_input may still be read by the device
@@ -212,6 +213,15 @@ void clear_stamps(DevSet& s, int from, int to) {
   for (int i = from; i <= to; ++i) reinterpret_cast<volatile uint64_t*>(s.h_stamp)[i] = 0;
 }
 
+StampSpan stamp_span(const DevSet& s, int from, int to) { return {s.h_stamp + from, uint32_t(to - from + 1)}; }
+
+// The times from .. to are about to be taken anew.  An idle set's read as not taken from now on; kernels of an
+// earlier sequence may still write them otherwise, and the new sequence's first kernel clears them.
+void renew_stamps(DevSet& s, int from, int to) {
+  if (!s.in_flight) clear_stamps(s, from, to);
+  s.in_flight = true;
+}
+
 fdas_status stamp(fdas_ctx* ctx, DevSet& s, Stamp at) {
   HIPCK(ctx, launch_stamp(s.stream, s.h_stamp + at));
   return FDAS_OK;
@@ -245,7 +255,7 @@ float since_epoch(const fdas_ctx* ctx, const DevSet& s, int at) {
 // Waits for the set's stream: lists and stamps are in host memory, the staged spectrum has been read.
 fdas_status drain(fdas_ctx* ctx, DevSet& s) {
   HIPCK(ctx, hipStreamSynchronize(s.stream));
-  s.input_pending = false;
+  s.input_pending = s.in_flight = false;
   return FDAS_OK;
 }
 
@@ -334,10 +344,10 @@ void fill_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr) {
 }
 
 // Takes the pack's jobs to the device, with the counters cleared when a summing pass is among them.
-fdas_status put_jobs(fdas_ctx* ctx, DevSet& s, uint64_t* stamp = nullptr, uint64_t* stamp2 = nullptr) {
+fdas_status put_jobs(fdas_ctx* ctx, DevSet& s, const StampOps& times = StampOps{}) {
   ZeroSpan zero;
   if (s.pack.n_sel) zero = {s.counts, ctx->cfg.n_harmonics * kPlaneCounters};
-  HIPCK(ctx, launch_put_jobs(s.pack, s.d_ftc, s.d_hsum, s.d_sel, zero, s.stream, stamp, stamp2));
+  HIPCK(ctx, launch_put_jobs(s.pack, s.d_ftc, s.d_hsum, s.d_sel, zero, s.stream, times));
   s.pack.n_ftc = s.pack.n_sel = 0;
   return FDAS_OK;
 }
@@ -371,43 +381,61 @@ fdas_status run_hsum(fdas_ctx* ctx, DevSet& s) {
   return FDAS_OK;
 }
 
-// Convolution alone.  start: the sequence starts here (no input step before it).
+// Times of a sequence that begins with a convolution and ends at `last`.  start: it starts here (no input step
+// before it).
+StampOps ftc_stamps(DevSet& s, bool start, int last) {
+  renew_stamps(s, start ? ST_START : ST_INPUT, last);
+  StampOps t;
+  t.stamp = s.h_stamp + ST_INPUT;
+  if (start) t.stamp2 = s.h_stamp + ST_START;
+  t.clear = stamp_span(s, ST_FTC_K, last);
+  return t;
+}
+
+// Convolution alone.
 fdas_status enqueue_ftc(fdas_ctx* ctx, DevSet& s, fdas_part part, bool start) {
-  clear_stamps(s, start ? ST_START : ST_INPUT, ST_FTC);
+  const StampOps times = ftc_stamps(s, start, ST_FTC);
   s.ftc_to_hsum = false;
-  uint64_t* const at_start = start ? s.h_stamp + ST_START : nullptr;
   uint32_t n_jobs, n_items;
   fdas_status st = fill_ftc(ctx, s, part, &n_jobs, &n_items);
   if (st != FDAS_OK) return st;
-  // (with no jobs in the pack the kernel takes the stamps only)
-  if ((st = put_jobs(ctx, s, s.h_stamp + ST_INPUT, at_start)) != FDAS_OK) return st;
+  // (with no jobs in the pack the kernel sees to the times only)
+  if ((st = put_jobs(ctx, s, times)) != FDAS_OK) return st;
   if ((st = run_ftc(ctx, s, n_jobs, n_items)) != FDAS_OK) return st;
   return stamp(ctx, s, ST_FTC);
 }
 
-// A summing pass on its own: the convolution's end is kept, the pass's times are not taken yet.
-void restart_hsum_stamps(DevSet& s) {
-  if (s.ftc_to_hsum) s.h_stamp[ST_FTC] = s.h_stamp[ST_HSUM_K0];
+// Times of a summing pass on its own: the convolution's end is kept, the pass's are not taken yet.
+StampOps hsum_stamps(DevSet& s) {
+  StampOps t;
+  if (s.ftc_to_hsum && s.in_flight) {
+    t.keep_from = s.h_stamp + ST_HSUM_K0;
+    t.keep_to = s.h_stamp + ST_FTC;
+  } else if (s.ftc_to_hsum) {
+    s.h_stamp[ST_FTC] = s.h_stamp[ST_HSUM_K0];
+  }
   s.ftc_to_hsum = false;
-  clear_stamps(s, ST_HSUM_K0, ST_COUNT - 1);
+  renew_stamps(s, ST_HSUM_K0, ST_COUNT - 1);
+  t.clear = stamp_span(s, ST_HSUM_K0, ST_COUNT - 1);
+  return t;
 }
 
 fdas_status enqueue_hsum(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr) {
-  restart_hsum_stamps(s);
+  const StampOps times = hsum_stamps(s);
   fill_hsum(ctx, s, part, thr);
-  const fdas_status st = put_jobs(ctx, s);
+  const fdas_status st = put_jobs(ctx, s, times);
   return st == FDAS_OK ? run_hsum(ctx, s) : st;
 }
 
 // Convolution and summing of one launch, their jobs taken to the device together.
 fdas_status enqueue_search(fdas_ctx* ctx, DevSet& s, fdas_part part, const float* thr, bool start) {
-  clear_stamps(s, start ? ST_START : ST_INPUT, ST_COUNT - 1);
+  const StampOps times = ftc_stamps(s, start, ST_COUNT - 1);
   s.ftc_to_hsum = true;
   uint32_t n_jobs, n_items;
   fdas_status st = fill_ftc(ctx, s, part, &n_jobs, &n_items);
   if (st != FDAS_OK) return st;
   fill_hsum(ctx, s, part, thr);
-  if ((st = put_jobs(ctx, s, s.h_stamp + ST_INPUT, start ? s.h_stamp + ST_START : nullptr)) != FDAS_OK) return st;
+  if ((st = put_jobs(ctx, s, times)) != FDAS_OK) return st;
   if ((st = run_ftc(ctx, s, n_jobs, n_items)) != FDAS_OK) return st;
   return run_hsum(ctx, s);
 }
@@ -622,6 +650,7 @@ extern "C" fdas_status fdas_create(const fdas_config* cfg, fdas_log_fn log, void
       return bail(fail(ctx, FDAS_EDEVICE, "stream creation failed"));
     if ((st = host_alloc(ctx, &s.h_stamp, ST_COUNT, hipHostMallocCoherent)) != FDAS_OK) return bail(st);
     clear_stamps(s, 0, ST_COUNT - 1);
+    static_assert(ST_COUNT <= 64, "cleared by one workgroup's threads");
     if (N * sizeof(float2) <= kStagedInput && (st = host_alloc(ctx, &s.h_input, N)) != FDAS_OK) return bail(st);
     if (hipEventCreateWithFlags(&s.hsum_done, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&s.staged_ftc, hipEventDisableTiming) != hipSuccess)
@@ -760,7 +789,7 @@ static fdas_status upload_input(fdas_ctx* ctx, DevSet& s, const void* src, hipMe
   const size_t bytes = sizeof(float2) * ctx->geo.n_bins;
   fdas_status st;
   if (s.input_pending && (st = drain(ctx, s)) != FDAS_OK) return st;
-  clear_stamps(s, 0, ST_COUNT - 1);
+  renew_stamps(s, 0, ST_COUNT - 1);
   s.ftc_to_hsum = false;
   const float2* from = nullptr;
   if (kind == hipMemcpyHostToDevice && s.h_input) {
@@ -772,9 +801,9 @@ static fdas_status upload_input(fdas_ctx* ctx, DevSet& s, const void* src, hipMe
   }
   if (from) {
     HIPCK(ctx, launch_copy_spectrum(from, s.input, ctx->geo.n_bins, s.stream, s.h_stamp + ST_START,
-                                    s.h_stamp + ST_INPUT));
+                                    s.h_stamp + ST_INPUT, stamp_span(s, ST_FTC_K, ST_COUNT - 1)));
   } else {
-    if ((st = stamp(ctx, s, ST_START)) != FDAS_OK) return st;
+    HIPCK(ctx, launch_stamp(s.stream, s.h_stamp + ST_START, nullptr, stamp_span(s, ST_INPUT, ST_COUNT - 1)));
     HIPCK(ctx, hipMemcpyAsync(s.input, src, bytes, kind, s.stream));
   }
   s.has_input = true;
@@ -980,9 +1009,9 @@ extern "C" fdas_status fdas_inject_fop(fdas_ctx* ctx, const float* fop, int set)
   HIPCK(ctx, hipSetDevice(ctx->cfg.device));
   const size_t n = size_t(ctx->cfg.n_templates) * ctx->geo.n_bins;
   fdas_status st;
-  clear_stamps(s, ST_START, ST_FTC);
+  renew_stamps(s, ST_START, ST_FTC);
   s.ftc_to_hsum = false;
-  HIPCK(ctx, launch_stamp(s.stream, s.h_stamp + ST_START, s.h_stamp + ST_INPUT));
+  HIPCK(ctx, launch_stamp(s.stream, s.h_stamp + ST_START, s.h_stamp + ST_INPUT, stamp_span(s, ST_FTC_K, ST_FTC)));
   HIPCK(ctx, hipMemcpyAsync(s.fop, fop, n * sizeof(float), hipMemcpyHostToDevice, s.stream));
   if ((st = stamp(ctx, s, ST_FTC)) != FDAS_OK) return st;
   s.fop_valid = true;
@@ -1102,11 +1131,11 @@ extern "C" fdas_status fdas_quantile_thresholds(fdas_ctx* ctx, uint32_t n_per_pl
     if ((st = drain(ctx, s)) != FDAS_OK) return st;
     deliver_early(ctx, s);
   }
-  restart_hsum_stamps(s);
+  const StampOps times = hsum_stamps(s);
   s.cands_valid = false;  // the lists will belong to these thresholds, not to a search
   std::vector<float> thr(H, -INFINITY);
   fill_hsum(ctx, s, part, thr.data());
-  if ((st = put_jobs(ctx, s)) != FDAS_OK) return st;
+  if ((st = put_jobs(ctx, s, times)) != FDAS_OK) return st;
   const uint32_t nb = hmax_blocks(N, nr);
   HIPCK(ctx, launch_hmax(s.fop, N, ctx->cfg.n_templates, rb, nr, H, s.quant, s.stream));
   HIPCK(ctx, launch_quantile_bound(s.quant, nb, uint32_t(std::min<uint64_t>(want, UINT32_MAX)), H, s.d_hsum, s.d_sel,

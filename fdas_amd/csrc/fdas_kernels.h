@@ -91,15 +91,29 @@ struct ZeroSpan {
   uint32_t* p = nullptr;
   uint32_t n = 0;
 };
+// Times that a sequence has not reached are cleared by its first kernel, in the stream's order: the host cannot, while
+// an earlier sequence may still write them.
+struct StampSpan {
+  uint64_t* p = nullptr;
+  uint32_t n = 0;  // at most a workgroup of put_jobs, copy_spectrum or stamp_kernel (64)
+};
+// What put_jobs does with a sequence's times: *keep_to = *keep_from, then the clearing, then the stamps.
+struct StampOps {
+  uint64_t* stamp = nullptr;
+  uint64_t* stamp2 = nullptr;
+  StampSpan clear;
+  const uint64_t* keep_from = nullptr;
+  uint64_t* keep_to = nullptr;
+};
 hipError_t launch_put_jobs(const JobPack& pack, FtcJob* d_ftc, HsumJob* d_hsum, SelectJob* d_sel, ZeroSpan zero,
-                           hipStream_t stream, uint64_t* stamp = nullptr, uint64_t* stamp2 = nullptr);
+                           hipStream_t stream, const StampOps& times = StampOps{});
 
 // n spectrum bins from device or pinned host memory (8-byte aligned); `end`: the last workgroup's end.
 hipError_t launch_copy_spectrum(const float2* src, float2* dst, uint32_t n, hipStream_t stream, uint64_t* stamp,
-                                uint64_t* end);
+                                uint64_t* end, StampSpan clear);
 
 // A stamp where no kernel of the sequence starts.
-hipError_t launch_stamp(hipStream_t stream, uint64_t* stamp, uint64_t* stamp2 = nullptr);
+hipError_t launch_stamp(hipStream_t stream, uint64_t* stamp, uint64_t* stamp2 = nullptr, StampSpan clear = StampSpan{});
 
 // One launch running both the FT convolution of ftc_jobs (1024-point tiles)
 // and the harmonic summing of hsum_jobs (n_harmonics planes) over a FOP written

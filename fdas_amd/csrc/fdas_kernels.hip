@@ -29,6 +29,10 @@ __device__ __forceinline__ void put_stamp(uint64_t* stamp) {
   if (stamp && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *stamp = wall_clock64();
 }
 
+__device__ __forceinline__ void clear_stamps(StampSpan s) {
+  if (blockIdx.x == 0 && threadIdx.x < s.n) s.p[threadIdx.x] = 0;
+}
+
 __device__ __forceinline__ uint32_t find_job_ftc(const FtcJob* __restrict__ jobs, uint32_t n_jobs, uint32_t item) {
   uint32_t lo = 0, hi = n_jobs;
   while (hi - lo > 1) {
@@ -1775,10 +1779,14 @@ hipError_t launch_zero_u32(uint32_t* p, uint32_t n, hipStream_t stream) {
 static_assert(sizeof(JobPack) <= 3584, "job descriptors must fit a kernel argument block");
 
 __global__ __launch_bounds__(256) void put_jobs_kernel(JobPack pack, FtcJob* ftc, HsumJob* hsum, SelectJob* sel,
-                                                       ZeroSpan zero, uint64_t* stamp,
-                                                       uint64_t* stamp2) {
-  put_stamp(stamp);
-  put_stamp(stamp2);
+                                                       ZeroSpan zero, StampOps times) {
+  put_stamp(times.stamp);
+  put_stamp(times.stamp2);
+  if (times.keep_from) {  // one of the times cleared below
+    if (blockIdx.x == 0 && threadIdx.x == 0) *times.keep_to = *times.keep_from;
+    __syncthreads();
+  }
+  clear_stamps(times.clear);
   const uint32_t tid = blockIdx.x * 256u + threadIdx.x, stride = gridDim.x * 256u;
   for (uint32_t i = tid; i < zero.n; i += stride) zero.p[i] = 0u;
   auto copy = [&](const void* src, void* dst, uint32_t bytes) {
@@ -1793,17 +1801,18 @@ __global__ __launch_bounds__(256) void put_jobs_kernel(JobPack pack, FtcJob* ftc
 }
 
 hipError_t launch_put_jobs(const JobPack& pack, FtcJob* d_ftc, HsumJob* d_hsum, SelectJob* d_sel, ZeroSpan zero,
-                           hipStream_t stream, uint64_t* stamp, uint64_t* stamp2) {
+                           hipStream_t stream, const StampOps& times) {
   const uint32_t blocks = min(1u + zero.n / 1024u, 64u);
-  hipLaunchKernelGGL(put_jobs_kernel, dim3(blocks), dim3(256), 0, stream, pack, d_ftc, d_hsum, d_sel, zero, stamp,
-                     stamp2);
+  hipLaunchKernelGGL(put_jobs_kernel, dim3(blocks), dim3(256), 0, stream, pack, d_ftc, d_hsum, d_sel, zero, times);
   return hipGetLastError();
 }
 
 // Bound by the source: pinned host memory or HBM.
 __global__ __launch_bounds__(256) void copy_spectrum_kernel(const float2* __restrict__ src, float2* __restrict__ dst,
-                                                            uint32_t n, uint64_t* stamp, uint64_t* end) {
+                                                            uint32_t n, uint64_t* stamp, uint64_t* end,
+                                                            StampSpan clear) {
   put_stamp(stamp);
+  clear_stamps(clear);
   const uint32_t step = gridDim.x * 256u;
   for (uint64_t i0 = blockIdx.x * 256u + threadIdx.x; i0 < n; i0 += 4ull * step) {
     float2 v[4];
@@ -1817,20 +1826,21 @@ __global__ __launch_bounds__(256) void copy_spectrum_kernel(const float2* __rest
 }
 
 hipError_t launch_copy_spectrum(const float2* src, float2* dst, uint32_t n, hipStream_t stream, uint64_t* stamp,
-                                uint64_t* end) {
+                                uint64_t* end, StampSpan clear) {
   if (n == 0) return hipSuccess;
   const uint32_t blocks = min((n + 1023u) / 1024u, 2048u);
-  copy_spectrum_kernel<<<blocks, 256, 0, stream>>>(src, dst, n, stamp, end);
+  copy_spectrum_kernel<<<blocks, 256, 0, stream>>>(src, dst, n, stamp, end, clear);
   return hipGetLastError();
 }
 
-__global__ void stamp_kernel(uint64_t* stamp, uint64_t* stamp2) {
+__global__ void stamp_kernel(uint64_t* stamp, uint64_t* stamp2, StampSpan clear) {
   put_stamp(stamp);
   put_stamp(stamp2);
+  clear_stamps(clear);
 }
 
-hipError_t launch_stamp(hipStream_t stream, uint64_t* stamp, uint64_t* stamp2) {
-  stamp_kernel<<<1, 64, 0, stream>>>(stamp, stamp2);
+hipError_t launch_stamp(hipStream_t stream, uint64_t* stamp, uint64_t* stamp2, StampSpan clear) {
+  stamp_kernel<<<1, 64, 0, stream>>>(stamp, stamp2, clear);
   return hipGetLastError();
 }
 

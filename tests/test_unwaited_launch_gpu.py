@@ -1,5 +1,7 @@
 """GPU test of calls on a buffer set whose launch has not been waited for."""
 
+import time
+
 import numpy as np
 import pytest
 
@@ -57,3 +59,30 @@ def test_quantile_thresholds_before_wait_leave_the_launch_its_lists(search):
     assert f.retrieve_candidates(*summed, FDAS.A) and f.wait(FDAS.A), f.last_error
     assert all(np.array_equal(a, b) for a, b in zip(got, summed))
     assert not np.array_equal(got[0], want[0])
+
+
+def test_stage_times_of_a_pass_after_an_unwaited_launch(search):
+    """The convolution's time stays that of the launch, and the summing's are those of the later pass, though the
+    launch's kernels may still be writing theirs when the pass is enqueued."""
+    f, x, thr = search
+    loc_pwr = arrays(f)
+    assert f.launch(x, thr, *loc_pwr, 2, FDAS.A) and f.wait(FDAS.A), f.last_error
+    for passes in (lambda: f.perform_harmonic_summing(thr, 2, FDAS.A),
+                   lambda: f.quantile_thresholds(3, 2, FDAS.A) is not None,
+                   lambda: f.perform_harmonic_summing(thr, 2, FDAS.A) and f.perform_harmonic_summing(thr, 2, FDAS.A)):
+        for _ in range(5):
+            t0 = time.perf_counter()
+            assert f.launch_resident(thr, *loc_pwr, 2, FDAS.A) and passes(), f.last_error
+            wall = 1e3 * (time.perf_counter() - t0)
+            ms = f.stage_times(FDAS.A)
+            assert ms[1] > 0 and ms[2] > 0 and ms[3] > 0, ms
+            assert ms[0] + ms[1] + ms[2] + ms[3] <= ms[5] + 1e-3 and ms[5] <= wall, (ms, wall)
+            assert f.wait(FDAS.A), f.last_error
+    # a launch over an unwaited one: the later one's times
+    for again in (lambda: f.launch_resident(thr, *loc_pwr, 2, FDAS.A), lambda: f.launch(x, thr, *loc_pwr, 2, FDAS.A)):
+        assert f.launch_resident(thr, *loc_pwr, 2, FDAS.A)
+        t0 = time.perf_counter()
+        assert again() and f.wait(FDAS.A), f.last_error
+        wall = 1e3 * (time.perf_counter() - t0)
+        ms = f.stage_times(FDAS.A)
+        assert ms[1] > 0 and ms[2] > 0 and ms[3] > 0 and ms[:4].sum() <= ms[5] + 1e-3 and ms[5] <= wall, (ms, wall)
