@@ -32,8 +32,12 @@ constexpr uint32_t kMaxFtcJobs = 64;  // row groups per FT-convolution launch
 
 // Device times of a launch (clock ticks, in pinned host memory, 0: not taken): START, INPUT (spectrum in place),
 // FTC_K (FT-convolution kernel start), FTC (its end where no summing follows at once), HSUM_K0 (harmonic-summing
-// kernel start), HSUM_K1 (selection start), then the end of each plane's selection.
-enum Stamp { ST_START = 0, ST_INPUT, ST_FTC_K, ST_FTC, ST_HSUM_K0, ST_HSUM_K1, ST_ENDS, ST_COUNT = ST_ENDS + kMaxHarmonics };
+// kernel start), HSUM_K1 (selection start), then the end of each plane's selection.  TAKEN is no time of its own: the
+// kernel after a staged spectrum's copy has started, and the staging buffer may be rewritten.
+enum Stamp {
+  ST_START = 0, ST_INPUT, ST_FTC_K, ST_FTC, ST_HSUM_K0, ST_HSUM_K1, ST_ENDS, ST_COUNT = ST_ENDS + kMaxHarmonics,
+  ST_TAKEN = ST_COUNT, ST_WORDS
+};
 
 // Host spectra up to this size are taken through pinned memory by a kernel; larger ones by a copy command.  Launch and
 // wait with 5 templates, by copy command and by kernel: 74 and 44 us at 4096 bins, 73 and 62 at 32768, 109 and 93 at
@@ -66,7 +70,7 @@ struct DevSet {
   uint32_t* h_quant = nullptr;     // [4H] mirror of quant's tail
 
   hipStream_t stream = nullptr;
-  uint64_t* h_stamp = nullptr;       // [ST_COUNT] pinned
+  uint64_t* h_stamp = nullptr;       // [ST_WORDS] pinned
   bool in_flight = false;            // work was enqueued since the stream was last waited for
   bool ftc_to_hsum = false;          // the summing followed the convolution at once: its start is the other's end
   float2* h_input = nullptr;         // pinned staging of small host spectra
@@ -259,6 +263,24 @@ fdas_status drain(fdas_ctx* ctx, DevSet& s) {
   return FDAS_OK;
 }
 
+// Waits until the device has read the staged spectrum, not for the work behind it: a launch over one that was not
+// waited for is enqueued while that one runs.
+fdas_status wait_taken(fdas_ctx* ctx, DevSet& s) {
+  const volatile uint64_t* taken = s.h_stamp + ST_TAKEN;
+  for (uint32_t spin = 1; s.input_pending && !*taken; ++spin) {
+    if (spin % 256 != 0) continue;
+    const hipError_t e = hipStreamQuery(s.stream);  // idle: whatever was enqueued has run
+    if (e == hipErrorNotReady) {
+      (void)hipGetLastError();
+      continue;
+    }
+    HIPCK(ctx, e);
+    break;
+  }
+  s.input_pending = false;
+  return FDAS_OK;
+}
+
 // The convolution jobs of the part.  Planned once per part and template bank: the
 // row grouping (a dynamic program over the rows, about 35 us on the host for 85) depends on
 // nothing else that changes between launches.
@@ -387,7 +409,7 @@ StampOps ftc_stamps(DevSet& s, bool start, int last) {
   renew_stamps(s, start ? ST_START : ST_INPUT, last);
   StampOps t;
   t.stamp = s.h_stamp + ST_INPUT;
-  if (start) t.stamp2 = s.h_stamp + ST_START;
+  t.stamp2 = s.h_stamp + (start ? ST_START : ST_TAKEN);
   t.clear = stamp_span(s, ST_FTC_K, last);
   return t;
 }
@@ -648,7 +670,7 @@ extern "C" fdas_status fdas_create(const fdas_config* cfg, fdas_log_fn log, void
     std::memset(s.h_counts, 0, sizeof(uint32_t) * H);
     if (hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) != hipSuccess)
       return bail(fail(ctx, FDAS_EDEVICE, "stream creation failed"));
-    if ((st = host_alloc(ctx, &s.h_stamp, ST_COUNT, hipHostMallocCoherent)) != FDAS_OK) return bail(st);
+    if ((st = host_alloc(ctx, &s.h_stamp, ST_WORDS, hipHostMallocCoherent)) != FDAS_OK) return bail(st);
     clear_stamps(s, 0, ST_COUNT - 1);
     static_assert(ST_COUNT <= 64, "cleared by one workgroup's threads");
     if (N * sizeof(float2) <= kStagedInput && (st = host_alloc(ctx, &s.h_input, N)) != FDAS_OK) return bail(st);
@@ -784,16 +806,19 @@ static bool readable_spectrum(const fdas_ctx* ctx, const void* src, size_t bytes
 
 // The spectrum into the set's buffer.  By a kernel, which the next one follows within 2 us, where it can be read:
 // device memory, and host memory up to kStagedInput after a copy to pinned memory, as the runtime also makes one; a
-// copy command's completion signal takes about 10 us to let the next kernel start.
+// copy command's completion signal takes about 10 us to let the next kernel start.  A launch over one that was not
+// waited for takes 55 us of the host at 131,072 bins (130 when it waited for all of that one's kernels); a third one
+// waits until the second one's copy, behind the first one's kernels, has run.
 static fdas_status upload_input(fdas_ctx* ctx, DevSet& s, const void* src, hipMemcpyKind kind) {
   const size_t bytes = sizeof(float2) * ctx->geo.n_bins;
   fdas_status st;
-  if (s.input_pending && (st = drain(ctx, s)) != FDAS_OK) return st;
+  if (s.input_pending && (st = wait_taken(ctx, s)) != FDAS_OK) return st;
   renew_stamps(s, 0, ST_COUNT - 1);
   s.ftc_to_hsum = false;
   const float2* from = nullptr;
   if (kind == hipMemcpyHostToDevice && s.h_input) {
     std::memcpy(s.h_input, src, bytes);
+    *static_cast<volatile uint64_t*>(s.h_stamp + ST_TAKEN) = 0;
     s.input_pending = true;
     from = s.h_input;
   } else if (kind == hipMemcpyDeviceToDevice && readable_spectrum(ctx, src, bytes)) {

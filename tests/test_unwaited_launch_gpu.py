@@ -86,3 +86,29 @@ def test_stage_times_of_a_pass_after_an_unwaited_launch(search):
         wall = 1e3 * (time.perf_counter() - t0)
         ms = f.stage_times(FDAS.A)
         assert ms[1] > 0 and ms[2] > 0 and ms[3] > 0 and ms[:4].sum() <= ms[5] + 1e-3 and ms[5] <= wall, (ms, wall)
+
+
+def test_a_launch_over_an_unwaited_one_does_not_wait_for_it(search):
+    """Only the copy of the first spectrum has to be over before the second one is staged.  With every bin detected a
+    launch's kernels take many times as long as the host needs to enqueue one."""
+    f, x, thr = search
+    dense = np.zeros(H, np.float32)
+    loc_pwr = arrays(f)
+    second, device = [], []
+    for _ in range(15):
+        assert f.launch(x, dense, *loc_pwr, 2, FDAS.A), f.last_error
+        t0 = time.perf_counter()
+        assert f.launch(x, dense, *loc_pwr, 2, FDAS.A), f.last_error
+        second.append(1e3 * (time.perf_counter() - t0))
+        f.wait(FDAS.A)  # False: the spill lists overflow
+        device.append(f.stage_times(FDAS.A)[5])
+    print(f"second launch {np.median(second):.3f} ms on the host, kernels {np.median(device):.3f} ms")
+    assert np.median(second) < 0.5 * np.median(device)
+    # several in a row: each spectrum was copied before the next took its place
+    for seeds in ((3, 4, 2), (2, 3, 4)):
+        want, got = arrays(f), arrays(f)
+        xs = [spectrum(N, s) for s in seeds]
+        assert f.launch(xs[-1], thr, *want, 2, FDAS.A) and f.wait(FDAS.A), f.last_error
+        for y in xs:
+            assert f.launch(y, thr, *got, 2, FDAS.A), f.last_error
+        assert f.wait(FDAS.A) and all(np.array_equal(a, b) for a, b in zip(got, want)), f.last_error
