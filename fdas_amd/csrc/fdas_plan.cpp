@@ -135,6 +135,26 @@ void make_twiddles(uint32_t tile, std::vector<float2>& tw1, std::vector<float2>&
   }
 }
 
+LineTables line_tables(const uint32_t (&len)[2]) {
+  LineTables t;
+  for (int i = 0; i < 2; ++i) {
+    if (i == 1 && len[1] == len[0]) {
+      t.w1[1] = t.w1[0];
+      t.w2[1] = t.w2[0];
+      continue;
+    }
+    if (len[i] <= 16) continue;
+    std::vector<float2> w1, w2;
+    make_twiddles(len[i], w1, w2);
+    t.w1[i] = uint32_t(t.data.size());
+    t.data.insert(t.data.end(), w1.begin(), w1.end());
+    if (len[i] <= 256) continue;
+    t.w2[i] = uint32_t(t.data.size());
+    t.data.insert(t.data.end(), w2.begin(), w2.end());
+  }
+  return t;
+}
+
 uint32_t hsum_rows_for(uint32_t n_bins, uint32_t n_rows) {
   const uint64_t row_blocks = uint64_t((n_bins + kHsumBinsPerBlock - 1) / kHsumBinsPerBlock) * n_rows;
   return std::min(kHsumRowsPerBlock, std::max(1u, uint32_t(std::lround(std::sqrt(double(row_blocks) / 100.0)))));

@@ -55,6 +55,15 @@ std::vector<std::complex<double>> taps_to_spectra(const float* taps_c64, uint32_
 // Twiddle tables of the S-point tile transform: w1[k][b] = W_S^(b k), w2[k][d] = W_(S/16)^(d k).
 void make_twiddles(uint32_t tile, std::vector<float2>& tw1, std::vector<float2>& tw2);
 
+// The front end's twiddle tables, one after another, for its column (len[0]) and row (len[1]) transforms.  A line
+// of L = 16 NT points reads w1 where NT > 1 and w2 where it takes three passes (L > 256); no other table is made,
+// and two transforms of one length share theirs.
+struct LineTables {
+  std::vector<float2> data;
+  uint32_t w1[2] = {0, 0}, w2[2] = {0, 0};  // where each begins
+};
+LineTables line_tables(const uint32_t (&len)[2]);
+
 // Rows per summing workgroup for a launch of one trial.  Short chunks fill the
 // chip where a plane is small (a chunk's rows follow one another, and each waits
 // for its loads); tall ones re-read fewer sub-harmonic rows and send fewer additions
