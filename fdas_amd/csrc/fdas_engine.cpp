@@ -460,6 +460,7 @@ fdas_status group_reserve(fdas_engine* e, GroupBuf& g, uint32_t n_ftc, uint32_t 
 
 // Fills the host job arrays of a group of placed trials (mem, input, h_lists set)
 // and its launch list: FT-convolution jobs grouped by tile, summing jobs by H.
+// A trial without lists (autotuning) gets no selection jobs.
 fdas_status build_group(fdas_engine* e, GroupBuf& g, const std::vector<Trial*>& trials) {
   const uint32_t cap = e->cfg.cands_per_harmonic, ccap = cap + kSelectPool;
   uint32_t n_ftc = 0, n_sel = 0;
@@ -515,6 +516,7 @@ fdas_status build_group(fdas_engine* e, GroupBuf& g, const std::vector<Trial*>& 
       for (uint32_t k = 0; k < H; ++k) j.thr[k] = t->req.thresholds[k];
       L.n_blocks += (j.n_bins + kHsumBinsPerBlock - 1) / kHsumBinsPerBlock * j.n_row_chunks;
       L.whole_groups = L.whole_groups && hsum_whole_groups(j.n_bins);
+      if (!t->h_lists) continue;
       for (uint32_t p = 0; p < H; ++p) {
         SelectJob& q = g.h_sel[js++];
         q.spill_key = j.spill_key + size_t(p) * spill;
@@ -1095,7 +1097,7 @@ bool admit(fdas_engine* e, fdas_engine::Ctx& c, bool others_in_flight, bool& mem
   std::vector<Trial*> ptrs;
   // Uploads go on a stream of their own, beside the kernels of the groups in flight.
   for (Trial& t : picked) {
-    t.h_lists = c.h_lists + off;
+    if (c.h_lists) t.h_lists = c.h_lists + off;
     off += t.lay.host_bytes;
     if (t.req.flags & FDAS_REQ_DEVICE_SPECTRUM) {
       t.input = static_cast<const float2*>(t.req.spectrum);
