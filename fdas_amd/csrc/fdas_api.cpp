@@ -116,6 +116,7 @@ struct fdas_ctx {
   DevSet set[2];
   uint64_t epoch = 0;       // device clock at creation
   double clock_khz = 1e5;
+  uint32_t n_cu = 256;
   bool sync_pipeline = false;
   // print_stats state; the reference keeps it file-static (FDAS.cpp:640-641)
   float pipeline_start = 0.f;
@@ -290,7 +291,7 @@ const std::vector<FtcJob>& ftc_jobs(const fdas_ctx* ctx, DevSet& s, fdas_part pa
   uint32_t rb, nr;
   part_rows(ctx, part, &rb, &nr);
   jobs = plan_ftc_rows(ctx->cfg.tile, ctx->geo.n_bins, ctx->cfg.max_taps, s.row_taps, rb, nr, kMaxFtcJobs);
-  fit_ftc_items(jobs, ftconv_slots(ctx->cfg.tile));
+  fit_ftc_items(jobs, ftconv_slots(ctx->cfg.tile, ctx->n_cu));
   uint32_t item = 0;
   for (FtcJob& j : jobs) {
     j.spectrum = s.input;
@@ -647,6 +648,9 @@ extern "C" fdas_status fdas_create(const fdas_config* cfg, fdas_log_fn log, void
   int khz = 0;
   if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, cfg->device) == hipSuccess && khz > 0)
     ctx->clock_khz = khz;
+  int n_cu = 0;
+  if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, cfg->device) == hipSuccess && n_cu > 0)
+    ctx->n_cu = uint32_t(n_cu);
 
   const size_t N = cfg->n_bins, T = cfg->n_templates, H = cfg->n_harmonics, cap = cfg->cands_per_harmonic;
   for (auto& s : ctx->set) {

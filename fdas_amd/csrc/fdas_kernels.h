@@ -27,10 +27,10 @@ int ftconv_threads(int tile);
 // its own, or a signal on the dispatch, that keeps the second kernel waiting for 5 to 9 us; with three events in it a
 // launch of 32768 bins took 106 us, and 88 without.
 
-// Workgroups of the FT-convolution kernel that run at once on the 256 CUs, at three
+// Workgroups of the FT-convolution kernel that run at once on n_cu CUs, at three
 // waves per SIMD: 12 one-wave workgroups per CU for 1024-point tiles, 6 and 3 of two
 // and four waves for 2048 and 4096.
-inline uint32_t ftconv_slots(uint32_t tile) { return 256u * 12u * 1024u / tile; }
+inline uint32_t ftconv_slots(uint32_t tile, uint32_t n_cu) { return n_cu * 12u * 1024u / tile; }
 
 // Fused FT convolution over a list of jobs (all with the same tile size).
 hipError_t launch_ftconv(int tile, const FtcJob* d_jobs, uint32_t n_jobs, uint32_t n_items, const float2* tw1,
