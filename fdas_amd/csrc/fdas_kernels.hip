@@ -10,7 +10,6 @@
 //  select_kernel  per-plane cap (strongest first) and (row, bin) ordering of the
 //                 detections; replaces the reference's overwrite-oldest ring
 //                 (detect.cl.mako:106-115) with a deterministic rule.
-#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <climits>
