@@ -62,7 +62,7 @@ MEASURED_VALU = {("ftconv1w_kernel", 8): 1050779416, ("hsum_kernel<8>", 8): 4220
 VALU_ISSUE_PER_S = 256 * 4 * 2.4e9 / 4
 # Shader clock the kernel runs at (amd-smi median while it runs alone, bench.py --forms batched,power);
 # profiles/power_clock_n2p21_t85_tile1024.txt.  The FT convolution holds the board at its power limit.
-MEASURED_CLOCK_GHZ = {"ftconv1w_kernel": 2.112, "hsum_kernel<8>": 2.385}
+MEASURED_CLOCK_GHZ = {"ftconv1w_kernel": 2.112, "hsum_kernel<8>": 2.378}
 FP32_PEAK_TFLOPS = 157.3
 N_METRIC = 1 << 21
 T_METRIC = 85

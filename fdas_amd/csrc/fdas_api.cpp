@@ -3,9 +3,10 @@
 // Mirrors the reference host class FDAS (fdas/src/host/FDAS.cpp): a context
 // owns the device, two buffer sets A/B with their own stream, the resident
 // template spectra, the FOP and the candidate buffers.  Where the reference
-// sequences ~40 OpenCL kernels over on-chip channels, one set here runs three
-// HIP kernels in order on its stream: fused FT convolution, harmonic summing
-// with compaction, and per-plane selection.
+// sequences ~40 OpenCL kernels over on-chip channels, one set here runs seven
+// HIP kernels in order on its stream: spectrum copy, job descriptors, fused FT
+// convolution, harmonic summing with thresholding, and per-plane selection
+// (histogram, compaction, final).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

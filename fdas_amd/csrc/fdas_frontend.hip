@@ -15,9 +15,10 @@
 // Bound by memory passes: a workgroup of cols_kernel takes kCols neighbouring
 // columns and one of rows_kernel a few neighbouring rows together with the rows
 // that mirror them, so both transposes and the split happen in the two passes
-// that the transforms need anyway.  N = 2^22: 41 us of kernels, 3.4 TB/s, and 50 us
-// the call, against 88 and 97 us with separate transposes and split (six passes of
-// 2 x 8N bytes); N = 2^15: 20 us the call, against 32.
+// that the transforms need anyway.  N = 2^22: 41 us of kernels, 3.4 TB/s, against 88
+// with separate transposes and split (six passes of 2 x 8N bytes); the call takes 51 us,
+// against 95, on buffers that stay in the last-level cache, and 64, against 98, on
+// others each time; N = 2^15: 20 us, against 31, on either.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -141,8 +142,8 @@ __device__ __forceinline__ uint32_t die_units(uint32_t blk, uint32_t n) {
 }
 
 // Columns of one cols_kernel workgroup and rows of one rows_kernel workgroup (half of
-// them mirrors).  At N = 2^22 the call took 52 us with 4 and 8, 52 with 8 and 8, 56 with 4
-// and 4, 55 with 8 and 4; at 2^20 31, 33, 31, 32.
+// them mirrors).  At N = 2^22, on buffers that stay in the last-level cache, the call took
+// 52 us with 4 and 8, 52 with 8 and 8, 56 with 4 and 4, 55 with 8 and 4; at 2^20 31, 33, 31, 32.
 constexpr int kCols = 4;
 constexpr int kRows = 8;
 

@@ -347,7 +347,7 @@ __device__ __forceinline__ uint32_t wave_prefix_small(uint32_t v, uint32_t& tota
 // planes 1.645 -> 1.617 ms (memory bound), 2^20 x 85 x 16 1.54 -> 1.48.
 template <int H>
 struct HsumStage {
-  static constexpr uint32_t kGroups = H <= 8 ? 24 : 12;  // LDS for 5 and 4 workgroups per CU
+  static constexpr uint32_t kGroups = H <= 8 ? 24 : 12;  // 27.8 KB at 8 planes, 27.9 at 16: 5 workgroups per CU
   float sum[kHsumThreads / 64][H][kGroups][kHsumBinsPerThread];
   uint32_t key[kHsumThreads / 64][H][kGroups];  // row << kKeyBinBits | f0
   uint32_t n[H][kHsumThreads / 64];             // groups of each wave, at the end
@@ -725,9 +725,10 @@ __device__ __forceinline__ void hsum_block(HsumStage<H>& st, const HsumJob* __re
   flush_rest(st, job, wn);
 }
 
-// Up to 8 planes are held to the registers of 5 and 6 waves per SIMD, as many as the LDS allows from 5 planes on, and
-// 15 and 16 planes to 128 registers: four waves per SIMD in place of three, 1.49 -> 1.30 ms per 8 trials of 2^20 bins
-// x 85 rows x 16 planes.
+// Up to 4 planes are held to the registers of 6 waves per SIMD and 5 to 8 planes to those of 5, at 8 planes as many
+// as the LDS allows; 15 and 16 planes to 128 registers: four waves per SIMD in place of three, 1.49 -> 1.30 ms per 8
+// trials of 2^20 bins x 85 rows x 16 planes.  9 to 14 planes take what they need: 105 to 136 registers, four waves up
+// to 12 planes and three at 13 and 14.
 template <int H>
 __global__ __launch_bounds__(kHsumThreads) __attribute__((amdgpu_waves_per_eu(H >= 15 ? 4 : H > 8 ? 1 : H > 4 ? 5 : 6))) void hsum_kernel(
     const HsumJob* __restrict__ jobs, uint32_t n_jobs, uint64_t* stamp) {
@@ -1740,8 +1741,10 @@ hipError_t launch_select(const SelectJob* d_jobs, uint32_t n_jobs, uint32_t cap,
   if (cap > kSelectMaxCap) return hipErrorInvalidValue;
   hipLaunchKernelGGL(cand_hist_kernel, dim3(kSelectSlices, n_jobs), dim3(256), 0, stream, d_jobs, stamp);
   hipLaunchKernelGGL(cand_compact_kernel, dim3(kSelectSlices, n_jobs), dim3(256), 0, stream, d_jobs);
-  // The workgroup grows with the list.  With 1024 / 512 / 256 threads a cap of 4096 took 28 / 30 / 38 us and one
-  // of 512 took 11 / 10 / 11 us, where the small workgroup needs a quarter of the CU beside other kernels.
+  // The workgroup grows with the list.  With 256 / 512 / 1024 threads this kernel takes, for 8 planes and a cap of 512,
+  // 9.4 / 11.6 / 10.5 us at 32,768 bins x 85 rows and 8.5 / 12.0 / 11.2 at 2^21; a cap of 1024 12.2 / 12.5 / 10.9 and
+  // 11.3 / 13.2 / 12.2, where the small workgroup needs a quarter of the CU beside other kernels; a cap of 2048 at
+  // 32,768 bins 25 / 17 / 15; a cap of 4096 at 2^21 42 / 25 / 23.
   if (cap <= 1024) select_final_kernel<256, 1024><<<n_jobs, 256, 0, stream>>>(d_jobs, ends);
   else if (cap <= 4096) select_final_kernel<1024, 4096><<<n_jobs, 1024, 0, stream>>>(d_jobs, ends);
   else select_final_kernel<1024, 8192><<<n_jobs, 1024, 0, stream>>>(d_jobs, ends);

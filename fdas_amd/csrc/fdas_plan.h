@@ -33,12 +33,12 @@ std::vector<FtcJob> plan_ftc_rows(uint32_t tile, uint32_t n_bins, uint32_t max_t
 // latency, not the number of rows in a row, sets the span; launches with more
 // items than that at 16 rows keep 16, which spend the fewest forward transforms.
 // Measured, us per launch (1 trial), at 16 rows / at the count chosen here:
-//   4,999 bins x 33 templates, tile 1024: 28 / 8 (1 row)
-//   32,768 x 85, tile 2048: 39 / 15 (2; 1 row, two rounds of workgroups: 21)
-//   20,011 x 169, tile 4096: 49 / 17 (2)
-//   131,072 x 85, tile 2048: 42 / 29 (8); tile 1024: 38 / 27 (6)
-// (2048 and 4096 with two waves per SIMD; three since), and where one round needs
-// more than 16 rows, 16 are the fastest or within 3 %.
+//   4,999 bins x 33 templates, tile 1024: 26 / 6.6 (1 row)
+//   32,768 x 85, tile 1024: 33 / 12.8 (2; 1 row, two rounds of workgroups: 15.5); tile 2048: 40 / 13.0 (1)
+//   20,011 x 169, tile 4096: 53 / 15.7 (2; 1 row: 18.9)
+//   131,072 x 85, tile 1024: 38 / 24.6 (5); tile 2048: 45 / 24.8 (4); tile 4096: 53 / 26.4 (4)
+// and where one round needs more than 16 rows, 16 are the fastest or within 3 %
+// (700,001 x 85, tile 2048: 6 / 8 / 12 / 16 rows 100 / 97 / 102 / 98).
 // The FOP does not depend on it.
 void fit_ftc_items(std::vector<FtcJob>& jobs, uint32_t slots);
 
@@ -73,6 +73,11 @@ LineTables line_tables(const uint32_t (&len)[2]);
 // 5.7 / 9.0 / 15 / 21; 20,011 x 169 15 / 14 / 23 / 31; 32,768 x 85 12.7 / 10.6 / 18 / 22;
 // 100,003 x 85 31 / 22 / 17 / 17; 262,144 x 85 70 / 44 / 33 / 34; 700,001 x 85
 // 175 / 105 / 72 / 65; 2^21 x 85 510 / 302 / 200 / 196, and 203 at 15.
+// The rule does not look at the number of planes.  Against the fastest of 1, 2, 4, 8,
+// 11 and 16 rows on a spectrum with a tone that every plane detects, it is within
+// 25 % at 1 and 2 planes and within 10 % at 4 and 8; at 12 and 16 fewer rows would be
+// faster: 100,003 x 85 at 4 rows 28 and 33 us against 34 and 44, 2^21 x 85 at 8 rows
+// 340 and 439 against 389 and 504.
 uint32_t hsum_rows_for(uint32_t n_bins, uint32_t n_rows);
 
 // HSUM workgroup row chunking for a part of n_rows rows (at most `target` rows per workgroup).

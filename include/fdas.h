@@ -187,9 +187,11 @@ void fdas_print_events(fdas_ctx* ctx, int set);
 fdas_status fdas_quantile_thresholds(fdas_ctx* ctx, uint32_t n_per_plane, fdas_part part, int set, float* thresholds);
 
 /* Device durations in ms of the last run on `set` (the device clock as the
- * launches' kernels start; a stage includes the gap before the next): [0] input, [1] FT-convolution kernel, [2] harmonic-summing kernel,
- * [3] candidate selection, [4] candidate read-back (0: the selection writes the
- * lists to host memory), [5] total. */
+ * run's kernels start; a stage includes the gap before the next one, and the
+ * selection, with both sets in use, the time it runs behind the other set's
+ * convolution): [0] input, [1] FT-convolution kernel, [2] harmonic-summing
+ * kernel, [3] candidate selection, [4] candidate read-back (0: the selection
+ * writes the lists to host memory), [5] total. */
 fdas_status fdas_get_stage_times(fdas_ctx* ctx, int set, float* ms6);
 
 /* Device enumeration for the platform / device selectors of
