@@ -312,6 +312,9 @@ struct fdas_engine {
   std::vector<Ctx> ctxs;
   uint64_t launch_seq = 0;
   std::vector<fdas_plan*> plans;   // live plans, which hold arena memory (guarded by api_mu)
+  // Served groups and plans are never on the device together (see wait_turn): the end of the last plan launched and
+  // of the last group served, nullptr once waited for (guarded by api_mu).
+  hipEvent_t last_plan = nullptr, last_served = nullptr;
   fdas_engine_stats stats{};
 };
 
@@ -581,6 +584,17 @@ fdas_status enqueue_group(fdas_engine* e, GroupBuf& g, hipEvent_t wait_before, b
   }
   EHIP(e, launch_select(g.d_sel, g.n_sel, e->cfg.cands_per_harmonic, B));
   EHIP(e, hipEventRecord(g.ev_done, B));
+  return FDAS_OK;
+}
+
+// Before work of one kind (plans, served groups) is enqueued: waits for the last work of the other, so that the two are
+// never on the device together.  A run that served random requests while random plans, eager and captured, were
+// launched on the same engine hung, with the served groups' uploads on a stream of their own; the cause was not found,
+// and the same run passed with the uploads on the convolution stream.  Either kind alone keeps its streams and its
+// speed.  Every wait is for work that is already on its stream.  Caller holds api_mu.
+fdas_status wait_turn(fdas_engine* e, hipEvent_t& other) {
+  if (other) EHIP(e, hipEventSynchronize(other));
+  other = nullptr;
   return FDAS_OK;
 }
 
@@ -1093,6 +1107,7 @@ bool admit(fdas_engine* e, fdas_engine::Ctx& c, bool others_in_flight, bool& mem
     if (host_alloc(e, &c.h_lists, lists, hipHostMallocCoherent) == FDAS_OK) c.h_lists_cap = lists;
   }
   fdas_status st = c.h_lists ? FDAS_OK : FDAS_ENOMEM;
+  if (st == FDAS_OK) st = wait_turn(e, e->last_plan);
   uint64_t off = 0;
   std::vector<Trial*> ptrs;
   // Uploads go on a stream of their own, beside the kernels of the groups in flight.
@@ -1130,6 +1145,7 @@ bool admit(fdas_engine* e, fdas_engine::Ctx& c, bool others_in_flight, bool& mem
     }
     return true;
   }
+  e->last_served = c.buf.ev_done;
   c.trials = std::move(picked);
   c.busy = true;
   c.seq = ++e->launch_seq;
@@ -1149,9 +1165,12 @@ void scheduler_loop(fdas_engine* e) {
       for (auto& c : e->ctxs)
         if (c.busy && (!oldest || c.seq < oldest->seq)) oldest = &c;
       if (!oldest) break;
-      if (hipEventQuery(oldest->buf.ev_done) != hipSuccess) {
-        (void)hipGetLastError();  // "not ready" must not reach the next launch's error check
-        break;
+      {
+        std::lock_guard<std::mutex> lk(e->api_mu);  // not beside a plan's capture
+        if (hipEventQuery(oldest->buf.ev_done) != hipSuccess) {
+          (void)hipGetLastError();  // "not ready" must not reach the next launch's error check
+          break;
+        }
       }
       complete_ctx(e, *oldest);
       progress = true;
@@ -1641,6 +1660,8 @@ fdas_status fdas_plan_launch(fdas_plan* p) {
   if (p->launched) return fail(e, FDAS_ESTATE, "plan already launched; wait for it first");
   std::lock_guard<std::mutex> lk(e->api_mu);
   EHIP(e, hipSetDevice(e->cfg.device));
+  const fdas_status turn = wait_turn(e, e->last_served);
+  if (turn != FDAS_OK) return turn;
   // Host spectra go to the plan's device copies first (outside any graph).
   for (Trial& t : p->trials)
     if (!(t.req.flags & FDAS_REQ_DEVICE_SPECTRUM))
@@ -1670,6 +1691,7 @@ fdas_status fdas_plan_launch(fdas_plan* p) {
     p->eager_timed = true;
   }
   EHIP(e, hipEventRecord(p->ev_end, e->s_ftc));
+  e->last_plan = p->ev_end;
   p->launched = true;
   p->n_launches += 1;
   return FDAS_OK;
@@ -1732,6 +1754,7 @@ fdas_status fdas_plan_get_info(const fdas_plan* p, fdas_plan_info* out) {
 static void plan_release(fdas_engine* e, fdas_plan* p) {
   (void)hipSetDevice(e->cfg.device);
   if (p->launched) (void)hipEventSynchronize(p->ev_end);
+  if (e->last_plan == p->ev_end) e->last_plan = nullptr;
   if (p->exec) (void)hipGraphExecDestroy(p->exec);
   if (p->graph) (void)hipGraphDestroy(p->graph);
   for (auto& b : p->bufs) free_group(b);

@@ -426,7 +426,8 @@ void fdas_plan_destroy(fdas_plan* plan);
 
 /* Serving: trials are queued, admitted while the HBM budget and the groups in
  * flight allow, and launched in groups formed from whatever is waiting, so
- * requests that arrive while others run join the next group.  `result` (and
+ * requests that arrive while others run join the next group.  Served groups and
+ * plans of one engine take turns on the device.  `result` (and
  * its key/power arrays and the request's spectrum) must stay valid until the
  * result is returned by fdas_engine_poll.  Calls are thread-safe. */
 fdas_status fdas_engine_submit(fdas_engine* eng, const fdas_request* req, fdas_result* result);

@@ -1,15 +1,47 @@
 // Host-side test of the engine's own code under sanitizers, with a HIP runtime of host memory in which every kernel
 // launch only reads its job descriptors (and the selection writes one entry per list): autotuning, an eager plan
-// twice, a changed request and served requests.
+// twice, a changed request, served requests, and plans launched while requests are served.  An event counts as
+// reached 1 ms after its record, so that work is in flight for a while: kernels of plans (launched by the main thread)
+// and of served groups (by the scheduler's) must not be in flight together.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
+#include <thread>
 #include <vector>
 
 #include "fdas.h"
 #include "fdas_kernels.h"
+
+static int failures = 0;
+#define CHECK(cond)                                                                   \
+  do {                                                                                \
+    if (!(cond)) ++failures, std::printf("FAIL line %d: %s\n", __LINE__, #cond);      \
+  } while (0)
+
+typedef std::chrono::steady_clock Clock;
+static const std::thread::id main_thread = std::this_thread::get_id();
+static int kind() { return std::this_thread::get_id() == main_thread ? 0 : 1; }
+static std::mutex mu;
+static int n_launched[2] = {0, 0}, n_reached[2] = {0, 0};  // kernels launched; known to have ended
+struct Event {
+  int kind = 0, launched = 0;
+  Clock::time_point at{};
+};
+static void launched() {
+  std::lock_guard<std::mutex> lk(mu);
+  const int k = kind();
+  CHECK(n_reached[1 - k] == n_launched[1 - k]);  // nothing of the other kind is in flight
+  ++n_launched[k];
+}
+static void reached(const Event& e) {
+  std::lock_guard<std::mutex> lk(mu);
+  if (e.launched > n_reached[e.kind]) n_reached[e.kind] = e.launched;
+}
 
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n) { return *p = std::malloc(n), *p ? hipSuccess : hipErrorOutOfMemory; }
@@ -24,12 +56,22 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) { return st
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "error"; }
-hipError_t hipEventCreate(hipEvent_t* e) { return *e = reinterpret_cast<hipEvent_t>(std::malloc(1)), hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { return *e = reinterpret_cast<hipEvent_t>(new Event), hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
-hipError_t hipEventDestroy(hipEvent_t e) { return std::free(e), hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { return delete reinterpret_cast<Event*>(e), hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
+  std::lock_guard<std::mutex> lk(mu);
+  *reinterpret_cast<Event*>(e) = {kind(), n_launched[kind()], Clock::now() + std::chrono::milliseconds(1)};
+  return hipSuccess;
+}
+hipError_t hipEventQuery(hipEvent_t e) {
+  if (Clock::now() < reinterpret_cast<Event*>(e)->at) return hipErrorNotReady;
+  return reached(*reinterpret_cast<Event*>(e)), hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t e) {
+  std::this_thread::sleep_until(reinterpret_cast<Event*>(e)->at);
+  return reached(*reinterpret_cast<Event*>(e)), hipSuccess;
+}
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 1.f, hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = reinterpret_cast<hipStream_t>(std::malloc(1)), hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { return std::free(s), hipSuccess; }
@@ -43,20 +85,16 @@ hipError_t hipGraphInstantiate(hipGraphExec_t*, hipGraph_t, hipGraphNode_t*, cha
 hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipErrorNotSupported; }
 }
 
-static int failures = 0;
-#define CHECK(cond)                                                                   \
-  do {                                                                                \
-    if (!(cond)) ++failures, std::printf("FAIL line %d: %s\n", __LINE__, #cond);      \
-  } while (0)
-
 namespace fdas {
 hipError_t launch_ftconv(int, const FtcJob* j, uint32_t n, uint32_t items, const float2*, const float2*, uint32_t,
                          hipStream_t, uint64_t*) {
+  launched();
   CHECK(n > 0 && j[n - 1].item_begin + j[n - 1].n_tiles * j[n - 1].n_chunks == items);
   for (uint32_t i = 0; i < n; ++i) CHECK(j[i].spectrum && j[i].fop && j[i].hperm);
   return hipSuccess;
 }
 hipError_t launch_hsum(const HsumJob* j, uint32_t n, uint32_t blocks, uint32_t H, hipStream_t, uint64_t*) {
+  launched();
   for (uint32_t i = 0; i < n; ++i) {
     CHECK(j[i].n_harmonics == H && j[i].block_begin < blocks);
     j[i].counts[(H - 1) * kPlaneCounters] = 0;
@@ -66,6 +104,7 @@ hipError_t launch_hsum(const HsumJob* j, uint32_t n, uint32_t blocks, uint32_t H
   return hipSuccess;
 }
 hipError_t launch_select(const SelectJob* j, uint32_t n, uint32_t cap, hipStream_t, uint64_t*, uint64_t*) {
+  launched();
   for (uint32_t i = 0; i < n; ++i) {
     CHECK(j[i].cap == cap);
     j[i].hist[kSelectBins - 1] = 0;
@@ -147,16 +186,39 @@ int main() {
       req[3].thresholds[0] = 77.f;
       CHECK(fdas_plan_set_request(plan, 3, nullptr, req[3].thresholds) == FDAS_OK);
     }
-    fdas_plan_destroy(plan);
-    for (uint32_t i = 0; i < R; ++i) CHECK(fdas_engine_submit(e, &req[i], &res[i]) == FDAS_OK);
-    for (uint32_t got = 0; got < R;) {
-      fdas_result* done[R];
-      uint32_t n = 0;
-      CHECK(fdas_engine_poll(e, done, R, &n, 1000) == FDAS_OK && n > 0);
-      if (n == 0) break;
-      for (uint32_t i = 0; i < n; ++i) complete(*done[i]);
-      got += n;
+    // requests served while plans run: submitted before, between and after their launches
+    fdas_result planned[R];
+    std::vector<std::vector<uint32_t>> pkey(key);
+    std::vector<std::vector<float>> ppower(power);
+    for (uint32_t i = 0; i < R; ++i) {
+      planned[i] = res[i];
+      planned[i].key = pkey[i].data();
+      planned[i].power = ppower[i].data();
     }
+    fdas_plan* second = nullptr;
+    CHECK(fdas_plan_create(e, req, R, 0, &second) == FDAS_OK);
+    for (int round = 0; round < 4; ++round) {
+      for (uint32_t i = 0; i < R; ++i) {
+        CHECK(fdas_engine_submit(e, &req[i], &res[i]) == FDAS_OK);
+        if (i == 1) CHECK(fdas_plan_launch(plan) == FDAS_OK);
+        if (i == 3) CHECK(fdas_plan_launch(second) == FDAS_OK);
+        if (round % 2) std::this_thread::sleep_for(std::chrono::microseconds(300));
+      }
+      for (fdas_plan* p : {plan, second}) {
+        CHECK(fdas_plan_wait(p, planned) == FDAS_OK);
+        for (const fdas_result& r : planned) complete(r);
+      }
+      for (uint32_t got = 0; got < R;) {
+        fdas_result* done[R];
+        uint32_t n = 0;
+        CHECK(fdas_engine_poll(e, done, R, &n, 1000) == FDAS_OK && n > 0);
+        if (n == 0) break;
+        for (uint32_t i = 0; i < n; ++i) complete(*done[i]);
+        got += n;
+      }
+    }
+    fdas_plan_destroy(plan);
+    fdas_plan_destroy(second);
     fdas_engine_destroy(e);
   }
   if (failures == 0) std::printf("engine host test ok\n");

@@ -1,4 +1,4 @@
-"""The engine's host code (autotuning, plans, serving) under AddressSanitizer and UndefinedBehaviorSanitizer, linked to
+"""The engine's host code (autotuning, plans, serving, both at once) under AddressSanitizer and UndefinedBehaviorSanitizer, linked to
 a HIP runtime of host memory (tests/cpp/engine_host_test.cpp).  CPU only: no kernel is built."""
 
 import shutil
