@@ -1051,6 +1051,7 @@ bool admit(fdas_engine* e, fdas_engine::Ctx& c, bool others_in_flight, bool& mem
   }
   bool progress = false;
   std::lock_guard<std::mutex> lk_api(e->api_mu);
+  fdas_status st = wait_turn(e, e->last_plan);  // before anything is allocated or freed for the group, too
   while (picked.size() < e->cfg.group_trials) {
     Trial t;
     {
@@ -1106,8 +1107,7 @@ bool admit(fdas_engine* e, fdas_engine::Ctx& c, bool others_in_flight, bool& mem
     c.h_lists_cap = 0;
     if (host_alloc(e, &c.h_lists, lists, hipHostMallocCoherent) == FDAS_OK) c.h_lists_cap = lists;
   }
-  fdas_status st = c.h_lists ? FDAS_OK : FDAS_ENOMEM;
-  if (st == FDAS_OK) st = wait_turn(e, e->last_plan);
+  if (st == FDAS_OK && !c.h_lists) st = FDAS_ENOMEM;
   uint64_t off = 0;
   std::vector<Trial*> ptrs;
   // Uploads go on a stream of their own, beside the kernels of the groups in flight.
